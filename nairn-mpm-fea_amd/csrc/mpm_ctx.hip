@@ -23,10 +23,8 @@ using mpmi::fail_global;
 void mpmi::set_positions(MpmCtx *c) {
     double **cur = c->parity == 0 ? c->posA : c->posB;
     double **nxt = c->parity == 0 ? c->posB : c->posA;
-    for (int a = 0; a < 3; a++) {
-        c->kp.f[MPF_POS_X + a] = cur[a];
-        c->kp.posn[a] = nxt[a];
-    }
+    c->kp.pos = cur[0];            // each buffer's three rows are n entries apart
+    c->kp.posNew = nxt[0];
 }
 using mpmi::set_positions;
 using mpmi::check_run;
@@ -282,6 +280,7 @@ void mpmi::fill_grid(KGrid &g, int dim, const MpmGridDesc *grid, const MpmRunPar
     g.tilesTotal = g.ntiles;
     g.xmin = grid->xmin; g.ymin = grid->ymin; g.zmin = grid->zmin;
     g.dx = grid->dx; g.dy = grid->dy; g.dz = grid->dz;
+    g.rdx[0] = 1. / g.dx; g.rdx[1] = 1. / g.dy; g.rdx[2] = dim == 3 ? 1. / g.dz : 0.;
     g.timestep = run->timestep; g.strainFirst = run->strainFirst; g.strainLast = run->strainLast;
     g.gridDamping = run->gridDamping; g.particleDamping = run->particleDamping;
     g.damped = run->gridDamping != 0. || run->particleDamping != 0.;
@@ -951,9 +950,9 @@ int mpmi::place_particles(MpmCtx *c, int64_t n) {
         if (c->run.shape == MPMGPU_SHAPE_LCPDI) HIPCHECK(c, hipMalloc(&c->cbuf, (size_t)9 * n * sizeof(double)));
         c->ncap = n;
     }
-    for (int a = 0; a < 9; a++) c->kp.cpr[a] = c->cbuf ? c->cbuf + (size_t)a * n : nullptr;
+    c->kp.semi = c->cbuf;
     size_t nn = (size_t)n;
-    for (int f = 0; f < MPF_NUM_FIELDS; f++) c->kp.f[f] = c->pbuf + f * nn;
+    c->kp.d = c->kp.pos = c->pbuf;
     for (int a = 0; a < 3; a++) {
         c->posA[a] = c->pbuf + (MPF_POS_X + a) * nn;
         c->posB[a] = c->pbuf + (MPF_NUM_FIELDS + a) * nn;
@@ -1064,7 +1063,8 @@ int mpmgpu_upload_particles(MpmCtx *c, int64_t n, const double *dfields, const i
     // uniform particle size lets the kernels skip the lp arrays
     c->kg.uniformLp = 1;
     if (n > 0) {
-        for (int a = 0; a < 3; a++) c->kg.lp[a] = dfields[(MPF_LP_X + a) * nn];
+        const double lp0[3] = {dfields[MPF_LP_X * nn], dfields[MPF_LP_Y * nn], dfields[MPF_LP_Z * nn]};
+        set_particle_size(c->kg, lp0);
         for (int64_t i = 0; i < n && c->kg.uniformLp; i++)
             for (int a = 0; a < 3; a++)
                 if (dfields[(MPF_LP_X + a) * nn + i] != c->kg.lp[a]) { c->kg.uniformLp = 0; break; }
@@ -1078,7 +1078,8 @@ int mpmgpu_upload_particles(MpmCtx *c, int64_t n, const double *dfields, const i
             int k = (int)(&gi - c->inst.data());
             if (!seen[k]) {
                 seen[k] = 1;
-                for (int a = 0; a < 3; a++) gi.lp[a] = dfields[(MPF_LP_X + a) * nn + i];
+                const double lp0[3] = {dfields[MPF_LP_X * nn + i], dfields[MPF_LP_Y * nn + i], dfields[MPF_LP_Z * nn + i]};
+                set_particle_size(gi, lp0);
             } else if (gi.uniformLp) {
                 for (int a = 0; a < 3; a++)
                     if (dfields[(MPF_LP_X + a) * nn + i] != gi.lp[a]) { gi.uniformLp = 0; break; }
@@ -1640,7 +1641,7 @@ int mpmgpu_download_particles(MpmCtx *c, double *dfields, int32_t *ifields) {
     // rows back to upload order through the scratch row
     hipStream_t s = c->stream;
     for (int f = 0; f < MPF_NUM_FIELDS; f++) {
-        launch_scatter_row(c->kp.f[f], c->scr, c->kb.home, (long long)nn, s);
+        launch_scatter_row(c->kp.f(f), c->scr, c->kb.home, (long long)nn, s);
         HIPCHECK(c, hipMemcpyAsync(dfields + f * nn, c->scr, nn * sizeof(double), hipMemcpyDeviceToHost, s));
     }
     if (ifields) {

@@ -55,6 +55,8 @@ struct KGrid {
     const int *tileType;
     int ntypes, types[4], anyMixed;
     double lp[3];
+    // reciprocals found once on the host: 1/d of the cell sizes and, with uniformLp, 1/(4 lp), 1/(2 lp)
+    double rdx[3], rlp4[3], rlp2[3];
     // material velocity fields (multimaterial mode when nfields > 1)
     int nfields;
     int fieldOf[MPMGPU_MAX_MATERIALS];   // material -> field
@@ -81,12 +83,19 @@ struct KGrid {
     const int *matInst;        // material -> instance
 };
 
+// Particle rows, n entries apart: the MPF_* fields at d (positions at pos, which alternates between two
+// buffers), the end-of-step positions and lCPDI's semi-side vectors. Kept as bases and one length:
+// a pointer per row held 110 scalar registers over a kernel.
 struct KPart {
-    double *f[MPF_NUM_FIELDS]; // f[MPF_POS_*] is the start-of-step position
-    double *posn[3];           // end-of-step position (written by the particle update)
-    double *cpr[9];            // lCPDI: semi-side vectors r1, r2, r3 of the step (null otherwise)
+    double *d;
+    double *pos;               // three rows: start-of-step position
+    double *posNew;            // three rows: end-of-step position (written by the particle update)
+    double *semi;              // nine rows, lCPDI: semi-side vectors r1, r2, r3 of the step (null otherwise)
     int *elem, *mat, *id, *left;
     long long n;
+    __host__ __device__ double *f(int r) const { return (r <= MPF_POS_Z ? pos : d) + r * n; }
+    __host__ __device__ double *posn(int a) const { return posNew + a * n; }
+    __host__ __device__ double *cpr(int a) const { return semi + a * n; }
 };
 
 struct KBins {
@@ -116,6 +125,15 @@ struct KBins {
     int ntall;                 // (field, tile) pairs: nfields * tilesTotal
     int slot;                  // the launch's cursor (set by the launch functions)
 };
+
+// the particle size of a grid whose particles share one (uniformLp), with its reciprocals
+inline void set_particle_size(KGrid &g, const double lp[3]) {
+    for (int a = 0; a < 3; a++) {
+        g.lp[a] = lp[a];
+        g.rlp4[a] = 1. / (4. * lp[a]);
+        g.rlp2[a] = 2. * g.rlp4[a];
+    }
+}
 
 // launches of the tile kernels in one step, each with its own cursors (cleared when the list is built)
 // (the XPIC iterations share one slot, whose cursors each iteration's node pass clears again)

@@ -3,18 +3,18 @@
 // Layout: particles stay in structure-of-arrays form; every step they are binned by cell with a
 // stable counting sort into tiles of TileGeom<DIM> cells (tile-major cell keys), which gives a
 // sorted slot -> particle map (order[]). Particle-to-grid sums never use floating-point atomics:
-// a tile kernel stages its particles' per-axis GIMP factors in LDS; then one wave handles one
-// cell at a time with each lane owning one of the 64 candidate node offsets, sums the cell's
-// particles in sorted order in registers and adds the sum to the wave's own LDS copy of the
-// tile's node footprint (wave_cells). The copies are added in wave order and the footprint sums
-// of each tile go to a partial buffer that a node kernel adds in fixed tile order. Results are
-// therefore deterministic; they differ from the reference's single-patch sums by summation
-// order only.
+// each wave of a tile's block takes a layer of the tile's cells, stages its particles' per-axis shape
+// factors in LDS, sums each cell's particles at the cell's candidate nodes in sorted order on the
+// matrix cores (WaveScatter) and adds the sums to the wave's own LDS copy of the tile's node
+// footprint. The copies are added in wave order and the footprint sums of each tile go to a partial
+// buffer that a node kernel adds in fixed tile order. Results are therefore deterministic; they
+// differ from the reference's single-patch sums by summation order only.
 //
 // Reference tasks (paths relative to the reference root, NairnMPM/src/NairnMPM_Class/):
 //   k_p2g_mass    MassAndMomentumTask.cpp:48-127      (+ InitializationTask xi, :43-85)
 //   k_node_mass   PostExtrapolationTask.cpp:46-165 + GridValueCalculation (UpdateStrainsFirstTask.cpp:120)
-//   k_usf_force   UpdateStrainsFirstTask.cpp:101-168 + GridForcesTask.cpp:40-153
+//   k_usf         UpdateStrainsFirstTask.cpp:101-168
+//   k_p2g_force   GridForcesTask.cpp:40-153
 //   k_node_force  PostForcesTask.cpp:43-111 + UpdateMomentaTask.cpp:44-64 + GridValueCalculation
 //   k_g2p_p2g     UpdateParticlesTask.cpp:44-298 + UpdateStrainsLastContactTask.cpp:60-142
 //   k_node_mom2   UpdateStrainsLastContactTask.cpp:139-149 + GridValueCalculation
@@ -28,6 +28,10 @@
 #include "mpm_kernels.h"
 
 #define NT 256
+// records (particles, or lCPDI corners) that a wave of a scatter stages at a time, two rounds per 64
+// lanes, and the length of its rows: 16 words read from four rows by one instruction lie on different banks
+#define WREC 32
+#define WROW (WREC + 4)
 
 // The kernels of one tile shape: this file builds shape 0, and mpm_kernels_s1.hip builds shape 1
 // by defining MPM_TILE_SHAPE before including it. Each goes into its own namespace.
@@ -85,16 +89,36 @@ __device__ __forceinline__ KNodes field_view(const KGrid &g, const KNodes &N, in
     return v;
 }
 
-// grid of the instance that owns context tile tg (the kernel's grid for one instance)
-__device__ __forceinline__ KGrid tile_grid(const KGrid &g0, int tg) {
-    if (!g0.inst) return g0;
-    return g0.inst[g0.tileInst[tg]];
+// A grid read as constant memory, which no kernel writes: an instance's from the table, or the kernel's
+// own from its arguments (every kernel's first). With a uniform instance the words come by scalar loads
+// into scalar registers; read as ordinary memory they took vector registers (about 90 live through a
+// tile kernel, a wave per SIMD), also where there is one grid and the table is never read.
+typedef const __attribute__((address_space(4))) KGrid *GridPtr;
+
+__device__ __forceinline__ KGrid grid_copy(GridPtr p) {
+    typedef const __attribute__((address_space(4))) unsigned long long *Words;
+    static_assert(sizeof(KGrid) % 8 == 0, "whole words");
+    const Words s = (Words)p;
+    union { KGrid g; unsigned long long w[sizeof(KGrid) / 8]; } u;
+#pragma unroll
+    for (unsigned k = 0; k < sizeof(KGrid) / 8; k++) u.w[k] = s[k];
+    return u.g;
+}
+__device__ __forceinline__ int const_int(const int *p) {
+    return *(const __attribute__((address_space(4))) int *)p;
 }
 
-// grid of the instance that owns context node ng (node ranges are padded to NT per instance)
+// grid of the instance that owns context tile tg (the kernel's grid for one instance)
+__device__ __forceinline__ GridPtr tile_grid_ptr(const KGrid &g0, int tg) {
+    if (!g0.inst) return (GridPtr)__builtin_amdgcn_kernarg_segment_ptr();
+    return (GridPtr)(g0.inst + const_int(g0.tileInst + tg));
+}
+
+// grid of the instance that owns context node ng (node ranges are padded to NT per instance, so a
+// block's nodes belong to one)
 __device__ __forceinline__ KGrid node_grid(const KGrid &g0, long long ng) {
     if (!g0.inst) return g0;
-    return g0.inst[g0.nodeBlockInst[ng / 256]];
+    return grid_copy((GridPtr)(g0.inst + const_int(g0.nodeBlockInst + __builtin_amdgcn_readfirstlane((int)(ng / 256)))));
 }
 
 __device__ __forceinline__ void elem_ijk(const KGrid &g, int e, int &i, int &j, int &k) {
@@ -137,7 +161,7 @@ __device__ __forceinline__ void particle_factors(const KGrid &g, const KPart &P,
     }
     double lpx, lpy, lpz;
     if (g.uniformLp) { lpx = g.lp[0]; lpy = g.lp[1]; lpz = g.lp[2]; }
-    else { lpx = P.f[MPF_LP_X][p]; lpy = P.f[MPF_LP_Y][p]; lpz = P.f[MPF_LP_Z][p]; }
+    else { lpx = P.f(MPF_LP_X)[p]; lpy = P.f(MPF_LP_Y)[p]; lpz = P.f(MPF_LP_Z)[p]; }
     if (DIM == 3) {
         gimp_axis3(xi[0], lpx, 1. / (4. * lpx), S[0], dS[0]);
         gimp_axis3(xi[1], lpy, 1. / (4. * lpy), S[1], dS[1]);
@@ -173,19 +197,13 @@ __device__ __forceinline__ int find_cell(double x, double xmin, double d, int n,
 
 // semi-side vectors from the particle's F and size (GetSemiSideVectors, GetParticleSize)
 template <int DIM>
-__device__ __forceinline__ void cpdi_semi_sides(const KGrid &g, const KPart &P, int p, int ei, int ej, int ek,
-                                                double r[9]) {
+__device__ __forceinline__ void cpdi_semi_sides_of(const KGrid &g, const KPart &P, int p, int ei, int ej, int ek,
+                                                   const double ep[6], const double wr[3], double r[9]) {
     double lpx, lpy, lpz;
     if (g.uniformLp) { lpx = g.lp[0]; lpy = g.lp[1]; lpz = g.lp[2]; }
-    else { lpx = P.f[MPF_LP_X][p]; lpy = P.f[MPF_LP_Y][p]; lpz = P.f[MPF_LP_Z][p]; }
+    else { lpx = P.f(MPF_LP_X)[p]; lpy = P.f(MPF_LP_Y)[p]; lpz = P.f(MPF_LP_Z)[p]; }
     double psx = ((g.xmin + (double)(ei + 1) * g.dx) - (g.xmin + (double)ei * g.dx)) * (0.5 * lpx);
     double psy = ((g.ymin + (double)(ej + 1) * g.dy) - (g.ymin + (double)ej * g.dy)) * (0.5 * lpy);
-    double ep[6] = {P.f[MPF_EP_XX][p], P.f[MPF_EP_YY][p], P.f[MPF_EP_ZZ][p], 0., 0., P.f[MPF_EP_XY][p]};
-    double wr[3] = {0., 0., P.f[MPF_WR_XY][p]};
-    if (DIM == 3) {
-        ep[3] = P.f[MPF_EP_YZ][p]; ep[4] = P.f[MPF_EP_XZ][p];
-        wr[0] = P.f[MPF_WR_YZ][p]; wr[1] = P.f[MPF_WR_XZ][p];
-    }
     double F[3][3];
     get_F3(ep, wr, F);
     if (DIM == 3) {
@@ -198,6 +216,18 @@ __device__ __forceinline__ void cpdi_semi_sides(const KGrid &g, const KPart &P, 
         r[3] = F[0][1] * psy; r[4] = F[1][1] * psy; r[5] = 0.;
         r[6] = r[7] = r[8] = 0.;
     }
+}
+
+template <int DIM>
+__device__ __forceinline__ void cpdi_semi_sides(const KGrid &g, const KPart &P, int p, int ei, int ej, int ek,
+                                                double r[9]) {
+    double ep[6] = {P.f(MPF_EP_XX)[p], P.f(MPF_EP_YY)[p], P.f(MPF_EP_ZZ)[p], 0., 0., P.f(MPF_EP_XY)[p]};
+    double wr[3] = {0., 0., P.f(MPF_WR_XY)[p]};
+    if (DIM == 3) {
+        ep[3] = P.f(MPF_EP_YZ)[p]; ep[4] = P.f(MPF_EP_XZ)[p];
+        wr[0] = P.f(MPF_WR_YZ)[p]; wr[1] = P.f(MPF_WR_XZ)[p];
+    }
+    cpdi_semi_sides_of<DIM>(g, P, p, ei, ej, ek, ep, wr, r);
 }
 
 // linear function of element node (jx,jy,jz) at natural coordinates x (EightNodeIsoparamBrick.cpp:87-108,
@@ -233,7 +263,7 @@ __device__ __forceinline__ long long foot_node(const KGrid &g, int s, int ox, in
     return ((long long)k * g.nny + j) * g.nnx + i;
 }
 
-// corner c of a particle (the body of cpdi_corners for one corner); false if the corner is unusable
+// corner c of a particle; false if the corner is unusable
 template <int DIM>
 __device__ __forceinline__ bool cpdi_corner(const KGrid &g, const double pos[3], const double r[9], int ei, int ej,
                                             int ek, int c, double xi[3], int off[3]) {
@@ -270,8 +300,8 @@ __device__ __forceinline__ bool cpdi_particle(const KGrid &g, const KPart &P, in
                                               CpdiCorners &cc) {
     double r[9];
 #pragma unroll
-    for (int a = 0; a < 9; a++) r[a] = P.cpr[a][p];
-    double pos[3] = {P.f[MPF_POS_X][p], P.f[MPF_POS_Y][p], DIM == 3 ? P.f[MPF_POS_Z][p] : 0.};
+    for (int a = 0; a < 9; a++) r[a] = P.cpr(a)[p];
+    double pos[3] = {P.f(MPF_POS_X)[p], P.f(MPF_POS_Y)[p], DIM == 3 ? P.f(MPF_POS_Z)[p] : 0.};
     bool ok = true;
     constexpr int NCOR = DIM == 3 ? 8 : 4;
 #pragma unroll
@@ -305,11 +335,8 @@ __device__ __forceinline__ void cpdi_wg_listed(const double r[9], int c, double 
     }
 }
 
-// Corner tables of the lCPDI scatters. A scatter lane owns candidate node offset o1 - 1 per axis
-// (o1 = 0..3); corner c's element holds the nodes at offsets off and off + 1, where the corner's
-// linear factors are 1 - xi and 1 + xi. The table of an axis holds those two factors at o1 = off + 1
-// and off + 2 and zeros elsewhere, so a lane reads the corner's function for its node with one load
-// per axis, zero for nodes outside the element. Built by one thread per (particle, corner).
+// linear factors of corner c at its particle's candidate node offsets o1 - 1 per axis (o1 = 0..3): the
+// corner's element holds the nodes at offsets off and off + 1, where they are 1 - xi and 1 + xi
 template <int DIM>
 __device__ __forceinline__ void cpdi_table(const double xi[3], const int off[3], double (*T)[4]) {
 #pragma unroll
@@ -319,40 +346,250 @@ __device__ __forceinline__ void cpdi_table(const double xi[3], const int off[3],
             T[a][o] = o == off[a] + 1 ? 1. - xi[a] : (o == off[a] + 2 ? 1. + xi[a] : 0.);
 }
 
-// Merged weight (and gradient) of the lane's node over the corners of one staged particle, summed
-// in corner order; corners whose element lacks the node or whose function is below 1e-15 add
-// nothing (GetCPDIFunctions, MoreMPMElementBase.cpp:581-656). The corner function 1/8 t1 t2 t3
-// (1/4 t1 t2 in 2D) is formed without its power-of-two factor, which is exact to move: the
-// threshold is scaled by 8 (4), the weight sum by 1/8 (1/4) once at the end, and the staged
-// gradient weights carry it (cpdi_wg_staged). The weight is then the same to the last bit.
-template <int DIM, bool GRAD>
-__device__ __forceinline__ void cpdi_table_node(const double (*T)[DIM][4], const double (*wg)[3], int o1x, int o1y,
-                                                int o1z, double &w, double gr[3]) {
-    constexpr int NCOR = DIM == 3 ? 8 : 4;
-    constexpr double thr = (DIM == 3 ? 8. : 4.) * 1e-15;
-    constexpr double wscale = DIM == 3 ? 0.125 * 0.125 : 0.25 * 0.25;   // ws times the corner factor
-    double sum = 0.;
-    if (GRAD) gr[0] = gr[1] = gr[2] = 0.;
-#pragma unroll
-    for (int c = 0; c < NCOR; c++) {
-        double f = DIM == 3 ? T[c][0][o1x] * T[c][1][o1y] * T[c][2][o1z] : T[c][0][o1x] * T[c][1][o1y];
-        f = f < thr ? 0. : f;
-        sum = c == 0 ? f : sum + f;
-        if (GRAD) {
-            gr[0] = fma(wg[c][0], f, gr[0]);
-            gr[1] = fma(wg[c][1], f, gr[1]);
-            if (DIM == 3) gr[2] = fma(wg[c][2], f, gr[2]);
-        }
-    }
-    w = wscale * sum;
-}
-
 // gradient weight of corner c as the scatters stage it: times the corner function's factor
 template <int DIM>
 __device__ __forceinline__ void cpdi_wg_staged(const double r[9], int c, double w[3]) {
     cpdi_wg_listed<DIM>(r, c, w);
 #pragma unroll
     for (int a = 0; a < 3; a++) w[a] *= DIM == 3 ? 0.125 : 0.25;
+}
+
+// ---------------------------------------------------------------------------------------
+// Shape factors of the step's passes (uGIMP and classic). Every pass needs them for every particle,
+// and evaluated as the reference writes them (particle_factors below: four candidates per axis, a
+// division for each natural coordinate and size, an integer division per axis for the cell) they
+// were most of the vector work of a pass (about 700 of the mass scatter's 1,500 VALU operations per
+// particle). Here the cell comes from the particle's bin key, the divisions are done with the
+// reciprocals of the cell size and the particle size kept in KGrid, and an axis evaluates the
+// three nodes that can lie in the support: with a = |xi| they are the near one at distance 1 - a,
+// the other node of the cell at 1 + a, and the outer one at 3 - a on the near one's side.
+
+// The rows with an opaque length: their addresses are then formed where a particle's words are read
+// (scalar additions) instead of being held in registers over the particle loop.
+__device__ __forceinline__ KPart local_rows(const KPart &P) {
+    KPart q = P;
+    asm volatile("" : "+s"(q.n));
+    return q;
+}
+
+// the particle's cell within its tile, from its bin key
+template <int DIM>
+__device__ __forceinline__ void tile_cell(int key, int tall, int &lx, int &ly, int &lz) {
+    using G = TileGeom<DIM>;
+    const int l = key - tall * G::NC;
+    lx = l % G::TX;
+    ly = (l / G::TX) % G::TY;
+    lz = DIM == 3 ? l / (G::TX * G::TY) : 0;
+}
+
+// Natural coordinate of x in cell c of one axis (node coordinates xmin + i*d) and 2 over the cell's
+// size. The quotient (2x - xmn - xmx)/(xmx - xmn) is found from r = 1/d: a Newton step gives the
+// reciprocal of the cell's own (rounded) size and one more of the quotient gives the correctly
+// rounded value, so a particle on the edge of a support lies exactly where the division puts it.
+__device__ __forceinline__ double natural_coord(double x, double xmin, double d, double r, int c, double &invd) {
+    const double mn = xmin + (double)c * d, mx = xmin + (double)(c + 1) * d;
+    const double w = mx - mn, n = 2. * x - mn - mx;
+    const double y = fma(r, fma(-w, r, 1.), r);
+    const double q = n * y;
+    invd = 2. * y;
+    return fma(fma(-q, w, n), y, q);
+}
+
+// values and derivatives (natural coordinates, towards the near node) at the three nodes of an axis
+struct AxisFactors {
+    double sn, sm, sx;         // near, the cell's other node, outer
+    double dn, dm, dx;       // magnitudes with the sign of the derivative left of the node
+    int w;                     // 1 when xi >= 0: near is candidate offset 1, outer 2, other 0
+    __device__ __forceinline__ double s4(int o) const {      // factor at candidate offset o - 1
+        return o == 0 ? (w ? 0. : sx) : o == 1 ? (w ? sm : sn) : o == 2 ? (w ? sn : sm) : (w ? sx : 0.);
+    }
+    __device__ __forceinline__ double d4(int o) const {
+        return o == 0 ? (w ? 0. : dx) : o == 1 ? (w ? dm : dn) : o == 2 ? (w ? -dn : -dm) : (w ? -dx : 0.);
+    }
+    __device__ __forceinline__ double s3(int j) const {      // factor at window node w + j
+        return j == 1 ? sn : ((j == 0) == (w != 0)) ? sm : sx;
+    }
+    __device__ __forceinline__ double d3(int j) const {
+        return j == 0 ? (w ? dm : dx) : j == 1 ? (w ? -dn : dn) : (w ? -dx : -dm);
+    }
+};
+
+// uGIMP factor and derivative at distance xp (zero outside, and for a NaN position)
+__device__ __forceinline__ void gimp_any(double xp, double lp, double inv, double i2lp, double &s, double &d) {
+    const double q1 = 2. - lp, q2 = 2. + lp, arg = (q2 - xp) * inv;
+    s = xp < lp ? ((4. - lp) * lp - xp * xp) * inv : xp <= q1 ? 0.5 * (2. - xp) : 2. * lp * arg * arg;
+    d = xp < lp ? -xp * i2lp : xp <= q1 ? -0.5 : -arg;
+    if (!(xp < q2)) { s = 0.; d = 0.; }
+}
+
+// lp: half size of the particle; inv = 1/(4 lp) (the 3D z axis takes lp.y's, as in the reference);
+// i2lp = 1/(2 lp) of the axis itself. INSIDE: |xi| <= 1; without it any coordinate (a position
+// outside the cell that its element names, or NaN), equal to the other for |xi| <= 1.
+template <bool INSIDE>
+__device__ __forceinline__ void axis_factors(double xi, double lp, double inv, double i2lp, AxisFactors &f) {
+    const double a = fabs(xi);
+    f.w = xi >= 0. ? 1 : 0;
+    if (!INSIDE) {
+        gimp_any(fabs(1. - a), lp, inv, i2lp, f.sn, f.dn);
+        gimp_any(1. + a, lp, inv, i2lp, f.sm, f.dm);
+        gimp_any(fabs(3. - a), lp, inv, i2lp, f.sx, f.dx);
+        if (a > 1.) f.dn = -f.dn;
+        if (a > 3.) f.dx = -f.dx;
+        return;
+    }
+    const double x0 = 1. - a, x1 = 1. + a, x2 = 3. - a, q1 = 2. - lp, q2 = 2. + lp;
+    const double a1 = (q2 - x1) * inv, a2 = (q2 - x2) * inv;
+    f.sn = x0 < lp ? ((4. - lp) * lp - x0 * x0) * inv : 0.5 * (2. - x0);
+    f.dn = x0 < lp ? -x0 * i2lp : -0.5;
+    f.sm = x1 <= q1 ? 0.5 * (2. - x1) : 2. * lp * a1 * a1;
+    f.dm = x1 <= q1 ? -0.5 : -a1;
+    f.sx = x2 < q2 ? 2. * lp * a2 * a2 : 0.;
+    f.dx = x2 < q2 ? -a2 : 0.;
+}
+
+// the element's linear functions (classic MPM)
+__device__ __forceinline__ void linear_factors(double xi, AxisFactors &f) {
+    const double n = 0.5 * (1. + fabs(xi)), o = 0.5 * (1. - fabs(xi));
+    f.w = xi >= 0. ? 1 : 0;
+    f.sn = n >= 0. ? n : 0.;
+    f.sm = o >= 0. ? o : 0.;
+    f.dn = n >= 0. ? -0.5 : 0.;
+    f.dm = o >= 0. ? -0.5 : 0.;
+    f.sx = f.dx = 0.;
+}
+
+// The axes of particle p in cell (cx, cy, cz). The grid's words are read here, through an opaque
+// pointer (scalar loads once per 64 particles): held over the particle loop they and the row
+// addresses overran the scalar registers.
+template <int DIM>
+__device__ __forceinline__ void particle_axes(GridPtr gp, const KPart &P, int p, int cx, int cy, int cz,
+                                              const double pos[3], AxisFactors f[DIM], double invd[DIM]) {
+    asm volatile("" : "+s"(gp));
+    double xi[DIM];
+    xi[0] = natural_coord(pos[0], gp->xmin, gp->dx, gp->rdx[0], cx, invd[0]);
+    xi[1] = natural_coord(pos[1], gp->ymin, gp->dy, gp->rdx[1], cy, invd[1]);
+    if constexpr (DIM == 3) xi[2] = natural_coord(pos[2], gp->zmin, gp->dz, gp->rdx[2], cz, invd[2]);
+    if (gp->shape == MPMGPU_SHAPE_LINEAR) {
+#pragma unroll
+        for (int a = 0; a < DIM; a++) linear_factors(xi[a], f[a]);
+        return;
+    }
+    bool inside = true;
+#pragma unroll
+    for (int a = 0; a < DIM; a++) inside = inside && fabs(xi[a]) <= 1.;
+    // z takes 1/(4 lp.y) in 3D (EightNodeIsoparamBrick.cpp:303)
+    if (gp->uniformLp && __all(inside)) {
+#pragma unroll
+        for (int a = 0; a < DIM; a++) axis_factors<true>(xi[a], gp->lp[a], gp->rlp4[a == 2 ? 1 : a], gp->rlp2[a], f[a]);
+        return;
+    }
+    const KPart R = local_rows(P);
+#pragma unroll
+    for (int a = 0; a < DIM; a++) {
+        const double lp = R.f(MPF_LP_X + a)[p], own = 1. / (4. * lp);
+        const double inv = a == 2 ? 1. / (4. * R.f(MPF_LP_Y)[p]) : own;
+        axis_factors<false>(xi[a], lp, inv, 2. * own, f[a]);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
+// Support window of one particle: with a half size lp <= 1 (natural units) a particle with xi < 0
+// touches no node at offset 2 and one with xi >= 0 none at offset -1, so three offsets per axis
+// starting at w = 0 (offsets -1..1) or w = 1 (0..2) hold every node of its support. The window's
+// factors are zero for nodes outside the support, and derivatives times 2/dx.
+template <int DIM>
+__device__ __forceinline__ void particle_window(const AxisFactors f[DIM], const double invd[DIM], int w[3],
+                                                double Sw[3][3], double Dw[3][3]) {
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+        w[a] = 0;
+#pragma unroll
+        for (int j = 0; j < 3; j++) {
+            if (a >= DIM) { Sw[a][j] = j == 1 ? 1. : 0.; Dw[a][j] = 0.; continue; }
+            w[a] = f[a < DIM ? a : 0].w;
+            Sw[a][j] = f[a < DIM ? a : 0].s3(j);
+            Dw[a][j] = f[a < DIM ? a : 0].d3(j) * invd[a < DIM ? a : 0];
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------------------
+// lCPDI, a lane per particle corner: a wave takes eight particles (sixteen in 2D) of its cells at a time
+// (their corners are adjacent lanes), and the scatters take the corners as records (WaveScatter, PPR = NCOR).
+template <int DIM> struct Corners {
+    static constexpr int N = DIM == 3 ? 8 : 4, PB = 64 / N;    // corners, particles per 64 lanes
+    static constexpr double W = 1. / N, WW = W * W;             // a corner's share; times its function's factor
+};
+
+// n/d from r = 1/d, correctly rounded as a division
+__device__ __forceinline__ double quotient(double n, double d, double r) {
+    const double q = n * r;
+    return fma(fma(-q, d, n), r, q);
+}
+
+// corner c of a particle at pos in cell (cx, cy, cz): cpdi_corner without its divisions
+template <int DIM>
+__device__ __forceinline__ bool corner_lane(GridPtr gp, const double pos[DIM], const double r[9], int cx, int cy, int cz,
+                                            int c, double xi[3], int off[3]) {
+    asm volatile("" : "+s"(gp));
+    const int q = c & 3;
+    const double s1 = (q == 1 || q == 2) ? 1. : -1.;
+    const double s2 = q >= 2 ? 1. : -1.;
+    const double s3 = c >= 4 ? 1. : -1.;
+    const double mn[3] = {gp->xmin, gp->ymin, gp->zmin}, d[3] = {gp->dx, gp->dy, gp->dz};
+    const int n[3] = {gp->nx, gp->ny, gp->nz}, cell[3] = {cx, cy, cz};
+    bool ok = true;
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+        if (a >= DIM) { xi[a] = 0.; off[a] = 0; continue; }
+        double x = pos[a < DIM ? a : 0] + s1 * r[a] + s2 * r[3 + a];
+        if (DIM == 3) x += s3 * r[6 + a];
+        int e = (int)quotient(x - mn[a], d[a], gp->rdx[a]);      // find_cell
+        if (e < 0 || e >= n[a]) {
+            if (x == mn[a] + n[a] * d[a]) e = n[a] - 1;
+            else { ok = false; e = e < 0 ? 0 : n[a] - 1; }
+        }
+        off[a] = e - cell[a];
+        if (off[a] < -1 || off[a] > 1) { ok = false; off[a] = off[a] < -1 ? -1 : 1; }
+        double invd;
+        xi[a] = natural_coord(x, mn[a], d[a], gp->rdx[a], cell[a] + off[a], invd);
+    }
+    return ok;
+}
+
+// A corner's rows at record i: 1 - xi and 1 + xi at the candidates of its element, zeros elsewhere. The
+// reference leaves a corner's node out when its function is below 1e-15; here a factor below 2e-15 is
+// zero, which drops the nodes of a corner on its element's edge (to rounding) likewise, and elsewhere
+// differs by weights of that size. The factors 1/8 (2D: 1/4) of the function and of the corner's share
+// are in the payload.
+template <int DIM, int NU>
+__device__ __forceinline__ void stage_corner(double (*S)[WROW], int i, const double xi[3], const int off[3],
+                                             const double u[NU]) {
+#pragma unroll
+    for (int a = 0; a < DIM; a++) {
+        double lo = 1. - xi[a], hi = 1. + xi[a];
+        lo = lo < 2e-15 ? 0. : lo;
+        hi = hi < 2e-15 ? 0. : hi;
+#pragma unroll
+        for (int o = 0; o < 4; o++) S[a * 4 + o][i] = o == off[a] + 1 ? lo : (o == off[a] + 2 ? hi : 0.);
+    }
+#pragma unroll
+    for (int q = 0; q < NU; q++) S[4 * DIM + q][i] = u[q];
+}
+
+// sum over the corner lanes of a particle, the total in each of them
+template <int CTRL> __device__ __forceinline__ double dpp_double(double v) {
+    union { double d; int i[2]; } t;
+    t.d = v;
+    t.i[0] = __builtin_amdgcn_update_dpp(0, t.i[0], CTRL, 0xf, 0xf, true);
+    t.i[1] = __builtin_amdgcn_update_dpp(0, t.i[1], CTRL, 0xf, 0xf, true);
+    return t.d;
+}
+template <int DIM> __device__ __forceinline__ double corner_sum(double v) {
+    v += dpp_double<0xB1>(v);      // quad_perm 1,0,3,2
+    v += dpp_double<0x4E>(v);      // quad_perm 2,3,0,1
+    if (DIM == 3) v += dpp_double<0x141>(v);   // mirror within eight lanes
+    return v;
 }
 
 // ---------------------------------------------------------------------------------------
@@ -538,7 +775,7 @@ __global__ void k_tile_need(KGrid g0, KBins B) {
     if (tall >= B.ntall) return;
     const int fld = tall / g0.tilesTotal;
     const int tg = tall - fld * g0.tilesTotal;
-    const KGrid g = tile_grid(g0, tg);
+    const KGrid g = g0.inst ? g0.inst[g0.tileInst[tg]] : g0;   // (a thread per tile)
     const int t = tg - g.tileBase;
     const int tx = t % g.ntx, ty = (t / g.ntx) % g.nty, tz = DIM == 3 ? t / (g.ntx * g.nty) : 0;
     int need = 0;
@@ -570,146 +807,312 @@ __device__ __forceinline__ void for_each_tile(const KBins &B, F &tile) {
     while (li < n) {
         int next = 0;
         if (threadIdx.x == 0) next = (int)gridDim.x + cur + 8 * atomicAdd(cursor, 1);
-        tile(B.tiles[li]);
+        // one tile per block: a scalar for the compiler, so an instance's grid and the node views
+        // built from it stay in scalar registers
+        tile(__builtin_amdgcn_readfirstlane(B.tiles[li]));
         if (threadIdx.x == 0) s_li = next;
         __syncthreads();
-        li = s_li;
+        li = __builtin_amdgcn_readfirstlane(s_li);
         __syncthreads();
     }
 }
 
 // ---------------------------------------------------------------------------------------
-// Deterministic per-wave scatter. Wave w of the block takes the tile's cells w, w+NW, ... in
-// order; for one cell, lane l owns the candidate node offset (l%4-1, (l/4)%4-1, l/16-1) (2D: the
-// first 16 lanes, (l%4-1, l/4-1)), so the 64 lanes write 64 different nodes. The lane sums the
-// cell's staged particles in sorted order in registers, then adds the sum to the wave's own
-// accumulator copy in LDS. The copies are added in wave order at the end. Every node value is
-// therefore the same fixed-order sum on every run.
 #define NW (NT / 64)
 
-// Footprint columns one wave's cells touch: wave w takes cells c = w, w+NW, ..., whose x index
-// runs from w to w + TX - NW (TX is a multiple of NW), so with node offsets -1..2 its accumulator
-// needs footprint columns w .. w + WX - 1 only.
+// A wave takes a run of the tile's cells, in sorted order: its layer z = w in 3D, its rows y = 2w and
+// 2w + 1 in 2D. The wave's copy of the footprint covers the planes (3D) or rows (2D) that its cells
+// reach, from LPW * w.
 template <int DIM> struct WaveFoot {
-    static_assert(TileGeom<DIM>::TX % NW == 0, "tile width must be a multiple of the waves per block");
-    static constexpr int WX = TileGeom<DIM>::TX - NW + 4;
-    static constexpr int SIZE = WX * TileGeom<DIM>::FY * TileGeom<DIM>::FZ;
+    using G = TileGeom<DIM>;
+    static constexpr int LPW = (DIM == 3 ? G::TZ : G::TY) / NW;     // layers of cells per wave
+    static_assert(LPW * NW == (DIM == 3 ? G::TZ : G::TY), "tile layers against the waves per block");
+    static constexpr int WX = G::FX, LAYERS = LPW + 3;
+    // words from one layer to the next: in 3D chosen so that the 64 additions of one instruction of a
+    // matrix-core scatter fall on few banks more than twice (the least for 64 doubles)
+    static constexpr int LAYER = DIM == 3 ? WX * G::FY + (G::TX == 8 ? 1 : 0) : WX;
+    static constexpr int SIZE = LAYERS * LAYER;
 };
 
-template <int DIM, int NQ, typename Load, typename Add>
-__device__ __forceinline__ void wave_cells(const int *s_cs, int r0, int r1,
-                                           double (*s_acc)[NQ][WaveFoot<DIM>::SIZE], Load load, Add add) {
-    using G = TileGeom<DIM>;
-    const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
-    const int o1x = l & 3, o1y = (l >> 2) & 3, o1z = DIM == 3 ? (l >> 4) : 1;   // offset + 1
-    if constexpr (DIM == 2) {
-        // A 2D cell has 16 candidate nodes, so a wave takes four cells per pass: lane group
-        // l / 16 one cell, lane l % 16 its candidate. The wave's cells sit at x = w + NW a
-        // (a < A) on every row; the four cells of a pass are 4 cells apart in x or y, so they
-        // touch different nodes and their sums go to different slots of the wave's copy. Each
-        // node's slot takes its cells in a fixed pass order.
-        constexpr int A = G::TX / NW;
-        static_assert(A == 4 || (A == 2 && G::TY == 8), "2D tiles 4*NW cells wide, or 2*NW wide and 8 high");
-        constexpr int PASSES = A * G::TY / 4;
-        const int grp = l >> 4;
-        const int lx = w + NW * (A == 4 ? grp : (grp & 1));
-#pragma unroll 1
-        for (int it = 0; it < PASSES; it++) {
-            const int ly = A == 4 ? it : it + 4 * (grp >> 1);
-            const int c = ly * G::TX + lx;
-            const int b = max(s_cs[c], r0), e = min(s_cs[c + 1], r1);
-            if (__ballot(b < e) == 0ull) continue;      // none of the four cells has particles here
-            double acc[NQ];
-#pragma unroll
-            for (int q = 0; q < NQ; q++) acc[q] = 0.;
-            int k = b;
-            for (; k + 4 <= e; k += 4) {
-                auto a0 = load(k - r0, o1x, o1y, o1z);
-                auto a1 = load(k + 1 - r0, o1x, o1y, o1z);
-                auto a2 = load(k + 2 - r0, o1x, o1y, o1z);
-                auto a3 = load(k + 3 - r0, o1x, o1y, o1z);
-                add(a0, acc, lx, ly, 0);
-                add(a1, acc, lx, ly, 0);
-                add(a2, acc, lx, ly, 0);
-                add(a3, acc, lx, ly, 0);
-            }
-            for (; k < e; k++) {
-                auto a0 = load(k - r0, o1x, o1y, o1z);
-                add(a0, acc, lx, ly, 0);
-            }
-            if (b < e) {
-                const int slot = (ly + o1y) * WaveFoot<DIM>::WX + (lx + o1x - w);
-#pragma unroll
-                for (int q = 0; q < NQ; q++) s_acc[w][q][slot] += acc[q];
-            }
-            __builtin_amdgcn_wave_barrier();
-        }
-        return;
+// Scatters on the matrix cores. A cell's sums over its particles at the candidate nodes are a
+// contraction: with per-axis factors X, Y, Z and a payload u_q, node (ix, iy, iz) of component q
+// gains sum_p (X_p[ix] Y_p[iy]) (Z_p[iz] u_pq), a 16 x K by K x 16 product over the cell's particles
+// with rows (iy, ix) and columns (iz, q): v_mfma_f64_16x16x4 for four particles at a time, with four
+// LDS reads and two multiplications, where a lane per node read seven words and issued six FP64
+// operations for each particle. In 2D the columns are the components alone: v_mfma_f64_4x4x4, whose
+// four blocks take the rows iy. Sums keep a fixed order: a matrix instruction adds its four products
+// one after another (measured equal to a chain of FMAs bit for bit; a missing fourth adds zero), a
+// cell takes its particles in upload order, and a cell's result is added to the wave's own LDS copy,
+// one address per lane, by LDS additions that a wave issues in cell order; the copies are added in
+// wave order. Every node value is therefore the same on every run.
+//
+// A wave works on its own: it takes its particles 64 at a time (a lane each for the loads and the
+// shape factors), stages their factors in its own LDS rows and scatters its own cells, so no barrier
+// stands between loads, factors and sums and the waves of a CU overlap them. The rows hold WREC
+// records, so that three blocks fit in a CU's LDS. On the 128^3 J2 block the mass scatter went from
+// 0.65 to 0.36 ms per launch, the force scatter from 0.83 to 0.55 and the particle update from 0.92
+// to 0.67; on 86k lCPDI particles from 0.13, 0.18 and 0.18 to 0.075, 0.073 and 0.090.
+typedef double mat4d __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ void lds_add(double *a, double v) {
+    __hip_atomic_fetch_add(a, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+// LDS words written by some lanes of a wave are read by others: a wave's LDS instructions execute in
+// order, so only the compiler has to keep them so
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// The cells of a wave taken one after another as their particles are staged. bounds: lane it holds the
+// start of the wave's it-th cell, lane it + ITS its end; it: the cell reached; open: its sums (in the
+// caller's registers) have begun; at: its offset in the wave's copy.
+template <int DIM> struct WaveCells {
+    static constexpr int ITS = TileGeom<DIM>::NC / NW;
+    static_assert(ITS <= 32, "bounds held by the lanes of a wave");
+    int bounds, it, at;
+    bool open;
+    int b, e;                   // the wave's particles: sorted slots b..e-1
+    __device__ __forceinline__ void begin(const int *s_cs) {
+        const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
+        bounds = s_cs[w * ITS + l % ITS + (l / ITS > 0 ? 1 : 0)];
+        it = 0;
+        open = false;
+        b = start(0);
+        e = end(ITS - 1);
     }
-    const bool lane_on = true;
-    for (int c = w; c < G::NC; c += NW) {
-        int b = max(s_cs[c], r0), e = min(s_cs[c + 1], r1);
-        if (b >= e) continue;
-        int lx = c % G::TX, ly = (c / G::TX) % G::TY, lz = DIM == 3 ? c / (G::TX * G::TY) : 0;
-        double acc[NQ];
-#pragma unroll
-        for (int q = 0; q < NQ; q++) acc[q] = 0.;
-        if (lane_on) {
-            // records of four particles are read before they are added, in particle order
-            int k = b;
-            for (; k + 4 <= e; k += 4) {
-                auto a0 = load(k - r0, o1x, o1y, o1z);
-                auto a1 = load(k + 1 - r0, o1x, o1y, o1z);
-                auto a2 = load(k + 2 - r0, o1x, o1y, o1z);
-                auto a3 = load(k + 3 - r0, o1x, o1y, o1z);
-                add(a0, acc, lx, ly, lz);
-                add(a1, acc, lx, ly, lz);
-                add(a2, acc, lx, ly, lz);
-                add(a3, acc, lx, ly, lz);
+    __device__ __forceinline__ int start(int i) const { return __builtin_amdgcn_readlane(bounds, i); }
+    __device__ __forceinline__ int end(int i) const { return __builtin_amdgcn_readlane(bounds, i + ITS); }
+};
+
+// visits the cells with particles among the staged slots r0..r1-1: first(kb, ke, open) begins a cell
+// with particles kb..ke-1 of them (open: the one before it still has to be added to the copy),
+// more(kb, ke) goes on with one that an earlier round began
+template <int DIM, typename First, typename More>
+__device__ __forceinline__ void wave_walk(WaveCells<DIM> &W, int r0, int r1, First first, More more) {
+    using G = TileGeom<DIM>;
+    while (W.it < WaveCells<DIM>::ITS) {
+        const int s = W.start(W.it), e = W.end(W.it);
+        if (s >= r1) break;
+        const int kb = max(s, r0) - r0, ke = min(e, r1) - r0;
+        if (kb < ke) {
+            if (s < r0 && W.open) more(kb, ke);
+            else {
+                first(kb, ke, W.open);
+                W.open = true;
+                W.at = (W.it / G::TX) * WaveFoot<DIM>::WX + W.it % G::TX;
             }
-            for (; k < e; k++) {
-                auto a0 = load(k - r0, o1x, o1y, o1z);
-                add(a0, acc, lx, ly, lz);
-            }
-            const int row = DIM == 3 ? (lz + o1z) * G::FY + (ly + o1y) : ly + o1y;   // footprint row
-            const int slot = row * WaveFoot<DIM>::WX + (lx + o1x - w);
-#pragma unroll
-            for (int q = 0; q < NQ; q++) s_acc[w][q][slot] += acc[q];
         }
-        __builtin_amdgcn_wave_barrier();
+        if (e > r1) break;
+        W.it++;
     }
 }
 
-// particle records of the scatters: per-axis factors of the lane's candidate and the payload
-struct RecMass { double wx, wy, wz, mp, vx, vy, vz; };
-struct RecForce { double wx, wy, wz, dx, dy, dz, s0, s1, s2, s3, s4, s5; };
-struct RecForce2 { double2 x, y, z; double a[6]; };
-// with external particle loads or tractions: pFext and the particle's traction force at the node
-struct RecForceX : RecForce { double e[3], t[3]; };
-struct RecForce2X : RecForce2 { double e[3], t[3]; };
+// Mass- and momentum-like sums of NQ components. S: rows STR apart, 4*DIM of factors [axis*4 + candidate]
+// [record] and NQ of payload [q][record], rounded up to fours (a row beyond NQ is read and its result
+// dropped). Four components are one 16x16x4 product, up to eight are two with the same rows. A
+// particle has PPR records: itself, or its lCPDI corners (a corner's linear functions are a product of
+// axis factors too, zero at the candidates its element lacks). A cell's first records are read before
+// the cell before it is added to the copy, so the reads pass over the matrix instructions' latency.
+struct NoExtra {
+    template <typename... T> __device__ __forceinline__ void operator()(T &&...) const {}
+};
+template <int DIM> struct MatSums { typedef mat4d T; };     // of one component block of a cell, per lane
+template <> struct MatSums<2> { typedef double T; };
 
+template <int DIM, int NQ, int PPR, int STR> struct WaveScatter {
+    using F = WaveFoot<DIM>;
+    static constexpr int NB = (NQ + 3) / 4;
+    const double *plo, *phi;    // this lane's record of a quad in the rows of its lo and hi candidate
+    double *acc;
+    int k4, lo, hi;
+    typename MatSums<DIM>::T c[NB];
+    struct Quad { double x, y, z, v[NB]; };
+    __device__ __forceinline__ void begin(const double *S, double (*s_acc)[NQ][F::SIZE]) {
+        const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
+        lo = l & 3;
+        hi = (l >> 2) & 3;
+        k4 = l >> 4;
+        plo = S + lo * STR + k4;
+        phi = S + hi * STR + k4;
+        // 3D: result register r, lane l: node (ix = k4, iy = r, iz = hi) of component lo (block 1: 4 + lo);
+        // 2D: lane l: node (ix = k4, iy = hi)
+        acc = &s_acc[w][lo < NQ ? lo : 0][hi * F::LAYER + k4];
+    }
+    __device__ __forceinline__ Quad read(int k) const {
+        Quad t;
+        t.x = plo[k]; t.y = phi[4 * STR + k];
+        t.z = DIM == 3 ? phi[8 * STR + k] : 1.;
+#pragma unroll
+        for (int b = 0; b < NB; b++) t.v[b] = plo[(4 * DIM + 4 * b) * STR + k];
+        return t;
+    }
+    // records k..k+3 of a cell whose records end before e; those beyond the end count as zero
+    __device__ __forceinline__ Quad load(int k, int e) const {
+        if (PPR % 4 == 0 || k + 4 <= e) return read(k);
+        Quad t = read(min(k + k4, e - 1) - k4);
+        t.x = k + k4 < e ? t.x : 0.;
+        return t;
+    }
+    __device__ __forceinline__ void fold(const Quad &t) {
+        const double a = t.x * t.y;
+#pragma unroll
+        for (int b = 0; b < NB; b++) {
+            if constexpr (DIM == 3) c[b] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, t.z * t.v[b], c[b], 0, 0, 0);
+            else c[b] = __builtin_amdgcn_mfma_f64_4x4x4f64(a, t.v[b], c[b], 0, 0, 0);
+        }
+    }
+    __device__ __forceinline__ void flush(int at) const {
+#pragma unroll
+        for (int b = 0; b < NB; b++) {
+            if (4 * b + lo >= NQ) continue;
+            double *p = acc + b * 4 * F::SIZE + at;
+            if constexpr (DIM == 3) {
+#pragma unroll
+                for (int r = 0; r < 4; r++) lds_add(p + r * F::WX, c[b][r]);
+            } else lds_add(p, c[b]);
+        }
+    }
+    // particles r0..r1-1 are staged, from record 0; extra(kb, ke, lo, hi, k4, c) after each cell's sums
+    template <typename Extra> __device__ __forceinline__ void scatter(WaveCells<DIM> &W, int r0, int r1, Extra extra) {
+        auto add = [&](int k, int e) {
+#pragma unroll 1
+            for (; k < e; k += 4) fold(load(k, e));
+        };
+        wave_walk(W, r0, r1,
+            [&](int kb, int ke, bool open) {
+                const Quad t0 = load(kb * PPR, ke * PPR);
+                if (open) flush(W.at);
+#pragma unroll
+                for (int b = 0; b < NB; b++) c[b] = typename MatSums<DIM>::T{};
+                fold(t0);
+                add(kb * PPR + 4, ke * PPR);
+                extra(kb, ke, lo, hi, k4, c[0]);
+            },
+            [&](int kb, int ke) {
+                add(kb * PPR, ke * PPR);
+                extra(kb, ke, lo, hi, k4, c[0]);
+            });
+    }
+    __device__ __forceinline__ void scatter(WaveCells<DIM> &W, int r0, int r1) { scatter(W, r0, r1, NoExtra()); }
+    __device__ __forceinline__ void finish(const WaveCells<DIM> &W) const {
+        if (W.open) flush(W.at);
+    }
+};
+
+// The force scatter's sums: node (ix, iy, iz) of component q gains, per particle,
+// a_q0 X'YZ + a_q1 XY'Z + a_q2 XYZ' (the rows of the symmetric a: xx, yy, xy, zz, xz, yz): three of the
+// products above, with rows X'Y, XY' and XY and columns Z a_q0, Z a_q1 and Z' a_q2 (2D: two). F: 4*DIM
+// rows of (factor, derivative) pairs [axis*4 + candidate][record]; a: the terms' rows; both STR apart.
+// With loads (FX) e holds 3 rows of pFext, added times XYZ, and trac adds a particle's own nodal forces.
+template <int DIM, bool FX, int STR> struct WaveForce {
+    using F = WaveFoot<DIM>;
+    const double2 *flo, *fhi;
+    const double *a0, *a1, *a2, *eq;
+    double *acc;
+    int k4, q, hi;
+    bool on;
+    typename MatSums<DIM>::T c;
+    struct Quad { double2 x, y, z; double a0, a1, a2, e; };
+    __device__ __forceinline__ void begin(const double2 *S, const double *a, const double *e, double (*s_acc)[NQ_FORCE][F::SIZE]) {
+        const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
+        const int lo = l & 3;
+        hi = (l >> 2) & 3;
+        k4 = l >> 4;
+        on = lo < DIM;
+        q = on ? lo : 0;
+        flo = S + lo * STR + k4;
+        fhi = S + hi * STR + k4;
+        a0 = a + (q == 0 ? 0 : q == 1 ? 2 : 4) * STR + k4;
+        a1 = a + (q == 0 ? 2 : q == 1 ? 1 : 5) * STR + k4;
+        a2 = a + (DIM == 2 ? 0 : q == 0 ? 4 : q == 1 ? 5 : 3) * STR + k4;
+        eq = FX ? e + q * STR + k4 : nullptr;
+        // 3D: result register r, lane l: node (ix = k4, iy = r, iz = hi); 2D: lane l: node (ix = k4, iy = hi)
+        acc = &s_acc[w][q][hi * F::LAYER + k4];
+    }
+    __device__ __forceinline__ Quad read(int k) const {
+        Quad t;
+        t.x = flo[k]; t.y = fhi[4 * STR + k];
+        if (DIM == 3) { t.z = fhi[8 * STR + k]; t.a2 = a2[k]; }
+        t.a0 = a0[k]; t.a1 = a1[k];
+        t.e = FX ? eq[k] : 0.;
+        return t;
+    }
+    __device__ __forceinline__ Quad load(int k, int e) const {
+        if (k + 4 <= e) return read(k);
+        Quad t = read(min(k + k4, e - 1) - k4);
+        if (k + k4 >= e) t.x = make_double2(0., 0.);
+        return t;
+    }
+    __device__ __forceinline__ void fold(const Quad &t) {
+        if constexpr (DIM == 3) {
+            c = __builtin_amdgcn_mfma_f64_16x16x4f64(t.x.y * t.y.x, t.z.x * t.a0, c, 0, 0, 0);
+            c = __builtin_amdgcn_mfma_f64_16x16x4f64(t.x.x * t.y.y, t.z.x * t.a1, c, 0, 0, 0);
+            const double b = FX ? fma(t.z.x, t.e, t.z.y * t.a2) : t.z.y * t.a2;
+            c = __builtin_amdgcn_mfma_f64_16x16x4f64(t.x.x * t.y.x, b, c, 0, 0, 0);
+        } else {
+            c = __builtin_amdgcn_mfma_f64_4x4x4f64(t.x.y * t.y.x, t.a0, c, 0, 0, 0);
+            c = __builtin_amdgcn_mfma_f64_4x4x4f64(t.x.x * t.y.y, t.a1, c, 0, 0, 0);
+            if (FX) c = __builtin_amdgcn_mfma_f64_4x4x4f64(t.x.x * t.y.x, t.e, c, 0, 0, 0);
+        }
+    }
+    __device__ __forceinline__ void flush(int at) const {
+        if (!on) return;
+        if constexpr (DIM == 3) {
+#pragma unroll
+            for (int r = 0; r < 4; r++) lds_add(acc + at + r * F::WX, c[r]);
+        } else lds_add(acc + at, c);
+    }
+    template <typename Trac> __device__ __forceinline__ void scatter(WaveCells<DIM> &W, int r0, int r1, Trac trac) {
+        auto add = [&](int k, int e) {
+#pragma unroll 1
+            for (; k < e; k += 4) fold(load(k, e));
+        };
+        wave_walk(W, r0, r1,
+            [&](int kb, int ke, bool open) {
+                const Quad t = load(kb, ke);
+                if (open) flush(W.at);
+                c = typename MatSums<DIM>::T{};
+                fold(t);
+                add(kb + 4, ke);
+                if (FX) trac(kb, ke, q, hi, k4, c);
+            },
+            [&](int kb, int ke) {
+                add(kb, ke);
+                if (FX) trac(kb, ke, q, hi, k4, c);
+            });
+    }
+    __device__ __forceinline__ void finish(const WaveCells<DIM> &W) const {
+        if (W.open) flush(W.at);
+    }
+};
+
+// a wave's own copy (the wave's later LDS instructions follow in order)
 template <int DIM, int NQ>
-__device__ __forceinline__ void zero_acc(double (*s_acc)[NQ][WaveFoot<DIM>::SIZE]) {
-    double *a = &s_acc[0][0][0];
-    for (int i = threadIdx.x; i < NW * NQ * WaveFoot<DIM>::SIZE; i += NT) a[i] = 0.;
+__device__ __forceinline__ void zero_wave_acc(double (*s_acc)[NQ][WaveFoot<DIM>::SIZE]) {
+    double *a = &s_acc[threadIdx.x >> 6][0][0];
+    for (int i = threadIdx.x & 63; i < NQ * WaveFoot<DIM>::SIZE; i += 64) a[i] = 0.;
+    wave_sync();
 }
 
 // add the wave copies that cover each footprint node in wave order and store the tile's sums
 template <int DIM, int NQ>
 __device__ __forceinline__ void write_partials(const KNodes &N, int t, double (*s_acc)[NQ][WaveFoot<DIM>::SIZE]) {
     using G = TileGeom<DIM>;
-    constexpr int WX = WaveFoot<DIM>::WX;
+    using W = WaveFoot<DIM>;
     for (int s = threadIdx.x; s < G::FOOT; s += NT) {
-        const int fx = s % G::FX, row = s / G::FX;
+        const int in = DIM == 3 ? s % (G::FX * G::FY) : s % G::FX, layer = DIM == 3 ? s / (G::FX * G::FY) : s / G::FX;
 #pragma unroll
         for (int q = 0; q < NQ; q++) {
             double v = 0.;
             bool first = true;
 #pragma unroll
             for (int w = 0; w < NW; w++) {
-                const int c = fx - w;
-                if (c < 0 || c >= WX) continue;
-                const double a = s_acc[w][q][row * WX + c];
+                const int c = layer - W::LPW * w;
+                if (c < 0 || c >= W::LAYERS) continue;
+                const double a = s_acc[w][q][c * W::LAYER + in];
                 v = first ? a : v + a;
                 first = false;
             }
@@ -729,135 +1132,171 @@ __device__ __forceinline__ void load_tile_starts(const KBins &B, int t, int *s_c
 // P2G #1: mass and momentum (MassAndMomentumTask -> NodalPoint::AddMassMomentum,
 // NodalPointMPM.cpp:419-453). The point count of a node is not summed: every particle has
 // mp > 0 and every in-support weight is > 0, so numberPoints > 0 exactly when the mass is > 0.
-template <int DIM, int SH>
-__global__ __launch_bounds__(NT) void k_p2g_mass(KGrid g0, KPart P, KBins B, KNodes N, KStats st) {
+
+// uGIMP and classic: the words of a lane's particle that the mass scatter and the particle update need
+template <int DIM> struct MassWords { int p, key; double x[DIM], m, v[DIM]; };
+
+template <int DIM>
+__device__ __forceinline__ void load_mass_words(const KPart &rows, const KBins &B, int k, int e, MassWords<DIM> &t) {
+    const KPart P = local_rows(rows);
+    t.p = k < e ? B.order[k] : -1;
+    if (t.p < 0) return;
+    t.key = B.key[t.p];
+#pragma unroll
+    for (int a = 0; a < DIM; a++) {
+        t.x[a] = P.f(MPF_POS_X + a)[t.p];
+        t.v[a] = P.f(MPF_VEL_X + a)[t.p];
+    }
+    t.m = P.f(MPF_MASS)[t.p];
+}
+
+// a particle's factor rows and payload at record i of its wave's rows
+template <int DIM, int NU>
+__device__ __forceinline__ void stage_factors(double (*S)[WROW], int i, const AxisFactors f[DIM], const double u[NU]) {
+#pragma unroll
+    for (int a = 0; a < DIM; a++) {
+        AxisFactors t = f[a];
+        asm volatile("" : "+v"(t.w));          // formed here, not held from before the rounds
+#pragma unroll
+        for (int o = 0; o < 4; o++) S[a * 4 + o][i] = t.s4(o);
+    }
+#pragma unroll
+    for (int q = 0; q < NU; q++) S[4 * DIM + q][i] = u[q];
+}
+
+template <int DIM>
+__global__ __launch_bounds__(NT, G2P_WAVES) void k_p2g_mass(KGrid g0, KPart P, KBins B, KNodes N) {
     using G = TileGeom<DIM>;
-    constexpr bool CP = SH == MPMGPU_SHAPE_LCPDI;
-    constexpr int NCOR = DIM == 3 ? 8 : 4;
-    // particles staged per chunk (three blocks per CU); lCPDI: one thread per particle corner
-    constexpr int CH = CP ? NT / NCOR : NT / 2;
     __shared__ int s_cs[G::NC + 1];
-    __shared__ double s_S[CP ? 1 : DIM * 4][CH + 1];   // [axis*4 + offset][particle]
-    __shared__ double s_ct[CP ? CH : 1][NCOR][DIM][4];
-    __shared__ double s_q[4][CH + 1];
+    __shared__ double s_S[NW][4 * DIM + 4][WROW];       // per wave: [axis*4 + offset][record], then mass and momentum
     __shared__ double s_acc[NW][NQ_MASS][WaveFoot<DIM>::SIZE];
+    const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
     auto tile = [&](const int tall) {      // (field, context tile) pair
-        const KGrid g = tile_grid(g0, tall % g0.tilesTotal);
+        const int tc = tall % g0.tilesTotal;
+        const GridPtr gp = tile_grid_ptr(g0, tc);
+        const KGrid g = grid_copy(gp);
         load_tile_starts<DIM>(B, tall, s_cs);
-        const int tb = s_cs[0], te = s_cs[G::NC];
-        if (tb == te) return;
-        zero_acc<DIM, NQ_MASS>(s_acc);
-        auto scatter = [&](int c0, int c1) {
-            wave_cells<DIM, NQ_MASS>(s_cs, c0, c1, s_acc,
-                [&](int lq, int ix, int iy, int iz) {
-                    RecMass r;
-                    if (CP) {
-                        double gr[3];
-                        cpdi_table_node<DIM, false>(s_ct[lq], nullptr, ix, iy, iz, r.wx, gr);
-                        r.wy = 1.; r.wz = 1.;
-                    } else {
-                        r.wx = s_S[ix][lq]; r.wy = s_S[4 + iy][lq]; r.wz = DIM == 3 ? s_S[(DIM - 1) * 4 + iz][lq] : 1.;
-                    }
-                    r.mp = s_q[0][lq]; r.vx = s_q[1][lq]; r.vy = s_q[2][lq]; r.vz = s_q[3][lq];
-                    return r;
-                },
-                [&](const RecMass &r, double *acc, int, int, int) {
-                    // lCPDI: merged weight (zero for non-member nodes) times mp; otherwise the
-                    // product of the staged factors, mp included
-                    const double fnmp = CP ? r.wx * r.mp : (DIM == 3 ? r.wx * (r.wy * r.wz) : r.wx * r.wy);
-                    acc[0] += fnmp;
-                    acc[1] = fma(fnmp, r.vx, acc[1]);
-                    acc[2] = fma(fnmp, r.vy, acc[2]);
-                    acc[3] = fma(fnmp, r.vz, acc[3]);
-                });
-        };
-        if (!CP) {
-            // Rounds of 2*NT slots: every thread first loads the particle words of its two slots of
-            // the round (tb + t and tb + t + NT), so the round's global loads overlap; then the four
-            // chunks of CH slots are staged from registers by the half of the block that holds them.
-            for (int r0 = tb; r0 < te; r0 += 2 * NT) {
-                int rp[2], re[2];
-                double rx[2][3], rm[2], rv[2][3];
+        if (s_cs[0] == s_cs[G::NC]) return;
+        int ox, oy, oz;
+        tile_origin<DIM>(g, tc - g.tileBase, ox, oy, oz);
+        WaveCells<DIM> W;
+        W.begin(s_cs);
+        WaveScatter<DIM, NQ_MASS, 1, WROW> sc;
+        sc.begin(&s_S[w][0][0], s_acc);
+        MassWords<DIM> cur;
+        load_mass_words<DIM>(P, B, W.b + l, W.e, cur);
+        zero_wave_acc<DIM, NQ_MASS>(s_acc);
+        for (int r = W.b; r < W.e; r += 64) {
+            AxisFactors f[DIM];
+            double u[4];
+            if (cur.p >= 0) {
+                int lx, ly, lz;
+                double invd[DIM];
+                tile_cell<DIM>(cur.key, tall, lx, ly, lz);
+                particle_axes<DIM>(gp, P, cur.p, ox + lx, oy + ly, oz + lz, cur.x, f, invd);
+                u[0] = cur.m;
 #pragma unroll
-                for (int j = 0; j < 2; j++) {
-                    const int k = r0 + threadIdx.x + j * NT;
-                    rp[j] = k < te ? B.order[k] : -1;
-                }
-#pragma unroll
-                for (int j = 0; j < 2; j++) {
-                    const int p = rp[j];
-                    if (p < 0) continue;
-                    re[j] = P.elem[p];
-#pragma unroll
-                    for (int a = 0; a < 3; a++) {
-                        rx[j][a] = a < DIM ? P.f[MPF_POS_X + a][p] : 0.;
-                        rv[j][a] = a < DIM ? P.f[MPF_VEL_X + a][p] : 0.;
-                    }
-                    rm[j] = P.f[MPF_MASS][p];
-                }
-#pragma unroll
-                for (int c = 0; c < 4; c++) {
-                    const int c0 = r0 + c * CH;
-                    if (c0 >= te) break;
-                    const int j = c >> 1;
-                    if ((int)(threadIdx.x / CH) == (c & 1) && rp[j] >= 0) {
-                        const int i = threadIdx.x - (c & 1) * CH;
-                        int ei, ej, ek;
-                        elem_ijk(g, re[j], ei, ej, ek);
-                        // factors with zeros outside the support; the x factor carries mp
-                        double xi[3], invd[3], S[3][4], dS[3][4];
-                        particle_xi<DIM>(g, ei, ej, ek, rx[j][0], rx[j][1], rx[j][2], xi, invd);
-                        particle_factors<DIM>(g, P, rp[j], xi, S, dS);
-#pragma unroll
-                        for (int a = 0; a < DIM; a++)
-#pragma unroll
-                            for (int o = 0; o < 4; o++) {
-                                const double v = S[a][o] >= 0. ? S[a][o] : 0.;
-                                s_S[a * 4 + o][i] = a == 0 ? v * rm[j] : v;
-                            }
-                        s_q[0][i] = rm[j];
-                        s_q[1][i] = rv[j][0]; s_q[2][i] = rv[j][1]; s_q[3][i] = rv[j][2];
-                    }
-                    __syncthreads();
-                    scatter(c0, min(c0 + CH, te));
-                    __syncthreads();
-                }
+                for (int a = 0; a < 3; a++) u[1 + a] = a < DIM ? cur.m * cur.v[a < DIM ? a : 0] : 0.;
             }
-        } else {
-            const int i = threadIdx.x / NCOR, c = threadIdx.x % NCOR;
-            for (int c0 = tb; c0 < te; c0 += CH) {
-                const int k = c0 + i;
-                bool ok = true;
-                if (k < te) {
-                    const int p = B.order[k];
-                    int ei, ej, ek;
-                    elem_ijk(g, P.elem[p], ei, ej, ek);
-                    double pos[3] = {P.f[MPF_POS_X][p], P.f[MPF_POS_Y][p], DIM == 3 ? P.f[MPF_POS_Z][p] : 0.};
-                    // InitializationTask -> GetCPDINodesAndWeights: semi-side vectors of the step (each
-                    // corner's thread builds them; the first keeps them for the step's other passes)
-                    double r[9];
-                    cpdi_semi_sides<DIM>(g, P, p, ei, ej, ek, r);
-                    double xi[3];
-                    int off[3];
-                    ok = cpdi_corner<DIM>(g, pos, r, ei, ej, ek, c, xi, off);
-                    cpdi_table<DIM>(xi, off, s_ct[i][c]);
-                    if (c == 0) {
-#pragma unroll
-                        for (int a = 0; a < 9; a++) P.cpr[a][p] = r[a];
-                        s_q[0][i] = P.f[MPF_MASS][p];
-                        s_q[1][i] = P.f[MPF_VEL_X][p];
-                        s_q[2][i] = P.f[MPF_VEL_Y][p];
-                        s_q[3][i] = DIM == 3 ? P.f[MPF_VEL_Z][p] : 0.;
-                    }
-                }
-                // one count per particle with an unusable corner (its corner threads are adjacent lanes)
-                const unsigned long long bad = __ballot(!ok);
-                if (c == 0 && ((bad >> (threadIdx.x & 63)) & ((1ull << NCOR) - 1ull))) atomicAdd(st.cpdiErr, 1ull);
-                __syncthreads();
-                scatter(c0, min(c0 + CH, te));
-                __syncthreads();
+            for (int r0 = r; r0 < min(r + 64, W.e); r0 += WREC) {
+                if (l / WREC == (r0 - r) / WREC && cur.p >= 0) stage_factors<DIM, 4>(s_S[w], l % WREC, f, u);
+                // the next particles' loads pass over the last scatter
+                if (r0 + WREC >= min(r + 64, W.e)) load_mass_words<DIM>(P, B, r + 64 + l, W.e, cur);
+                wave_sync();
+                sc.scatter(W, r0, min(r0 + WREC, W.e));
+                wave_sync();
             }
         }
+        sc.finish(W);
+        __syncthreads();
+        write_partials<DIM, NQ_MASS>(N, tall, s_acc);
+    };
+    for_each_tile(B, tile);
+}
+
+// strains and rotations in the order of get_F3 (2D: those out of the plane are zero)
+template <int DIM>
+__device__ __forceinline__ void load_deformation(const KPart &P, int p, double ep[6], double wr[3]) {
+#pragma unroll
+    for (int a = 0; a < 6; a++) ep[a] = DIM == 3 || a < 3 || a == 5 ? P.f(MPF_EP_XX + a)[p] : 0.;
+#pragma unroll
+    for (int a = 0; a < 3; a++) wr[a] = DIM == 3 || a == 2 ? P.f(MPF_WR_YZ + a)[p] : 0.;
+}
+
+// lCPDI: the words of a lane's particle; F gives the semi-side vectors of the step
+template <int DIM> struct CornerMassWords { int p, key; double x[DIM], m, v[DIM], ep[6], wr[3]; };
+
+template <int DIM>
+__device__ __forceinline__ void load_corner_mass(const KPart &rows, const KBins &B, int k, int e, CornerMassWords<DIM> &t) {
+    const KPart P = local_rows(rows);
+    t.p = k < e ? B.order[k] : -1;
+    if (t.p < 0) return;
+    t.key = B.key[t.p];
+#pragma unroll
+    for (int a = 0; a < DIM; a++) {
+        t.x[a] = P.f(MPF_POS_X + a)[t.p];
+        t.v[a] = P.f(MPF_VEL_X + a)[t.p];
+    }
+    load_deformation<DIM>(P, t.p, t.ep, t.wr);
+    t.m = P.f(MPF_MASS)[t.p];
+}
+
+template <int DIM>
+__global__ __launch_bounds__(NT, G2P_WAVES) void k_p2g_mass_corners(KGrid g0, KPart P, KBins B, KNodes N, KStats st) {
+    using G = TileGeom<DIM>;
+    __shared__ int s_cs[G::NC + 1];
+    __shared__ double s_S[NW][4 * DIM + 4][WROW];       // per wave: [axis*4 + offset][corner], then mass and momentum over 64
+    __shared__ double s_acc[NW][NQ_MASS][WaveFoot<DIM>::SIZE];
+    const int w = threadIdx.x >> 6, l = threadIdx.x & 63, i = l / Corners<DIM>::N, c = l % Corners<DIM>::N;
+    auto tile = [&](const int tall) {      // (field, context tile) pair
+        const int tc = tall % g0.tilesTotal;
+        const GridPtr gp = tile_grid_ptr(g0, tc);
+        const KGrid g = grid_copy(gp);
+        load_tile_starts<DIM>(B, tall, s_cs);
+        if (s_cs[0] == s_cs[G::NC]) return;
+        int ox, oy, oz;
+        tile_origin<DIM>(g, tc - g.tileBase, ox, oy, oz);
+        WaveCells<DIM> W;
+        W.begin(s_cs);
+        WaveScatter<DIM, NQ_MASS, Corners<DIM>::N, WROW> sc;
+        sc.begin(&s_S[w][0][0], s_acc);
+        CornerMassWords<DIM> cur;
+        load_corner_mass<DIM>(P, B, W.b + i, W.e, cur);
+        zero_wave_acc<DIM, NQ_MASS>(s_acc);
+        for (int r = W.b; r < W.e; r += Corners<DIM>::PB) {
+            double xi[3], u[4];
+            int off[3];
+            bool ok = true;
+            if (cur.p >= 0) {
+                int lx, ly, lz;
+                tile_cell<DIM>(cur.key, tall, lx, ly, lz);
+                // InitializationTask -> GetCPDINodesAndWeights: semi-side vectors of the step (each
+                // corner's lane builds them; the first keeps them for the step's other passes)
+                double s[9];
+                cpdi_semi_sides_of<DIM>(g, P, cur.p, ox + lx, oy + ly, oz + lz, cur.ep, cur.wr, s);
+                ok = corner_lane<DIM>(gp, cur.x, s, ox + lx, oy + ly, oz + lz, c, xi, off);
+                if (c == 0) {
+#pragma unroll
+                    for (int a = 0; a < 9; a++) P.cpr(a)[cur.p] = s[a];
+                }
+                u[0] = Corners<DIM>::WW * cur.m;
+#pragma unroll
+                for (int a = 0; a < 3; a++) u[1 + a] = a < DIM ? u[0] * cur.v[a < DIM ? a : 0] : 0.;
+            }
+            // one count per particle with an unusable corner
+            const unsigned long long bad = __ballot(!ok);
+            if (c == 0 && ((bad >> l) & ((1ull << Corners<DIM>::N) - 1))) atomicAdd(st.cpdiErr, 1ull);
+            for (int r0 = r; r0 < min(r + Corners<DIM>::PB, W.e); r0 += WREC / Corners<DIM>::N) {
+                if (l / WREC == (r0 - r) / (WREC / Corners<DIM>::N) && cur.p >= 0) stage_corner<DIM, 4>(s_S[w], l % WREC, xi, off, u);
+                // the next particles' loads pass over the last scatter
+                if (r0 + WREC / Corners<DIM>::N >= min(r + Corners<DIM>::PB, W.e)) load_corner_mass<DIM>(P, B, r + Corners<DIM>::PB + i, W.e, cur);
+                wave_sync();
+                sc.scatter(W, r0, min(r0 + WREC / Corners<DIM>::N, W.e));
+                wave_sync();
+            }
+        }
+        sc.finish(W);
+        __syncthreads();
         write_partials<DIM, NQ_MASS>(N, tall, s_acc);
     };
     for_each_tile(B, tile);
@@ -947,7 +1386,7 @@ __device__ __forceinline__ void load_foot(const KGrid &g, int ox, int oy, int oz
 }
 
 // lCPDI gathers corner by corner. A node's merged weight and gradient are sums over the corners
-// whose element holds it (cpdi_table_node), so a gather over the merged node list is the same sum taken
+// whose element holds it, so a gather over the merged node list is the same sum taken
 // corner by corner: sum_n w(n) v(n) = ws sum_c sum_j cfn_c(j) v(n_cj) and
 // sum_n v(n) grad(n) = sum_c (sum_j cfn_c(j) v(n_cj)) wg_c, where j runs over the nodes of corner c's
 // element (cfn below 1e-15 left out, as in the reference's list). Each corner is built on the fly.
@@ -1004,41 +1443,16 @@ __device__ __forceinline__ void cpdi_corner_sum(const double xi[3], const int of
     }
 }
 
-// Support window of one particle: with a half size lp <= 1 (natural units) a particle with xi < 0
-// touches no node at offset 2 and one with xi >= 0 none at offset -1, so three offsets per axis
-// starting at w = 0 (offsets -1..1) or w = 1 (0..2) hold every node of its support. The window's
-// factors are stored with zeros for nodes outside the support, and derivatives times 2/dx.
-template <int DIM>
-__device__ __forceinline__ void support_window(const double xi[3], const double S[3][4], const double dS[3][4],
-                                               const double invd[3], int w[3], double Sw[3][3], double Dw[3][3]) {
-#pragma unroll
-    for (int a = 0; a < 3; a++) {
-        w[a] = a < DIM && xi[a] >= 0. ? 1 : 0;
-#pragma unroll
-        for (int j = 0; j < 3; j++) {
-            if (a >= DIM) { Sw[a][j] = j == 1 ? 1. : 0.; Dw[a][j] = 0.; continue; }
-            const double sv = w[a] ? S[a][j + 1] : S[a][j];
-            const double dv = w[a] ? dS[a][j + 1] : dS[a][j];
-            const bool in = sv >= 0.;
-            Sw[a][j] = in ? sv : 0.;
-            Dw[a][j] = in ? dv * invd[a] : 0.;
-        }
-    }
-}
-
 // velocity gradient of one particle from footprint velocities over its support window
 // (MatPoint3D::ExtrapVelocityGradient, MatPoint3D.cpp:62-94; MatPoint2D.cpp:57-89)
 template <int DIM>
-__device__ __forceinline__ void velocity_gradient(const double xi[3], const double S[3][4], const double dS[3][4],
-                                                  const double invd[3], int lx, int ly, int lz,
-                                                  const double (*s_v)[TileGeom<DIM>::FOOT], double L[3][3]) {
+__device__ __forceinline__ void velocity_gradient(const int w[3], const double Sw[3][3], const double Dw[3][3], int lx,
+                                                  int ly, int lz, const double (*s_v)[TileGeom<DIM>::FOOT],
+                                                  double L[3][3]) {
 #pragma unroll
     for (int a = 0; a < 3; a++)
 #pragma unroll
         for (int b = 0; b < 3; b++) L[a][b] = 0.;
-    int w[3];
-    double Sw[3][3], Dw[3][3];
-    support_window<DIM>(xi, S, dS, invd, w, Sw, Dw);
     constexpr int NZ = DIM == 3 ? 3 : 1;
 #pragma unroll 1
     for (int jz = 0; jz < NZ; jz++)
@@ -1071,7 +1485,7 @@ __device__ __forceinline__ void scale_gradient(double L[3][3], double f) {
 // velocity gradient of particle p from footprint velocities (lx,ly,lz = its cell in the tile):
 // the support window of its shape functions, or lCPDI nodes in list order
 template <int DIM, int SH>
-__device__ __forceinline__ void particle_gradient(const KGrid &g, const KPart &P, int p, int ei, int ej, int ek,
+__device__ __forceinline__ void particle_gradient(const KGrid &g, GridPtr gp, const KPart &P, int p, int ei, int ej, int ek,
                                                   int lx, int ly, int lz, const double (*s_v)[TileGeom<DIM>::FOOT],
                                                   double L[3][3]) {
     if (SH == MPMGPU_SHAPE_LCPDI) {
@@ -1081,8 +1495,8 @@ __device__ __forceinline__ void particle_gradient(const KGrid &g, const KPart &P
             for (int b = 0; b < 3; b++) L[a][b] = 0.;
         double r[9];
 #pragma unroll
-        for (int a = 0; a < 9; a++) r[a] = P.cpr[a][p];
-        const double pos[3] = {P.f[MPF_POS_X][p], P.f[MPF_POS_Y][p], DIM == 3 ? P.f[MPF_POS_Z][p] : 0.};
+        for (int a = 0; a < 9; a++) r[a] = P.cpr(a)[p];
+        const double pos[3] = {P.f(MPF_POS_X)[p], P.f(MPF_POS_Y)[p], DIM == 3 ? P.f(MPF_POS_Z)[p] : 0.};
         const double inv = cpdi_inv_measure<DIM>(r);
         constexpr int NCOR = DIM == 3 ? 8 : 4;
 #pragma unroll 1
@@ -1098,11 +1512,13 @@ __device__ __forceinline__ void particle_gradient(const KGrid &g, const KPart &P
                 for (int b = 0; b < DIM; b++) L[a][b] = fma(vc[a], w[b], L[a][b]);
         }
     } else {
-        double xi[3], invd[3], S[3][4], dS[3][4];
-        particle_xi<DIM>(g, ei, ej, ek, P.f[MPF_POS_X][p], P.f[MPF_POS_Y][p],
-                         DIM == 3 ? P.f[MPF_POS_Z][p] : 0., xi, invd);
-        particle_factors<DIM>(g, P, p, xi, S, dS);
-        velocity_gradient<DIM>(xi, S, dS, invd, lx, ly, lz, s_v, L);
+        const double pos[3] = {P.f(MPF_POS_X)[p], P.f(MPF_POS_Y)[p], DIM == 3 ? P.f(MPF_POS_Z)[p] : 0.};
+        AxisFactors f[DIM];
+        double invd[DIM], Sw[3][3], Dw[3][3];
+        int w[3];
+        particle_axes<DIM>(gp, P, p, ei, ej, ek, pos, f, invd);
+        particle_window<DIM>(f, invd, w, Sw, Dw);
+        velocity_gradient<DIM>(w, Sw, Dw, lx, ly, lz, s_v, L);
     }
 }
 
@@ -1115,15 +1531,16 @@ __device__ __forceinline__ bool alt_rows(int type, double h0) {
 }
 
 template <int DIM>
-__device__ __forceinline__ void load_state(const KPart &P, int p, int type, PState &s) {
-    s.ep[0] = P.f[MPF_EP_XX][p]; s.ep[1] = P.f[MPF_EP_YY][p]; s.ep[2] = P.f[MPF_EP_ZZ][p];
-    s.ep[5] = P.f[MPF_EP_XY][p]; s.wr[2] = P.f[MPF_WR_XY][p];
-    s.sp[0] = P.f[MPF_SP_XX][p]; s.sp[1] = P.f[MPF_SP_YY][p]; s.sp[2] = P.f[MPF_SP_ZZ][p];
-    s.sp[5] = P.f[MPF_SP_XY][p];
+__device__ __forceinline__ void load_state(const KPart &rows, int p, int type, PState &s) {
+    const KPart P = local_rows(rows);
+    s.ep[0] = P.f(MPF_EP_XX)[p]; s.ep[1] = P.f(MPF_EP_YY)[p]; s.ep[2] = P.f(MPF_EP_ZZ)[p];
+    s.ep[5] = P.f(MPF_EP_XY)[p]; s.wr[2] = P.f(MPF_WR_XY)[p];
+    s.sp[0] = P.f(MPF_SP_XX)[p]; s.sp[1] = P.f(MPF_SP_YY)[p]; s.sp[2] = P.f(MPF_SP_ZZ)[p];
+    s.sp[5] = P.f(MPF_SP_XY)[p];
     if (DIM == 3) {
-        s.ep[3] = P.f[MPF_EP_YZ][p]; s.ep[4] = P.f[MPF_EP_XZ][p];
-        s.wr[0] = P.f[MPF_WR_YZ][p]; s.wr[1] = P.f[MPF_WR_XZ][p];
-        s.sp[3] = P.f[MPF_SP_YZ][p]; s.sp[4] = P.f[MPF_SP_XZ][p];
+        s.ep[3] = P.f(MPF_EP_YZ)[p]; s.ep[4] = P.f(MPF_EP_XZ)[p];
+        s.wr[0] = P.f(MPF_WR_YZ)[p]; s.wr[1] = P.f(MPF_WR_XZ)[p];
+        s.sp[3] = P.f(MPF_SP_YZ)[p]; s.sp[4] = P.f(MPF_SP_XZ)[p];
     } else {
         s.ep[3] = s.ep[4] = 0.; s.wr[0] = s.wr[1] = 0.; s.sp[3] = s.sp[4] = 0.;
     }
@@ -1131,37 +1548,38 @@ __device__ __forceinline__ void load_state(const KPart &P, int p, int type, PSta
 #pragma unroll
     for (int c = 0; c < 6; c++) s.alt[c] = 0.;
     if (type != MPMGPU_MAT_ISOTROPIC) {
-        s.P = P.f[MPF_PRESSURE][p];
-        s.h0 = P.f[MPF_HIST0][p];
+        s.P = P.f(MPF_PRESSURE)[p];
+        s.h0 = P.f(MPF_HIST0)[p];
         if (alt_rows(type, s.h0)) {
-            s.alt[0] = P.f[MPF_ALT_XX][p]; s.alt[1] = P.f[MPF_ALT_YY][p]; s.alt[2] = P.f[MPF_ALT_ZZ][p];
-            s.alt[5] = P.f[MPF_ALT_XY][p];
-            if (DIM == 3) { s.alt[3] = P.f[MPF_ALT_YZ][p]; s.alt[4] = P.f[MPF_ALT_XZ][p]; }
+            s.alt[0] = P.f(MPF_ALT_XX)[p]; s.alt[1] = P.f(MPF_ALT_YY)[p]; s.alt[2] = P.f(MPF_ALT_ZZ)[p];
+            s.alt[5] = P.f(MPF_ALT_XY)[p];
+            if (DIM == 3) { s.alt[3] = P.f(MPF_ALT_YZ)[p]; s.alt[4] = P.f(MPF_ALT_XZ)[p]; }
         }
-        if (type == MPMGPU_MAT_NEOHOOKEAN || type == MPMGPU_MAT_MOONEY) s.h1 = P.f[MPF_HIST1][p];
+        if (type == MPMGPU_MAT_NEOHOOKEAN || type == MPMGPU_MAT_MOONEY) s.h1 = P.f(MPF_HIST1)[p];
     }
 }
 
 template <int DIM>
-__device__ __forceinline__ void store_state(const KPart &P, int p, int type, const PState &s) {
-    P.f[MPF_EP_XX][p] = s.ep[0]; P.f[MPF_EP_YY][p] = s.ep[1]; P.f[MPF_EP_ZZ][p] = s.ep[2];
-    P.f[MPF_EP_XY][p] = s.ep[5]; P.f[MPF_WR_XY][p] = s.wr[2];
-    P.f[MPF_SP_XX][p] = s.sp[0]; P.f[MPF_SP_YY][p] = s.sp[1]; P.f[MPF_SP_ZZ][p] = s.sp[2];
-    P.f[MPF_SP_XY][p] = s.sp[5];
+__device__ __forceinline__ void store_state(const KPart &rows, int p, int type, const PState &s) {
+    const KPart P = local_rows(rows);
+    P.f(MPF_EP_XX)[p] = s.ep[0]; P.f(MPF_EP_YY)[p] = s.ep[1]; P.f(MPF_EP_ZZ)[p] = s.ep[2];
+    P.f(MPF_EP_XY)[p] = s.ep[5]; P.f(MPF_WR_XY)[p] = s.wr[2];
+    P.f(MPF_SP_XX)[p] = s.sp[0]; P.f(MPF_SP_YY)[p] = s.sp[1]; P.f(MPF_SP_ZZ)[p] = s.sp[2];
+    P.f(MPF_SP_XY)[p] = s.sp[5];
     if (DIM == 3) {
-        P.f[MPF_EP_YZ][p] = s.ep[3]; P.f[MPF_EP_XZ][p] = s.ep[4];
-        P.f[MPF_WR_YZ][p] = s.wr[0]; P.f[MPF_WR_XZ][p] = s.wr[1];
-        P.f[MPF_SP_YZ][p] = s.sp[3]; P.f[MPF_SP_XZ][p] = s.sp[4];
+        P.f(MPF_EP_YZ)[p] = s.ep[3]; P.f(MPF_EP_XZ)[p] = s.ep[4];
+        P.f(MPF_WR_YZ)[p] = s.wr[0]; P.f(MPF_WR_XZ)[p] = s.wr[1];
+        P.f(MPF_SP_YZ)[p] = s.sp[3]; P.f(MPF_SP_XZ)[p] = s.sp[4];
     }
     if (type != MPMGPU_MAT_ISOTROPIC) {
-        P.f[MPF_PRESSURE][p] = s.P;
+        P.f(MPF_PRESSURE)[p] = s.P;
         if (alt_rows(type, s.h0)) {
-            P.f[MPF_ALT_XX][p] = s.alt[0]; P.f[MPF_ALT_YY][p] = s.alt[1]; P.f[MPF_ALT_ZZ][p] = s.alt[2];
-            P.f[MPF_ALT_XY][p] = s.alt[5];
-            if (DIM == 3) { P.f[MPF_ALT_YZ][p] = s.alt[3]; P.f[MPF_ALT_XZ][p] = s.alt[4]; }
-            P.f[MPF_HIST0][p] = s.h0;
+            P.f(MPF_ALT_XX)[p] = s.alt[0]; P.f(MPF_ALT_YY)[p] = s.alt[1]; P.f(MPF_ALT_ZZ)[p] = s.alt[2];
+            P.f(MPF_ALT_XY)[p] = s.alt[5];
+            if (DIM == 3) { P.f(MPF_ALT_YZ)[p] = s.alt[3]; P.f(MPF_ALT_XZ)[p] = s.alt[4]; }
+            P.f(MPF_HIST0)[p] = s.h0;
         }
-        if (type == MPMGPU_MAT_NEOHOOKEAN || type == MPMGPU_MAT_MOONEY) P.f[MPF_HIST1][p] = s.h1;
+        if (type == MPMGPU_MAT_NEOHOOKEAN || type == MPMGPU_MAT_MOONEY) P.f(MPF_HIST1)[p] = s.h1;
     }
 }
 
@@ -1177,7 +1595,8 @@ __global__ __launch_bounds__(NT, 2) void k_usf(KGrid g0, KPart P, KBins B, KNode
     auto tile = [&](const int tall) {      // (field, context tile) pair
         if (only >= 0 && g0.tileType[tall % g0.tilesTotal] != only) return;   // another launch's type
         const int fld = tall / g0.tilesTotal;
-        const KGrid g = tile_grid(g0, tall - fld * g0.tilesTotal);
+        const GridPtr gp = tile_grid_ptr(g0, tall - fld * g0.tilesTotal);
+        const KGrid g = grid_copy(gp);
         const int t = tall - fld * g0.tilesTotal - g.tileBase;
         const KNodes Nf = field_view(g, N, fld);
         load_tile_starts<DIM>(B, tall, s_cs);
@@ -1193,10 +1612,10 @@ __global__ __launch_bounds__(NT, 2) void k_usf(KGrid g0, KPart P, KBins B, KNode
         __syncthreads();
         for (int k = tb + threadIdx.x; k < te; k += NT) {
             int p = B.order[k];
-            int ei, ej, ek;
-            elem_ijk(g, P.elem[p], ei, ej, ek);
+            int lx, ly, lz;
+            tile_cell<DIM>(B.key[p], tall, lx, ly, lz);
             double L[3][3];
-            particle_gradient<DIM, SH>(g, P, p, ei, ej, ek, ei - ox, ej - oy, DIM == 3 ? ek - oz : 0, s_v, L);
+            particle_gradient<DIM, SH>(g, gp, P, p, ox + lx, oy + ly, oz + lz, lx, ly, lz, s_v, L);
             scale_gradient<DIM>(L, g.strainFirst);
             const MpmMaterial &m = mats[P.mat[p]];
             const int mtype = MAT ? MAT : m.type;
@@ -1212,195 +1631,219 @@ __global__ __launch_bounds__(NT, 2) void k_usf(KGrid g0, KPart P, KBins B, KNode
 // internal-force scatter (GridForcesTask::Execute, GridForcesTask.cpp:40-153 ->
 // MatPoint3D::GetFintPlusFext, MatPoint3D.cpp:248-270; MatPoint2D.cpp:242-263) with the stress
 // just updated by k_usf; FX adds N * pFext of the loaded particles (pFext is zero otherwise)
-template <int DIM, int SH, bool FX>
-__global__ __launch_bounds__(NT) void k_p2g_force(KGrid g0, KPart P, KBins B, KNodes N, KLoads L,
-                                                  const int *loaded) {
+
+// uGIMP and classic: stages -mp times the stress terms (xx, yy, xy, zz, xz, yz of sigma - P; 2D: three)
+// and the factor pairs of one particle at record i of its wave's rows
+template <int DIM>
+__device__ __forceinline__ void stage_force(double2 (*F)[WROW], double (*A)[WROW], int i, const AxisFactors f[DIM],
+                                            const double invd[DIM], const double s[6]) {
+#pragma unroll
+    for (int a = 0; a < DIM; a++) {
+        AxisFactors t = f[a];
+        asm volatile("" : "+v"(t.w));          // formed here, not held from before the rounds (48 registers)
+#pragma unroll
+        for (int o = 0; o < 4; o++) F[a * 4 + o][i] = make_double2(t.s4(o), t.d4(o) * invd[a]);
+    }
+#pragma unroll
+    for (int c = 0; c < (DIM == 3 ? 6 : 3); c++) A[c][i] = s[c];
+}
+
+// lane (q, iz, ix) of a scatter adds the traction tables of a cell's staged particles to its nodes
+__device__ __forceinline__ void add_tractions(const KLoads &L, const int *tt, int kb, int ke, int q, int iz, int ix,
+                                              mat4d &c) {
+    if (q > 2) return;
+    for (int s = kb; s < ke; s++) {
+        if (tt[s] < 0) continue;
+        const double *tab = L.ttab + (size_t)(3 * tt[s] + q) * TRAC_NODES + iz * 16 + ix;
+#pragma unroll
+        for (int r = 0; r < 4; r++) c[r] += tab[r * 4];
+    }
+}
+
+// 2D: lane (q, iy, ix)
+__device__ __forceinline__ void add_tractions(const KLoads &L, const int *tt, int kb, int ke, int q, int iy, int ix,
+                                              double &c) {
+    if (q > 1) return;
+    for (int s = kb; s < ke; s++)
+        if (tt[s] >= 0) c += L.ttab[(size_t)(3 * tt[s] + q) * TRAC_NODES + iy * 4 + ix];
+}
+
+template <int DIM> struct ForceWords { int p, key; double x[DIM], m, pr, s[6]; };
+
+template <int DIM>
+__device__ __forceinline__ void load_force_words(const KPart &rows, const KBins &B, int k, int e, ForceWords<DIM> &t) {
+    const KPart P = local_rows(rows);
+    t.p = k < e ? B.order[k] : -1;
+    if (t.p < 0) return;
+    t.key = B.key[t.p];
+#pragma unroll
+    for (int a = 0; a < DIM; a++) t.x[a] = P.f(MPF_POS_X + a)[t.p];
+    t.m = P.f(MPF_MASS)[t.p];
+    t.pr = P.f(MPF_PRESSURE)[t.p];         // stays 0 for small-strain elastic particles
+    t.s[0] = P.f(MPF_SP_XX)[t.p]; t.s[1] = P.f(MPF_SP_YY)[t.p]; t.s[2] = P.f(MPF_SP_XY)[t.p];
+    if (DIM == 3) { t.s[3] = P.f(MPF_SP_ZZ)[t.p]; t.s[4] = P.f(MPF_SP_XZ)[t.p]; t.s[5] = P.f(MPF_SP_YZ)[t.p]; }
+}
+
+template <int DIM, bool FX>
+__global__ __launch_bounds__(NT, FX ? 2 : G2P_WAVES) void k_p2g_force(KGrid g0, KPart P, KBins B, KNodes N, KLoads L,
+                                                                       const int *loaded) {
     using G = TileGeom<DIM>;
-    constexpr bool CP = SH == MPMGPU_SHAPE_LCPDI;
-    constexpr int NCOR = DIM == 3 ? 8 : 4;
-    constexpr int CH = CP ? NT / NCOR : NT / 2;   // particles staged per chunk (lCPDI: a thread per corner)
-    constexpr int NA = DIM == 3 ? 6 : 3;      // -mp times the stress terms (shape-function path)
     __shared__ int s_cs[G::NC + 1];
-    // shape-function path: per axis and candidate offset, the factor and its derivative times
-    // 2/dx (zero outside the support), read as one pair
-    __shared__ double2 s_F[CP ? 1 : CH][DIM][4];
-    __shared__ double s_a[CP ? 1 : CH][NA];
-    __shared__ double s_ct[CP ? CH : 1][NCOR][DIM][4];
-    __shared__ double s_cwg[CP ? CH : 1][NCOR][3];
-    __shared__ double s_st[CP ? CH : 1][NA];
-    __shared__ double s_e[FX ? CH : 1][3];    // pFext of the staged particles
-    __shared__ int s_tt[FX ? CH : 1];         // their traction tables (-1: none)
+    __shared__ double2 s_F[NW][4 * DIM][WROW]; // per wave: [axis*4 + offset][record] (factor, derivative)
+    __shared__ double s_a[NW][6][WROW];
+    __shared__ double s_e[FX ? NW : 1][3][WROW];   // pFext of the staged particles
+    __shared__ int s_tt[FX ? NW : 1][WREC];        // their traction tables (-1: none)
     __shared__ double s_acc[NW][NQ_FORCE][WaveFoot<DIM>::SIZE];
-    using R1 = std::conditional_t<FX, RecForceX, RecForce>;
-    using R2 = std::conditional_t<FX, RecForce2X, RecForce2>;
-    // MatPtLoadBC's pFext of particle p (0 when it carries no load) and its traction table
-    auto stage_fext = [&](int slot, int p) {
-        const int q = L.map[B.home[p]];
-#pragma unroll
-        for (int c = 0; c < 3; c++) s_e[slot][c] = q >= 0 ? L.fext[3 * q + c] : 0.;
-        s_tt[slot] = q >= 0 && L.nt > 0 ? L.tslot[q] : -1;
-    };
-    // the staged particle's traction force at candidate node (ix, iy, iz) (zero without tractions)
-    auto trac = [&](int lq, int ix, int iy, int iz, double t[3]) {
-        const int tt = s_tt[lq];
-        const int o = DIM == 3 ? (iz * 4 + iy) * 4 + ix : iy * 4 + ix;
-        const double *tab = L.ttab + (size_t)3 * (tt < 0 ? 0 : tt) * TRAC_NODES + o;
-#pragma unroll
-        for (int c = 0; c < 3; c++) t[c] = tt >= 0 && c < DIM ? tab[c * TRAC_NODES] : 0.;
-    };
+    const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
     auto tile = [&](const int tall) {      // (field, context tile) pair
         // with loads: the launch with the load term takes the marked tiles, the other the rest
         if (loaded && (loaded[tall] != 0) != FX) return;
-        const int fld = tall / g0.tilesTotal;
-        const KGrid g = tile_grid(g0, tall - fld * g0.tilesTotal);
+        const int tc = tall % g0.tilesTotal;
+        const GridPtr gp = tile_grid_ptr(g0, tc);
+        const KGrid g = grid_copy(gp);
         load_tile_starts<DIM>(B, tall, s_cs);
-        const int tb = s_cs[0], te = s_cs[G::NC];
-        if (tb == te) return;
-        zero_acc<DIM, NQ_FORCE>(s_acc);
-        for (int c0 = tb; c0 < te; c0 += CH) {
-            if (CP) {
-                // thread (i, c): corner c of staged particle i; the first corner's thread stages the stress
-                const int i = threadIdx.x / NCOR, c = threadIdx.x % NCOR;
-                const int k = c0 + i;
-                if (k < te) {
-                    const int p = B.order[k];
-                    int ei, ej, ek;
-                    elem_ijk(g, P.elem[p], ei, ej, ek);
-                    double r[9];
-#pragma unroll
-                    for (int a = 0; a < 9; a++) r[a] = P.cpr[a][p];
-                    double pos[3] = {P.f[MPF_POS_X][p], P.f[MPF_POS_Y][p], DIM == 3 ? P.f[MPF_POS_Z][p] : 0.};
-                    double xi[3], w[3];
-                    int off[3];
-                    cpdi_corner<DIM>(g, pos, r, ei, ej, ek, c, xi, off);
-                    cpdi_table<DIM>(xi, off, s_ct[i][c]);
-                    cpdi_wg_staged<DIM>(r, c, w);
-                    s_cwg[i][c][0] = w[0]; s_cwg[i][c][1] = w[1]; s_cwg[i][c][2] = w[2];
-                    if (c == 0) {
-                        if constexpr (FX) stage_fext(i, p);
-                        const double Pr = P.f[MPF_PRESSURE][p];
-                        const double negmp = -P.f[MPF_MASS][p];
-                        s_st[i][0] = negmp * (P.f[MPF_SP_XX][p] - Pr);
-                        s_st[i][1] = negmp * (P.f[MPF_SP_YY][p] - Pr);
-                        s_st[i][2] = negmp * P.f[MPF_SP_XY][p];
-                        if constexpr (DIM == 3) {
-                            s_st[i][3] = negmp * (P.f[MPF_SP_ZZ][p] - Pr);
-                            s_st[i][4] = negmp * P.f[MPF_SP_XZ][p];
-                            s_st[i][5] = negmp * P.f[MPF_SP_YZ][p];
-                        }
-                    }
+        if (s_cs[0] == s_cs[G::NC]) return;
+        int ox, oy, oz;
+        tile_origin<DIM>(g, tc - g.tileBase, ox, oy, oz);
+        WaveCells<DIM> W;
+        W.begin(s_cs);
+        WaveForce<DIM, FX, WROW> sc;
+        sc.begin(&s_F[w][0][0], &s_a[w][0][0], &s_e[FX ? w : 0][0][0], s_acc);
+        // tractions: lane (q, iz, ix), in 2D (q, iy, ix), adds the tables of the cell's particles to its nodes
+        auto trac = [&](int kb, int ke, int q, int hi, int ix, auto &c) {
+            if (L.nt == 0) return;
+            add_tractions(L, s_tt[FX ? w : 0], kb, ke, q, hi, ix, c);
+        };
+        zero_wave_acc<DIM, NQ_FORCE>(s_acc);
+        for (int r = W.b; r < W.e; r += 64) {
+            ForceWords<DIM> cur;        // (loading them a round ahead costs the registers of the third wave per SIMD)
+            load_force_words<DIM>(P, B, r + l, W.e, cur);
+            AxisFactors f[DIM];
+            double invd[DIM], s[6];
+            if (cur.p >= 0) {
+                int lx, ly, lz;
+                tile_cell<DIM>(cur.key, tall, lx, ly, lz);
+                particle_axes<DIM>(gp, P, cur.p, ox + lx, oy + ly, oz + lz, cur.x, f, invd);
+                s[0] = -cur.m * (cur.s[0] - cur.pr);
+                s[1] = -cur.m * (cur.s[1] - cur.pr);
+                s[2] = -cur.m * cur.s[2];
+                if (DIM == 3) {
+                    s[3] = -cur.m * (cur.s[3] - cur.pr);
+                    s[4] = -cur.m * cur.s[4];
+                    s[5] = -cur.m * cur.s[5];
                 }
             }
-            int k = c0 + threadIdx.x;
-            if (!CP && threadIdx.x < CH && k < te) {
-                int p = B.order[k];
-                int ei, ej, ek;
-                elem_ijk(g, P.elem[p], ei, ej, ek);
-                double Pr = P.f[MPF_PRESSURE][p];      // stays 0 for small-strain elastic particles
-                const double negmp = -P.f[MPF_MASS][p];
-                const double sxx = P.f[MPF_SP_XX][p] - Pr, syy = P.f[MPF_SP_YY][p] - Pr, sxy = P.f[MPF_SP_XY][p];
-                {
-                    double xi[3], invd[3], S[3][4], dS[3][4];
-                    particle_xi<DIM>(g, ei, ej, ek, P.f[MPF_POS_X][p], P.f[MPF_POS_Y][p],
-                                     DIM == 3 ? P.f[MPF_POS_Z][p] : 0., xi, invd);
-                    particle_factors<DIM>(g, P, p, xi, S, dS);
-#pragma unroll
-                    for (int a = 0; a < DIM; a++)
-#pragma unroll
-                        for (int o = 0; o < 4; o++) {
-                            const bool in = S[a][o] >= 0.;
-                            s_F[threadIdx.x][a][o] = make_double2(in ? S[a][o] : 0., in ? dS[a][o] * invd[a] : 0.);
-                        }
-                    if constexpr (FX) stage_fext(threadIdx.x, p);
-                    s_a[threadIdx.x][0] = negmp * sxx;
-                    s_a[threadIdx.x][1] = negmp * syy;
-                    s_a[threadIdx.x][2] = negmp * sxy;
-                    if (DIM == 3) {
-                        s_a[threadIdx.x][3] = negmp * (P.f[MPF_SP_ZZ][p] - Pr);
-                        s_a[threadIdx.x][4] = negmp * P.f[MPF_SP_XZ][p];
-                        s_a[threadIdx.x][5] = negmp * P.f[MPF_SP_YZ][p];
-                    }
-                }
-            }
-            __syncthreads();
-            if (!CP) {
-                // f = -mp (sigma - P) . grad N; grad N from the staged factor pairs, accumulated with FMA
-                wave_cells<DIM, NQ_FORCE>(s_cs, c0, min(c0 + CH, te), s_acc,
-                    [&](int lq, int ix, int iy, int iz) {
-                        R2 r;
-                        r.x = s_F[lq][0][ix];
-                        r.y = s_F[lq][1][iy];
-                        r.z = DIM == 3 ? s_F[lq][DIM - 1][iz] : make_double2(1., 0.);
-#pragma unroll
-                        for (int q = 0; q < NA; q++) r.a[q] = s_a[lq][q];
-                        if constexpr (FX) {
-                            r.e[0] = s_e[lq][0]; r.e[1] = s_e[lq][1]; r.e[2] = s_e[lq][2];
-                            trac(lq, ix, iy, iz, r.t);
-                        }
-                        return r;
-                    },
-                    [&](const R2 &r, double *acc, int, int, int) {
-                        if constexpr (FX) {
-                            // + N pFext, N the product of the axis factors, + the traction force
-                            const double w = DIM == 3 ? r.x.x * (r.y.x * r.z.x) : r.x.x * r.y.x;
-                            acc[0] = fma(r.e[0], w, acc[0]) + r.t[0];
-                            acc[1] = fma(r.e[1], w, acc[1]) + r.t[1];
-                            if (DIM == 3) acc[2] = fma(r.e[2], w, acc[2]) + r.t[2];
-                        }
-                        if (DIM == 3) {
-                            const double gx = r.x.y * (r.y.x * r.z.x);
-                            const double gy = r.y.y * (r.x.x * r.z.x);
-                            const double gz = r.z.y * (r.x.x * r.y.x);
-                            // a: xx, yy, xy, zz, xz, yz
-                            acc[0] = fma(r.a[0], gx, fma(r.a[2], gy, fma(r.a[4], gz, acc[0])));
-                            acc[1] = fma(r.a[2], gx, fma(r.a[1], gy, fma(r.a[5], gz, acc[1])));
-                            acc[2] = fma(r.a[4], gx, fma(r.a[5], gy, fma(r.a[3], gz, acc[2])));
-                        } else {
-                            const double gx = r.x.y * r.y.x;
-                            const double gy = r.y.y * r.x.x;
-                            acc[0] = fma(r.a[0], gx, fma(r.a[2], gy, acc[0]));
-                            acc[1] = fma(r.a[2], gx, fma(r.a[1], gy, acc[1]));
-                        }
-                    });
-                __syncthreads();
-                continue;
-            }
-            wave_cells<DIM, NQ_FORCE>(s_cs, c0, min(c0 + CH, te), s_acc,
-                [&](int lq, int ix, int iy, int iz) {
-                    R1 r;
-                    {
-                        double gr[3];
-                        cpdi_table_node<DIM, true>(s_ct[lq], s_cwg[lq], ix, iy, iz, r.wx, gr);
-                        r.wy = r.wz = 1.;
-                        r.dx = gr[0]; r.dy = gr[1]; r.dz = gr[2];
-                    }
-                    r.s0 = s_st[lq][0]; r.s1 = s_st[lq][1]; r.s2 = s_st[lq][2];
-                    if constexpr (DIM == 3) { r.s3 = s_st[lq][3]; r.s4 = s_st[lq][4]; r.s5 = s_st[lq][5]; }
-                    else { r.s3 = r.s4 = r.s5 = 0.; }
+            for (int r0 = r; r0 < min(r + 64, W.e); r0 += WREC) {
+                if (l / WREC == (r0 - r) / WREC && cur.p >= 0) {
+                    stage_force<DIM>(s_F[w], s_a[w], l % WREC, f, invd, s);
                     if constexpr (FX) {
-                        r.e[0] = s_e[lq][0]; r.e[1] = s_e[lq][1]; r.e[2] = s_e[lq][2];
-                        trac(lq, ix, iy, iz, r.t);
+                        // MatPtLoadBC's pFext of the particle (0 when it carries no load) and its traction table
+                        const int q = L.map[B.home[cur.p]];
+#pragma unroll
+                        for (int c = 0; c < 3; c++) s_e[w][c][l % WREC] = q >= 0 ? L.fext[3 * q + c] : 0.;
+                        s_tt[w][l % WREC] = q >= 0 && L.nt > 0 ? L.tslot[q] : -1;
                     }
-                    return r;
-                },
-                [&](const R1 &r, double *acc, int, int, int) {
-                    if constexpr (FX) {              // + N pFext, N the merged corner weight, + traction
-                        acc[0] = fma(r.e[0], r.wx, acc[0]) + r.t[0];
-                        acc[1] = fma(r.e[1], r.wx, acc[1]) + r.t[1];
-                        if (DIM == 3) acc[2] = fma(r.e[2], r.wx, acc[2]) + r.t[2];
-                    }
-                    // s: -mp times xx, yy, xy, zz, xz, yz of sigma - P; non-member nodes have zero gradient
-                    if (DIM == 3) {
-                        acc[0] = fma(r.s0, r.dx, fma(r.s2, r.dy, fma(r.s4, r.dz, acc[0])));
-                        acc[1] = fma(r.s2, r.dx, fma(r.s1, r.dy, fma(r.s5, r.dz, acc[1])));
-                        acc[2] = fma(r.s4, r.dx, fma(r.s5, r.dy, fma(r.s3, r.dz, acc[2])));
-                    } else {
-                        acc[0] = fma(r.s0, r.dx, fma(r.s2, r.dy, acc[0]));
-                        acc[1] = fma(r.s2, r.dx, fma(r.s1, r.dy, acc[1]));
-                    }
-                });
-            __syncthreads();
+                }
+                wave_sync();
+                sc.scatter(W, r0, min(r0 + WREC, W.e), trac);
+                wave_sync();
+            }
         }
+        sc.finish(W);
+        __syncthreads();
+        write_partials<DIM, NQ_FORCE>(N, tall, s_acc);
+    };
+    for_each_tile(B, tile);
+}
+
+// lCPDI: a corner's payload is the force -mp (sigma - P) . its gradient weight (+ pFext)
+template <int DIM> struct CornerForceWords { int p, key; double x[DIM], m, pr, s[6], r[9]; };
+
+template <int DIM>
+__device__ __forceinline__ void load_corner_force(const KPart &rows, const KBins &B, int k, int e, CornerForceWords<DIM> &t) {
+    const KPart P = local_rows(rows);
+    t.p = k < e ? B.order[k] : -1;
+    if (t.p < 0) return;
+    t.key = B.key[t.p];
+#pragma unroll
+    for (int a = 0; a < DIM; a++) t.x[a] = P.f(MPF_POS_X + a)[t.p];
+#pragma unroll
+    for (int a = 0; a < 9; a++) t.r[a] = DIM == 3 || (a < 6 && a % 3 < 2) ? P.cpr(a)[t.p] : 0.;
+    t.m = P.f(MPF_MASS)[t.p];
+    t.pr = P.f(MPF_PRESSURE)[t.p];
+    t.s[0] = P.f(MPF_SP_XX)[t.p]; t.s[1] = P.f(MPF_SP_YY)[t.p]; t.s[2] = P.f(MPF_SP_XY)[t.p];
+    if (DIM == 3) { t.s[3] = P.f(MPF_SP_ZZ)[t.p]; t.s[4] = P.f(MPF_SP_XZ)[t.p]; t.s[5] = P.f(MPF_SP_YZ)[t.p]; }
+}
+
+template <int DIM, bool FX>
+__global__ __launch_bounds__(NT, FX ? 2 : G2P_WAVES) void k_p2g_force_corners(KGrid g0, KPart P, KBins B, KNodes N, KLoads L,
+                                                                        const int *loaded) {
+    using G = TileGeom<DIM>;
+    __shared__ int s_cs[G::NC + 1];
+    __shared__ double s_S[NW][4 * DIM + 4][WROW];
+    __shared__ int s_tt[FX ? NW : 1][WREC / Corners<DIM>::N];    // traction tables of the staged particles (-1: none)
+    __shared__ double s_acc[NW][NQ_FORCE][WaveFoot<DIM>::SIZE];
+    const int w = threadIdx.x >> 6, l = threadIdx.x & 63, i = l / Corners<DIM>::N, c = l % Corners<DIM>::N;
+    auto tile = [&](const int tall) {      // (field, context tile) pair
+        if (loaded && (loaded[tall] != 0) != FX) return;
+        const int tc = tall % g0.tilesTotal;
+        const GridPtr gp = tile_grid_ptr(g0, tc);
+        const KGrid g = grid_copy(gp);
+        load_tile_starts<DIM>(B, tall, s_cs);
+        if (s_cs[0] == s_cs[G::NC]) return;
+        int ox, oy, oz;
+        tile_origin<DIM>(g, tc - g.tileBase, ox, oy, oz);
+        WaveCells<DIM> W;
+        W.begin(s_cs);
+        WaveScatter<DIM, NQ_FORCE, Corners<DIM>::N, WROW> sc;
+        sc.begin(&s_S[w][0][0], s_acc);
+        auto trac = [&](int kb, int ke, int q, int hi, int ix, auto &f) {
+            if (!FX || L.nt == 0) return;
+            add_tractions(L, s_tt[FX ? w : 0], kb, ke, q, hi, ix, f);
+        };
+        zero_wave_acc<DIM, NQ_FORCE>(s_acc);
+        CornerForceWords<DIM> cur;
+        load_corner_force<DIM>(P, B, W.b + i, W.e, cur);
+        for (int r = W.b; r < W.e; r += Corners<DIM>::PB) {
+            double xi[3], u[3];
+            int off[3], tt = -1;
+            if (cur.p >= 0) {
+                int lx, ly, lz;
+                tile_cell<DIM>(cur.key, tall, lx, ly, lz);
+                corner_lane<DIM>(gp, cur.x, cur.r, ox + lx, oy + ly, oz + lz, c, xi, off);
+                double wg[3];
+                cpdi_wg_staged<DIM>(cur.r, c, wg);
+                const double xx = -cur.m * (cur.s[0] - cur.pr), yy = -cur.m * (cur.s[1] - cur.pr), xy = -cur.m * cur.s[2];
+                if constexpr (DIM == 3) {
+                    const double zz = -cur.m * (cur.s[3] - cur.pr), xz = -cur.m * cur.s[4], yz = -cur.m * cur.s[5];
+                    u[0] = fma(xx, wg[0], fma(xy, wg[1], xz * wg[2]));
+                    u[1] = fma(xy, wg[0], fma(yy, wg[1], yz * wg[2]));
+                    u[2] = fma(xz, wg[0], fma(yz, wg[1], zz * wg[2]));
+                } else {
+                    u[0] = fma(xx, wg[0], xy * wg[1]);
+                    u[1] = fma(xy, wg[0], yy * wg[1]);
+                    u[2] = 0.;
+                }
+                if constexpr (FX) {
+                    const int q = L.map[B.home[cur.p]];
+#pragma unroll
+                    for (int a = 0; a < 3; a++) u[a] = q >= 0 ? fma(Corners<DIM>::WW, L.fext[3 * q + a], u[a]) : u[a];
+                    tt = q >= 0 && L.nt > 0 ? L.tslot[q] : -1;
+                }
+            }
+            for (int r0 = r; r0 < min(r + Corners<DIM>::PB, W.e); r0 += WREC / Corners<DIM>::N) {
+                if (l / WREC == (r0 - r) / (WREC / Corners<DIM>::N) && cur.p >= 0) {
+                    stage_corner<DIM, 3>(s_S[w], l % WREC, xi, off, u);
+                    if (FX && c == 0) s_tt[FX ? w : 0][i % (WREC / Corners<DIM>::N)] = tt;
+                }
+                if (r0 + WREC / Corners<DIM>::N >= min(r + Corners<DIM>::PB, W.e)) load_corner_force<DIM>(P, B, r + Corners<DIM>::PB + i, W.e, cur);
+                wave_sync();
+                sc.scatter(W, r0, min(r0 + WREC / Corners<DIM>::N, W.e), trac);
+                wave_sync();
+            }
+        }
+        sc.finish(W);
+        __syncthreads();
         write_partials<DIM, NQ_FORCE>(N, tall, s_acc);
     };
     for_each_tile(B, tile);
@@ -1447,6 +1890,106 @@ __global__ void k_node_force(KGrid g0, KBins B, KNodes N) {
 }
 
 // ---------------------------------------------------------------------------------------
+// sums of NV footprint rows over a particle's support window
+template <int DIM, int NV>
+__device__ __forceinline__ void gather_window(const int w[3], const double Sw[3][3], int lx, int ly, int lz,
+                                              const double (*s_n)[TileGeom<DIM>::FOOT], double out[NV]) {
+#pragma unroll
+    for (int v = 0; v < NV; v++) out[v] = 0.;
+    constexpr int NZ = DIM == 3 ? 3 : 1;
+#pragma unroll
+    for (int jz = 0; jz < NZ; jz++) {
+#pragma unroll
+        for (int jy = 0; jy < 3; jy++)
+#pragma unroll
+            for (int jx = 0; jx < 3; jx++) {
+                const double fi = DIM == 3 ? Sw[0][jx] * (Sw[1][jy] * Sw[2][jz]) : Sw[0][jx] * Sw[1][jy];
+                const int s = foot_slot<DIM>(lx + w[0] + jx - 1, ly + w[1] + jy - 1, DIM == 3 ? lz + w[2] + jz - 1 : 0);
+#pragma unroll
+                for (int v = 0; v < NV; v++) out[v] = fma(s_n[v][s], fi, out[v]);
+            }
+        __builtin_amdgcn_sched_barrier(0);     // a plane's reads at a time: all 27 nodes' would not fit in registers
+    }
+    // the sums are formed here, not put off past a branch that follows (with the words held meanwhile)
+#pragma unroll
+    for (int v = 0; v < NV; v++) asm volatile("" : "+v"(out[v]));
+}
+
+// footprint velocities and accelerations f/m (zero outside the grid and on nodes without mass, which
+// no particle of the tile touches)
+template <int DIM>
+__device__ __forceinline__ void load_foot_va(const KGrid &g, const KNodes &Nf, int ox, int oy, int oz,
+                                             double (*s_n)[TileGeom<DIM>::FOOT]) {
+    const long long nn = g.nstride;
+    for (int s = threadIdx.x; s < TileGeom<DIM>::FOOT; s += NT) {
+        const long long n = foot_node<DIM>(g, s, ox, oy, oz);
+        const double m = n >= 0 ? Nf.mass[n] : 0.;
+        const double r = m > 0. ? 1. / m : 0.;
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+            s_n[c][s] = n >= 0 ? Nf.vk[c * nn + n] : 0.;
+            s_n[3 + c][s] = n >= 0 ? Nf.ftot[c * nn + n] * r : 0.;
+        }
+    }
+}
+
+// the same as (velocity, acceleration) pairs, one 16-byte LDS read each (the gather's reads kept the
+// LDS busy for almost half of the kernel's time)
+template <int DIM>
+__device__ __forceinline__ void load_foot_pairs(const KGrid &g, const KNodes &Nf, int ox, int oy, int oz,
+                                                double2 (*s_n)[TileGeom<DIM>::FOOT]) {
+    const long long nn = g.nstride;
+    for (int s = threadIdx.x; s < TileGeom<DIM>::FOOT; s += NT) {
+        const long long n = foot_node<DIM>(g, s, ox, oy, oz);
+        const double m = n >= 0 ? Nf.mass[n] : 0.;
+        const double r = m > 0. ? 1. / m : 0.;
+#pragma unroll
+        for (int c = 0; c < 3; c++)
+            s_n[c][s] = n >= 0 ? make_double2(Nf.vk[c * nn + n], Nf.ftot[c * nn + n] * r) : make_double2(0., 0.);
+    }
+}
+
+template <int DIM>
+__device__ __forceinline__ void gather_pairs(const int w[3], const double Sw[3][3], int lx, int ly, int lz,
+                                             const double2 (*s_n)[TileGeom<DIM>::FOOT], double v[3], double a[3]) {
+#pragma unroll
+    for (int c = 0; c < 3; c++) v[c] = a[c] = 0.;
+    constexpr int NZ = DIM == 3 ? 3 : 1;
+#pragma unroll
+    for (int jz = 0; jz < NZ; jz++) {
+#pragma unroll
+        for (int jy = 0; jy < 3; jy++)
+#pragma unroll
+            for (int jx = 0; jx < 3; jx++) {
+                const double fi = DIM == 3 ? Sw[0][jx] * (Sw[1][jy] * Sw[2][jz]) : Sw[0][jx] * Sw[1][jy];
+                const int s = foot_slot<DIM>(lx + w[0] + jx - 1, ly + w[1] + jy - 1, DIM == 3 ? lz + w[2] + jz - 1 : 0);
+#pragma unroll
+                for (int c = 0; c < DIM; c++) {
+                    const double2 t = s_n[c][s];
+                    v[c] = fma(t.x, fi, v[c]);
+                    a[c] = fma(t.y, fi, a[c]);
+                }
+            }
+        __builtin_amdgcn_sched_barrier(0);     // a plane's reads at a time: all 27 nodes' would not fit in registers
+    }
+    // the sums are formed here, not put off past a branch that follows (with the words held meanwhile)
+#pragma unroll
+    for (int c = 0; c < 3; c++) asm volatile("" : "+v"(v[c]), "+v"(a[c]));
+}
+
+// footprint XPIC increments (zero outside the grid and on nodes without particles)
+template <int DIM>
+__device__ __forceinline__ void load_foot_prev(const KGrid &g, const KNodes &Nf, int ox, int oy, int oz,
+                                               double (*s_n)[TileGeom<DIM>::FOOT]) {
+    const long long nn = g.nstride;
+    for (int s = threadIdx.x; s < TileGeom<DIM>::FOOT; s += NT) {
+        const long long n = foot_node<DIM>(g, s, ox, oy, oz);
+        const bool on = n >= 0 && Nf.cnt[n] > 0;
+#pragma unroll
+        for (int c = 0; c < 3; c++) s_n[c][s] = on ? Nf.vprev[c * nn + n] : 0.;
+    }
+}
+
 // Particle update (FLIP, no damping) fused with the momentum re-extrapolation of the USL pass
 // with start-of-step shape functions (MatVelocityField::IncrementNodalVelAcc,
 // MatVelocityField.cpp:410-426; MatPoint3D::MoveParticle, MatPoint3D.cpp:104-194;
@@ -1455,206 +1998,204 @@ __global__ void k_node_force(KGrid g0, KBins B, KNodes N) {
 // mode > 0 and by XPIC(-mode) for mode < 0 with the damping of the grid (zero damping gives the
 // same numbers as none). The FLIP instances keep their registers for the common update.
 enum { G2P_FLIP = 0, G2P_FLIP_DAMPED = 1, G2P_SERIES = 2 };
-template <int DIM, int SH, int MOVE>
-__global__ __launch_bounds__(NT, SH == MPMGPU_SHAPE_LCPDI ? 1 : G2P_WAVES) void k_g2p_p2g(KGrid g0, KPart P, KBins B, KNodes N,
-                                                                                  const MpmMaterial *mats, int mode) {
+template <int DIM, int MOVE>
+__device__ __forceinline__ void move_particle(const KGrid &g, const KPart &P, const MpmMaterial *mats, int mode, int p,
+                                              const double pos[3], const double vold[3], const double Svk[3],
+                                              const double Sacc[3], double vnew[3], double xnew[3]) {
     constexpr bool DAMP = MOVE != G2P_FLIP;
+    const double dt = g.timestep;
+    // particle damping: the material's own <PDamping> in place of the run's
+    // (MaterialBase::GetMaterialDamping, MaterialBaseMPM.cpp:742-744)
+    double alphaP = 0.;
+    if (DAMP) {
+        const MpmMaterial &mt = mats[P.mat[p]];
+        alphaP = mt.usePDamping ? mt.pdamping : g.particleDamping;
+    }
+    // MatPoint3D::MoveParticle (MatPoint3D.cpp:104-194): Adamp0 = alpha_p v + alpha_g vm
+    // (the DAMP instance; zero damping gives delV = Sacc dt for FLIP)
+    if (MOVE != G2P_SERIES) {
+        // FLIP: vm = S(v - a dt), v += (Sa - Adamp0) dt, x += (vm + delV/2) dt (:104-160)
+#pragma unroll
+        for (int c = 0; c < DIM; c++) {
+            double vm = Svk[c] - Sacc[c] * dt;
+            double delV = DAMP ? (Sacc[c] - (vold[c] * alphaP + vm * g.gridDamping)) * dt
+                               : Sacc[c] * dt;
+            vnew[c] = vold[c] + delV;
+            double delXRate = vm + 0.5 * delV;
+            xnew[c] = pos[c] + delXRate * dt;
+        }
+    } else {
+        // FMPM(k) (mode k): vm = S v+(k), v = vm - Adamp0 dt, x += (v(n) + v(n+1)) dt/2
+        // (:122-137); XPIC(k) (mode -k): vm = S(v(k) + a dt), v = vm - Adamp0 dt,
+        // x += (vm + delV/2) dt (:152-170)
+#pragma unroll
+        for (int c = 0; c < DIM; c++) {
+            const double vm = Svk[c];
+            const double adamp = DAMP ? vold[c] * alphaP + vm * g.gridDamping : 0.;
+            if (mode > 0) {
+                vnew[c] = vm + adamp * -dt;
+                const double delXRate = vold[c] + vnew[c];
+                xnew[c] = pos[c] + delXRate * (0.5 * dt);
+            } else {
+                vnew[c] = vm - adamp * dt;
+                const double delV = vnew[c] - vold[c];
+                const double delXRate = vm + 0.5 * delV;
+                xnew[c] = pos[c] + delXRate * dt;
+            }
+        }
+    }
+}
+
+template <int DIM>
+__device__ __forceinline__ void store_move(const KPart &rows, int p, const double vnew[3], const double xnew[3]) {
+    const KPart P = local_rows(rows);
+#pragma unroll
+    for (int c = 0; c < DIM; c++) {
+        P.f(MPF_VEL_X + c)[p] = vnew[c];
+        P.posn(c)[p] = xnew[c];
+    }
+}
+
+// uGIMP and classic: a wave gathers, moves and scatters its particles 64 at a time
+template <int DIM, int MOVE>
+__global__ __launch_bounds__(NT, G2P_WAVES) void k_g2p_p2g(KGrid g0, KPart P, KBins B, KNodes N, const MpmMaterial *mats,
+                                                            int mode) {
     using G = TileGeom<DIM>;
-    constexpr bool CP = SH == MPMGPU_SHAPE_LCPDI;
-    constexpr int NCOR = DIM == 3 ? 8 : 4;
-    // particles per scatter round: half the block, or (lCPDI) as many as the corner tables hold
-    constexpr int SUB = CP ? NT / NCOR : NT / 2;
     __shared__ int s_cs[G::NC + 1];
-    __shared__ double s_n[6][G::FOOT];         // v(3), f/m(3)
-    __shared__ double s_S[CP ? 1 : DIM * 4][SUB + 1];   // [axis*4 + offset][particle]
-    __shared__ double s_ct[CP ? SUB : 1][NCOR][DIM][4];
-    __shared__ double s_q[4][SUB + 1];
+    __shared__ double2 s_n[3][G::FOOT];        // (velocity, f/m) of each component
+    __shared__ double s_S[NW][4 * DIM + 4][WROW];       // [axis*4 + offset][record], then the momentum (the last row is not used)
     __shared__ double s_acc[NW][NQ_MOM][WaveFoot<DIM>::SIZE];
+    const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
     auto tile = [&](const int tall) {      // (field, context tile) pair
         const int fld = tall / g0.tilesTotal;
-        const KGrid g = tile_grid(g0, tall - fld * g0.tilesTotal);
-        const int t = tall - fld * g0.tilesTotal - g.tileBase;
+        const int tc = tall - fld * g0.tilesTotal;
+        const GridPtr gp = tile_grid_ptr(g0, tc);
+        const KGrid g = grid_copy(gp);
         const KNodes Nf = field_view(g, N, fld);
         load_tile_starts<DIM>(B, tall, s_cs);
-        const int tb = s_cs[0], te = s_cs[G::NC];
-        if (tb == te) return;
+        if (s_cs[0] == s_cs[G::NC]) return;
         int ox, oy, oz;
-        tile_origin<DIM>(g, t, ox, oy, oz);
-        {
-            // footprint velocities and accelerations f/m (zero outside the grid and on nodes without
-            // mass, which no particle of the tile touches)
-            const long long nn = g.nstride;
-            for (int s = threadIdx.x; s < G::FOOT; s += NT) {
-                const long long n = foot_node<DIM>(g, s, ox, oy, oz);
-                const double m = n >= 0 ? Nf.mass[n] : 0.;
-                const double r = m > 0. ? 1. / m : 0.;
-#pragma unroll
-                for (int c = 0; c < 3; c++) {
-                    s_n[c][s] = n >= 0 ? Nf.vk[c * nn + n] : 0.;
-                    s_n[3 + c][s] = n >= 0 ? Nf.ftot[c * nn + n] * r : 0.;
-                }
-            }
-        }
-        zero_acc<DIM, NQ_MOM>(s_acc);
+        tile_origin<DIM>(g, tc - g.tileBase, ox, oy, oz);
+        WaveCells<DIM> W;
+        W.begin(s_cs);
+        WaveScatter<DIM, NQ_MOM, 1, WROW> sc;
+        sc.begin(&s_S[w][0][0], s_acc);
+        MassWords<DIM> cur;
+        load_mass_words<DIM>(P, B, W.b + l, W.e, cur);
+        load_foot_pairs<DIM>(g, Nf, ox, oy, oz, s_n);
+        zero_wave_acc<DIM, NQ_MOM>(s_acc);
         __syncthreads();
-        const double dt = g.timestep;
-        for (int c0 = tb; c0 < te; c0 += NT) {
-            const int c1 = min(c0 + NT, te);
-            const int k = c0 + threadIdx.x;
-            double S[3][4], q4[4];
-            CpdiCorners cc;
-            if (k < c1) {
-                int p = B.order[k];
-                // every word of the particle is loaded before anything is stored, so the loads are
-                // issued together (a later load could not move above a store to another row)
-                const int e0 = P.elem[p];
-                double pos[3] = {P.f[MPF_POS_X][p], P.f[MPF_POS_Y][p], DIM == 3 ? P.f[MPF_POS_Z][p] : 0.};
-                double vold[3] = {P.f[MPF_VEL_X][p], P.f[MPF_VEL_Y][p], DIM == 3 ? P.f[MPF_VEL_Z][p] : 0.};
-                const double mp = P.f[MPF_MASS][p];
-                int ei, ej, ek;
-                elem_ijk(g, e0, ei, ej, ek);
-                int lx = ei - ox, ly = ej - oy, lz = DIM == 3 ? ek - oz : 0;
-                double Svk[3] = {0., 0., 0.}, Sacc[3] = {0., 0., 0.};
-                if (CP) {
-                    cpdi_particle<DIM>(g, P, p, ei, ej, ek, cc);
-                    constexpr int NCOR = DIM == 3 ? 8 : 4;
-                    constexpr double ws = DIM == 3 ? 0.125 : 0.25;
-                    double sum[6] = {0., 0., 0., 0., 0., 0.};
-#pragma unroll
-                    for (int c = 0; c < NCOR; c++) {
-                        double vc[6];
-                        cpdi_corner_sum<DIM, 6>(cc.xi[c], cc.off[c], lx, ly, lz, s_n, vc);
-#pragma unroll
-                        for (int v = 0; v < 6; v++) sum[v] += vc[v];
-                    }
-#pragma unroll
-                    for (int a = 0; a < 3; a++) { Svk[a] = ws * sum[a]; Sacc[a] = ws * sum[3 + a]; }
-                } else {
-                double xi[3], invd[3], dS[3][4];
-                particle_xi<DIM>(g, ei, ej, ek, pos[0], pos[1], pos[2], xi, invd);
-                particle_factors<DIM>(g, P, p, xi, S, dS);
-                int w[3];
-                double Sw[3][3], Dw[3][3];
-                support_window<DIM>(xi, S, dS, invd, w, Sw, Dw);
-                constexpr int NZ = DIM == 3 ? 3 : 1;
-#pragma unroll
-                for (int jz = 0; jz < NZ; jz++)
-#pragma unroll
-                    for (int jy = 0; jy < 3; jy++)
-#pragma unroll
-                        for (int jx = 0; jx < 3; jx++) {
-                            const double fi = DIM == 3 ? Sw[0][jx] * (Sw[1][jy] * Sw[2][jz]) : Sw[0][jx] * Sw[1][jy];
-                            const int s = foot_slot<DIM>(lx + w[0] + jx - 1, ly + w[1] + jy - 1,
-                                                         DIM == 3 ? lz + w[2] + jz - 1 : 0);
-                            Svk[0] = fma(s_n[0][s], fi, Svk[0]);
-                            Svk[1] = fma(s_n[1][s], fi, Svk[1]);
-                            Svk[2] = fma(s_n[2][s], fi, Svk[2]);
-                            Sacc[0] = fma(s_n[3][s], fi, Sacc[0]);
-                            Sacc[1] = fma(s_n[4][s], fi, Sacc[1]);
-                            Sacc[2] = fma(s_n[5][s], fi, Sacc[2]);
-                        }
+        for (int r = W.b; r < W.e; r += 64) {
+            AxisFactors f[DIM];
+            double u[3];
+            if (cur.p >= 0) {
+                int lx, ly, lz;
+                tile_cell<DIM>(cur.key, tall, lx, ly, lz);
+                int wd[3];
+                double invd[DIM], Svk[3], Sacc[3], vnew[3], xnew[3];
+                {
+                    double Sw[3][3], Dw[3][3];
+                    particle_axes<DIM>(gp, P, cur.p, ox + lx, oy + ly, oz + lz, cur.x, f, invd);
+                    particle_window<DIM>(f, invd, wd, Sw, Dw);
+                    gather_pairs<DIM>(wd, Sw, lx, ly, lz, s_n, Svk, Sacc);
                 }
-                double vnew[3] = {0., 0., 0.};
-                // particle damping: the material's own <PDamping> in place of the run's
-                // (MaterialBase::GetMaterialDamping, MaterialBaseMPM.cpp:742-744)
-                double alphaP = 0.;
-                if (DAMP) {
-                    const MpmMaterial &mt = mats[P.mat[p]];
-                    alphaP = mt.usePDamping ? mt.pdamping : g.particleDamping;
-                }
-                // MatPoint3D::MoveParticle (MatPoint3D.cpp:104-194): Adamp0 = alpha_p v + alpha_g vm
-                // (the DAMP instance; zero damping gives delV = Sacc dt for FLIP)
-                if (MOVE != G2P_SERIES) {
-                    // FLIP: vm = S(v - a dt), v += (Sa - Adamp0) dt, x += (vm + delV/2) dt (:104-160)
+                move_particle<DIM, MOVE>(g, P, mats, mode, cur.p, cur.x, cur.v, Svk, Sacc, vnew, xnew);
+                store_move<DIM>(P, cur.p, vnew, xnew);
 #pragma unroll
-                    for (int c = 0; c < DIM; c++) {
-                        double vm = Svk[c] - Sacc[c] * dt;
-                        double delV = DAMP ? (Sacc[c] - (vold[c] * alphaP + vm * g.gridDamping)) * dt
-                                           : Sacc[c] * dt;
-                        vnew[c] = vold[c] + delV;
-                        P.f[MPF_VEL_X + c][p] = vnew[c];
-                        double delXRate = vm + 0.5 * delV;
-                        P.posn[c][p] = pos[c] + delXRate * dt;
-                    }
-                } else {
-                    // FMPM(k) (mode k): vm = S v+(k), v = vm - Adamp0 dt, x += (v(n) + v(n+1)) dt/2
-                    // (:122-137); XPIC(k) (mode -k): vm = S(v(k) + a dt), v = vm - Adamp0 dt,
-                    // x += (vm + delV/2) dt (:152-170)
-#pragma unroll
-                    for (int c = 0; c < DIM; c++) {
-                        const double vm = Svk[c];
-                        const double adamp = DAMP ? vold[c] * alphaP + vm * g.gridDamping : 0.;
-                        if (mode > 0) {
-                            vnew[c] = vm + adamp * -dt;
-                            const double delXRate = vold[c] + vnew[c];
-                            P.posn[c][p] = pos[c] + delXRate * (0.5 * dt);
-                        } else {
-                            vnew[c] = vm - adamp * dt;
-                            const double delV = vnew[c] - vold[c];
-                            const double delXRate = vm + 0.5 * delV;
-                            P.posn[c][p] = pos[c] + delXRate * dt;
-                        }
-                        P.f[MPF_VEL_X + c][p] = vnew[c];
-                    }
-                }
-                q4[0] = mp;
-                q4[1] = vnew[0]; q4[2] = vnew[1]; q4[3] = vnew[2];
+                for (int c = 0; c < 3; c++) u[c] = c < DIM ? cur.m * vnew[c] : 0.;
             }
-            for (int h = 0; h < NT / SUB; h++) {
-                const int r0 = c0 + h * SUB, r1 = min(r0 + SUB, c1);
-                if (r0 >= r1) break;
-                if ((int)(threadIdx.x / SUB) == h && k < c1) {
-                    const int i = threadIdx.x - h * SUB;
-                    if (CP) {
-                        // the tables are built here, at the thread's turn (an empty asm makes the corner
-                        // coordinates opaque, so the compiler cannot build them once before the rounds
-                        // and hold all of them in registers)
-#pragma unroll
-                        for (int c = 0; c < NCOR; c++) {
-                            double xo[3];
-#pragma unroll
-                            for (int a = 0; a < 3; a++) {
-                                xo[a] = cc.xi[c][a];
-                                asm volatile("" : "+v"(xo[a]));
-                            }
-                            cpdi_table<DIM>(xo, cc.off[c], s_ct[i][c]);
-                        }
-                    } else {
-                        // factors with zeros outside the support; the x factor carries mp
-#pragma unroll
-                        for (int a = 0; a < DIM; a++)
-#pragma unroll
-                            for (int o = 0; o < 4; o++) {
-                                const double v = S[a][o] >= 0. ? S[a][o] : 0.;
-                                s_S[a * 4 + o][i] = a == 0 ? v * q4[0] : v;
-                            }
-                    }
-#pragma unroll
-                    for (int q = 0; q < 4; q++) s_q[q][i] = q4[q];
-                }
-                __syncthreads();
-                wave_cells<DIM, NQ_MOM>(s_cs, r0, r1, s_acc,
-                    [&](int lq, int ix, int iy, int iz) {
-                        RecMass r;
-                        if (CP) {
-                            double gr[3];
-                            cpdi_table_node<DIM, false>(s_ct[lq], nullptr, ix, iy, iz, r.wx, gr);
-                            r.wy = 1.; r.wz = 1.;
-                        } else {
-                            r.wx = s_S[ix][lq]; r.wy = s_S[4 + iy][lq]; r.wz = DIM == 3 ? s_S[(DIM - 1) * 4 + iz][lq] : 1.;
-                        }
-                        r.mp = s_q[0][lq]; r.vx = s_q[1][lq]; r.vy = s_q[2][lq]; r.vz = s_q[3][lq];
-                        return r;
-                    },
-                    [&](const RecMass &r, double *acc, int, int, int) {
-                        const double fnmp = CP ? r.wx * r.mp : (DIM == 3 ? r.wx * (r.wy * r.wz) : r.wx * r.wy);
-                        acc[0] = fma(r.vx, fnmp, acc[0]);
-                        acc[1] = fma(r.vy, fnmp, acc[1]);
-                        acc[2] = fma(r.vz, fnmp, acc[2]);
-                    });
-                __syncthreads();
+            for (int r0 = r; r0 < min(r + 64, W.e); r0 += WREC) {
+                if (l / WREC == (r0 - r) / WREC && cur.p >= 0) stage_factors<DIM, 3>(s_S[w], l % WREC, f, u);
+                // the next particles' loads pass over the last scatter
+                if (r0 + WREC >= min(r + 64, W.e)) load_mass_words<DIM>(P, B, r + 64 + l, W.e, cur);
+                wave_sync();
+                sc.scatter(W, r0, min(r0 + WREC, W.e));
+                wave_sync();
             }
         }
+        sc.finish(W);
+        __syncthreads();
+        write_partials<DIM, NQ_MOM>(N, tall, s_acc);
+    };
+    for_each_tile(B, tile);
+}
+
+// lCPDI: the gather is taken corner by corner, a lane each, and added over the particle's lanes
+template <int DIM> struct CornerMoveWords { int p, key; double x[DIM], m, v[DIM], r[9]; };
+
+template <int DIM>
+__device__ __forceinline__ void load_corner_move(const KPart &rows, const KBins &B, int k, int e, CornerMoveWords<DIM> &t) {
+    const KPart P = local_rows(rows);
+    t.p = k < e ? B.order[k] : -1;
+    if (t.p < 0) return;
+    t.key = B.key[t.p];
+#pragma unroll
+    for (int a = 0; a < DIM; a++) {
+        t.x[a] = P.f(MPF_POS_X + a)[t.p];
+        t.v[a] = P.f(MPF_VEL_X + a)[t.p];
+    }
+#pragma unroll
+    for (int a = 0; a < 9; a++) t.r[a] = DIM == 3 || (a < 6 && a % 3 < 2) ? P.cpr(a)[t.p] : 0.;
+    t.m = P.f(MPF_MASS)[t.p];
+}
+
+template <int DIM, int MOVE>
+__global__ __launch_bounds__(NT, G2P_WAVES) void k_g2p_p2g_corners(KGrid g0, KPart P, KBins B, KNodes N,
+                                                             const MpmMaterial *mats, int mode) {
+    using G = TileGeom<DIM>;
+    __shared__ int s_cs[G::NC + 1];
+    __shared__ double s_n[6][G::FOOT];         // v(3), f/m(3)
+    __shared__ double s_S[NW][4 * DIM + 4][WROW];
+    __shared__ double s_acc[NW][NQ_MOM][WaveFoot<DIM>::SIZE];
+    const int w = threadIdx.x >> 6, l = threadIdx.x & 63, i = l / Corners<DIM>::N, c = l % Corners<DIM>::N;
+    auto tile = [&](const int tall) {      // (field, context tile) pair
+        const int fld = tall / g0.tilesTotal;
+        const int tc = tall - fld * g0.tilesTotal;
+        const GridPtr gp = tile_grid_ptr(g0, tc);
+        const KGrid g = grid_copy(gp);
+        const KNodes Nf = field_view(g, N, fld);
+        load_tile_starts<DIM>(B, tall, s_cs);
+        if (s_cs[0] == s_cs[G::NC]) return;
+        int ox, oy, oz;
+        tile_origin<DIM>(g, tc - g.tileBase, ox, oy, oz);
+        WaveCells<DIM> W;
+        W.begin(s_cs);
+        WaveScatter<DIM, NQ_MOM, Corners<DIM>::N, WROW> sc;
+        sc.begin(&s_S[w][0][0], s_acc);
+        CornerMoveWords<DIM> cur;
+        load_corner_move<DIM>(P, B, W.b + i, W.e, cur);
+        load_foot_va<DIM>(g, Nf, ox, oy, oz, s_n);
+        zero_wave_acc<DIM, NQ_MOM>(s_acc);
+        __syncthreads();
+        for (int r = W.b; r < W.e; r += Corners<DIM>::PB) {
+            double xi[3], u[3];
+            int off[3];
+            if (cur.p >= 0) {
+                int lx, ly, lz;
+                tile_cell<DIM>(cur.key, tall, lx, ly, lz);
+                corner_lane<DIM>(gp, cur.x, cur.r, ox + lx, oy + ly, oz + lz, c, xi, off);
+                double vc[6], Svk[3], Sacc[3], vnew[3], xnew[3];
+                cpdi_corner_sum<DIM, 6>(xi, off, lx, ly, lz, s_n, vc);
+#pragma unroll
+                for (int a = 0; a < 3; a++) {
+                    Svk[a] = Corners<DIM>::W * corner_sum<DIM>(vc[a]);
+                    Sacc[a] = Corners<DIM>::W * corner_sum<DIM>(vc[3 + a]);
+                }
+                move_particle<DIM, MOVE>(g, P, mats, mode, cur.p, cur.x, cur.v, Svk, Sacc, vnew, xnew);
+                if (c == 0) store_move<DIM>(P, cur.p, vnew, xnew);
+#pragma unroll
+                for (int a = 0; a < 3; a++) u[a] = a < DIM ? Corners<DIM>::WW * cur.m * vnew[a] : 0.;
+            }
+            for (int r0 = r; r0 < min(r + Corners<DIM>::PB, W.e); r0 += WREC / Corners<DIM>::N) {
+                if (l / WREC == (r0 - r) / (WREC / Corners<DIM>::N) && cur.p >= 0) stage_corner<DIM, 3>(s_S[w], l % WREC, xi, off, u);
+                if (r0 + WREC / Corners<DIM>::N >= min(r + Corners<DIM>::PB, W.e)) load_corner_move<DIM>(P, B, r + Corners<DIM>::PB + i, W.e, cur);
+                wave_sync();
+                sc.scatter(W, r0, min(r0 + WREC / Corners<DIM>::N, W.e));
+                wave_sync();
+            }
+        }
+        sc.finish(W);
+        __syncthreads();
         write_partials<DIM, NQ_MOM>(N, tall, s_acc);
     };
     for_each_tile(B, tile);
@@ -1733,143 +2274,113 @@ __global__ void k_xpic_init(KGrid g0, KBins B, KNodes N, int fmpm) {
 // node i gains sum_p mp S_ip (sum_j S_jp vprev_j), the particle's gather of the last increment
 // scattered as a momentum; the node pass divides by m_i. Shape functions are those of the step's
 // start, as in every pass of the step.
-template <int DIM, int SH>
-__global__ __launch_bounds__(NT, SH == MPMGPU_SHAPE_LCPDI ? 1 : G2P_WAVES) void k_xpic_p2g(KGrid g0, KPart P, KBins B, KNodes N) {
+// uGIMP and classic: a wave gathers and scatters its particles 64 at a time
+template <int DIM>
+__global__ __launch_bounds__(NT, G2P_WAVES) void k_xpic_p2g(KGrid g0, KPart P, KBins B, KNodes N) {
     using G = TileGeom<DIM>;
-    constexpr bool CP = SH == MPMGPU_SHAPE_LCPDI;
-    constexpr int NCOR = DIM == 3 ? 8 : 4;
-    constexpr int SUB = CP ? NT / NCOR : NT / 2;
     __shared__ int s_cs[G::NC + 1];
     __shared__ double s_n[3][G::FOOT];         // vprev
-    __shared__ double s_S[CP ? 1 : DIM * 4][SUB + 1];
-    __shared__ double s_ct[CP ? SUB : 1][NCOR][DIM][4];
-    __shared__ double s_q[4][SUB + 1];
+    __shared__ double s_S[NW][4 * DIM + 4][WROW];       // [axis*4 + offset][record], then the momentum (the last row is not used)
     __shared__ double s_acc[NW][NQ_MOM][WaveFoot<DIM>::SIZE];
-    auto tile = [&](const int tall) {
+    const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
+    auto tile = [&](const int tall) {      // (field, context tile) pair
         const int fld = tall / g0.tilesTotal;
-        const KGrid g = tile_grid(g0, tall - fld * g0.tilesTotal);
-        const int t = tall - fld * g0.tilesTotal - g.tileBase;
+        const int tc = tall - fld * g0.tilesTotal;
+        const GridPtr gp = tile_grid_ptr(g0, tc);
+        const KGrid g = grid_copy(gp);
         const KNodes Nf = field_view(g, N, fld);
         load_tile_starts<DIM>(B, tall, s_cs);
-        const int tb = s_cs[0], te = s_cs[G::NC];
-        if (tb == te) return;
+        if (s_cs[0] == s_cs[G::NC]) return;
         int ox, oy, oz;
-        tile_origin<DIM>(g, t, ox, oy, oz);
-        {
-            // footprint increments (zero outside the grid and on nodes without particles)
-            const long long nn = g.nstride;
-            for (int s = threadIdx.x; s < G::FOOT; s += NT) {
-                const long long n = foot_node<DIM>(g, s, ox, oy, oz);
-                const bool on = n >= 0 && Nf.cnt[n] > 0;
-#pragma unroll
-                for (int c = 0; c < 3; c++) s_n[c][s] = on ? Nf.vprev[c * nn + n] : 0.;
-            }
-        }
-        zero_acc<DIM, NQ_MOM>(s_acc);
+        tile_origin<DIM>(g, tc - g.tileBase, ox, oy, oz);
+        WaveCells<DIM> W;
+        W.begin(s_cs);
+        WaveScatter<DIM, NQ_MOM, 1, WROW> sc;
+        sc.begin(&s_S[w][0][0], s_acc);
+        MassWords<DIM> cur;
+        load_mass_words<DIM>(P, B, W.b + l, W.e, cur);
+        load_foot_prev<DIM>(g, Nf, ox, oy, oz, s_n);
+        zero_wave_acc<DIM, NQ_MOM>(s_acc);
         __syncthreads();
-        for (int c0 = tb; c0 < te; c0 += NT) {
-            const int c1 = min(c0 + NT, te);
-            const int k = c0 + threadIdx.x;
-            double S[3][4], q4[4];
-            CpdiCorners cc;
-            if (k < c1) {
-                const int p = B.order[k];
-                const int e0 = P.elem[p];
-                const double pos[3] = {P.f[MPF_POS_X][p], P.f[MPF_POS_Y][p], DIM == 3 ? P.f[MPF_POS_Z][p] : 0.};
-                const double mp = P.f[MPF_MASS][p];
-                int ei, ej, ek;
-                elem_ijk(g, e0, ei, ej, ek);
-                const int lx = ei - ox, ly = ej - oy, lz = DIM == 3 ? ek - oz : 0;
-                double u[3] = {0., 0., 0.};
-                if (CP) {
-                    cpdi_particle<DIM>(g, P, p, ei, ej, ek, cc);
-                    constexpr double ws = DIM == 3 ? 0.125 : 0.25;
-                    double sum[3] = {0., 0., 0.};
+        for (int r = W.b; r < W.e; r += 64) {
+            AxisFactors f[DIM];
+            double u[3];
+            if (cur.p >= 0) {
+                int lx, ly, lz;
+                tile_cell<DIM>(cur.key, tall, lx, ly, lz);
+                int wd[3];
+                double invd[DIM], Sw[3][3], Dw[3][3], v[3];
+                particle_axes<DIM>(gp, P, cur.p, ox + lx, oy + ly, oz + lz, cur.x, f, invd);
+                particle_window<DIM>(f, invd, wd, Sw, Dw);
+                gather_window<DIM, 3>(wd, Sw, lx, ly, lz, s_n, v);
 #pragma unroll
-                    for (int c = 0; c < NCOR; c++) {
-                        double vc[3];
-                        cpdi_corner_sum<DIM, 3>(cc.xi[c], cc.off[c], lx, ly, lz, s_n, vc);
-#pragma unroll
-                        for (int v = 0; v < 3; v++) sum[v] += vc[v];
-                    }
-#pragma unroll
-                    for (int a = 0; a < 3; a++) u[a] = ws * sum[a];
-                } else {
-                    double xi[3], invd[3], dS[3][4];
-                    particle_xi<DIM>(g, ei, ej, ek, pos[0], pos[1], pos[2], xi, invd);
-                    particle_factors<DIM>(g, P, p, xi, S, dS);
-                    int w[3];
-                    double Sw[3][3], Dw[3][3];
-                    support_window<DIM>(xi, S, dS, invd, w, Sw, Dw);
-                    constexpr int NZ = DIM == 3 ? 3 : 1;
-#pragma unroll
-                    for (int jz = 0; jz < NZ; jz++)
-#pragma unroll
-                        for (int jy = 0; jy < 3; jy++)
-#pragma unroll
-                            for (int jx = 0; jx < 3; jx++) {
-                                const double fi = DIM == 3 ? Sw[0][jx] * (Sw[1][jy] * Sw[2][jz]) : Sw[0][jx] * Sw[1][jy];
-                                const int s = foot_slot<DIM>(lx + w[0] + jx - 1, ly + w[1] + jy - 1,
-                                                             DIM == 3 ? lz + w[2] + jz - 1 : 0);
-                                u[0] = fma(s_n[0][s], fi, u[0]);
-                                u[1] = fma(s_n[1][s], fi, u[1]);
-                                u[2] = fma(s_n[2][s], fi, u[2]);
-                            }
-                }
-                q4[0] = mp;
-                q4[1] = u[0]; q4[2] = u[1]; q4[3] = u[2];
+                for (int c = 0; c < 3; c++) u[c] = c < DIM ? cur.m * v[c] : 0.;
             }
-            for (int h = 0; h < NT / SUB; h++) {
-                const int r0 = c0 + h * SUB, r1 = min(r0 + SUB, c1);
-                if (r0 >= r1) break;
-                if ((int)(threadIdx.x / SUB) == h && k < c1) {
-                    const int i = threadIdx.x - h * SUB;
-                    if (CP) {
-#pragma unroll
-                        for (int c = 0; c < NCOR; c++) {
-                            double xo[3];
-#pragma unroll
-                            for (int a = 0; a < 3; a++) {
-                                xo[a] = cc.xi[c][a];
-                                asm volatile("" : "+v"(xo[a]));
-                            }
-                            cpdi_table<DIM>(xo, cc.off[c], s_ct[i][c]);
-                        }
-                    } else {
-#pragma unroll
-                        for (int a = 0; a < DIM; a++)
-#pragma unroll
-                            for (int o = 0; o < 4; o++) {
-                                const double v = S[a][o] >= 0. ? S[a][o] : 0.;
-                                s_S[a * 4 + o][i] = a == 0 ? v * q4[0] : v;
-                            }
-                    }
-#pragma unroll
-                    for (int q = 0; q < 4; q++) s_q[q][i] = q4[q];
-                }
-                __syncthreads();
-                wave_cells<DIM, NQ_MOM>(s_cs, r0, r1, s_acc,
-                    [&](int lq, int ix, int iy, int iz) {
-                        RecMass r;
-                        if (CP) {
-                            double gr[3];
-                            cpdi_table_node<DIM, false>(s_ct[lq], nullptr, ix, iy, iz, r.wx, gr);
-                            r.wy = 1.; r.wz = 1.;
-                        } else {
-                            r.wx = s_S[ix][lq]; r.wy = s_S[4 + iy][lq]; r.wz = DIM == 3 ? s_S[(DIM - 1) * 4 + iz][lq] : 1.;
-                        }
-                        r.mp = s_q[0][lq]; r.vx = s_q[1][lq]; r.vy = s_q[2][lq]; r.vz = s_q[3][lq];
-                        return r;
-                    },
-                    [&](const RecMass &r, double *acc, int, int, int) {
-                        const double fnmp = CP ? r.wx * r.mp : (DIM == 3 ? r.wx * (r.wy * r.wz) : r.wx * r.wy);
-                        acc[0] = fma(r.vx, fnmp, acc[0]);
-                        acc[1] = fma(r.vy, fnmp, acc[1]);
-                        acc[2] = fma(r.vz, fnmp, acc[2]);
-                    });
-                __syncthreads();
+            for (int r0 = r; r0 < min(r + 64, W.e); r0 += WREC) {
+                if (l / WREC == (r0 - r) / WREC && cur.p >= 0) stage_factors<DIM, 3>(s_S[w], l % WREC, f, u);
+                // the next particles' loads pass over the last scatter
+                if (r0 + WREC >= min(r + 64, W.e)) load_mass_words<DIM>(P, B, r + 64 + l, W.e, cur);
+                wave_sync();
+                sc.scatter(W, r0, min(r0 + WREC, W.e));
+                wave_sync();
             }
         }
+        sc.finish(W);
+        __syncthreads();
+        write_partials<DIM, NQ_MOM>(N, tall, s_acc);
+    };
+    for_each_tile(B, tile);
+}
+
+template <int DIM>
+__global__ __launch_bounds__(NT, G2P_WAVES) void k_xpic_p2g_corners(KGrid g0, KPart P, KBins B, KNodes N) {
+    using G = TileGeom<DIM>;
+    __shared__ int s_cs[G::NC + 1];
+    __shared__ double s_n[3][G::FOOT];         // vprev
+    __shared__ double s_S[NW][4 * DIM + 4][WROW];
+    __shared__ double s_acc[NW][NQ_MOM][WaveFoot<DIM>::SIZE];
+    const int w = threadIdx.x >> 6, l = threadIdx.x & 63, i = l / Corners<DIM>::N, c = l % Corners<DIM>::N;
+    auto tile = [&](const int tall) {      // (field, context tile) pair
+        const int fld = tall / g0.tilesTotal;
+        const int tc = tall - fld * g0.tilesTotal;
+        const GridPtr gp = tile_grid_ptr(g0, tc);
+        const KGrid g = grid_copy(gp);
+        const KNodes Nf = field_view(g, N, fld);
+        load_tile_starts<DIM>(B, tall, s_cs);
+        if (s_cs[0] == s_cs[G::NC]) return;
+        int ox, oy, oz;
+        tile_origin<DIM>(g, tc - g.tileBase, ox, oy, oz);
+        WaveCells<DIM> W;
+        W.begin(s_cs);
+        WaveScatter<DIM, NQ_MOM, Corners<DIM>::N, WROW> sc;
+        sc.begin(&s_S[w][0][0], s_acc);
+        CornerMoveWords<DIM> cur;
+        load_corner_move<DIM>(P, B, W.b + i, W.e, cur);
+        load_foot_prev<DIM>(g, Nf, ox, oy, oz, s_n);
+        zero_wave_acc<DIM, NQ_MOM>(s_acc);
+        __syncthreads();
+        for (int r = W.b; r < W.e; r += Corners<DIM>::PB) {
+            double xi[3], u[3];
+            int off[3];
+            if (cur.p >= 0) {
+                int lx, ly, lz;
+                tile_cell<DIM>(cur.key, tall, lx, ly, lz);
+                corner_lane<DIM>(gp, cur.x, cur.r, ox + lx, oy + ly, oz + lz, c, xi, off);
+                double vc[3];
+                cpdi_corner_sum<DIM, 3>(xi, off, lx, ly, lz, s_n, vc);
+#pragma unroll
+                for (int a = 0; a < 3; a++) u[a] = a < DIM ? Corners<DIM>::WW * cur.m * (Corners<DIM>::W * corner_sum<DIM>(vc[a])) : 0.;
+            }
+            for (int r0 = r; r0 < min(r + Corners<DIM>::PB, W.e); r0 += WREC / Corners<DIM>::N) {
+                if (l / WREC == (r0 - r) / (WREC / Corners<DIM>::N) && cur.p >= 0) stage_corner<DIM, 3>(s_S[w], l % WREC, xi, off, u);
+                if (r0 + WREC / Corners<DIM>::N >= min(r + Corners<DIM>::PB, W.e)) load_corner_move<DIM>(P, B, r + Corners<DIM>::PB + i, W.e, cur);
+                wave_sync();
+                sc.scatter(W, r0, min(r0 + WREC / Corners<DIM>::N, W.e));
+                wave_sync();
+            }
+        }
+        sc.finish(W);
+        __syncthreads();
         write_partials<DIM, NQ_MOM>(N, tall, s_acc);
     };
     for_each_tile(B, tile);
@@ -1934,7 +2445,8 @@ __global__ __launch_bounds__(NT, 2) void k_usl_reset(KGrid g0, KPart P, KBins B,
     auto tile = [&](const int tall) {      // (field, context tile) pair
         if (only >= 0 && g0.tileType[tall % g0.tilesTotal] != only) return;   // another launch's type
         const int fld = tall / g0.tilesTotal;
-        const KGrid g = tile_grid(g0, tall - fld * g0.tilesTotal);
+        const GridPtr gp = tile_grid_ptr(g0, tall - fld * g0.tilesTotal);
+        const KGrid g = grid_copy(gp);
         const int t = tall - fld * g0.tilesTotal - g.tileBase;
         const KNodes Nf = field_view(g, N, fld);
         load_tile_starts<DIM>(B, tall, s_cs);
@@ -1950,14 +2462,14 @@ __global__ __launch_bounds__(NT, 2) void k_usl_reset(KGrid g0, KPart P, KBins B,
         __syncthreads();
         for (int k = tb + threadIdx.x; k < te; k += NT) {
             int p = B.order[k];
-            int e = P.elem[p];
+            int lx, ly, lz;
+            tile_cell<DIM>(B.key[p], tall, lx, ly, lz);
             // the end-of-step position is loaded here, before the state stores below, so its load is
             // issued with the others instead of after them
-            double pos[3] = {P.posn[0][p], P.posn[1][p], DIM == 3 ? P.posn[2][p] : 0.};
-            int ei, ej, ek;
-            elem_ijk(g, e, ei, ej, ek);
+            double pos[3] = {P.posn(0)[p], P.posn(1)[p], DIM == 3 ? P.posn(2)[p] : 0.};
+            int ei = ox + lx, ej = oy + ly, ek = oz + lz;
             double L[3][3];
-            particle_gradient<DIM, SH>(g, P, p, ei, ej, ek, ei - ox, ej - oy, DIM == 3 ? ek - oz : 0, s_v, L);
+            particle_gradient<DIM, SH>(g, gp, P, p, ei, ej, ek, lx, ly, lz, s_v, L);
             scale_gradient<DIM>(L, g.strainLast);
             const MpmMaterial &m = mats[P.mat[p]];
             const int mtype = MAT ? MAT : m.type;
@@ -2008,7 +2520,7 @@ __global__ __launch_bounds__(NT, 2) void k_usl_reset(KGrid g0, KPart P, KBins B,
                     }
                 }
                 if (!left) {
-                    e = (int)(num - 1);
+                    const int e = (int)(num - 1);
                     P.elem[p] = e;
                     elem_ijk(g, e, ei, ej, ek);
                 } else {
@@ -2027,9 +2539,9 @@ __global__ __launch_bounds__(NT, 2) void k_usl_reset(KGrid g0, KPart P, KBins B,
                     double dtt = g.timestep;
                     double outside[3] = {pos[0], pos[1], pos[2]};
                     double inside[3];
-                    inside[0] = outside[0] - dtt * P.f[MPF_VEL_X][p];
-                    inside[1] = outside[1] - dtt * P.f[MPF_VEL_Y][p];
-                    inside[2] = DIM == 3 ? outside[2] - dtt * P.f[MPF_VEL_Z][p] : 0.;
+                    inside[0] = outside[0] - dtt * P.f(MPF_VEL_X)[p];
+                    inside[1] = outside[1] - dtt * P.f(MPF_VEL_Y)[p];
+                    inside[2] = DIM == 3 ? outside[2] - dtt * P.f(MPF_VEL_Z)[p] : 0.;
                     if (!pt_in_elem<DIM>(g, ei, ej, ek, inside)) {
                         inside[0] = ((g.xmin + (double)ei * g.dx) + (g.xmin + (double)(ei + 1) * g.dx)) / 2.;
                         inside[1] = ((g.ymin + (double)ej * g.dy) + (g.ymin + (double)(ej + 1) * g.dy)) / 2.;
@@ -2041,9 +2553,9 @@ __global__ __launch_bounds__(NT, 2) void k_usl_reset(KGrid g0, KPart P, KBins B,
                         if (pt_in_elem<DIM>(g, ei, ej, ek, mid)) { inside[0] = mid[0]; inside[1] = mid[1]; inside[2] = mid[2]; }
                         else { outside[0] = mid[0]; outside[1] = mid[1]; outside[2] = mid[2]; }
                     }
-                    P.posn[0][p] = inside[0];
-                    P.posn[1][p] = inside[1];
-                    if (DIM == 3) P.posn[2][p] = inside[2];
+                    P.posn(0)[p] = inside[0];
+                    P.posn(1)[p] = inside[1];
+                    if (DIM == 3) P.posn(2)[p] = inside[2];
                 }
             }
             int key = cell_key<DIM>(g, fld, ei, ej, DIM == 3 ? ek : 0);
@@ -2061,145 +2573,113 @@ __global__ __launch_bounds__(NT, 2) void k_usl_reset(KGrid g0, KPart P, KBins B,
 // volume sum N Vp, displacement sum (x - x0) N mp and volume gradient sum grad N Vp, with
 // Vp = det(F) mp / rho (MatPoint3D::GetVolume, MatPoint2D::GetVolume) and the start-of-step
 // shape functions. The displacement uses the new positions in the USL pass.
-struct RecContact { double wx, wy, wz, dx, dy, dz, vp, mp, ux, uy, uz; };
+// Seven components are two products with the same rows. A particle's records are its lCPDI corners
+// (weights and the gradient weight times Vp), or, for uGIMP and classic, four: its factors with the
+// volume and the displacement's momentum-like terms, and with each axis's derivative in turn, which
+// carry the three components of the volume gradient (2D: the last is zero).
+template <int DIM> struct ContactWords { int p, key; double x[DIM], m, ep[6], wr[3], u[DIM], rho; };
+
+template <int DIM>
+__device__ __forceinline__ void load_contact_words(const KPart &rows, const KBins &B, const MpmMaterial *mats, int newPositions,
+                                                   int k, int e, ContactWords<DIM> &t) {
+    const KPart P = local_rows(rows);
+    t.p = k < e ? B.order[k] : -1;
+    if (t.p < 0) return;
+    t.key = B.key[t.p];
+#pragma unroll
+    for (int a = 0; a < DIM; a++) {
+        t.x[a] = P.f(MPF_POS_X + a)[t.p];
+        t.u[a] = (newPositions ? P.posn(a)[t.p] : t.x[a]) - P.f(MPF_ORIG_X + a)[t.p];
+    }
+    load_deformation<DIM>(P, t.p, t.ep, t.wr);
+    t.m = P.f(MPF_MASS)[t.p];
+    t.rho = mats[P.mat[t.p]].rho;
+}
 
 template <int DIM, int SH>
-__global__ __launch_bounds__(NT) void k_p2g_contact(KGrid g0, KPart P, KBins B, KNodes N, const MpmMaterial *mats,
-                                                    int newPositions) {
+__global__ __launch_bounds__(NT, MPM_TILE_SHAPE == 0 ? 2 : 1) void k_p2g_contact(KGrid g0, KPart P, KBins B, KNodes N, const MpmMaterial *mats,
+                                                        int newPositions) {
     using G = TileGeom<DIM>;
     constexpr bool CP = SH == MPMGPU_SHAPE_LCPDI;
-    constexpr int NCOR = DIM == 3 ? 8 : 4;
-    constexpr int CH = CP ? NT / NCOR : NT / 2;   // lCPDI: a thread per particle corner
+    constexpr int PPR = CP ? Corners<DIM>::N : 4, PB = 64 / PPR;     // records per particle, particles per 64 lanes
     __shared__ int s_cs[G::NC + 1];
-    __shared__ double s_S[CP ? 1 : CH][DIM][4];
-    __shared__ double s_dS[CP ? 1 : CH][DIM][4];
-    __shared__ double s_ct[CP ? CH : 1][NCOR][DIM][4];
-    __shared__ double s_cwg[CP ? CH : 1][NCOR][3];
-    __shared__ double s_q[CH][5];              // Vp, mp, displacement
+    __shared__ double s_S[NW][4 * DIM + 8][WROW];
     __shared__ double s_acc[NW][NQ_CONTACT][WaveFoot<DIM>::SIZE];
-    __shared__ double s_id[DIM][G::TX];
+    const int w = threadIdx.x >> 6, l = threadIdx.x & 63, i = l / PPR, c = l % PPR;
     auto tile = [&](const int tall) {      // (field, context tile) pair
-        const int fld = tall / g0.tilesTotal;
-        const KGrid g = tile_grid(g0, tall - fld * g0.tilesTotal);
-        const int t = tall - fld * g0.tilesTotal - g.tileBase;
+        const int tc = tall % g0.tilesTotal;
+        const GridPtr gp = tile_grid_ptr(g0, tc);
+        const KGrid g = grid_copy(gp);
         load_tile_starts<DIM>(B, tall, s_cs);
-        const int tb = s_cs[0], te = s_cs[G::NC];
-        if (tb == te) return;
+        if (s_cs[0] == s_cs[G::NC]) return;
         int ox, oy, oz;
-        tile_origin<DIM>(g, t, ox, oy, oz);
-        if (threadIdx.x < G::TX) {
-            int i = threadIdx.x;
-            s_id[0][i] = 2.0 / ((g.xmin + (double)(ox + i + 1) * g.dx) - (g.xmin + (double)(ox + i) * g.dx));
-            if (i < G::TY) s_id[1][i] = 2.0 / ((g.ymin + (double)(oy + i + 1) * g.dy) - (g.ymin + (double)(oy + i) * g.dy));
-            if (DIM == 3 && i < G::TZ)
-                s_id[DIM - 1][i] = 2.0 / ((g.zmin + (double)(oz + i + 1) * g.dz) - (g.zmin + (double)(oz + i) * g.dz));
-        }
-        zero_acc<DIM, NQ_CONTACT>(s_acc);
-        // staging thread: particle si of the chunk, and (lCPDI) its corner sc; the particle's own
-        // quantities are staged by its first thread
-        const int si = CP ? threadIdx.x / NCOR : threadIdx.x, sc = CP ? threadIdx.x % NCOR : 0;
-        for (int c0 = tb; c0 < te; c0 += CH) {
-            const int k = c0 + si;
-            if (si < CH && k < te) {
-                const int p = B.order[k];
-                int ei, ej, ek;
-                elem_ijk(g, P.elem[p], ei, ej, ek);
-                double pos[3] = {P.f[MPF_POS_X][p], P.f[MPF_POS_Y][p], DIM == 3 ? P.f[MPF_POS_Z][p] : 0.};
-                if (CP) {
-                    double r[9];
+        tile_origin<DIM>(g, tc - g.tileBase, ox, oy, oz);
+        WaveCells<DIM> W;
+        W.begin(s_cs);
+        WaveScatter<DIM, NQ_CONTACT, PPR, WROW> sc;
+        sc.begin(&s_S[w][0][0], s_acc);
+        ContactWords<DIM> cur;
+        load_contact_words<DIM>(P, B, mats, newPositions, W.b + i, W.e, cur);
+        zero_wave_acc<DIM, NQ_CONTACT>(s_acc);
+        for (int r = W.b; r < W.e; r += PB) {
+            double xi[3], u[NQ_CONTACT], invd[DIM];
+            int off[3];
+            AxisFactors f[DIM];
+            if (cur.p >= 0) {
+                int lx, ly, lz;
+                tile_cell<DIM>(cur.key, tall, lx, ly, lz);
+                double Fm[3][3], J;
+                get_F3(cur.ep, cur.wr, Fm);
+                if (DIM == 3)
+                    J = Fm[0][0] * (Fm[1][1] * Fm[2][2] - Fm[2][1] * Fm[1][2])
+                        - Fm[0][1] * (Fm[1][0] * Fm[2][2] - Fm[2][0] * Fm[1][2])
+                        + Fm[0][2] * (Fm[1][0] * Fm[2][1] - Fm[2][0] * Fm[1][1]);
+                else J = Fm[0][0] * Fm[1][1] - Fm[1][0] * Fm[0][1];
+                const double Vp = J * cur.m / cur.rho;
+                if constexpr (CP) {
+                    double s[9], wg[3];
 #pragma unroll
-                    for (int a = 0; a < 9; a++) r[a] = P.cpr[a][p];
-                    double xi[3], w[3];
-                    int off[3];
-                    cpdi_corner<DIM>(g, pos, r, ei, ej, ek, sc, xi, off);
-                    cpdi_table<DIM>(xi, off, s_ct[si][sc]);
-                    cpdi_wg_staged<DIM>(r, sc, w);
-                    s_cwg[si][sc][0] = w[0]; s_cwg[si][sc][1] = w[1]; s_cwg[si][sc][2] = w[2];
-                } else {
-                    double xi[3], invd[3], S[3][4], dS[3][4];
-                    particle_xi<DIM>(g, ei, ej, ek, pos[0], pos[1], pos[2], xi, invd);
-                    particle_factors<DIM>(g, P, p, xi, S, dS);
+                    for (int a = 0; a < 9; a++) s[a] = DIM == 3 || (a < 6 && a % 3 < 2) ? P.cpr(a)[cur.p] : 0.;
+                    corner_lane<DIM>(gp, cur.x, s, ox + lx, oy + ly, oz + lz, c, xi, off);
+                    cpdi_wg_staged<DIM>(s, c, wg);
+                    u[0] = Corners<DIM>::WW * Vp;
 #pragma unroll
-                    for (int a = 0; a < DIM; a++)
-#pragma unroll
-                        for (int o = 0; o < 4; o++) {
-                            s_S[threadIdx.x][a][o] = S[a][o];
-                            s_dS[threadIdx.x][a][o] = dS[a][o];
-                        }
-                }
-                if (sc == 0) {
-                    double mp = P.f[MPF_MASS][p];
-                    double rho = mats[P.mat[p]].rho;
-                    double Vp;
-                    if (DIM == 3) {
-                        double Fm[3][3];
-                        double ep[6] = {P.f[MPF_EP_XX][p], P.f[MPF_EP_YY][p], P.f[MPF_EP_ZZ][p],
-                                        P.f[MPF_EP_YZ][p], P.f[MPF_EP_XZ][p], P.f[MPF_EP_XY][p]};
-                        double wr[3] = {P.f[MPF_WR_YZ][p], P.f[MPF_WR_XZ][p], P.f[MPF_WR_XY][p]};
-                        get_F3(ep, wr, Fm);
-                        Vp = (Fm[0][0] * (Fm[1][1] * Fm[2][2] - Fm[2][1] * Fm[1][2])
-                            - Fm[0][1] * (Fm[1][0] * Fm[2][2] - Fm[2][0] * Fm[1][2])
-                            + Fm[0][2] * (Fm[1][0] * Fm[2][1] - Fm[2][0] * Fm[1][1])) * mp / rho;
-                    } else {
-                        double exy = P.f[MPF_EP_XY][p], wxy = P.f[MPF_WR_XY][p];
-                        double f00 = 1. + P.f[MPF_EP_XX][p], f11 = 1. + P.f[MPF_EP_YY][p];
-                        double f01 = 0.5 * (exy - wxy), f10 = 0.5 * (exy + wxy);
-                        Vp = (f00 * f11 - f10 * f01) * mp / rho;
+                    for (int a = 0; a < 3; a++) {
+                        u[1 + a] = a < DIM ? Corners<DIM>::WW * cur.m * cur.u[a < DIM ? a : 0] : 0.;
+                        u[4 + a] = wg[a] * Vp;
                     }
-                    s_q[si][0] = Vp;
-                    s_q[si][1] = mp;
+                } else {
+                    particle_axes<DIM>(gp, P, cur.p, ox + lx, oy + ly, oz + lz, cur.x, f, invd);
+                    u[0] = c == 0 ? Vp : 0.;
 #pragma unroll
-                    for (int a = 0; a < 3; a++)
-                        s_q[si][2 + a] = a < DIM ? (newPositions ? P.posn[a][p] : pos[a]) - P.f[MPF_ORIG_X + a][p] : 0.;
+                    for (int a = 0; a < 3; a++) {
+                        u[1 + a] = a < DIM && c == 0 ? cur.m * cur.u[a < DIM ? a : 0] : 0.;
+                        u[4 + a] = a < DIM && c == 1 + a ? Vp : 0.;
+                    }
                 }
             }
-            __syncthreads();
-            wave_cells<DIM, NQ_CONTACT>(s_cs, c0, min(c0 + CH, te), s_acc,
-                [&](int lq, int ix, int iy, int iz) {
-                    RecContact r;
-                    if (CP) {
-                        double gr[3];
-                        cpdi_table_node<DIM, true>(s_ct[lq], s_cwg[lq], ix, iy, iz, r.wx, gr);
-                        r.wy = r.wz = 1.;
-                        r.dx = gr[0]; r.dy = gr[1]; r.dz = gr[2];
-                    } else {
-                        r.wx = s_S[lq][0][ix]; r.wy = s_S[lq][1][iy];
-                        r.dx = s_dS[lq][0][ix]; r.dy = s_dS[lq][1][iy];
-                        if (DIM == 3) { r.wz = s_S[lq][DIM - 1][iz]; r.dz = s_dS[lq][DIM - 1][iz]; }
-                        else { r.wz = 1.; r.dz = 0.; }
+            for (int r0 = r; r0 < min(r + PB, W.e); r0 += WREC / PPR) {
+                if (l / WREC == (r0 - r) / (WREC / PPR) && cur.p >= 0) {
+                    if constexpr (CP) stage_corner<DIM, NQ_CONTACT>(s_S[w], l % WREC, xi, off, u);
+                    else {
+#pragma unroll
+                        for (int a = 0; a < DIM; a++)
+#pragma unroll
+                            for (int o = 0; o < 4; o++)
+                                s_S[w][a * 4 + o][l % WREC] = c == 1 + a ? f[a].d4(o) * invd[a] : f[a].s4(o);
+#pragma unroll
+                        for (int q = 0; q < NQ_CONTACT; q++) s_S[w][4 * DIM + q][l % WREC] = u[q];
                     }
-                    r.vp = s_q[lq][0]; r.mp = s_q[lq][1];
-                    r.ux = s_q[lq][2]; r.uy = s_q[lq][3]; r.uz = s_q[lq][4];
-                    return r;
-                },
-                [&](const RecContact &r, double *acc, int lx, int ly, int lz) {
-                    bool on = r.wx >= 0. && r.wy >= 0. && r.wz >= 0.;
-                    double vp = on ? r.vp : 0., mp = on ? r.mp : 0.;
-                    double fn, gx, gy, gz;
-                    if (CP) {
-                        fn = r.wx; gx = r.dx; gy = r.dy; gz = DIM == 3 ? r.dz : 0.;
-                    } else if (DIM == 3) {
-                        fn = r.wx * r.wy * r.wz;
-                        gx = r.dx * r.wy * r.wz * s_id[0][lx];
-                        gy = r.wx * r.dy * r.wz * s_id[1][ly];
-                        gz = r.wx * r.wy * r.dz * s_id[DIM - 1][lz];
-                    } else {
-                        fn = r.wx * r.wy;
-                        gx = r.dx * r.wy * s_id[0][lx];
-                        gy = r.wx * r.dy * s_id[1][ly];
-                        gz = 0.;
-                    }
-                    acc[0] = fma(fn, vp, acc[0]);
-                    const double fnmp = fn * mp;
-                    acc[1] = fma(r.ux, fnmp, acc[1]);
-                    acc[2] = fma(r.uy, fnmp, acc[2]);
-                    acc[3] = fma(r.uz, fnmp, acc[3]);
-                    acc[4] = fma(gx, vp, acc[4]);
-                    acc[5] = fma(gy, vp, acc[5]);
-                    acc[6] = fma(gz, vp, acc[6]);
-                });
-            __syncthreads();
+                }
+                if (r0 + WREC / PPR >= min(r + PB, W.e))
+                    load_contact_words<DIM>(P, B, mats, newPositions, r + PB + i, W.e, cur);
+                wave_sync();
+                sc.scatter(W, r0, min(r0 + WREC / PPR, W.e));
+                wave_sync();
+            }
         }
+        sc.finish(W);
+        __syncthreads();
         write_partials<DIM, NQ_CONTACT>(N, tall, s_acc);
     };
     for_each_tile(B, tile);
@@ -2458,7 +2938,7 @@ __device__ __forceinline__ bool lr_member(const KGrid &g, const KPart &P, int p,
         return in;
     }
     double xi[3], invd[3], S[3][4], dS[3][4];
-    particle_xi<DIM>(g, ei, ej, ek, P.f[MPF_POS_X][p], P.f[MPF_POS_Y][p], DIM == 3 ? P.f[MPF_POS_Z][p] : 0., xi, invd);
+    particle_xi<DIM>(g, ei, ej, ek, P.f(MPF_POS_X)[p], P.f(MPF_POS_Y)[p], DIM == 3 ? P.f(MPF_POS_Z)[p] : 0., xi, invd);
     particle_factors<DIM>(g, P, p, xi, S, dS);
     bool in = true;
 #pragma unroll
@@ -2536,10 +3016,10 @@ template <int DIM>
 __device__ __forceinline__ double lr_radius(const KGrid &g, const KPart &P, int p, const double n[3]) {
     double lpx, lpy, lpz;
     if (g.uniformLp) { lpx = g.lp[0]; lpy = g.lp[1]; lpz = g.lp[2]; }
-    else { lpx = P.f[MPF_LP_X][p]; lpy = P.f[MPF_LP_Y][p]; lpz = P.f[MPF_LP_Z][p]; }
+    else { lpx = P.f(MPF_LP_X)[p]; lpy = P.f(MPF_LP_Y)[p]; lpz = P.f(MPF_LP_Z)[p]; }
     const double psx = g.dx * (0.5 * lpx), psy = g.dy * (0.5 * lpy);      // GetParticleSize
     if (DIM == 2) {
-        const double exx = P.f[MPF_EP_XX][p], eyy = P.f[MPF_EP_YY][p], exy = P.f[MPF_EP_XY][p], wxy = P.f[MPF_WR_XY][p];
+        const double exx = P.f(MPF_EP_XX)[p], eyy = P.f(MPF_EP_YY)[p], exy = P.f(MPF_EP_XY)[p], wxy = P.f(MPF_WR_XY)[p];
         const double F00 = 1. + exx, F01 = 0.5 * (exy - wxy), F10 = 0.5 * (exy + wxy), F11 = 1. + eyy;
         const double rdet2D = 1. / (F00 * F11 - F01 * F10);
         const double n0x = (F11 * n[0] - F10 * n[1]) * rdet2D;
@@ -2549,9 +3029,9 @@ __device__ __forceinline__ double lr_radius(const KGrid &g, const KPart &P, int 
     const double psz = g.dz * (0.5 * lpz);
     double ep[6], wr[3], m[3][3];
 #pragma unroll
-    for (int c = 0; c < 6; c++) ep[c] = P.f[MPF_EP_XX + c][p];
+    for (int c = 0; c < 6; c++) ep[c] = P.f(MPF_EP_XX + c)[p];
 #pragma unroll
-    for (int c = 0; c < 3; c++) wr[c] = P.f[MPF_WR_YZ + c][p];
+    for (int c = 0; c < 3; c++) wr[c] = P.f(MPF_WR_YZ + c)[p];
     get_F3(ep, wr, m);
     double inv[3][3] = {{m[1][1] * m[2][2] - m[2][1] * m[1][2], -(m[0][1] * m[2][2] - m[2][1] * m[0][2]),
                          m[0][1] * m[1][2] - m[1][1] * m[0][2]},
@@ -2578,9 +3058,9 @@ __global__ __launch_bounds__(NT) void k_contact_normals(KGrid g, KPart P, KBins 
     int *list = s_list[w];
     const int count = N.clist[0];
     const long long nn = g.nstride;
-    const double *px = newPos ? P.posn[0] : P.f[MPF_POS_X];
-    const double *py = newPos ? P.posn[1] : P.f[MPF_POS_Y];
-    const double *pz = DIM == 3 ? (newPos ? P.posn[2] : P.f[MPF_POS_Z]) : nullptr;
+    const double *px = newPos ? P.posn(0) : P.f(MPF_POS_X);
+    const double *py = newPos ? P.posn(1) : P.f(MPF_POS_Y);
+    const double *pz = DIM == 3 ? (newPos ? P.posn(2) : P.f(MPF_POS_Z)) : nullptr;
     const bool logistic = g.normals == 6;
     for (int e = blockIdx.x * NW + w; e < count; e += gridDim.x * NW) {
         const long long n = N.clist[1 + e];
@@ -2848,11 +3328,11 @@ void launch_p2g_mass(int dim, const KGrid &g, const KPart &p, const KBins &b, co
     (void)mats;
     const bool cp = g.shape == MPMGPU_SHAPE_LCPDI;
     if (dim == 3) {
-        if (cp) TILE_LAUNCH((k_p2g_mass<3, MPMGPU_SHAPE_LCPDI>), tb, s, g, p, tb, nd, st);
-        else TILE_LAUNCH((k_p2g_mass<3, MPMGPU_SHAPE_UGIMP>), tb, s, g, p, tb, nd, st);
+        if (cp) TILE_LAUNCH(k_p2g_mass_corners<3>, tb, s, g, p, tb, nd, st);
+        else TILE_LAUNCH(k_p2g_mass<3>, tb, s, g, p, tb, nd);
     } else {
-        if (cp) TILE_LAUNCH((k_p2g_mass<2, MPMGPU_SHAPE_LCPDI>), tb, s, g, p, tb, nd, st);
-        else TILE_LAUNCH((k_p2g_mass<2, MPMGPU_SHAPE_UGIMP>), tb, s, g, p, tb, nd, st);
+        if (cp) TILE_LAUNCH(k_p2g_mass_corners<2>, tb, s, g, p, tb, nd, st);
+        else TILE_LAUNCH(k_p2g_mass<2>, tb, s, g, p, tb, nd);
     }
 }
 
@@ -2968,7 +3448,7 @@ __device__ int surface_info(const KGrid &g, const KPart &P, int p, int ei, int e
         // the undeformed semi sides (GetUndeformedSemiSides)
         double lpx, lpy, lpz;
         if (g.uniformLp) { lpx = g.lp[0]; lpy = g.lp[1]; lpz = g.lp[2]; }
-        else { lpx = P.f[MPF_LP_X][p]; lpy = P.f[MPF_LP_Y][p]; lpz = P.f[MPF_LP_Z][p]; }
+        else { lpx = P.f(MPF_LP_X)[p]; lpy = P.f(MPF_LP_Y)[p]; lpz = P.f(MPF_LP_Z)[p]; }
         const double ux = ((g.xmin + (double)(ei + 1) * g.dx) - (g.xmin + (double)ei * g.dx)) * (0.5 * lpx);
         const double uy = ((g.ymin + (double)(ej + 1) * g.dy) - (g.ymin + (double)ej * g.dy)) * (0.5 * lpy);
         const double uz = DIM == 3 ? ((g.zmin + (double)(ek + 1) * g.dz) - (g.zmin + (double)ek * g.dz)) * (0.5 * lpz) : 0.;
@@ -2976,7 +3456,7 @@ __device__ int surface_info(const KGrid &g, const KPart &P, int p, int ei, int e
         for (int a = 0; a < 9; a++) r[a] = 0.;
         r1[0] = ux; r2[1] = uy; r3[2] = uz;
     }
-    const double pos[3] = {P.f[MPF_POS_X][p], P.f[MPF_POS_Y][p], DIM == 3 ? P.f[MPF_POS_Z][p] : 0.};
+    const double pos[3] = {P.f(MPF_POS_X)[p], P.f(MPF_POS_Y)[p], DIM == 3 ? P.f(MPF_POS_Z)[p] : 0.};
     const int nc = DIM == 3 ? 4 : 2;
     for (int k = 0; k < nc; k++) {
 #pragma unroll
@@ -3091,19 +3571,19 @@ void launch_p2g_force(int dim, const KGrid &g, const KPart &p, const KBins &b, c
         loaded = L.tflag[par];
         const KBins tl = tile_bins(b, TILE_SLOT_FORCE_LOADS);
         if (dim == 3) {
-            if (cp) TILE_LAUNCH((k_p2g_force<3, MPMGPU_SHAPE_LCPDI, true>), tl, s, g, p, tl, nd, L, loaded);
-            else TILE_LAUNCH((k_p2g_force<3, MPMGPU_SHAPE_UGIMP, true>), tl, s, g, p, tl, nd, L, loaded);
+            if (cp) TILE_LAUNCH((k_p2g_force_corners<3, true>), tl, s, g, p, tl, nd, L, loaded);
+            else TILE_LAUNCH((k_p2g_force<3, true>), tl, s, g, p, tl, nd, L, loaded);
         } else {
-            if (cp) TILE_LAUNCH((k_p2g_force<2, MPMGPU_SHAPE_LCPDI, true>), tl, s, g, p, tl, nd, L, loaded);
-            else TILE_LAUNCH((k_p2g_force<2, MPMGPU_SHAPE_UGIMP, true>), tl, s, g, p, tl, nd, L, loaded);
+            if (cp) TILE_LAUNCH((k_p2g_force_corners<2, true>), tl, s, g, p, tl, nd, L, loaded);
+            else TILE_LAUNCH((k_p2g_force<2, true>), tl, s, g, p, tl, nd, L, loaded);
         }
     }
     if (dim == 3) {
-        if (cp) TILE_LAUNCH((k_p2g_force<3, MPMGPU_SHAPE_LCPDI, false>), tb, s, g, p, tb, nd, L, loaded);
-        else TILE_LAUNCH((k_p2g_force<3, MPMGPU_SHAPE_UGIMP, false>), tb, s, g, p, tb, nd, L, loaded);
+        if (cp) TILE_LAUNCH((k_p2g_force_corners<3, false>), tb, s, g, p, tb, nd, L, loaded);
+        else TILE_LAUNCH((k_p2g_force<3, false>), tb, s, g, p, tb, nd, L, loaded);
     } else {
-        if (cp) TILE_LAUNCH((k_p2g_force<2, MPMGPU_SHAPE_LCPDI, false>), tb, s, g, p, tb, nd, L, loaded);
-        else TILE_LAUNCH((k_p2g_force<2, MPMGPU_SHAPE_UGIMP, false>), tb, s, g, p, tb, nd, L, loaded);
+        if (cp) TILE_LAUNCH((k_p2g_force_corners<2, false>), tb, s, g, p, tb, nd, L, loaded);
+        else TILE_LAUNCH((k_p2g_force<2, false>), tb, s, g, p, tb, nd, L, loaded);
     }
 }
 
@@ -3117,11 +3597,11 @@ static void g2p_move(int dim, const KGrid &g, const KPart &p, const KBins &tb, c
                      const MpmMaterial *mats, int mode, hipStream_t s) {
     const bool cp = g.shape == MPMGPU_SHAPE_LCPDI;
     if (dim == 3) {
-        if (cp) TILE_LAUNCH((k_g2p_p2g<3, MPMGPU_SHAPE_LCPDI, MOVE>), tb, s, g, p, tb, nd, mats, mode);
-        else TILE_LAUNCH((k_g2p_p2g<3, MPMGPU_SHAPE_UGIMP, MOVE>), tb, s, g, p, tb, nd, mats, mode);
+        if (cp) TILE_LAUNCH((k_g2p_p2g_corners<3, MOVE>), tb, s, g, p, tb, nd, mats, mode);
+        else TILE_LAUNCH((k_g2p_p2g<3, MOVE>), tb, s, g, p, tb, nd, mats, mode);
     } else {
-        if (cp) TILE_LAUNCH((k_g2p_p2g<2, MPMGPU_SHAPE_LCPDI, MOVE>), tb, s, g, p, tb, nd, mats, mode);
-        else TILE_LAUNCH((k_g2p_p2g<2, MPMGPU_SHAPE_UGIMP, MOVE>), tb, s, g, p, tb, nd, mats, mode);
+        if (cp) TILE_LAUNCH((k_g2p_p2g_corners<2, MOVE>), tb, s, g, p, tb, nd, mats, mode);
+        else TILE_LAUNCH((k_g2p_p2g<2, MOVE>), tb, s, g, p, tb, nd, mats, mode);
     }
 }
 
@@ -3322,12 +3802,12 @@ void launch_xpic(int dim, const KGrid &g, const KPart &p, const KBins &b, const 
     else hipLaunchKernelGGL(k_xpic_init<2>, ng, blk, 0, s, g, b, nd, fmpm ? 1 : 0);
     for (int it = 2; it <= order; it++) {
         if (dim == 3) {
-            if (cp) TILE_LAUNCH((k_xpic_p2g<3, MPMGPU_SHAPE_LCPDI>), tb, s, g, p, tb, nd);
-            else TILE_LAUNCH((k_xpic_p2g<3, MPMGPU_SHAPE_UGIMP>), tb, s, g, p, tb, nd);
+            if (cp) TILE_LAUNCH(k_xpic_p2g_corners<3>, tb, s, g, p, tb, nd);
+            else TILE_LAUNCH(k_xpic_p2g<3>, tb, s, g, p, tb, nd);
             hipLaunchKernelGGL(k_xpic_node<3>, ng, blk, 0, s, g, tb, nd);
         } else {
-            if (cp) TILE_LAUNCH((k_xpic_p2g<2, MPMGPU_SHAPE_LCPDI>), tb, s, g, p, tb, nd);
-            else TILE_LAUNCH((k_xpic_p2g<2, MPMGPU_SHAPE_UGIMP>), tb, s, g, p, tb, nd);
+            if (cp) TILE_LAUNCH(k_xpic_p2g_corners<2>, tb, s, g, p, tb, nd);
+            else TILE_LAUNCH(k_xpic_p2g<2>, tb, s, g, p, tb, nd);
             hipLaunchKernelGGL(k_xpic_node<2>, ng, blk, 0, s, g, tb, nd);
         }
         if (bc.nb) MPM_KNS::launch_vel_bcs(g, nd, bc, forcePass && !fmpm ? BC_PASS_XPIC_FORCE : BC_PASS_XPIC, par, s);

@@ -158,7 +158,7 @@ int relayout(MpmServer *s, const std::vector<Request *> &members) {
     nc->kg.matType = common;
     for (size_t k = 0; k < ni; k++) {
         nc->inst[k].uniformLp = members[k]->uniformLp;
-        for (int a = 0; a < 3; a++) nc->inst[k].lp[a] = members[k]->lp[a];
+        set_particle_size(nc->inst[k], members[k]->lp);
         nc->inst[k].matType = common;
     }
     if (hipMemcpyAsync(nc->dinst, nc->inst.data(), ni * sizeof(KGrid), hipMemcpyHostToDevice, nc->stream) !=
@@ -177,7 +177,7 @@ int relayout(MpmServer *s, const std::vector<Request *> &members) {
         if (r->placed) {
             KMove mv{};
             mv.sd = old->pbuf;
-            for (int a = 0; a < 3; a++) mv.spos[a] = old->kp.f[MPF_POS_X + a];
+            for (int a = 0; a < 3; a++) mv.spos[a] = old->kp.f(MPF_POS_X + a);
             mv.si = old->ibuf;
             mv.sn = old->kp.n;
             mv.soff = r->off;
@@ -260,7 +260,7 @@ int keep_result(MpmServer *s, Request *r) {
         return srv_fail(s, "out of device memory keeping a result");
     }
     for (int f = 0; f < MPF_NUM_FIELDS; f++)
-        if (hipMemcpyAsync(r->dd + f * n, c->kp.f[f] + r->off, n * sizeof(double), hipMemcpyDeviceToDevice,
+        if (hipMemcpyAsync(r->dd + f * n, c->kp.f(f) + r->off, n * sizeof(double), hipMemcpyDeviceToDevice,
                            c->stream) != hipSuccess)
             return srv_fail(s, "result copy failed");
     for (int q = 0; q < IROWS; q++) {

@@ -172,12 +172,12 @@ int mpmgpu_solve_static(const MpmGridDesc *grid, const MpmMaterial *mats, int32_
     // the particle rows are the caller's; the second position buffer and the bin rows are scratch
     const size_t nn = (size_t)n;
     KPart &P = c.kp;
-    for (int f = 0; f < MPF_NUM_FIELDS; f++) P.f[f] = dfields + f * nn;
+    P.d = dfields;
     for (int k = 0; k < 3; k++) {
         c.posA[k] = dfields + (MPF_POS_X + k) * nn;
         c.posB[k] = posB + k * nn;
     }
-    for (int k = 0; k < 9; k++) P.cpr[k] = cbuf ? cbuf + k * nn : nullptr;
+    P.semi = cbuf;
     P.elem = ifields + MPI_ELEM * nn;
     P.mat = ifields + MPI_MAT * nn;
     P.id = ifields + MPI_ID * nn;
@@ -210,7 +210,7 @@ int mpmgpu_solve_static(const MpmGridDesc *grid, const MpmMaterial *mats, int32_
     // kernels skip the size rows (as mpmgpu_upload_particles decides)
     c.kg.matType = hchk[CHK_MIXED_TYPE] ? 0 : mats[mat0].type;
     c.kg.uniformLp = hchk[CHK_MIXED_LP] ? 0 : 1;
-    for (int k = 0; k < 3; k++) c.kg.lp[k] = lp0[k];
+    set_particle_size(c.kg, lp0);
 
     // prepare as an upload does (the rows keep the caller's order: they are not sorted into tiles,
     // which changes no result), then step
