@@ -8,6 +8,7 @@
 #include <utility>
 #include <vector>
 
+#include "mpm_download.h"
 #include "mpm_events.h"
 #include "mpm_kernels.h"
 
@@ -50,6 +51,7 @@ struct MpmCtx {
     int *ibuf = nullptr;              // particle int fields
     double *cbuf = nullptr;           // lCPDI semi-side vectors of the step
     double *scr = nullptr;            // one particle row of scratch (row permutations)
+    RowDownload rows;                 // staging of mpmgpu_download_particles
     int sortInterval = 50;           // steps between sorts of the rows into tile order (0: never)
     int sinceSort = 0;
     // batch of independent instances (empty for one simulation)

@@ -1638,21 +1638,9 @@ int mpmgpu_download_particles(MpmCtx *c, double *dfields, int32_t *ifields) {
     size_t nn = (size_t)c->kp.n;
     if (nn == 0) return 0;
     set_positions(c);
-    // rows back to upload order through the scratch row
-    hipStream_t s = c->stream;
-    for (int f = 0; f < MPF_NUM_FIELDS; f++) {
-        launch_scatter_row(c->kp.f(f), c->scr, c->kb.home, (long long)nn, s);
-        HIPCHECK(c, hipMemcpyAsync(dfields + f * nn, c->scr, nn * sizeof(double), hipMemcpyDeviceToHost, s));
-    }
-    if (ifields) {
-        int *iscr = reinterpret_cast<int *>(c->scr);
-        for (int q = 0; q < MPI_NUM_FIELDS; q++) {
-            launch_scatter_irow(c->ibuf + q * nn, iscr, c->kb.home, (long long)nn, s);
-            HIPCHECK(c, hipMemcpyAsync(ifields + q * nn, iscr, nn * sizeof(int), hipMemcpyDeviceToHost, s));
-        }
-    }
-    HIPCHECK(c, hipGetLastError());
-    HIPCHECK(c, hipStreamSynchronize(s));
+    // rows back to upload order
+    HIPCHECK(c, c->rows.run(c->kp.pos, c->kp.d, c->ibuf, c->kb.home, reinterpret_cast<int *>(c->scr), (long long)nn, 0, 0,
+                            dfields, ifields, c->stream));
     return 0;
 }
 

@@ -3892,12 +3892,6 @@ __global__ void k_gather_row(const T *src, T *dst, const int *order, long long n
     if (k < n) dst[k] = src[order[k]];
 }
 
-template <typename T>
-__global__ void k_scatter_row(const T *src, T *dst, const int *home, long long n) {
-    const long long k = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k < n) dst[home[k]] = src[k];
-}
-
 __global__ void k_iota(int *a, long long n, int base) {
     const long long k = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (k < n) a[k] = base + (int)k;
@@ -3908,12 +3902,6 @@ void launch_gather_row(const double *src, double *dst, const int *order, long lo
 }
 void launch_gather_irow(const int *src, int *dst, const int *order, long long n, hipStream_t s) {
     if (n > 0) hipLaunchKernelGGL(k_gather_row<int>, dim3(blocks_for(n, NT)), dim3(NT), 0, s, src, dst, order, n);
-}
-void launch_scatter_row(const double *src, double *dst, const int *home, long long n, hipStream_t s) {
-    if (n > 0) hipLaunchKernelGGL(k_scatter_row<double>, dim3(blocks_for(n, NT)), dim3(NT), 0, s, src, dst, home, n);
-}
-void launch_scatter_irow(const int *src, int *dst, const int *home, long long n, hipStream_t s) {
-    if (n > 0) hipLaunchKernelGGL(k_scatter_row<int>, dim3(blocks_for(n, NT)), dim3(NT), 0, s, src, dst, home, n);
 }
 void launch_iota(int *a, long long n, int base, hipStream_t s) {
     if (n > 0) hipLaunchKernelGGL(k_iota, dim3(blocks_for(n, NT)), dim3(NT), 0, s, a, n, base);

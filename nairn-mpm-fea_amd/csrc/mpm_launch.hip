@@ -77,10 +77,4 @@ void launch_gather_row(const double *src, double *dst, const int *order, long lo
 void launch_gather_irow(const int *src, int *dst, const int *order, long long n, hipStream_t s) {
     mpmk_s0::launch_gather_irow(src, dst, order, n, s);
 }
-void launch_scatter_row(const double *src, double *dst, const int *home, long long n, hipStream_t s) {
-    mpmk_s0::launch_scatter_row(src, dst, home, n, s);
-}
-void launch_scatter_irow(const int *src, int *dst, const int *home, long long n, hipStream_t s) {
-    mpmk_s0::launch_scatter_irow(src, dst, home, n, s);
-}
 void launch_iota(int *a, long long n, int base, hipStream_t s) { mpmk_s0::launch_iota(a, n, base, s); }

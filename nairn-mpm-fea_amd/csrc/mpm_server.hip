@@ -83,6 +83,9 @@ struct MpmServer {
     double layoutSeconds = 0., stepSeconds = 0.;   // request-loop time in layouts and in batch steps
     int64_t deviceRowBytes = 0;                  // staged uploads and results held on the device
     hipStream_t upStream = nullptr;              // staging copies of submitting threads
+    std::mutex downMutex;                        // one collecting thread at a time uses the two below
+    hipStream_t downStream = nullptr;
+    RowDownload rows;
     std::string err;
     bool failed = false;
     std::thread loop;
@@ -386,7 +389,9 @@ int mpmgpu_server_create(const MpmServerParams *params, MpmServer **out) {
         p.memoryBudget = (int64_t)(0.9 * (double)freeB);
     }
     MpmServer *s = new MpmServer();
-    if (hipStreamCreateWithFlags(&s->upStream, hipStreamNonBlocking) != hipSuccess) {
+    if (hipStreamCreateWithFlags(&s->upStream, hipStreamNonBlocking) != hipSuccess ||
+        hipStreamCreateWithFlags(&s->downStream, hipStreamNonBlocking) != hipSuccess) {
+        if (s->upStream) (void)hipStreamDestroy(s->upStream);
         delete s;
         return create_fail("hipStreamCreate failed");
     }
@@ -577,34 +582,27 @@ int mpmgpu_server_collect(MpmServer *s, int64_t id, double *dfields, int32_t *if
         }
         r->state = MPMGPU_REQ_COLLECTED;       // the result rows are this thread's now
     }
+    // back to the solve's own order (upload-index row) and material numbering; the result rows are
+    // complete (the loop waits for their copies), and their order row is free for the places
     const size_t n = (size_t)r->n;
-    std::vector<double> d((size_t)MPF_NUM_FIELDS * n);
-    std::vector<int32_t> iv((size_t)IROWS * n);
-    bool ok = hipMemcpy(d.data(), r->dd, d.size() * sizeof(double), hipMemcpyDeviceToHost) == hipSuccess &&
-              hipMemcpy(iv.data(), r->di, iv.size() * sizeof(int), hipMemcpyDeviceToHost) == hipSuccess;
-    free_rows(r);
+    hipError_t rc;
     {
-        std::lock_guard<std::mutex> lk(s->m);
-        s->deviceRowBytes -= r->devBytes;
-        r->devBytes = 0;
-        if (!ok) {
-            s->err = "result download failed";
-            return 1;
-        }
+        std::lock_guard<std::mutex> lk(s->downMutex);
+        int dev = s->device;
+        (void)hipGetDevice(&dev);
+        rc = hipSetDevice(s->device);
+        if (rc == hipSuccess)
+            rc = s->rows.run(r->dd, r->dd, r->di, r->di + IROW_HOME * n, r->di + IROW_ORDER * n, r->n, r->homeBase,
+                             r->resultFirstMat, dfields, ifields, s->downStream);
+        if (dev != s->device) (void)hipSetDevice(dev);
     }
-    // back to the solve's own order (upload-index row) and material numbering
-    const int32_t *home = iv.data() + (size_t)IROW_HOME * n;
-    for (size_t i = 0; i < n; i++) {
-        const long long h = (long long)home[i] - r->homeBase;
-        if (h < 0 || h >= (long long)n) {
-            std::lock_guard<std::mutex> lk(s->m);
-            s->err = "particle rows of a solve left its range";
-            return 1;
-        }
-        for (int f = 0; f < MPF_NUM_FIELDS; f++) dfields[f * n + h] = d[f * n + i];
-        if (ifields)
-            for (int q = 0; q < MPI_NUM_FIELDS; q++)
-                ifields[q * n + h] = iv[q * n + i] - (q == MPI_MAT ? r->resultFirstMat : 0);
+    free_rows(r);
+    std::lock_guard<std::mutex> lk(s->m);
+    s->deviceRowBytes -= r->devBytes;
+    r->devBytes = 0;
+    if (rc != hipSuccess) {
+        s->err = rc == hipErrorInvalidValue ? "particle rows of a solve left its range" : "result download failed";
+        return 1;
     }
     return 0;
 }
@@ -635,6 +633,7 @@ void mpmgpu_server_destroy(MpmServer *s) {
     if (s->ctx) mpmgpu_destroy(s->ctx);
     for (auto &kv : s->reqs) free_rows(kv.second.get());
     if (s->upStream) (void)hipStreamDestroy(s->upStream);
+    if (s->downStream) (void)hipStreamDestroy(s->downStream);
     delete s;
 }
 

@@ -453,8 +453,8 @@ class Simulation:
         _check(library().mpmgpu_sync(self._h), self._h)
 
     def particles(self):
-        d = np.zeros((NUM_FIELDS, self.n), dtype=np.float64)
-        i = np.zeros((NUM_IFIELDS, self.n), dtype=np.int32)
+        d = np.empty((NUM_FIELDS, self.n), dtype=np.float64)       # every word is written below
+        i = np.empty((NUM_IFIELDS, self.n), dtype=np.int32)
         _check(library().mpmgpu_download_particles(self._h, _dptr(d), _iptr(i)), self._h)
         return d, i
 
@@ -642,8 +642,8 @@ class Server:
 
     def collect(self, rid: int):
         n = self._n[rid]
-        d = np.zeros((NUM_FIELDS, n), dtype=np.float64)
-        i = np.zeros((NUM_IFIELDS, n), dtype=np.int32)
+        d = np.empty((NUM_FIELDS, n), dtype=np.float64)
+        i = np.empty((NUM_IFIELDS, n), dtype=np.int32)
         self._ok(library().mpmgpu_server_collect(self._h, int(rid), _dptr(d), _iptr(i)))
         return d, i
 
