@@ -46,9 +46,19 @@
 namespace MPM_KNS {
 
 template <int DIM> using TileGeom = TileShape<DIM, MPM_TILE_SHAPE>;
-// waves per SIMD the uGIMP particle-update scatters are built for: shape 1's larger footprint
-// leaves LDS for two workgroups per CU
-#define G2P_WAVES (MPM_TILE_SHAPE == 0 ? 3 : 2)
+// Waves that share a tile in a scatter, and waves per SIMD their kernels are built for (shape 1's larger
+// footprint leaves LDS for two). Eight waves give a few full tiles more parallelism and, where the
+// registers allow two such blocks per CU, four waves per SIMD instead of three; each has its own staging
+// rows and footprint copy, so they need 1.5 times the LDS, and with 32 particles a wave (2D) half of its
+// lanes idle. us per launch with 4 and 8 waves: 7.08M uGIMP particles, update 670 and 600, mass 356 and
+// 375, force 540 and 870 (its registers and LDS then leave one block); 87k lCPDI particles, mass 74 and 59,
+// force 73 and 59, update 90 and 70 (16 waves: 60, 56, 69); 1.7M 2D particles, mass 73 and 110.
+// One choice per kernel: the order of a sum must not depend on the number of particles.
+#define WAVES4 (MPM_TILE_SHAPE == 0 ? 3 : 2)
+#define WAVES8 (MPM_TILE_SHAPE == 0 ? 4 : 2)
+constexpr int UGIMP_NW = 4;
+constexpr int G2P_NW(int dim) { return dim == 3 ? 8 : 4; }
+constexpr int CORNER_NW(int dim) { return dim == 3 ? 8 : 4; }
 
 template <int DIM>
 __device__ __forceinline__ void tile_origin(const KGrid &g, int t, int &ox, int &oy, int &oz) {
@@ -818,20 +828,20 @@ __device__ __forceinline__ void for_each_tile(const KBins &B, F &tile) {
 }
 
 // ---------------------------------------------------------------------------------------
-#define NW (NT / 64)
-
-// A wave takes a run of the tile's cells, in sorted order: its layer z = w in 3D, its rows y = 2w and
-// 2w + 1 in 2D. The wave's copy of the footprint covers the planes (3D) or rows (2D) that its cells
-// reach, from LPW * w.
-template <int DIM> struct WaveFoot {
+// NW waves share a tile in a scatter: each takes a run of the tile's cells, in sorted order, that is a
+// layer z or half of one in 3D (NW = 4 or 8) and two rows y in 2D (NW = 4). The wave's copy of the
+// footprint covers the planes and rows that its cells reach.
+template <int DIM, int NW> struct WaveFoot {
     using G = TileGeom<DIM>;
-    static constexpr int LPW = (DIM == 3 ? G::TZ : G::TY) / NW;     // layers of cells per wave
-    static_assert(LPW * NW == (DIM == 3 ? G::TZ : G::TY), "tile layers against the waves per block");
-    static constexpr int WX = G::FX, LAYERS = LPW + 3;
-    // words from one layer to the next: in 3D chosen so that the 64 additions of one instruction of a
-    // matrix-core scatter fall on few banks more than twice (the least for 64 doubles)
-    static constexpr int LAYER = DIM == 3 ? WX * G::FY + (G::TX == 8 ? 1 : 0) : WX;
-    static constexpr int SIZE = LAYERS * LAYER;
+    static constexpr int RW = DIM == 3 ? G::TY * G::TZ / NW : G::TY / NW;       // rows of cells per wave
+    static_assert(RW > 0 && G::TY % RW == 0 && RW * NW == (DIM == 3 ? G::TY * G::TZ : G::TY), "whole rows of a layer");
+    static constexpr int WPZ = G::TY / RW;                                      // waves per layer (3D)
+    static constexpr int WX = G::FX, WY = RW + 3, WZ = DIM == 3 ? 4 : 1;
+    static constexpr int PLANE = WX * WY;
+    static constexpr int SIZE = PLANE * WZ;
+    // first footprint row and plane of wave w
+    static __device__ __forceinline__ int y0(int w) { return DIM == 3 ? w % WPZ * RW : w * RW; }
+    static __device__ __forceinline__ int z0(int w) { return DIM == 3 ? w / WPZ : 0; }
 };
 
 // Scatters on the matrix cores. A cell's sums over its particles at the candidate nodes are a
@@ -850,8 +860,8 @@ template <int DIM> struct WaveFoot {
 // shape factors), stages their factors in its own LDS rows and scatters its own cells, so no barrier
 // stands between loads, factors and sums and the waves of a CU overlap them. The rows hold WREC
 // records, so that three blocks fit in a CU's LDS. On the 128^3 J2 block the mass scatter went from
-// 0.65 to 0.36 ms per launch, the force scatter from 0.83 to 0.55 and the particle update from 0.92
-// to 0.67; on 86k lCPDI particles from 0.13, 0.18 and 0.18 to 0.075, 0.073 and 0.090.
+// 0.65 to 0.35 ms per launch, the force scatter from 0.83 to 0.53 and the particle update from 0.92
+// to 0.60; on 87k lCPDI particles from 0.13, 0.18 and 0.18 to 0.059, 0.059 and 0.070.
 typedef double mat4d __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ void lds_add(double *a, double v) {
@@ -869,7 +879,7 @@ __device__ __forceinline__ void wave_sync() {
 // The cells of a wave taken one after another as their particles are staged. bounds: lane it holds the
 // start of the wave's it-th cell, lane it + ITS its end; it: the cell reached; open: its sums (in the
 // caller's registers) have begun; at: its offset in the wave's copy.
-template <int DIM> struct WaveCells {
+template <int DIM, int NW> struct WaveCells {
     static constexpr int ITS = TileGeom<DIM>::NC / NW;
     static_assert(ITS <= 32, "bounds held by the lanes of a wave");
     int bounds, it, at;
@@ -883,6 +893,8 @@ template <int DIM> struct WaveCells {
         b = start(0);
         e = end(ITS - 1);
     }
+    // the particle of sorted slot k (none beyond the wave's)
+    __device__ __forceinline__ int particle(const KBins &B, int k) const { return k < e ? B.order[k] : -1; }
     __device__ __forceinline__ int start(int i) const { return __builtin_amdgcn_readlane(bounds, i); }
     __device__ __forceinline__ int end(int i) const { return __builtin_amdgcn_readlane(bounds, i + ITS); }
 };
@@ -890,10 +902,10 @@ template <int DIM> struct WaveCells {
 // visits the cells with particles among the staged slots r0..r1-1: first(kb, ke, open) begins a cell
 // with particles kb..ke-1 of them (open: the one before it still has to be added to the copy),
 // more(kb, ke) goes on with one that an earlier round began
-template <int DIM, typename First, typename More>
-__device__ __forceinline__ void wave_walk(WaveCells<DIM> &W, int r0, int r1, First first, More more) {
+template <int DIM, int NW, typename First, typename More>
+__device__ __forceinline__ void wave_walk(WaveCells<DIM, NW> &W, int r0, int r1, First first, More more) {
     using G = TileGeom<DIM>;
-    while (W.it < WaveCells<DIM>::ITS) {
+    while (W.it < WaveCells<DIM, NW>::ITS) {
         const int s = W.start(W.it), e = W.end(W.it);
         if (s >= r1) break;
         const int kb = max(s, r0) - r0, ke = min(e, r1) - r0;
@@ -902,7 +914,7 @@ __device__ __forceinline__ void wave_walk(WaveCells<DIM> &W, int r0, int r1, Fir
             else {
                 first(kb, ke, W.open);
                 W.open = true;
-                W.at = (W.it / G::TX) * WaveFoot<DIM>::WX + W.it % G::TX;
+                W.at = (W.it / G::TX) * WaveFoot<DIM, NW>::WX + W.it % G::TX;
             }
         }
         if (e > r1) break;
@@ -922,8 +934,8 @@ struct NoExtra {
 template <int DIM> struct MatSums { typedef mat4d T; };     // of one component block of a cell, per lane
 template <> struct MatSums<2> { typedef double T; };
 
-template <int DIM, int NQ, int PPR, int STR> struct WaveScatter {
-    using F = WaveFoot<DIM>;
+template <int DIM, int NW, int NQ, int PPR, int STR> struct WaveScatter {
+    using F = WaveFoot<DIM, NW>;
     static constexpr int NB = (NQ + 3) / 4;
     const double *plo, *phi;    // this lane's record of a quad in the rows of its lo and hi candidate
     double *acc;
@@ -939,7 +951,7 @@ template <int DIM, int NQ, int PPR, int STR> struct WaveScatter {
         phi = S + hi * STR + k4;
         // 3D: result register r, lane l: node (ix = k4, iy = r, iz = hi) of component lo (block 1: 4 + lo);
         // 2D: lane l: node (ix = k4, iy = hi)
-        acc = &s_acc[w][lo < NQ ? lo : 0][hi * F::LAYER + k4];
+        acc = &s_acc[w][lo < NQ ? lo : 0][hi * (DIM == 3 ? F::PLANE : F::WX) + k4];
     }
     __device__ __forceinline__ Quad read(int k) const {
         Quad t;
@@ -976,7 +988,7 @@ template <int DIM, int NQ, int PPR, int STR> struct WaveScatter {
         }
     }
     // particles r0..r1-1 are staged, from record 0; extra(kb, ke, lo, hi, k4, c) after each cell's sums
-    template <typename Extra> __device__ __forceinline__ void scatter(WaveCells<DIM> &W, int r0, int r1, Extra extra) {
+    template <typename Extra> __device__ __forceinline__ void scatter(WaveCells<DIM, NW> &W, int r0, int r1, Extra extra) {
         auto add = [&](int k, int e) {
 #pragma unroll 1
             for (; k < e; k += 4) fold(load(k, e));
@@ -996,8 +1008,8 @@ template <int DIM, int NQ, int PPR, int STR> struct WaveScatter {
                 extra(kb, ke, lo, hi, k4, c[0]);
             });
     }
-    __device__ __forceinline__ void scatter(WaveCells<DIM> &W, int r0, int r1) { scatter(W, r0, r1, NoExtra()); }
-    __device__ __forceinline__ void finish(const WaveCells<DIM> &W) const {
+    __device__ __forceinline__ void scatter(WaveCells<DIM, NW> &W, int r0, int r1) { scatter(W, r0, r1, NoExtra()); }
+    __device__ __forceinline__ void finish(const WaveCells<DIM, NW> &W) const {
         if (W.open) flush(W.at);
     }
 };
@@ -1007,8 +1019,8 @@ template <int DIM, int NQ, int PPR, int STR> struct WaveScatter {
 // products above, with rows X'Y, XY' and XY and columns Z a_q0, Z a_q1 and Z' a_q2 (2D: two). F: 4*DIM
 // rows of (factor, derivative) pairs [axis*4 + candidate][record]; a: the terms' rows; both STR apart.
 // With loads (FX) e holds 3 rows of pFext, added times XYZ, and trac adds a particle's own nodal forces.
-template <int DIM, bool FX, int STR> struct WaveForce {
-    using F = WaveFoot<DIM>;
+template <int DIM, int NW, bool FX, int STR> struct WaveForce {
+    using F = WaveFoot<DIM, NW>;
     const double2 *flo, *fhi;
     const double *a0, *a1, *a2, *eq;
     double *acc;
@@ -1030,7 +1042,7 @@ template <int DIM, bool FX, int STR> struct WaveForce {
         a2 = a + (DIM == 2 ? 0 : q == 0 ? 4 : q == 1 ? 5 : 3) * STR + k4;
         eq = FX ? e + q * STR + k4 : nullptr;
         // 3D: result register r, lane l: node (ix = k4, iy = r, iz = hi); 2D: lane l: node (ix = k4, iy = hi)
-        acc = &s_acc[w][q][hi * F::LAYER + k4];
+        acc = &s_acc[w][q][hi * (DIM == 3 ? F::PLANE : F::WX) + k4];
     }
     __device__ __forceinline__ Quad read(int k) const {
         Quad t;
@@ -1065,7 +1077,7 @@ template <int DIM, bool FX, int STR> struct WaveForce {
             for (int r = 0; r < 4; r++) lds_add(acc + at + r * F::WX, c[r]);
         } else lds_add(acc + at, c);
     }
-    template <typename Trac> __device__ __forceinline__ void scatter(WaveCells<DIM> &W, int r0, int r1, Trac trac) {
+    template <typename Trac> __device__ __forceinline__ void scatter(WaveCells<DIM, NW> &W, int r0, int r1, Trac trac) {
         auto add = [&](int k, int e) {
 #pragma unroll 1
             for (; k < e; k += 4) fold(load(k, e));
@@ -1084,47 +1096,49 @@ template <int DIM, bool FX, int STR> struct WaveForce {
                 if (FX) trac(kb, ke, q, hi, k4, c);
             });
     }
-    __device__ __forceinline__ void finish(const WaveCells<DIM> &W) const {
+    __device__ __forceinline__ void finish(const WaveCells<DIM, NW> &W) const {
         if (W.open) flush(W.at);
     }
 };
 
 // a wave's own copy (the wave's later LDS instructions follow in order)
-template <int DIM, int NQ>
-__device__ __forceinline__ void zero_wave_acc(double (*s_acc)[NQ][WaveFoot<DIM>::SIZE]) {
+template <int DIM, int NW, int NQ>
+__device__ __forceinline__ void zero_wave_acc(double (*s_acc)[NQ][(WaveFoot<DIM, NW>::SIZE)]) {
     double *a = &s_acc[threadIdx.x >> 6][0][0];
-    for (int i = threadIdx.x & 63; i < NQ * WaveFoot<DIM>::SIZE; i += 64) a[i] = 0.;
+    for (int i = threadIdx.x & 63; i < NQ * WaveFoot<DIM, NW>::SIZE; i += 64) a[i] = 0.;
     wave_sync();
 }
 
 // add the wave copies that cover each footprint node in wave order and store the tile's sums
-template <int DIM, int NQ>
-__device__ __forceinline__ void write_partials(const KNodes &N, int t, double (*s_acc)[NQ][WaveFoot<DIM>::SIZE]) {
+template <int DIM, int NW, int NQ>
+__device__ __forceinline__ void write_partials(const KNodes &N, int t, double (*s_acc)[NQ][WaveFoot<DIM, NW>::SIZE]) {
     using G = TileGeom<DIM>;
-    using W = WaveFoot<DIM>;
-    for (int s = threadIdx.x; s < G::FOOT; s += NT) {
-        const int in = DIM == 3 ? s % (G::FX * G::FY) : s % G::FX, layer = DIM == 3 ? s / (G::FX * G::FY) : s / G::FX;
+    using W = WaveFoot<DIM, NW>;
+    for (int s = threadIdx.x; s < G::FOOT; s += 64 * NW) {
+        const int x = s % G::FX, y = DIM == 3 ? s / G::FX % G::FY : s / G::FX, z = DIM == 3 ? s / (G::FX * G::FY) : 0;
+        // every copy is read (a read in place of those that lack the node), so the reads are in flight together
+        int at[NW];
+#pragma unroll
+        for (int w = 0; w < NW; w++) {
+            const int r = y - W::y0(w), c = z - W::z0(w);
+            at[w] = r < 0 || r >= W::WY || c < 0 || c >= W::WZ ? -1 : c * W::PLANE + r * W::WX + x;
+        }
 #pragma unroll
         for (int q = 0; q < NQ; q++) {
-            double v = 0.;
-            bool first = true;
+            double a[NW], v = 0.;
 #pragma unroll
-            for (int w = 0; w < NW; w++) {
-                const int c = layer - W::LPW * w;
-                if (c < 0 || c >= W::LAYERS) continue;
-                const double a = s_acc[w][q][c * W::LAYER + in];
-                v = first ? a : v + a;
-                first = false;
-            }
+            for (int w = 0; w < NW; w++) a[w] = s_acc[w][q][at[w] < 0 ? 0 : at[w]];
+#pragma unroll
+            for (int w = 0; w < NW; w++) v = at[w] < 0 ? v : v + a[w];
             N.part[((size_t)t * NQMAX + q) * G::FOOT + s] = v;
         }
     }
 }
 
-template <int DIM>
+template <int DIM, int NTB = NT>
 __device__ __forceinline__ void load_tile_starts(const KBins &B, int t, int *s_cs) {
     using G = TileGeom<DIM>;
-    for (int i = threadIdx.x; i <= G::NC; i += NT) s_cs[i] = B.cellStart[t * G::NC + i];
+    for (int i = threadIdx.x; i <= G::NC; i += NTB) s_cs[i] = B.cellStart[t * G::NC + i];
     __syncthreads();
 }
 
@@ -1137,9 +1151,9 @@ __device__ __forceinline__ void load_tile_starts(const KBins &B, int t, int *s_c
 template <int DIM> struct MassWords { int p, key; double x[DIM], m, v[DIM]; };
 
 template <int DIM>
-__device__ __forceinline__ void load_mass_words(const KPart &rows, const KBins &B, int k, int e, MassWords<DIM> &t) {
+__device__ __forceinline__ void load_mass_words(const KPart &rows, const KBins &B, int p, MassWords<DIM> &t) {
     const KPart P = local_rows(rows);
-    t.p = k < e ? B.order[k] : -1;
+    t.p = p;
     if (t.p < 0) return;
     t.key = B.key[t.p];
 #pragma unroll
@@ -1165,27 +1179,29 @@ __device__ __forceinline__ void stage_factors(double (*S)[WROW], int i, const Ax
 }
 
 template <int DIM>
-__global__ __launch_bounds__(NT, G2P_WAVES) void k_p2g_mass(KGrid g0, KPart P, KBins B, KNodes N) {
+__global__ __launch_bounds__(64 * UGIMP_NW, WAVES4) void k_p2g_mass(KGrid g0, KPart P, KBins B, KNodes N) {
     using G = TileGeom<DIM>;
+    constexpr int NW = UGIMP_NW;
     __shared__ int s_cs[G::NC + 1];
     __shared__ double s_S[NW][4 * DIM + 4][WROW];       // per wave: [axis*4 + offset][record], then mass and momentum
-    __shared__ double s_acc[NW][NQ_MASS][WaveFoot<DIM>::SIZE];
+    __shared__ double s_acc[NW][NQ_MASS][WaveFoot<DIM, NW>::SIZE];
     const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
     auto tile = [&](const int tall) {      // (field, context tile) pair
         const int tc = tall % g0.tilesTotal;
         const GridPtr gp = tile_grid_ptr(g0, tc);
         const KGrid g = grid_copy(gp);
-        load_tile_starts<DIM>(B, tall, s_cs);
+        load_tile_starts<DIM, 64 * NW>(B, tall, s_cs);
         if (s_cs[0] == s_cs[G::NC]) return;
         int ox, oy, oz;
         tile_origin<DIM>(g, tc - g.tileBase, ox, oy, oz);
-        WaveCells<DIM> W;
+        WaveCells<DIM, NW> W;
         W.begin(s_cs);
-        WaveScatter<DIM, NQ_MASS, 1, WROW> sc;
+        WaveScatter<DIM, NW, NQ_MASS, 1, WROW> sc;
         sc.begin(&s_S[w][0][0], s_acc);
         MassWords<DIM> cur;
-        load_mass_words<DIM>(P, B, W.b + l, W.e, cur);
-        zero_wave_acc<DIM, NQ_MASS>(s_acc);
+        int ahead = W.particle(B, W.b + 64 + l);       // the order is read a round before the words
+        load_mass_words<DIM>(P, B, W.particle(B, W.b + l), cur);
+        zero_wave_acc<DIM, NW, NQ_MASS>(s_acc);
         for (int r = W.b; r < W.e; r += 64) {
             AxisFactors f[DIM];
             double u[4];
@@ -1201,7 +1217,10 @@ __global__ __launch_bounds__(NT, G2P_WAVES) void k_p2g_mass(KGrid g0, KPart P, K
             for (int r0 = r; r0 < min(r + 64, W.e); r0 += WREC) {
                 if (l / WREC == (r0 - r) / WREC && cur.p >= 0) stage_factors<DIM, 4>(s_S[w], l % WREC, f, u);
                 // the next particles' loads pass over the last scatter
-                if (r0 + WREC >= min(r + 64, W.e)) load_mass_words<DIM>(P, B, r + 64 + l, W.e, cur);
+                if (r0 + WREC >= min(r + 64, W.e)) {
+                    load_mass_words<DIM>(P, B, ahead, cur);
+                    ahead = W.particle(B, r + 2 * 64 + l);
+                }
                 wave_sync();
                 sc.scatter(W, r0, min(r0 + WREC, W.e));
                 wave_sync();
@@ -1209,7 +1228,7 @@ __global__ __launch_bounds__(NT, G2P_WAVES) void k_p2g_mass(KGrid g0, KPart P, K
         }
         sc.finish(W);
         __syncthreads();
-        write_partials<DIM, NQ_MASS>(N, tall, s_acc);
+        write_partials<DIM, NW, NQ_MASS>(N, tall, s_acc);
     };
     for_each_tile(B, tile);
 }
@@ -1227,9 +1246,9 @@ __device__ __forceinline__ void load_deformation(const KPart &P, int p, double e
 template <int DIM> struct CornerMassWords { int p, key; double x[DIM], m, v[DIM], ep[6], wr[3]; };
 
 template <int DIM>
-__device__ __forceinline__ void load_corner_mass(const KPart &rows, const KBins &B, int k, int e, CornerMassWords<DIM> &t) {
+__device__ __forceinline__ void load_corner_mass(const KPart &rows, const KBins &B, int p, CornerMassWords<DIM> &t) {
     const KPart P = local_rows(rows);
-    t.p = k < e ? B.order[k] : -1;
+    t.p = p;
     if (t.p < 0) return;
     t.key = B.key[t.p];
 #pragma unroll
@@ -1242,27 +1261,29 @@ __device__ __forceinline__ void load_corner_mass(const KPart &rows, const KBins 
 }
 
 template <int DIM>
-__global__ __launch_bounds__(NT, G2P_WAVES) void k_p2g_mass_corners(KGrid g0, KPart P, KBins B, KNodes N, KStats st) {
+__global__ __launch_bounds__(64 * CORNER_NW(DIM), WAVES8) void k_p2g_mass_corners(KGrid g0, KPart P, KBins B, KNodes N, KStats st) {
     using G = TileGeom<DIM>;
+    constexpr int NW = CORNER_NW(DIM);
     __shared__ int s_cs[G::NC + 1];
     __shared__ double s_S[NW][4 * DIM + 4][WROW];       // per wave: [axis*4 + offset][corner], then mass and momentum over 64
-    __shared__ double s_acc[NW][NQ_MASS][WaveFoot<DIM>::SIZE];
+    __shared__ double s_acc[NW][NQ_MASS][WaveFoot<DIM, NW>::SIZE];
     const int w = threadIdx.x >> 6, l = threadIdx.x & 63, i = l / Corners<DIM>::N, c = l % Corners<DIM>::N;
     auto tile = [&](const int tall) {      // (field, context tile) pair
         const int tc = tall % g0.tilesTotal;
         const GridPtr gp = tile_grid_ptr(g0, tc);
         const KGrid g = grid_copy(gp);
-        load_tile_starts<DIM>(B, tall, s_cs);
+        load_tile_starts<DIM, 64 * NW>(B, tall, s_cs);
         if (s_cs[0] == s_cs[G::NC]) return;
         int ox, oy, oz;
         tile_origin<DIM>(g, tc - g.tileBase, ox, oy, oz);
-        WaveCells<DIM> W;
+        WaveCells<DIM, NW> W;
         W.begin(s_cs);
-        WaveScatter<DIM, NQ_MASS, Corners<DIM>::N, WROW> sc;
+        WaveScatter<DIM, NW, NQ_MASS, Corners<DIM>::N, WROW> sc;
         sc.begin(&s_S[w][0][0], s_acc);
         CornerMassWords<DIM> cur;
-        load_corner_mass<DIM>(P, B, W.b + i, W.e, cur);
-        zero_wave_acc<DIM, NQ_MASS>(s_acc);
+        int ahead = W.particle(B, W.b + Corners<DIM>::PB + i);       // the order is read a round before the words
+        load_corner_mass<DIM>(P, B, W.particle(B, W.b + i), cur);
+        zero_wave_acc<DIM, NW, NQ_MASS>(s_acc);
         for (int r = W.b; r < W.e; r += Corners<DIM>::PB) {
             double xi[3], u[4];
             int off[3];
@@ -1289,7 +1310,10 @@ __global__ __launch_bounds__(NT, G2P_WAVES) void k_p2g_mass_corners(KGrid g0, KP
             for (int r0 = r; r0 < min(r + Corners<DIM>::PB, W.e); r0 += WREC / Corners<DIM>::N) {
                 if (l / WREC == (r0 - r) / (WREC / Corners<DIM>::N) && cur.p >= 0) stage_corner<DIM, 4>(s_S[w], l % WREC, xi, off, u);
                 // the next particles' loads pass over the last scatter
-                if (r0 + WREC / Corners<DIM>::N >= min(r + Corners<DIM>::PB, W.e)) load_corner_mass<DIM>(P, B, r + Corners<DIM>::PB + i, W.e, cur);
+                if (r0 + WREC / Corners<DIM>::N >= min(r + Corners<DIM>::PB, W.e)) {
+                    load_corner_mass<DIM>(P, B, ahead, cur);
+                    ahead = W.particle(B, r + 2 * Corners<DIM>::PB + i);
+                }
                 wave_sync();
                 sc.scatter(W, r0, min(r0 + WREC / Corners<DIM>::N, W.e));
                 wave_sync();
@@ -1297,7 +1321,7 @@ __global__ __launch_bounds__(NT, G2P_WAVES) void k_p2g_mass_corners(KGrid g0, KP
         }
         sc.finish(W);
         __syncthreads();
-        write_partials<DIM, NQ_MASS>(N, tall, s_acc);
+        write_partials<DIM, NW, NQ_MASS>(N, tall, s_acc);
     };
     for_each_tile(B, tile);
 }
@@ -1671,9 +1695,9 @@ __device__ __forceinline__ void add_tractions(const KLoads &L, const int *tt, in
 template <int DIM> struct ForceWords { int p, key; double x[DIM], m, pr, s[6]; };
 
 template <int DIM>
-__device__ __forceinline__ void load_force_words(const KPart &rows, const KBins &B, int k, int e, ForceWords<DIM> &t) {
+__device__ __forceinline__ void load_force_words(const KPart &rows, const KBins &B, int p, ForceWords<DIM> &t) {
     const KPart P = local_rows(rows);
-    t.p = k < e ? B.order[k] : -1;
+    t.p = p;
     if (t.p < 0) return;
     t.key = B.key[t.p];
 #pragma unroll
@@ -1685,15 +1709,16 @@ __device__ __forceinline__ void load_force_words(const KPart &rows, const KBins 
 }
 
 template <int DIM, bool FX>
-__global__ __launch_bounds__(NT, FX ? 2 : G2P_WAVES) void k_p2g_force(KGrid g0, KPart P, KBins B, KNodes N, KLoads L,
+__global__ __launch_bounds__(64 * UGIMP_NW, FX ? 2 : WAVES4) void k_p2g_force(KGrid g0, KPart P, KBins B, KNodes N, KLoads L,
                                                                        const int *loaded) {
     using G = TileGeom<DIM>;
+    constexpr int NW = UGIMP_NW;
     __shared__ int s_cs[G::NC + 1];
     __shared__ double2 s_F[NW][4 * DIM][WROW]; // per wave: [axis*4 + offset][record] (factor, derivative)
     __shared__ double s_a[NW][6][WROW];
     __shared__ double s_e[FX ? NW : 1][3][WROW];   // pFext of the staged particles
     __shared__ int s_tt[FX ? NW : 1][WREC];        // their traction tables (-1: none)
-    __shared__ double s_acc[NW][NQ_FORCE][WaveFoot<DIM>::SIZE];
+    __shared__ double s_acc[NW][NQ_FORCE][WaveFoot<DIM, NW>::SIZE];
     const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
     auto tile = [&](const int tall) {      // (field, context tile) pair
         // with loads: the launch with the load term takes the marked tiles, the other the rest
@@ -1701,23 +1726,25 @@ __global__ __launch_bounds__(NT, FX ? 2 : G2P_WAVES) void k_p2g_force(KGrid g0, 
         const int tc = tall % g0.tilesTotal;
         const GridPtr gp = tile_grid_ptr(g0, tc);
         const KGrid g = grid_copy(gp);
-        load_tile_starts<DIM>(B, tall, s_cs);
+        load_tile_starts<DIM, 64 * NW>(B, tall, s_cs);
         if (s_cs[0] == s_cs[G::NC]) return;
         int ox, oy, oz;
         tile_origin<DIM>(g, tc - g.tileBase, ox, oy, oz);
-        WaveCells<DIM> W;
+        WaveCells<DIM, NW> W;
         W.begin(s_cs);
-        WaveForce<DIM, FX, WROW> sc;
+        WaveForce<DIM, NW, FX, WROW> sc;
         sc.begin(&s_F[w][0][0], &s_a[w][0][0], &s_e[FX ? w : 0][0][0], s_acc);
         // tractions: lane (q, iz, ix), in 2D (q, iy, ix), adds the tables of the cell's particles to its nodes
         auto trac = [&](int kb, int ke, int q, int hi, int ix, auto &c) {
             if (L.nt == 0) return;
             add_tractions(L, s_tt[FX ? w : 0], kb, ke, q, hi, ix, c);
         };
-        zero_wave_acc<DIM, NQ_FORCE>(s_acc);
+        zero_wave_acc<DIM, NW, NQ_FORCE>(s_acc);
+        int ahead = W.particle(B, W.b + l);
         for (int r = W.b; r < W.e; r += 64) {
             ForceWords<DIM> cur;        // (loading them a round ahead costs the registers of the third wave per SIMD)
-            load_force_words<DIM>(P, B, r + l, W.e, cur);
+            load_force_words<DIM>(P, B, ahead, cur);
+            ahead = W.particle(B, r + 64 + l);
             AxisFactors f[DIM];
             double invd[DIM], s[6];
             if (cur.p >= 0) {
@@ -1751,7 +1778,7 @@ __global__ __launch_bounds__(NT, FX ? 2 : G2P_WAVES) void k_p2g_force(KGrid g0, 
         }
         sc.finish(W);
         __syncthreads();
-        write_partials<DIM, NQ_FORCE>(N, tall, s_acc);
+        write_partials<DIM, NW, NQ_FORCE>(N, tall, s_acc);
     };
     for_each_tile(B, tile);
 }
@@ -1760,9 +1787,9 @@ __global__ __launch_bounds__(NT, FX ? 2 : G2P_WAVES) void k_p2g_force(KGrid g0, 
 template <int DIM> struct CornerForceWords { int p, key; double x[DIM], m, pr, s[6], r[9]; };
 
 template <int DIM>
-__device__ __forceinline__ void load_corner_force(const KPart &rows, const KBins &B, int k, int e, CornerForceWords<DIM> &t) {
+__device__ __forceinline__ void load_corner_force(const KPart &rows, const KBins &B, int p, CornerForceWords<DIM> &t) {
     const KPart P = local_rows(rows);
-    t.p = k < e ? B.order[k] : -1;
+    t.p = p;
     if (t.p < 0) return;
     t.key = B.key[t.p];
 #pragma unroll
@@ -1776,34 +1803,36 @@ __device__ __forceinline__ void load_corner_force(const KPart &rows, const KBins
 }
 
 template <int DIM, bool FX>
-__global__ __launch_bounds__(NT, FX ? 2 : G2P_WAVES) void k_p2g_force_corners(KGrid g0, KPart P, KBins B, KNodes N, KLoads L,
+__global__ __launch_bounds__(64 * CORNER_NW(DIM), FX ? 2 : WAVES8) void k_p2g_force_corners(KGrid g0, KPart P, KBins B, KNodes N, KLoads L,
                                                                         const int *loaded) {
     using G = TileGeom<DIM>;
+    constexpr int NW = CORNER_NW(DIM);
     __shared__ int s_cs[G::NC + 1];
     __shared__ double s_S[NW][4 * DIM + 4][WROW];
     __shared__ int s_tt[FX ? NW : 1][WREC / Corners<DIM>::N];    // traction tables of the staged particles (-1: none)
-    __shared__ double s_acc[NW][NQ_FORCE][WaveFoot<DIM>::SIZE];
+    __shared__ double s_acc[NW][NQ_FORCE][WaveFoot<DIM, NW>::SIZE];
     const int w = threadIdx.x >> 6, l = threadIdx.x & 63, i = l / Corners<DIM>::N, c = l % Corners<DIM>::N;
     auto tile = [&](const int tall) {      // (field, context tile) pair
         if (loaded && (loaded[tall] != 0) != FX) return;
         const int tc = tall % g0.tilesTotal;
         const GridPtr gp = tile_grid_ptr(g0, tc);
         const KGrid g = grid_copy(gp);
-        load_tile_starts<DIM>(B, tall, s_cs);
+        load_tile_starts<DIM, 64 * NW>(B, tall, s_cs);
         if (s_cs[0] == s_cs[G::NC]) return;
         int ox, oy, oz;
         tile_origin<DIM>(g, tc - g.tileBase, ox, oy, oz);
-        WaveCells<DIM> W;
+        WaveCells<DIM, NW> W;
         W.begin(s_cs);
-        WaveScatter<DIM, NQ_FORCE, Corners<DIM>::N, WROW> sc;
+        WaveScatter<DIM, NW, NQ_FORCE, Corners<DIM>::N, WROW> sc;
         sc.begin(&s_S[w][0][0], s_acc);
         auto trac = [&](int kb, int ke, int q, int hi, int ix, auto &f) {
             if (!FX || L.nt == 0) return;
             add_tractions(L, s_tt[FX ? w : 0], kb, ke, q, hi, ix, f);
         };
-        zero_wave_acc<DIM, NQ_FORCE>(s_acc);
+        zero_wave_acc<DIM, NW, NQ_FORCE>(s_acc);
         CornerForceWords<DIM> cur;
-        load_corner_force<DIM>(P, B, W.b + i, W.e, cur);
+        int ahead = W.particle(B, W.b + Corners<DIM>::PB + i);       // the order is read a round before the words
+        load_corner_force<DIM>(P, B, W.particle(B, W.b + i), cur);
         for (int r = W.b; r < W.e; r += Corners<DIM>::PB) {
             double xi[3], u[3];
             int off[3], tt = -1;
@@ -1836,7 +1865,10 @@ __global__ __launch_bounds__(NT, FX ? 2 : G2P_WAVES) void k_p2g_force_corners(KG
                     stage_corner<DIM, 3>(s_S[w], l % WREC, xi, off, u);
                     if (FX && c == 0) s_tt[FX ? w : 0][i % (WREC / Corners<DIM>::N)] = tt;
                 }
-                if (r0 + WREC / Corners<DIM>::N >= min(r + Corners<DIM>::PB, W.e)) load_corner_force<DIM>(P, B, r + Corners<DIM>::PB + i, W.e, cur);
+                if (r0 + WREC / Corners<DIM>::N >= min(r + Corners<DIM>::PB, W.e)) {
+                    load_corner_force<DIM>(P, B, ahead, cur);
+                    ahead = W.particle(B, r + 2 * Corners<DIM>::PB + i);
+                }
                 wave_sync();
                 sc.scatter(W, r0, min(r0 + WREC / Corners<DIM>::N, W.e), trac);
                 wave_sync();
@@ -1844,7 +1876,7 @@ __global__ __launch_bounds__(NT, FX ? 2 : G2P_WAVES) void k_p2g_force_corners(KG
         }
         sc.finish(W);
         __syncthreads();
-        write_partials<DIM, NQ_FORCE>(N, tall, s_acc);
+        write_partials<DIM, NW, NQ_FORCE>(N, tall, s_acc);
     };
     for_each_tile(B, tile);
 }
@@ -1917,11 +1949,11 @@ __device__ __forceinline__ void gather_window(const int w[3], const double Sw[3]
 
 // footprint velocities and accelerations f/m (zero outside the grid and on nodes without mass, which
 // no particle of the tile touches)
-template <int DIM>
+template <int DIM, int NW>
 __device__ __forceinline__ void load_foot_va(const KGrid &g, const KNodes &Nf, int ox, int oy, int oz,
                                              double (*s_n)[TileGeom<DIM>::FOOT]) {
     const long long nn = g.nstride;
-    for (int s = threadIdx.x; s < TileGeom<DIM>::FOOT; s += NT) {
+    for (int s = threadIdx.x; s < TileGeom<DIM>::FOOT; s += 64 * NW) {
         const long long n = foot_node<DIM>(g, s, ox, oy, oz);
         const double m = n >= 0 ? Nf.mass[n] : 0.;
         const double r = m > 0. ? 1. / m : 0.;
@@ -1935,11 +1967,11 @@ __device__ __forceinline__ void load_foot_va(const KGrid &g, const KNodes &Nf, i
 
 // the same as (velocity, acceleration) pairs, one 16-byte LDS read each (the gather's reads kept the
 // LDS busy for almost half of the kernel's time)
-template <int DIM>
+template <int DIM, int NW>
 __device__ __forceinline__ void load_foot_pairs(const KGrid &g, const KNodes &Nf, int ox, int oy, int oz,
                                                 double2 (*s_n)[TileGeom<DIM>::FOOT]) {
     const long long nn = g.nstride;
-    for (int s = threadIdx.x; s < TileGeom<DIM>::FOOT; s += NT) {
+    for (int s = threadIdx.x; s < TileGeom<DIM>::FOOT; s += 64 * NW) {
         const long long n = foot_node<DIM>(g, s, ox, oy, oz);
         const double m = n >= 0 ? Nf.mass[n] : 0.;
         const double r = m > 0. ? 1. / m : 0.;
@@ -1978,11 +2010,11 @@ __device__ __forceinline__ void gather_pairs(const int w[3], const double Sw[3][
 }
 
 // footprint XPIC increments (zero outside the grid and on nodes without particles)
-template <int DIM>
+template <int DIM, int NW>
 __device__ __forceinline__ void load_foot_prev(const KGrid &g, const KNodes &Nf, int ox, int oy, int oz,
                                                double (*s_n)[TileGeom<DIM>::FOOT]) {
     const long long nn = g.nstride;
-    for (int s = threadIdx.x; s < TileGeom<DIM>::FOOT; s += NT) {
+    for (int s = threadIdx.x; s < TileGeom<DIM>::FOOT; s += 64 * NW) {
         const long long n = foot_node<DIM>(g, s, ox, oy, oz);
         const bool on = n >= 0 && Nf.cnt[n] > 0;
 #pragma unroll
@@ -2058,13 +2090,14 @@ __device__ __forceinline__ void store_move(const KPart &rows, int p, const doubl
 
 // uGIMP and classic: a wave gathers, moves and scatters its particles 64 at a time
 template <int DIM, int MOVE>
-__global__ __launch_bounds__(NT, G2P_WAVES) void k_g2p_p2g(KGrid g0, KPart P, KBins B, KNodes N, const MpmMaterial *mats,
+__global__ __launch_bounds__(64 * G2P_NW(DIM), WAVES8) void k_g2p_p2g(KGrid g0, KPart P, KBins B, KNodes N, const MpmMaterial *mats,
                                                             int mode) {
     using G = TileGeom<DIM>;
+    constexpr int NW = G2P_NW(DIM);
     __shared__ int s_cs[G::NC + 1];
     __shared__ double2 s_n[3][G::FOOT];        // (velocity, f/m) of each component
     __shared__ double s_S[NW][4 * DIM + 4][WROW];       // [axis*4 + offset][record], then the momentum (the last row is not used)
-    __shared__ double s_acc[NW][NQ_MOM][WaveFoot<DIM>::SIZE];
+    __shared__ double s_acc[NW][NQ_MOM][WaveFoot<DIM, NW>::SIZE];
     const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
     auto tile = [&](const int tall) {      // (field, context tile) pair
         const int fld = tall / g0.tilesTotal;
@@ -2072,18 +2105,19 @@ __global__ __launch_bounds__(NT, G2P_WAVES) void k_g2p_p2g(KGrid g0, KPart P, KB
         const GridPtr gp = tile_grid_ptr(g0, tc);
         const KGrid g = grid_copy(gp);
         const KNodes Nf = field_view(g, N, fld);
-        load_tile_starts<DIM>(B, tall, s_cs);
+        load_tile_starts<DIM, 64 * NW>(B, tall, s_cs);
         if (s_cs[0] == s_cs[G::NC]) return;
         int ox, oy, oz;
         tile_origin<DIM>(g, tc - g.tileBase, ox, oy, oz);
-        WaveCells<DIM> W;
+        WaveCells<DIM, NW> W;
         W.begin(s_cs);
-        WaveScatter<DIM, NQ_MOM, 1, WROW> sc;
+        WaveScatter<DIM, NW, NQ_MOM, 1, WROW> sc;
         sc.begin(&s_S[w][0][0], s_acc);
         MassWords<DIM> cur;
-        load_mass_words<DIM>(P, B, W.b + l, W.e, cur);
-        load_foot_pairs<DIM>(g, Nf, ox, oy, oz, s_n);
-        zero_wave_acc<DIM, NQ_MOM>(s_acc);
+        int ahead = W.particle(B, W.b + 64 + l);       // the order is read a round before the words
+        load_mass_words<DIM>(P, B, W.particle(B, W.b + l), cur);
+        load_foot_pairs<DIM, NW>(g, Nf, ox, oy, oz, s_n);
+        zero_wave_acc<DIM, NW, NQ_MOM>(s_acc);
         __syncthreads();
         for (int r = W.b; r < W.e; r += 64) {
             AxisFactors f[DIM];
@@ -2107,7 +2141,10 @@ __global__ __launch_bounds__(NT, G2P_WAVES) void k_g2p_p2g(KGrid g0, KPart P, KB
             for (int r0 = r; r0 < min(r + 64, W.e); r0 += WREC) {
                 if (l / WREC == (r0 - r) / WREC && cur.p >= 0) stage_factors<DIM, 3>(s_S[w], l % WREC, f, u);
                 // the next particles' loads pass over the last scatter
-                if (r0 + WREC >= min(r + 64, W.e)) load_mass_words<DIM>(P, B, r + 64 + l, W.e, cur);
+                if (r0 + WREC >= min(r + 64, W.e)) {
+                    load_mass_words<DIM>(P, B, ahead, cur);
+                    ahead = W.particle(B, r + 2 * 64 + l);
+                }
                 wave_sync();
                 sc.scatter(W, r0, min(r0 + WREC, W.e));
                 wave_sync();
@@ -2115,7 +2152,7 @@ __global__ __launch_bounds__(NT, G2P_WAVES) void k_g2p_p2g(KGrid g0, KPart P, KB
         }
         sc.finish(W);
         __syncthreads();
-        write_partials<DIM, NQ_MOM>(N, tall, s_acc);
+        write_partials<DIM, NW, NQ_MOM>(N, tall, s_acc);
     };
     for_each_tile(B, tile);
 }
@@ -2124,9 +2161,9 @@ __global__ __launch_bounds__(NT, G2P_WAVES) void k_g2p_p2g(KGrid g0, KPart P, KB
 template <int DIM> struct CornerMoveWords { int p, key; double x[DIM], m, v[DIM], r[9]; };
 
 template <int DIM>
-__device__ __forceinline__ void load_corner_move(const KPart &rows, const KBins &B, int k, int e, CornerMoveWords<DIM> &t) {
+__device__ __forceinline__ void load_corner_move(const KPart &rows, const KBins &B, int p, CornerMoveWords<DIM> &t) {
     const KPart P = local_rows(rows);
-    t.p = k < e ? B.order[k] : -1;
+    t.p = p;
     if (t.p < 0) return;
     t.key = B.key[t.p];
 #pragma unroll
@@ -2140,13 +2177,14 @@ __device__ __forceinline__ void load_corner_move(const KPart &rows, const KBins 
 }
 
 template <int DIM, int MOVE>
-__global__ __launch_bounds__(NT, G2P_WAVES) void k_g2p_p2g_corners(KGrid g0, KPart P, KBins B, KNodes N,
+__global__ __launch_bounds__(64 * CORNER_NW(DIM), WAVES8) void k_g2p_p2g_corners(KGrid g0, KPart P, KBins B, KNodes N,
                                                              const MpmMaterial *mats, int mode) {
     using G = TileGeom<DIM>;
+    constexpr int NW = CORNER_NW(DIM);
     __shared__ int s_cs[G::NC + 1];
     __shared__ double s_n[6][G::FOOT];         // v(3), f/m(3)
     __shared__ double s_S[NW][4 * DIM + 4][WROW];
-    __shared__ double s_acc[NW][NQ_MOM][WaveFoot<DIM>::SIZE];
+    __shared__ double s_acc[NW][NQ_MOM][WaveFoot<DIM, NW>::SIZE];
     const int w = threadIdx.x >> 6, l = threadIdx.x & 63, i = l / Corners<DIM>::N, c = l % Corners<DIM>::N;
     auto tile = [&](const int tall) {      // (field, context tile) pair
         const int fld = tall / g0.tilesTotal;
@@ -2154,18 +2192,19 @@ __global__ __launch_bounds__(NT, G2P_WAVES) void k_g2p_p2g_corners(KGrid g0, KPa
         const GridPtr gp = tile_grid_ptr(g0, tc);
         const KGrid g = grid_copy(gp);
         const KNodes Nf = field_view(g, N, fld);
-        load_tile_starts<DIM>(B, tall, s_cs);
+        load_tile_starts<DIM, 64 * NW>(B, tall, s_cs);
         if (s_cs[0] == s_cs[G::NC]) return;
         int ox, oy, oz;
         tile_origin<DIM>(g, tc - g.tileBase, ox, oy, oz);
-        WaveCells<DIM> W;
+        WaveCells<DIM, NW> W;
         W.begin(s_cs);
-        WaveScatter<DIM, NQ_MOM, Corners<DIM>::N, WROW> sc;
+        WaveScatter<DIM, NW, NQ_MOM, Corners<DIM>::N, WROW> sc;
         sc.begin(&s_S[w][0][0], s_acc);
         CornerMoveWords<DIM> cur;
-        load_corner_move<DIM>(P, B, W.b + i, W.e, cur);
-        load_foot_va<DIM>(g, Nf, ox, oy, oz, s_n);
-        zero_wave_acc<DIM, NQ_MOM>(s_acc);
+        int ahead = W.particle(B, W.b + Corners<DIM>::PB + i);       // the order is read a round before the words
+        load_corner_move<DIM>(P, B, W.particle(B, W.b + i), cur);
+        load_foot_va<DIM, NW>(g, Nf, ox, oy, oz, s_n);
+        zero_wave_acc<DIM, NW, NQ_MOM>(s_acc);
         __syncthreads();
         for (int r = W.b; r < W.e; r += Corners<DIM>::PB) {
             double xi[3], u[3];
@@ -2188,7 +2227,10 @@ __global__ __launch_bounds__(NT, G2P_WAVES) void k_g2p_p2g_corners(KGrid g0, KPa
             }
             for (int r0 = r; r0 < min(r + Corners<DIM>::PB, W.e); r0 += WREC / Corners<DIM>::N) {
                 if (l / WREC == (r0 - r) / (WREC / Corners<DIM>::N) && cur.p >= 0) stage_corner<DIM, 3>(s_S[w], l % WREC, xi, off, u);
-                if (r0 + WREC / Corners<DIM>::N >= min(r + Corners<DIM>::PB, W.e)) load_corner_move<DIM>(P, B, r + Corners<DIM>::PB + i, W.e, cur);
+                if (r0 + WREC / Corners<DIM>::N >= min(r + Corners<DIM>::PB, W.e)) {
+                    load_corner_move<DIM>(P, B, ahead, cur);
+                    ahead = W.particle(B, r + 2 * Corners<DIM>::PB + i);
+                }
                 wave_sync();
                 sc.scatter(W, r0, min(r0 + WREC / Corners<DIM>::N, W.e));
                 wave_sync();
@@ -2196,7 +2238,7 @@ __global__ __launch_bounds__(NT, G2P_WAVES) void k_g2p_p2g_corners(KGrid g0, KPa
         }
         sc.finish(W);
         __syncthreads();
-        write_partials<DIM, NQ_MOM>(N, tall, s_acc);
+        write_partials<DIM, NW, NQ_MOM>(N, tall, s_acc);
     };
     for_each_tile(B, tile);
 }
@@ -2276,12 +2318,13 @@ __global__ void k_xpic_init(KGrid g0, KBins B, KNodes N, int fmpm) {
 // start, as in every pass of the step.
 // uGIMP and classic: a wave gathers and scatters its particles 64 at a time
 template <int DIM>
-__global__ __launch_bounds__(NT, G2P_WAVES) void k_xpic_p2g(KGrid g0, KPart P, KBins B, KNodes N) {
+__global__ __launch_bounds__(64 * UGIMP_NW, WAVES4) void k_xpic_p2g(KGrid g0, KPart P, KBins B, KNodes N) {
     using G = TileGeom<DIM>;
+    constexpr int NW = UGIMP_NW;
     __shared__ int s_cs[G::NC + 1];
     __shared__ double s_n[3][G::FOOT];         // vprev
     __shared__ double s_S[NW][4 * DIM + 4][WROW];       // [axis*4 + offset][record], then the momentum (the last row is not used)
-    __shared__ double s_acc[NW][NQ_MOM][WaveFoot<DIM>::SIZE];
+    __shared__ double s_acc[NW][NQ_MOM][WaveFoot<DIM, NW>::SIZE];
     const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
     auto tile = [&](const int tall) {      // (field, context tile) pair
         const int fld = tall / g0.tilesTotal;
@@ -2289,18 +2332,19 @@ __global__ __launch_bounds__(NT, G2P_WAVES) void k_xpic_p2g(KGrid g0, KPart P, K
         const GridPtr gp = tile_grid_ptr(g0, tc);
         const KGrid g = grid_copy(gp);
         const KNodes Nf = field_view(g, N, fld);
-        load_tile_starts<DIM>(B, tall, s_cs);
+        load_tile_starts<DIM, 64 * NW>(B, tall, s_cs);
         if (s_cs[0] == s_cs[G::NC]) return;
         int ox, oy, oz;
         tile_origin<DIM>(g, tc - g.tileBase, ox, oy, oz);
-        WaveCells<DIM> W;
+        WaveCells<DIM, NW> W;
         W.begin(s_cs);
-        WaveScatter<DIM, NQ_MOM, 1, WROW> sc;
+        WaveScatter<DIM, NW, NQ_MOM, 1, WROW> sc;
         sc.begin(&s_S[w][0][0], s_acc);
         MassWords<DIM> cur;
-        load_mass_words<DIM>(P, B, W.b + l, W.e, cur);
-        load_foot_prev<DIM>(g, Nf, ox, oy, oz, s_n);
-        zero_wave_acc<DIM, NQ_MOM>(s_acc);
+        int ahead = W.particle(B, W.b + 64 + l);       // the order is read a round before the words
+        load_mass_words<DIM>(P, B, W.particle(B, W.b + l), cur);
+        load_foot_prev<DIM, NW>(g, Nf, ox, oy, oz, s_n);
+        zero_wave_acc<DIM, NW, NQ_MOM>(s_acc);
         __syncthreads();
         for (int r = W.b; r < W.e; r += 64) {
             AxisFactors f[DIM];
@@ -2319,7 +2363,10 @@ __global__ __launch_bounds__(NT, G2P_WAVES) void k_xpic_p2g(KGrid g0, KPart P, K
             for (int r0 = r; r0 < min(r + 64, W.e); r0 += WREC) {
                 if (l / WREC == (r0 - r) / WREC && cur.p >= 0) stage_factors<DIM, 3>(s_S[w], l % WREC, f, u);
                 // the next particles' loads pass over the last scatter
-                if (r0 + WREC >= min(r + 64, W.e)) load_mass_words<DIM>(P, B, r + 64 + l, W.e, cur);
+                if (r0 + WREC >= min(r + 64, W.e)) {
+                    load_mass_words<DIM>(P, B, ahead, cur);
+                    ahead = W.particle(B, r + 2 * 64 + l);
+                }
                 wave_sync();
                 sc.scatter(W, r0, min(r0 + WREC, W.e));
                 wave_sync();
@@ -2327,18 +2374,19 @@ __global__ __launch_bounds__(NT, G2P_WAVES) void k_xpic_p2g(KGrid g0, KPart P, K
         }
         sc.finish(W);
         __syncthreads();
-        write_partials<DIM, NQ_MOM>(N, tall, s_acc);
+        write_partials<DIM, NW, NQ_MOM>(N, tall, s_acc);
     };
     for_each_tile(B, tile);
 }
 
 template <int DIM>
-__global__ __launch_bounds__(NT, G2P_WAVES) void k_xpic_p2g_corners(KGrid g0, KPart P, KBins B, KNodes N) {
+__global__ __launch_bounds__(64 * CORNER_NW(DIM), WAVES8) void k_xpic_p2g_corners(KGrid g0, KPart P, KBins B, KNodes N) {
     using G = TileGeom<DIM>;
+    constexpr int NW = CORNER_NW(DIM);
     __shared__ int s_cs[G::NC + 1];
     __shared__ double s_n[3][G::FOOT];         // vprev
     __shared__ double s_S[NW][4 * DIM + 4][WROW];
-    __shared__ double s_acc[NW][NQ_MOM][WaveFoot<DIM>::SIZE];
+    __shared__ double s_acc[NW][NQ_MOM][WaveFoot<DIM, NW>::SIZE];
     const int w = threadIdx.x >> 6, l = threadIdx.x & 63, i = l / Corners<DIM>::N, c = l % Corners<DIM>::N;
     auto tile = [&](const int tall) {      // (field, context tile) pair
         const int fld = tall / g0.tilesTotal;
@@ -2346,18 +2394,19 @@ __global__ __launch_bounds__(NT, G2P_WAVES) void k_xpic_p2g_corners(KGrid g0, KP
         const GridPtr gp = tile_grid_ptr(g0, tc);
         const KGrid g = grid_copy(gp);
         const KNodes Nf = field_view(g, N, fld);
-        load_tile_starts<DIM>(B, tall, s_cs);
+        load_tile_starts<DIM, 64 * NW>(B, tall, s_cs);
         if (s_cs[0] == s_cs[G::NC]) return;
         int ox, oy, oz;
         tile_origin<DIM>(g, tc - g.tileBase, ox, oy, oz);
-        WaveCells<DIM> W;
+        WaveCells<DIM, NW> W;
         W.begin(s_cs);
-        WaveScatter<DIM, NQ_MOM, Corners<DIM>::N, WROW> sc;
+        WaveScatter<DIM, NW, NQ_MOM, Corners<DIM>::N, WROW> sc;
         sc.begin(&s_S[w][0][0], s_acc);
         CornerMoveWords<DIM> cur;
-        load_corner_move<DIM>(P, B, W.b + i, W.e, cur);
-        load_foot_prev<DIM>(g, Nf, ox, oy, oz, s_n);
-        zero_wave_acc<DIM, NQ_MOM>(s_acc);
+        int ahead = W.particle(B, W.b + Corners<DIM>::PB + i);       // the order is read a round before the words
+        load_corner_move<DIM>(P, B, W.particle(B, W.b + i), cur);
+        load_foot_prev<DIM, NW>(g, Nf, ox, oy, oz, s_n);
+        zero_wave_acc<DIM, NW, NQ_MOM>(s_acc);
         __syncthreads();
         for (int r = W.b; r < W.e; r += Corners<DIM>::PB) {
             double xi[3], u[3];
@@ -2373,7 +2422,10 @@ __global__ __launch_bounds__(NT, G2P_WAVES) void k_xpic_p2g_corners(KGrid g0, KP
             }
             for (int r0 = r; r0 < min(r + Corners<DIM>::PB, W.e); r0 += WREC / Corners<DIM>::N) {
                 if (l / WREC == (r0 - r) / (WREC / Corners<DIM>::N) && cur.p >= 0) stage_corner<DIM, 3>(s_S[w], l % WREC, xi, off, u);
-                if (r0 + WREC / Corners<DIM>::N >= min(r + Corners<DIM>::PB, W.e)) load_corner_move<DIM>(P, B, r + Corners<DIM>::PB + i, W.e, cur);
+                if (r0 + WREC / Corners<DIM>::N >= min(r + Corners<DIM>::PB, W.e)) {
+                    load_corner_move<DIM>(P, B, ahead, cur);
+                    ahead = W.particle(B, r + 2 * Corners<DIM>::PB + i);
+                }
                 wave_sync();
                 sc.scatter(W, r0, min(r0 + WREC / Corners<DIM>::N, W.e));
                 wave_sync();
@@ -2381,7 +2433,7 @@ __global__ __launch_bounds__(NT, G2P_WAVES) void k_xpic_p2g_corners(KGrid g0, KP
         }
         sc.finish(W);
         __syncthreads();
-        write_partials<DIM, NQ_MOM>(N, tall, s_acc);
+        write_partials<DIM, NW, NQ_MOM>(N, tall, s_acc);
     };
     for_each_tile(B, tile);
 }
@@ -2581,9 +2633,9 @@ template <int DIM> struct ContactWords { int p, key; double x[DIM], m, ep[6], wr
 
 template <int DIM>
 __device__ __forceinline__ void load_contact_words(const KPart &rows, const KBins &B, const MpmMaterial *mats, int newPositions,
-                                                   int k, int e, ContactWords<DIM> &t) {
+                                                   int p, ContactWords<DIM> &t) {
     const KPart P = local_rows(rows);
-    t.p = k < e ? B.order[k] : -1;
+    t.p = p;
     if (t.p < 0) return;
     t.key = B.key[t.p];
 #pragma unroll
@@ -2597,30 +2649,32 @@ __device__ __forceinline__ void load_contact_words(const KPart &rows, const KBin
 }
 
 template <int DIM, int SH>
-__global__ __launch_bounds__(NT, MPM_TILE_SHAPE == 0 ? 2 : 1) void k_p2g_contact(KGrid g0, KPart P, KBins B, KNodes N, const MpmMaterial *mats,
+__global__ __launch_bounds__(64 * UGIMP_NW, MPM_TILE_SHAPE == 0 ? 2 : 1) void k_p2g_contact(KGrid g0, KPart P, KBins B, KNodes N, const MpmMaterial *mats,
                                                         int newPositions) {
     using G = TileGeom<DIM>;
+    constexpr int NW = UGIMP_NW;
     constexpr bool CP = SH == MPMGPU_SHAPE_LCPDI;
     constexpr int PPR = CP ? Corners<DIM>::N : 4, PB = 64 / PPR;     // records per particle, particles per 64 lanes
     __shared__ int s_cs[G::NC + 1];
     __shared__ double s_S[NW][4 * DIM + 8][WROW];
-    __shared__ double s_acc[NW][NQ_CONTACT][WaveFoot<DIM>::SIZE];
+    __shared__ double s_acc[NW][NQ_CONTACT][WaveFoot<DIM, NW>::SIZE];
     const int w = threadIdx.x >> 6, l = threadIdx.x & 63, i = l / PPR, c = l % PPR;
     auto tile = [&](const int tall) {      // (field, context tile) pair
         const int tc = tall % g0.tilesTotal;
         const GridPtr gp = tile_grid_ptr(g0, tc);
         const KGrid g = grid_copy(gp);
-        load_tile_starts<DIM>(B, tall, s_cs);
+        load_tile_starts<DIM, 64 * NW>(B, tall, s_cs);
         if (s_cs[0] == s_cs[G::NC]) return;
         int ox, oy, oz;
         tile_origin<DIM>(g, tc - g.tileBase, ox, oy, oz);
-        WaveCells<DIM> W;
+        WaveCells<DIM, NW> W;
         W.begin(s_cs);
-        WaveScatter<DIM, NQ_CONTACT, PPR, WROW> sc;
+        WaveScatter<DIM, NW, NQ_CONTACT, PPR, WROW> sc;
         sc.begin(&s_S[w][0][0], s_acc);
         ContactWords<DIM> cur;
-        load_contact_words<DIM>(P, B, mats, newPositions, W.b + i, W.e, cur);
-        zero_wave_acc<DIM, NQ_CONTACT>(s_acc);
+        int ahead = W.particle(B, W.b + PB + i);       // the order is read a round before the words
+        load_contact_words<DIM>(P, B, mats, newPositions, W.particle(B, W.b + i), cur);
+        zero_wave_acc<DIM, NW, NQ_CONTACT>(s_acc);
         for (int r = W.b; r < W.e; r += PB) {
             double xi[3], u[NQ_CONTACT], invd[DIM];
             int off[3];
@@ -2671,8 +2725,10 @@ __global__ __launch_bounds__(NT, MPM_TILE_SHAPE == 0 ? 2 : 1) void k_p2g_contact
                         for (int q = 0; q < NQ_CONTACT; q++) s_S[w][4 * DIM + q][l % WREC] = u[q];
                     }
                 }
-                if (r0 + WREC / PPR >= min(r + PB, W.e))
-                    load_contact_words<DIM>(P, B, mats, newPositions, r + PB + i, W.e, cur);
+                if (r0 + WREC / PPR >= min(r + PB, W.e)) {
+                    load_contact_words<DIM>(P, B, mats, newPositions, ahead, cur);
+                    ahead = W.particle(B, r + 2 * PB + i);
+                }
                 wave_sync();
                 sc.scatter(W, r0, min(r0 + WREC / PPR, W.e));
                 wave_sync();
@@ -2680,7 +2736,7 @@ __global__ __launch_bounds__(NT, MPM_TILE_SHAPE == 0 ? 2 : 1) void k_p2g_contact
         }
         sc.finish(W);
         __syncthreads();
-        write_partials<DIM, NQ_CONTACT>(N, tall, s_acc);
+        write_partials<DIM, NW, NQ_CONTACT>(N, tall, s_acc);
     };
     for_each_tile(B, tile);
 }
@@ -3053,6 +3109,7 @@ __device__ __forceinline__ double lr_radius(const KGrid &g, const KPart &P, int 
 template <int DIM, int SH>
 __global__ __launch_bounds__(NT) void k_contact_normals(KGrid g, KPart P, KBins B, KNodes N, const MpmMaterial *mats,
                                                         KStats st, int newPos) {
+    constexpr int NW = NT / 64;
     __shared__ int s_list[NW][LR_MAX];
     const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
     int *list = s_list[w];
@@ -3320,7 +3377,8 @@ static KBins tile_bins(const KBins &b, int slot) {
     r.slot = slot;
     return r;
 }
-#define TILE_LAUNCH(KERNEL, B, S, ...) hipLaunchKernelGGL(KERNEL, tile_grid_dim(B), dim3(NT), 0, S, __VA_ARGS__)
+#define TILE_LAUNCH_NT(NT, KERNEL, B, S, ...) hipLaunchKernelGGL(KERNEL, tile_grid_dim(B), dim3(NT), 0, S, __VA_ARGS__)
+#define TILE_LAUNCH(KERNEL, B, S, ...) TILE_LAUNCH_NT(NT, KERNEL, B, S, __VA_ARGS__)
 
 void launch_p2g_mass(int dim, const KGrid &g, const KPart &p, const KBins &b, const KNodes &nd,
                      const MpmMaterial *mats, const KStats &st, hipStream_t s) {
@@ -3328,11 +3386,11 @@ void launch_p2g_mass(int dim, const KGrid &g, const KPart &p, const KBins &b, co
     (void)mats;
     const bool cp = g.shape == MPMGPU_SHAPE_LCPDI;
     if (dim == 3) {
-        if (cp) TILE_LAUNCH(k_p2g_mass_corners<3>, tb, s, g, p, tb, nd, st);
-        else TILE_LAUNCH(k_p2g_mass<3>, tb, s, g, p, tb, nd);
+        if (cp) TILE_LAUNCH_NT(64 * CORNER_NW(3), k_p2g_mass_corners<3>, tb, s, g, p, tb, nd, st);
+        else TILE_LAUNCH_NT(64 * UGIMP_NW, k_p2g_mass<3>, tb, s, g, p, tb, nd);
     } else {
-        if (cp) TILE_LAUNCH(k_p2g_mass_corners<2>, tb, s, g, p, tb, nd, st);
-        else TILE_LAUNCH(k_p2g_mass<2>, tb, s, g, p, tb, nd);
+        if (cp) TILE_LAUNCH_NT(64 * CORNER_NW(2), k_p2g_mass_corners<2>, tb, s, g, p, tb, nd, st);
+        else TILE_LAUNCH_NT(64 * UGIMP_NW, k_p2g_mass<2>, tb, s, g, p, tb, nd);
     }
 }
 
@@ -3571,19 +3629,19 @@ void launch_p2g_force(int dim, const KGrid &g, const KPart &p, const KBins &b, c
         loaded = L.tflag[par];
         const KBins tl = tile_bins(b, TILE_SLOT_FORCE_LOADS);
         if (dim == 3) {
-            if (cp) TILE_LAUNCH((k_p2g_force_corners<3, true>), tl, s, g, p, tl, nd, L, loaded);
-            else TILE_LAUNCH((k_p2g_force<3, true>), tl, s, g, p, tl, nd, L, loaded);
+            if (cp) TILE_LAUNCH_NT(64 * CORNER_NW(3), (k_p2g_force_corners<3, true>), tl, s, g, p, tl, nd, L, loaded);
+            else TILE_LAUNCH_NT(64 * UGIMP_NW, (k_p2g_force<3, true>), tl, s, g, p, tl, nd, L, loaded);
         } else {
-            if (cp) TILE_LAUNCH((k_p2g_force_corners<2, true>), tl, s, g, p, tl, nd, L, loaded);
-            else TILE_LAUNCH((k_p2g_force<2, true>), tl, s, g, p, tl, nd, L, loaded);
+            if (cp) TILE_LAUNCH_NT(64 * CORNER_NW(2), (k_p2g_force_corners<2, true>), tl, s, g, p, tl, nd, L, loaded);
+            else TILE_LAUNCH_NT(64 * UGIMP_NW, (k_p2g_force<2, true>), tl, s, g, p, tl, nd, L, loaded);
         }
     }
     if (dim == 3) {
-        if (cp) TILE_LAUNCH((k_p2g_force_corners<3, false>), tb, s, g, p, tb, nd, L, loaded);
-        else TILE_LAUNCH((k_p2g_force<3, false>), tb, s, g, p, tb, nd, L, loaded);
+        if (cp) TILE_LAUNCH_NT(64 * CORNER_NW(3), (k_p2g_force_corners<3, false>), tb, s, g, p, tb, nd, L, loaded);
+        else TILE_LAUNCH_NT(64 * UGIMP_NW, (k_p2g_force<3, false>), tb, s, g, p, tb, nd, L, loaded);
     } else {
-        if (cp) TILE_LAUNCH((k_p2g_force_corners<2, false>), tb, s, g, p, tb, nd, L, loaded);
-        else TILE_LAUNCH((k_p2g_force<2, false>), tb, s, g, p, tb, nd, L, loaded);
+        if (cp) TILE_LAUNCH_NT(64 * CORNER_NW(2), (k_p2g_force_corners<2, false>), tb, s, g, p, tb, nd, L, loaded);
+        else TILE_LAUNCH_NT(64 * UGIMP_NW, (k_p2g_force<2, false>), tb, s, g, p, tb, nd, L, loaded);
     }
 }
 
@@ -3597,11 +3655,11 @@ static void g2p_move(int dim, const KGrid &g, const KPart &p, const KBins &tb, c
                      const MpmMaterial *mats, int mode, hipStream_t s) {
     const bool cp = g.shape == MPMGPU_SHAPE_LCPDI;
     if (dim == 3) {
-        if (cp) TILE_LAUNCH((k_g2p_p2g_corners<3, MOVE>), tb, s, g, p, tb, nd, mats, mode);
-        else TILE_LAUNCH((k_g2p_p2g<3, MOVE>), tb, s, g, p, tb, nd, mats, mode);
+        if (cp) TILE_LAUNCH_NT(64 * CORNER_NW(3), (k_g2p_p2g_corners<3, MOVE>), tb, s, g, p, tb, nd, mats, mode);
+        else TILE_LAUNCH_NT(64 * G2P_NW(3), (k_g2p_p2g<3, MOVE>), tb, s, g, p, tb, nd, mats, mode);
     } else {
-        if (cp) TILE_LAUNCH((k_g2p_p2g_corners<2, MOVE>), tb, s, g, p, tb, nd, mats, mode);
-        else TILE_LAUNCH((k_g2p_p2g<2, MOVE>), tb, s, g, p, tb, nd, mats, mode);
+        if (cp) TILE_LAUNCH_NT(64 * CORNER_NW(2), (k_g2p_p2g_corners<2, MOVE>), tb, s, g, p, tb, nd, mats, mode);
+        else TILE_LAUNCH_NT(64 * G2P_NW(2), (k_g2p_p2g<2, MOVE>), tb, s, g, p, tb, nd, mats, mode);
     }
 }
 
@@ -3657,11 +3715,11 @@ void launch_p2g_contact(int dim, const KGrid &g, const KPart &p, const KBins &b,
     int np = newPositions ? 1 : 0;
     const bool cp = g.shape == MPMGPU_SHAPE_LCPDI;
     if (dim == 3) {
-        if (cp) TILE_LAUNCH((k_p2g_contact<3, MPMGPU_SHAPE_LCPDI>), tb, s, g, p, tb, nd, mats, np);
-        else TILE_LAUNCH((k_p2g_contact<3, MPMGPU_SHAPE_UGIMP>), tb, s, g, p, tb, nd, mats, np);
+        if (cp) TILE_LAUNCH_NT(64 * UGIMP_NW, (k_p2g_contact<3, MPMGPU_SHAPE_LCPDI>), tb, s, g, p, tb, nd, mats, np);
+        else TILE_LAUNCH_NT(64 * UGIMP_NW, (k_p2g_contact<3, MPMGPU_SHAPE_UGIMP>), tb, s, g, p, tb, nd, mats, np);
     } else {
-        if (cp) TILE_LAUNCH((k_p2g_contact<2, MPMGPU_SHAPE_LCPDI>), tb, s, g, p, tb, nd, mats, np);
-        else TILE_LAUNCH((k_p2g_contact<2, MPMGPU_SHAPE_UGIMP>), tb, s, g, p, tb, nd, mats, np);
+        if (cp) TILE_LAUNCH_NT(64 * UGIMP_NW, (k_p2g_contact<2, MPMGPU_SHAPE_LCPDI>), tb, s, g, p, tb, nd, mats, np);
+        else TILE_LAUNCH_NT(64 * UGIMP_NW, (k_p2g_contact<2, MPMGPU_SHAPE_UGIMP>), tb, s, g, p, tb, nd, mats, np);
     }
 }
 
@@ -3802,12 +3860,12 @@ void launch_xpic(int dim, const KGrid &g, const KPart &p, const KBins &b, const 
     else hipLaunchKernelGGL(k_xpic_init<2>, ng, blk, 0, s, g, b, nd, fmpm ? 1 : 0);
     for (int it = 2; it <= order; it++) {
         if (dim == 3) {
-            if (cp) TILE_LAUNCH(k_xpic_p2g_corners<3>, tb, s, g, p, tb, nd);
-            else TILE_LAUNCH(k_xpic_p2g<3>, tb, s, g, p, tb, nd);
+            if (cp) TILE_LAUNCH_NT(64 * CORNER_NW(3), k_xpic_p2g_corners<3>, tb, s, g, p, tb, nd);
+            else TILE_LAUNCH_NT(64 * UGIMP_NW, k_xpic_p2g<3>, tb, s, g, p, tb, nd);
             hipLaunchKernelGGL(k_xpic_node<3>, ng, blk, 0, s, g, tb, nd);
         } else {
-            if (cp) TILE_LAUNCH(k_xpic_p2g_corners<2>, tb, s, g, p, tb, nd);
-            else TILE_LAUNCH(k_xpic_p2g<2>, tb, s, g, p, tb, nd);
+            if (cp) TILE_LAUNCH_NT(64 * CORNER_NW(2), k_xpic_p2g_corners<2>, tb, s, g, p, tb, nd);
+            else TILE_LAUNCH_NT(64 * UGIMP_NW, k_xpic_p2g<2>, tb, s, g, p, tb, nd);
             hipLaunchKernelGGL(k_xpic_node<2>, ng, blk, 0, s, g, tb, nd);
         }
         if (bc.nb) MPM_KNS::launch_vel_bcs(g, nd, bc, forcePass && !fmpm ? BC_PASS_XPIC_FORCE : BC_PASS_XPIC, par, s);
