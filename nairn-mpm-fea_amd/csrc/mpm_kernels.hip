@@ -634,72 +634,167 @@ __global__ void k_bin_keys(KGrid g0, KPart P, KBins B) {
     wave_count(B.count, key);
 }
 
-#define SCAN_PER_THREAD 4
-#define SCAN_BLOCK (NT * SCAN_PER_THREAD)
+// Cell starts, in one launch: blocks take runs of SCAN_BLOCK keys in the order in which they start
+// (a ticket), publish their sum, and add up the sums before theirs until they meet a block that has
+// published its whole prefix (decoupled look-back; a block waits for blocks that started before it
+// only, so every wait ends). A run holds whole tiles, so its threads also list the non-empty ones.
+// state: 2 flag bits and 30 bits of sum (fewer than 2^30 particles fit in the device's memory), zeroed
+// with the ticket by k_bin_sort_cells. Three scan launches and a fourth for the list took 20 us of a
+// step on 885k particles (0.7M keys) and 11 on 4k; this one takes 10 and 6. It is latency: tickets on one
+// address, then one look at the sums of up to 256 blocks before; runs of 8,192 keys (four times the
+// tickets) took 20 us instead of 12 on 2.1M keys, and scans by shuffles instead of data-parallel moves 14.
+#define SCAN_NT 1024
+#define SCAN_ROUNDS 8              // of 256 keys per wave, four a lane
+#define SCAN_BLOCK (SCAN_NT * 4 * SCAN_ROUNDS)
+#define SCAN_SUM 0x40000000u
+#define SCAN_PREFIX 0x80000000u
+#define SCAN_VALUE 0x3fffffffu
 
-__device__ __forceinline__ int block_exclusive_scan(int v, int *s_tmp, int &total) {
-    // Hillis-Steele over the block in LDS
-    int tid = threadIdx.x;
-    s_tmp[tid] = v;
+__device__ __forceinline__ unsigned scan_wait(const unsigned *state) {
+    unsigned v;
+    while (!((v = __hip_atomic_load(state, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) & (SCAN_SUM | SCAN_PREFIX)))
+        __builtin_amdgcn_s_sleep(1);
+    return v;
+}
+
+// a lane's neighbour's value by a data-parallel move (zero where there is none)
+template <int CTRL, int ROWS = 0xf> __device__ __forceinline__ int dpp_int(int v) {
+    return __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xf, false);
+}
+// inclusive sum over the wave's lanes: within rows of 16, then each row's total to those after it
+__device__ __forceinline__ int wave_inclusive(int v) {
+    v += dpp_int<0x111>(v);
+    v += dpp_int<0x112>(v);
+    v += dpp_int<0x114>(v);
+    v += dpp_int<0x118>(v);
+    v += dpp_int<0x142, 0xa>(v);
+    v += dpp_int<0x143, 0xc>(v);
+    return v;
+}
+// sum over the aligned 16 or 32 lanes, in each of them
+template <int LANES> __device__ __forceinline__ int lanes_sum(int v) {
+    static_assert(LANES == 16 || LANES == 32, "a row or two");
+    v += dpp_int<0xB1>(v);
+    v += dpp_int<0x4E>(v);
+    v += dpp_int<0x141>(v);
+    v += dpp_int<0x140>(v);
+    return LANES == 32 ? v + __shfl_xor(v, 16) : v;
+}
+
+template <int NC>
+__global__ __launch_bounds__(SCAN_NT) void k_bin_scan(KBins B, int n, int nb) {
+    static_assert(256 % NC == 0 && 64 % (NC / 4) == 0, "whole tiles");
+    __shared__ int s_sum[SCAN_NT / 64];
+    __shared__ int s_block, s_before;
+    unsigned *state = reinterpret_cast<unsigned *>(B.blockSums);
+    const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
+    if (threadIdx.x == 0) s_block = atomicAdd(&B.blockSums[nb], 1);
     __syncthreads();
-    for (int off = 1; off < NT; off <<= 1) {
-        int add = tid >= off ? s_tmp[tid - off] : 0;
-        __syncthreads();
-        s_tmp[tid] += add;
-        __syncthreads();
+    const int blk = s_block, base = blk * SCAN_BLOCK + w * (256 * SCAN_ROUNDS) + l * 4;   // of this lane's first round
+    if (blk >= nb) return;               // (a ticket is taken once per block, so this does not happen)
+    const bool stopped = B.stop[0] != 0;
+    if (blk == 0) {
+        // the tile list is rebuilt; the tile kernels' cursors start again; one more step completed
+        if (threadIdx.x < TILE_SLOTS * 8) B.work[threadIdx.x * TILE_SLOT_STRIDE] = 0;
+        if (threadIdx.x == 0) {
+            __hip_atomic_store(B.ntiles, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (!stopped) B.stop[2] += 1;
+        }
     }
-    total = s_tmp[NT - 1];
-    int incl = s_tmp[tid];
+    int v[SCAN_ROUNDS][4], own[SCAN_ROUNDS], ex[SCAN_ROUNDS], sum = 0;     // keys, their sum, the wave's sum before
+#pragma unroll
+    for (int r = 0; r < SCAN_ROUNDS; r++) {
+        const int at = base + 256 * r;
+        if (at + 4 <= n) __builtin_memcpy(v[r], B.count + at, sizeof(v[r]));
+        else {
+#pragma unroll
+            for (int i = 0; i < 4; i++) v[r][i] = at + i < n ? B.count[at + i] : 0;
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < SCAN_ROUNDS; r++) {
+        own[r] = v[r][0] + v[r][1] + v[r][2] + v[r][3];
+        const int incl = wave_inclusive(own[r]);
+        ex[r] = sum + incl - own[r];
+        sum += __builtin_amdgcn_readlane(incl, 63);
+    }
+    if (l == 0) s_sum[w] = sum;
     __syncthreads();
-    return incl - v;
-}
-
-__global__ __launch_bounds__(NT) void k_scan_blocks(const int *in, int *out, int *blockSums, int n) {
-    __shared__ int s_tmp[NT];
-    int base = blockIdx.x * SCAN_BLOCK + threadIdx.x * SCAN_PER_THREAD;
-    int v[SCAN_PER_THREAD];
-    int sum = 0;
+    if (w == 0) {
+        // the waves' sums, then the sums of the blocks before
+        const int t = l < SCAN_NT / 64 ? s_sum[l] : 0, ti = wave_inclusive(t), total = __builtin_amdgcn_readlane(ti, 63);
+        if (l < SCAN_NT / 64) s_sum[l] = ti - t;
+        int before = 0;
+        if (blk > 0) {
+            if (l == 0)
+                __hip_atomic_store(&state[blk], SCAN_SUM | (unsigned)total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            // four blocks a lane, nearest first; those behind a whole prefix are in it already
+            int part = 0;
+            for (int at = blk - 1 - 4 * l;; at -= 256) {
+                unsigned s[4];
 #pragma unroll
-    for (int i = 0; i < SCAN_PER_THREAD; i++) {
-        v[i] = base + i < n ? in[base + i] : 0;
-        sum += v[i];
-    }
-    int total;
-    int ex = block_exclusive_scan(sum, s_tmp, total);
+                for (int i = 0; i < 4; i++) s[i] = at - i >= 0 ? scan_wait(&state[at - i]) : SCAN_PREFIX;
+                bool end = false;
+                int own = 0;
 #pragma unroll
-    for (int i = 0; i < SCAN_PER_THREAD; i++) {
-        if (base + i < n) out[base + i] = ex;
-        ex += v[i];
+                for (int i = 0; i < 4; i++) {
+                    own += end ? 0 : (int)(s[i] & SCAN_VALUE);
+                    end = end || (s[i] & SCAN_PREFIX);
+                }
+                const unsigned long long ends = __ballot(end);
+                if (l <= (ends ? __ffsll((long long)ends) - 1 : 63)) part += own;
+                if (ends) break;
+            }
+            before = __builtin_amdgcn_readlane(wave_inclusive(part), 63);
+            // the tile list's length was cleared by the first block: its prefix, or one that follows
+            // from it, has been read
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+        }
+        if (l == 0) {
+            __hip_atomic_store(&state[blk], SCAN_PREFIX | (unsigned)(before + total), __ATOMIC_RELEASE,
+                               __HIP_MEMORY_SCOPE_AGENT);
+            s_before = before;
+        }
     }
-    if (threadIdx.x == 0) blockSums[blockIdx.x] = total;
-}
-
-__global__ __launch_bounds__(NT) void k_scan_sums(int *blockSums, int nb, int *ntiles) {
-    __shared__ int s_tmp[NT];
-    if (threadIdx.x == 0) ntiles[0] = 0;      // the tile list is rebuilt after the scan
-    int carry = 0;
-    for (int b0 = 0; b0 < nb; b0 += NT) {
-        int i = b0 + threadIdx.x;
-        int v = i < nb ? blockSums[i] : 0;
-        int total;
-        int ex = block_exclusive_scan(v, s_tmp, total);
-        if (i < nb) blockSums[i] = ex + carry;
-        carry += total;
+    __syncthreads();
+    const int before = s_before + s_sum[w];
+    constexpr int TL = NC / 4;         // lanes of a tile; its first one lists it
+    unsigned on = 0;                   // per round
+    int listed = 0;
+#pragma unroll
+    for (int r = 0; r < SCAN_ROUNDS; r++) {
+        const int at = base + 256 * r, t = at / NC;
+        int c[4];
+        c[0] = before + ex[r];
+#pragma unroll
+        for (int i = 1; i < 4; i++) c[i] = c[i - 1] + v[r][i - 1];
+        if (at + 4 <= n) __builtin_memcpy(B.cellStart + at, c, sizeof(c));
+        else {
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                if (at + i < n) B.cellStart[at + i] = c[i];
+        }
+        const int in = lanes_sum<TL>(own[r]);
+        const bool mine = l % TL == 0 && t < B.ntall;
+        if (mine) B.tileOn[t] = !stopped && in > 0 ? 1 : 0;
+        if (mine && !stopped && in > 0) { on |= 1u << r; listed++; }
     }
-}
-
-__global__ void k_scan_add(int *out, const int *blockSums, int n) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) out[i] += blockSums[i / SCAN_BLOCK];
+    const int upto = wave_inclusive(listed), all = __builtin_amdgcn_readlane(upto, 63);
+    if (all == 0) return;
+    int slot = 0;
+    if (l == 0) slot = atomicAdd(B.ntiles, all);
+    slot = __shfl(slot, 0) + upto - listed;
+#pragma unroll
+    for (int r = 0; r < SCAN_ROUNDS; r++)
+        if (on >> r & 1u) B.tiles[slot++] = (base + 256 * r) / NC;
 }
 
 // Slots by key. The rows are kept in tile order, so the keys of a wave's 64 consecutive rows come
 // in runs; the first lane of each run takes the run's slots with one atomic, all runs of the wave
 // at once (one round trip per wave, not one per key). The order inside a cell is then fixed by
 // k_bin_sort_cells, so the slots' first placement does not change any result.
-__global__ void k_bin_scatter(KPart P, KBins B) {
+__device__ __forceinline__ void bin_scatter(const KPart &P, const KBins &B, long long p) {
     if (B.stop[0]) return;
-    const long long p = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     const bool valid = p < P.n;
     const int key = valid ? B.key[p] : -1;
     const int lane = (int)__lane_id();
@@ -723,65 +818,10 @@ __global__ void k_bin_scatter(KPart P, KBins B) {
     }
 }
 
-// the particles of a cell in upload order (their index at upload, which the memory order of the
-// rows does not change), so every sum over a cell's particles has the same order in any layout.
-// Most cells arrive in order already (their particles stayed put, in rows sorted by upload index):
-// a cell of up to 16 is checked with independent loads first and only sorted when it is not.
-__global__ void k_bin_sort_cells(KBins B) {
-    int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= B.nkeys) return;
-    int b = B.cellStart[c], e = B.cellStart[c + 1];
-    if (B.stop[0]) e = b;                    // stopped: nothing was scattered
-    bool sorted = false;
-    if (e - b <= 16) {
-        int h[16];
-#pragma unroll
-        for (int t = 0; t < 16; t++) h[t] = b + t < e ? B.shome[b + t] : 0x7fffffff;
-        sorted = true;
-#pragma unroll
-        for (int t = 1; t < 16; t++) sorted = sorted && h[t - 1] <= h[t];
-    }
-    if (!sorted) {
-        for (int i = b + 1; i < e; i++) {
-            const int v = B.order[i];
-            const int hv = B.shome[i];
-            int j = i - 1;
-            while (j >= b && B.shome[j] > hv) {
-                B.order[j + 1] = B.order[j];
-                B.shome[j + 1] = B.shome[j];
-                j--;
-            }
-            B.order[j + 1] = v;
-            B.shome[j + 1] = hv;
-        }
-    }
-    B.cursor[c] = 0;
-    B.count[c] = 0;
-}
-
-// list of the non-empty (field, tile) pairs; clears the lCPDI kernels' cursors
-__global__ void k_tile_list(KBins B, int nc) {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (blockIdx.x == 0 && threadIdx.x < TILE_SLOTS * 8) B.work[threadIdx.x * TILE_SLOT_STRIDE] = 0;
-    const bool stopped = B.stop[0] != 0;
-    if (t == 0 && !stopped) B.stop[2] += 1;   // one more step completed
-    const bool on = !stopped && t < B.ntall && B.cellStart[(size_t)(t + 1) * nc] > B.cellStart[(size_t)t * nc];
-    if (t < B.ntall) B.tileOn[t] = on ? 1 : 0;
-    const unsigned long long m = __ballot(on);
-    if (m == 0ull) return;
-    const int lane = (int)__lane_id();
-    const int leader = __ffsll((long long)m) - 1;
-    int base = 0;
-    if (lane == leader) base = atomicAdd(B.ntiles, __popcll(m));
-    base = __shfl(base, leader);
-    if (on) B.tiles[base + __popcll(m & ((1ull << lane) - 1ull))] = t;
-}
-
 // the (field, tile) pairs the next node passes visit (node_needed): needed = the pair or one of its
 // neighbours is non-empty; needAny = needed now or at the previous binning. A stopped run needs none.
 template <int DIM>
-__global__ void k_tile_need(KGrid g0, KBins B) {
-    const int tall = blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void tile_need(const KGrid &g0, const KBins &B, int tall) {
     if (tall >= B.ntall) return;
     const int fld = tall / g0.tilesTotal;
     const int tg = tall - fld * g0.tilesTotal;
@@ -800,6 +840,73 @@ __global__ void k_tile_need(KGrid g0, KBins B) {
     }
     B.needAny[tall] = need | B.need[tall];
     B.need[tall] = need;
+}
+
+// the first `need` blocks take the pairs, the others the particles (one launch: neither needs the other)
+template <int DIM>
+__global__ void k_bin_scatter(KGrid g0, KPart P, KBins B, int need) {
+    if ((int)blockIdx.x < need) tile_need<DIM>(g0, B, blockIdx.x * blockDim.x + threadIdx.x);
+    else bin_scatter(P, B, (long long)(blockIdx.x - need) * blockDim.x + threadIdx.x);
+}
+
+// the particles of a cell in upload order (their index at upload, which the memory order of the
+// rows does not change), so every sum over a cell's particles has the same order in any layout.
+// Up to 16 particles are read with independent loads and, unless they are in order already (they stayed
+// put, in rows sorted by upload index), each is written to its rank: the insertion sort in memory, which
+// larger cells still take, was a chain of loads and kept 885k particles of 8 a cell for 29 us once the
+// rows had moved since their last sort.
+template <int MOST>
+__device__ __forceinline__ void sort_few(const KBins &B, int b, int e) {
+    int h[MOST], o[MOST];
+#pragma unroll
+    for (int t = 0; t < MOST; t++) h[t] = b + t < e ? B.shome[b + t] : 0x7fffffff;
+    bool sorted = true;
+#pragma unroll
+    for (int t = 1; t < MOST; t++) sorted = sorted && h[t - 1] <= h[t];
+    if (sorted) return;
+#pragma unroll
+    for (int t = 0; t < MOST; t++) o[t] = b + t < e ? B.order[b + t] : 0;
+#pragma unroll
+    for (int t = 0; t < MOST; t++) {
+        int rank = 0;
+#pragma unroll
+        for (int u = 0; u < MOST; u++) rank += u != t && h[u] < h[t] ? 1 : 0;
+        if (b + t < e) { B.order[b + rank] = o[t]; B.shome[b + rank] = h[t]; }
+    }
+}
+
+__device__ __forceinline__ void sort_cell(const KBins &B, int b, int e) {
+    if (e - b <= 8) sort_few<8>(B, b, e);
+    else if (e - b <= 16) sort_few<16>(B, b, e);
+    else {
+        for (int i = b + 1; i < e; i++) {
+            const int v = B.order[i];
+            const int hv = B.shome[i];
+            int j = i - 1;
+            while (j >= b && B.shome[j] > hv) {
+                B.order[j + 1] = B.order[j];
+                B.shome[j + 1] = B.shome[j];
+                j--;
+            }
+            B.order[j + 1] = v;
+            B.shome[j + 1] = hv;
+        }
+    }
+}
+
+// Only listed tiles hold particles and counts; a stopped run lists none and clears every count.
+// Ends the binning: counts, cursors and the scan's words are zero for the next one.
+__global__ void k_bin_sort_cells(KBins B, int nc, int nb) {
+    const int i0 = blockIdx.x * blockDim.x + threadIdx.x, step = gridDim.x * blockDim.x;
+    for (int i = i0; i <= nb; i += step) B.blockSums[i] = 0;
+    const bool stopped = B.stop[0] != 0;
+    const int end = stopped ? B.nkeys : B.ntiles[0] * nc;
+    for (int i = i0; i < end; i += step) {
+        const int c = stopped ? i : B.tiles[i / nc] * nc + i % nc;
+        if (!stopped) sort_cell(B, B.cellStart[c], B.cellStart[c + 1]);
+        B.cursor[c] = 0;
+        B.count[c] = 0;
+    }
 }
 
 // A tile kernel's blocks walk the list of non-empty tiles, so no workgroup is spent on an empty
@@ -3341,6 +3448,7 @@ __global__ __launch_bounds__(NT) void k_contact_normals(KGrid g, KPart P, KBins 
 
 // ---------------------------------------------------------------------------------------
 // launchers
+static int g_cus = 256;
 static inline unsigned blocks_for(long long n, int bs) { return (unsigned)((n + bs - 1) / bs); }
 
 void launch_bin_keys(int dim, const KGrid &g, const KPart &p, const KBins &b, hipStream_t s) {
@@ -3350,20 +3458,21 @@ void launch_bin_keys(int dim, const KGrid &g, const KPart &p, const KBins &b, hi
 }
 
 void launch_bin_finish(int dim, const KGrid &g, const KPart &p, const KBins &b, hipStream_t s) {
-    int n = b.nkeys + 1;          // count[nkeys] stays zero, so cellStart[nkeys] = total
-    int nb = (n + SCAN_BLOCK - 1) / SCAN_BLOCK;
-    hipLaunchKernelGGL(k_scan_blocks, dim3(nb), dim3(NT), 0, s, b.count, b.cellStart, b.blockSums, n);
-    hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(NT), 0, s, b.blockSums, nb, b.ntiles);
-    hipLaunchKernelGGL(k_scan_add, dim3(blocks_for(n, NT)), dim3(NT), 0, s, b.cellStart, b.blockSums, n);
-    if (p.n > 0) hipLaunchKernelGGL(k_bin_scatter, dim3(blocks_for(p.n, NT)), dim3(NT), 0, s, p, b);
-    hipLaunchKernelGGL(k_bin_sort_cells, dim3(blocks_for(b.nkeys, NT)), dim3(NT), 0, s, b);
-    hipLaunchKernelGGL(k_tile_list, dim3(blocks_for(b.ntall, NT)), dim3(NT), 0, s, b,
-                       dim == 3 ? TileGeom<3>::NC : TileGeom<2>::NC);
-    if (dim == 3) hipLaunchKernelGGL(k_tile_need<3>, dim3(blocks_for(b.ntall, NT)), dim3(NT), 0, s, g, b);
-    else hipLaunchKernelGGL(k_tile_need<2>, dim3(blocks_for(b.ntall, NT)), dim3(NT), 0, s, g, b);
+    const int n = b.nkeys + 1;    // count[nkeys] stays zero, so cellStart[nkeys] = total
+    const int nb = (n + SCAN_BLOCK - 1) / SCAN_BLOCK;
+    constexpr int NC3 = TileGeom<3>::NC, NC2 = TileGeom<2>::NC;
+    const unsigned need = blocks_for(b.ntall, NT), rows = blocks_for(p.n, NT);
+    if (dim == 3) {
+        hipLaunchKernelGGL(k_bin_scan<NC3>, dim3(nb), dim3(SCAN_NT), 0, s, b, n, nb);
+        hipLaunchKernelGGL(k_bin_scatter<3>, dim3(need + rows), dim3(NT), 0, s, g, p, b, (int)need);
+    } else {
+        hipLaunchKernelGGL(k_bin_scan<NC2>, dim3(nb), dim3(SCAN_NT), 0, s, b, n, nb);
+        hipLaunchKernelGGL(k_bin_scatter<2>, dim3(need + rows), dim3(NT), 0, s, g, p, b, (int)need);
+    }
+    const unsigned cells = std::min<unsigned>(blocks_for(b.nkeys, NT), 16 * g_cus);
+    hipLaunchKernelGGL(k_bin_sort_cells, dim3(cells), dim3(NT), 0, s, b, dim == 3 ? NC3 : NC2, nb);
 }
 
-static int g_cus = 256;
 void set_tile_cus(int cus) { g_cus = cus > 0 ? cus : 256; }
 
 // workgroups of one tile-kernel launch: eight per CU (at least as many as the device holds at once
