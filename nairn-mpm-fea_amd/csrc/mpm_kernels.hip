@@ -131,6 +131,18 @@ __device__ __forceinline__ KGrid node_grid(const KGrid &g0, long long ng) {
     return grid_copy((GridPtr)(g0.inst + const_int(g0.nodeBlockInst + __builtin_amdgcn_readfirstlane((int)(ng / 256)))));
 }
 
+// Fields and node coordinates by 32-bit division (a 64-bit one is a hundred operations, and a node pass
+// had four): the device's memory holds fewer than 2^32 nodes of the 100 bytes and more that each takes.
+__device__ __forceinline__ int node_field(const KGrid &g0, long long nall) {
+    return g0.nfields == 1 ? 0 : (int)((unsigned)nall / (unsigned)g0.nstride);
+}
+__device__ __forceinline__ void node_ijk(const KGrid &g, long long n, int &i, int &j, int &k) {
+    const unsigned row = (unsigned)n / (unsigned)g.nnx, plane = row / (unsigned)g.nny;
+    i = (int)((unsigned)n - row * (unsigned)g.nnx);
+    j = (int)(row - plane * (unsigned)g.nny);
+    k = (int)plane;
+}
+
 __device__ __forceinline__ void elem_ijk(const KGrid &g, int e, int &i, int &j, int &k) {
     i = e % g.nx;
     int r = e / g.nx;
@@ -1438,23 +1450,39 @@ template <int DIM, int NQ>
 __device__ __forceinline__ void gather_partials(const KGrid &g, const KBins &B, const KNodes &N, int fld, int i,
                                                 int j, int k, double out[NQ]) {
     using G = TileGeom<DIM>;
-#pragma unroll
-    for (int q = 0; q < NQ; q++) out[q] = 0.;
-    int txh = min(g.ntx - 1, (i + 1) / G::TX), txl = i >= G::TX + 1 ? (i - 2) / G::TX : 0;
-    int tyh = min(g.nty - 1, (j + 1) / G::TY), tyl = j >= G::TY + 1 ? (j - 2) / G::TY : 0;
+    constexpr int NP = DIM == 3 ? 8 : 4;       // footprints overlap by less than a tile: two tiles an axis at most
+    const int txh = min(g.ntx - 1, (i + 1) / G::TX), txl = i >= G::TX + 1 ? (i - 2) / G::TX : 0;
+    const int tyh = min(g.nty - 1, (j + 1) / G::TY), tyl = j >= G::TY + 1 ? (j - 2) / G::TY : 0;
     int tzh = 0, tzl = 0;
     if (DIM == 3) { tzh = min(g.ntz - 1, (k + 1) / G::TZ); tzl = k >= G::TZ + 1 ? (k - 2) / G::TZ : 0; }
-    for (int tz = tzl; tz <= tzh; tz++)
-        for (int ty = tyl; ty <= tyh; ty++)
-            for (int tx = txl; tx <= txh; tx++) {
-                int t = (tz * g.nty + ty) * g.ntx + tx + g.tileBase + fld * g.tilesTotal;
-                if (!B.tileOn[t]) continue;
-                int fx = i - (tx * G::TX - 1), fy = j - (ty * G::TY - 1);   // slot in the footprint
-                int s = fy * G::FX + fx;
-                if (DIM == 3) s += (k - (tz * G::TZ - 1)) * G::FX * G::FY;
+    // the flags of all the tiles, then the sums of those that have particles, are read together
+    int t[NP];
+    bool on[NP];
 #pragma unroll
-                for (int q = 0; q < NQ; q++) out[q] += N.part[((size_t)t * NQMAX + q) * G::FOOT + s];
-            }
+    for (int c = 0; c < NP; c++) {
+        const int tx = txl + (c & 1), ty = tyl + (c >> 1 & 1), tz = tzl + (c >> 2);
+        const bool in = tx <= txh && ty <= tyh && tz <= tzh;
+        t[c] = (min(tz, tzh) * g.nty + min(ty, tyh)) * g.ntx + min(tx, txh) + g.tileBase + fld * g.tilesTotal;
+        on[c] = in & (B.tileOn[t[c]] != 0);
+    }
+    double v[NP][NQ];
+#pragma unroll
+    for (int c = 0; c < NP; c++) {
+#pragma unroll
+        for (int q = 0; q < NQ; q++) v[c][q] = 0.;
+        if (!on[c]) continue;
+        const int fx = i - ((txl + (c & 1)) * G::TX - 1), fy = j - ((tyl + (c >> 1 & 1)) * G::TY - 1);   // slot in the footprint
+        int s = fy * G::FX + fx;
+        if (DIM == 3) s += (k - ((tzl + (c >> 2)) * G::TZ - 1)) * G::FX * G::FY;
+#pragma unroll
+        for (int q = 0; q < NQ; q++) v[c][q] = N.part[((size_t)t[c] * NQMAX + q) * G::FOOT + s];
+    }
+#pragma unroll
+    for (int q = 0; q < NQ; q++) {
+        out[q] = v[0][q];
+#pragma unroll
+        for (int c = 1; c < NP; c++) out[q] += v[c][q];
+    }
 }
 
 // Node passes visit the nodes of the (field, tile) pairs that a non-empty pair's footprint reached at
@@ -1475,17 +1503,15 @@ template <int DIM>
 __global__ void k_node_mass(KGrid g0, KBins B, KNodes N) {
     long long nall = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (nall >= g0.nstride * g0.nfields) return;
-    const int fld = (int)(nall / g0.nstride);
+    const int fld = node_field(g0, nall);
     const long long ng = nall - (long long)fld * g0.nstride;
     const KGrid g = node_grid(g0, ng);
     const long long n = ng - g.nodeBase;
     if (n >= g.nnodes) return;                // padding between instances
     const KNodes Nf = field_view(g, N, fld);
     if (nall == 0 && N.clist) N.clist[0] = 0;   // contact-node list of the step (regression normals)
-    int i = (int)(n % g.nnx);
-    long long r = n / g.nnx;
-    int j = (int)(r % g.nny);
-    int k = (int)(r / g.nny);
+    int i, j, k;
+    node_ijk(g, n, i, j, k);
     if (!node_needed<DIM>(g, B, fld, i, j, k)) return;
     double a[NQ_MASS];
     gather_partials<DIM, NQ_MASS>(g, B, N, fld, i, j, k, a);
@@ -1994,16 +2020,14 @@ template <int DIM>
 __global__ void k_node_force(KGrid g0, KBins B, KNodes N) {
     long long nall = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (nall >= g0.nstride * g0.nfields) return;
-    const int fld = (int)(nall / g0.nstride);
+    const int fld = node_field(g0, nall);
     const long long ng = nall - (long long)fld * g0.nstride;
     const KGrid g = node_grid(g0, ng);
     const long long n = ng - g.nodeBase;
     if (n >= g.nnodes) return;                // padding between instances
     const KNodes Nf = field_view(g, N, fld);
-    int i = (int)(n % g.nnx);
-    long long r = n / g.nnx;
-    int j = (int)(r % g.nny);
-    int k = (int)(r / g.nny);
+    int i, j, k;
+    node_ijk(g, n, i, j, k);
     if (!node_needed<DIM>(g, B, fld, i, j, k)) return;
     double f[NQ_FORCE];
     gather_partials<DIM, NQ_FORCE>(g, B, N, fld, i, j, k, f);
@@ -2355,7 +2379,7 @@ template <int DIM>
 __global__ void k_node_mom2(KGrid g0, KBins B, KNodes N) {
     long long nall = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (nall >= g0.nstride * g0.nfields) return;
-    const int fld = (int)(nall / g0.nstride);
+    const int fld = node_field(g0, nall);
     const long long ng = nall - (long long)fld * g0.nstride;
     const KGrid g = node_grid(g0, ng);
     const long long n = ng - g.nodeBase;
@@ -2363,10 +2387,8 @@ __global__ void k_node_mom2(KGrid g0, KBins B, KNodes N) {
     const KNodes Nf = field_view(g, N, fld);
     int cnt = Nf.cnt[n];
     if (cnt <= 0) return;
-    int i = (int)(n % g.nnx);
-    long long r = n / g.nnx;
-    int j = (int)(r % g.nny);
-    int k = (int)(r / g.nny);
+    int i, j, k;
+    node_ijk(g, n, i, j, k);
     if (!node_needed<DIM>(g, B, fld, i, j, k)) return;
     double a[NQ_MOM];
     gather_partials<DIM, NQ_MOM>(g, B, N, fld, i, j, k, a);
@@ -2393,7 +2415,7 @@ template <int DIM>
 __global__ void k_xpic_init(KGrid g0, KBins B, KNodes N, int fmpm) {
     long long nall = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (nall >= g0.nstride * g0.nfields) return;
-    const int fld = (int)(nall / g0.nstride);
+    const int fld = node_field(g0, nall);
     const long long ng = nall - (long long)fld * g0.nstride;
     const KGrid g = node_grid(g0, ng);
     const long long n = ng - g.nodeBase;
@@ -2555,17 +2577,15 @@ __global__ void k_xpic_node(KGrid g0, KBins B, KNodes N) {
     if (blockIdx.x == 0 && threadIdx.x < 8) B.work[(TILE_SLOT_XPIC * 8 + threadIdx.x) * TILE_SLOT_STRIDE] = 0;
     long long nall = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (nall >= g0.nstride * g0.nfields) return;
-    const int fld = (int)(nall / g0.nstride);
+    const int fld = node_field(g0, nall);
     const long long ng = nall - (long long)fld * g0.nstride;
     const KGrid g = node_grid(g0, ng);
     const long long n = ng - g.nodeBase;
     if (n >= g.nnodes) return;
     const KNodes Nf = field_view(g, N, fld);
     if (Nf.cnt[n] <= 0) return;
-    int i = (int)(n % g.nnx);
-    long long r = n / g.nnx;
-    int j = (int)(r % g.nny);
-    int k = (int)(r / g.nny);
+    int i, j, k;
+    node_ijk(g, n, i, j, k);
     double a[NQ_MOM];
     gather_partials<DIM, NQ_MOM>(g, B, N, fld, i, j, k, a);
     const long long nn = g.nstride;
@@ -2852,16 +2872,14 @@ template <int DIM>
 __global__ void k_node_contact(KGrid g0, KBins B, KNodes N) {
     long long nall = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (nall >= g0.nstride * g0.nfields) return;
-    const int fld = (int)(nall / g0.nstride);
+    const int fld = node_field(g0, nall);
     const long long ng = nall - (long long)fld * g0.nstride;
     const KGrid g = node_grid(g0, ng);
     const long long n = ng - g.nodeBase;
     if (n >= g.nnodes) return;                // padding between instances
     const KNodes Nf = field_view(g, N, fld);
-    int i = (int)(n % g.nnx);
-    long long r = n / g.nnx;
-    int j = (int)(r % g.nny);
-    int k = (int)(r / g.nny);
+    int i, j, k;
+    node_ijk(g, n, i, j, k);
     if (!node_needed<DIM>(g, B, fld, i, j, k)) return;
     double a[NQ_CONTACT];
     gather_partials<DIM, NQ_CONTACT>(g, B, N, fld, i, j, k, a);
