@@ -105,15 +105,17 @@ __device__ __forceinline__ KNodes field_view(const KGrid &g, const KNodes &N, in
 // tile kernel, a wave per SIMD), also where there is one grid and the table is never read.
 typedef const __attribute__((address_space(4))) KGrid *GridPtr;
 
-__device__ __forceinline__ KGrid grid_copy(GridPtr p) {
+template <typename T>
+__device__ __forceinline__ T constant_copy(const __attribute__((address_space(4))) T *p) {
     typedef const __attribute__((address_space(4))) unsigned long long *Words;
-    static_assert(sizeof(KGrid) % 8 == 0, "whole words");
+    static_assert(sizeof(T) % 8 == 0, "whole words");
     const Words s = (Words)p;
-    union { KGrid g; unsigned long long w[sizeof(KGrid) / 8]; } u;
+    union { T t; unsigned long long w[sizeof(T) / 8]; } u;
 #pragma unroll
-    for (unsigned k = 0; k < sizeof(KGrid) / 8; k++) u.w[k] = s[k];
-    return u.g;
+    for (unsigned k = 0; k < sizeof(T) / 8; k++) u.w[k] = s[k];
+    return u.t;
 }
+__device__ __forceinline__ KGrid grid_copy(GridPtr p) { return constant_copy(p); }
 __device__ __forceinline__ int const_int(const int *p) {
     return *(const __attribute__((address_space(4))) int *)p;
 }
@@ -617,17 +619,24 @@ template <int DIM> __device__ __forceinline__ double corner_sum(double v) {
 // ---------------------------------------------------------------------------------------
 // binning: key + histogram, exclusive scan, scatter, per-cell sort (stable by particle index)
 
-// count[key] += 1 for every active lane, with one atomic per distinct key of the wave
-__device__ __forceinline__ void wave_count(int *count, int key) {
+// Runs of equal keys among a wave's active lanes, which are a prefix: whether the lane starts one, and its
+// length there. The rows are kept in tile order and a tile's particles are taken in sorted order, so keys
+// come in runs; a run takes one atomic, all runs of the wave at once (one after another, they were 40 us
+// of k_usl_reset's 830 on 7.08M particles and 17 of 131 on 1.7M in 2D).
+__device__ __forceinline__ bool run_start(int key, int &length) {
     const int lane = (int)__lane_id();
-    unsigned long long active = __ballot(1);
-    while (active) {
-        const int leader = __ffsll((long long)active) - 1;
-        const int lkey = __shfl(key, leader);
-        const unsigned long long same = __ballot(key == lkey) & active;
-        if (lane == leader) atomicAdd(&count[lkey], __popcll(same));
-        active &= ~same;
-    }
+    const int prev = __shfl_up(key, 1);
+    const bool start = lane == 0 || prev != key;
+    const int active = __popcll(__ballot(1));
+    const unsigned long long later = __ballot(start) & ~((2ull << lane) - 1ull);
+    length = (later ? __ffsll((long long)later) - 1 : active) - lane;
+    return start;
+}
+
+// count[key] += 1 for every active lane (a prefix of the wave's)
+__device__ __forceinline__ void wave_count(int *count, int key) {
+    int length;
+    if (run_start(key, length)) atomicAdd(&count[key], length);
 }
 
 template <int DIM>
@@ -1742,9 +1751,12 @@ __device__ __forceinline__ void store_state(const KPart &rows, int p, int type, 
 
 // ---------------------------------------------------------------------------------------
 // USF strain update, first half step (UpdateStrainsFirstTask::FullStrainUpdate,
-// UpdateStrainsFirstTask.cpp:101-168 -> MatPoint3D::UpdateStrain, MatPoint3D.cpp:45-60)
+// UpdateStrainsFirstTask.cpp:101-168 -> MatPoint3D::UpdateStrain, MatPoint3D.cpp:45-60). Bound by
+// memory: 735 MB for 2.1M J2 particles in 0.148 ms, 5.0 TB/s, with three waves per SIMD (two: 0.154).
+// The state is loaded before the gradient, which hides its latency (885k rubber particles: 123 and 120 us);
+// lCPDI's gradient is long and its registers are worth more.
 template <int DIM, int MAT, int SH>
-__global__ __launch_bounds__(NT, 2) void k_usf(KGrid g0, KPart P, KBins B, KNodes N, const MpmMaterial *mats,
+__global__ __launch_bounds__(NT, MAT == MPMGPU_MAT_ISOTROPIC || MAT == MPMGPU_MAT_ISOPLASTICITY ? 3 : 2) void k_usf(KGrid g0, KPart P, KBins B, KNodes N, const MpmMaterial *mats,
                                                int only) {
     using G = TileGeom<DIM>;
     __shared__ int s_cs[G::NC + 1];
@@ -1761,23 +1773,25 @@ __global__ __launch_bounds__(NT, 2) void k_usf(KGrid g0, KPart P, KBins B, KNode
         if (tb == te) return;
         int ox, oy, oz;
         tile_origin<DIM>(g, t, ox, oy, oz);
+        int p = tb + (int)threadIdx.x < te ? B.order[tb + threadIdx.x] : -1;
         {
             const double *src[3] = {Nf.vk, Nf.vk, Nf.vk};
             const long long st[3] = {0, g.nstride, 2 * g.nstride};
             load_foot<DIM, 3>(g, ox, oy, oz, src, st, s_v);
         }
         __syncthreads();
-        for (int k = tb + threadIdx.x; k < te; k += NT) {
-            int p = B.order[k];
+        for (int k = tb + threadIdx.x; k < te; k += NT, p = k < te ? B.order[k] : -1) {
+            const int mat = P.mat[p];
             int lx, ly, lz;
             tile_cell<DIM>(B.key[p], tall, lx, ly, lz);
+            const MpmMaterial &m = mats[mat];
+            const int mtype = MAT ? MAT : m.type;
+            PState s;
+            if (SH != MPMGPU_SHAPE_LCPDI) load_state<DIM>(P, p, mtype, s);
             double L[3][3];
             particle_gradient<DIM, SH>(g, gp, P, p, ox + lx, oy + ly, oz + lz, lx, ly, lz, s_v, L);
             scale_gradient<DIM>(L, g.strainFirst);
-            const MpmMaterial &m = mats[P.mat[p]];
-            const int mtype = MAT ? MAT : m.type;
-            PState s;
-            load_state<DIM>(P, p, mtype, s);
+            if (SH == MPMGPU_SHAPE_LCPDI) load_state<DIM>(P, p, mtype, s);
             constitutive<DIM, MAT>(L, m, s);
             store_state<DIM>(P, p, mtype, s);
         }
@@ -2633,27 +2647,29 @@ __global__ __launch_bounds__(NT, 2) void k_usl_reset(KGrid g0, KPart P, KBins B,
         if (tb == te) return;
         int ox, oy, oz;
         tile_origin<DIM>(g, t, ox, oy, oz);
+        int p = tb + (int)threadIdx.x < te ? B.order[tb + threadIdx.x] : -1;
         {
             const double *src[3] = {Nf.vk, Nf.vk, Nf.vk};
             const long long stt[3] = {0, g.nstride, 2 * g.nstride};
             load_foot<DIM, 3>(g, ox, oy, oz, src, stt, s_v);
         }
         __syncthreads();
-        for (int k = tb + threadIdx.x; k < te; k += NT) {
-            int p = B.order[k];
+        for (int k = tb + threadIdx.x; k < te; k += NT, p = k < te ? B.order[k] : -1) {
+            const int mat = P.mat[p];
             int lx, ly, lz;
             tile_cell<DIM>(B.key[p], tall, lx, ly, lz);
             // the end-of-step position is loaded here, before the state stores below, so its load is
             // issued with the others instead of after them
             double pos[3] = {P.posn(0)[p], P.posn(1)[p], DIM == 3 ? P.posn(2)[p] : 0.};
             int ei = ox + lx, ej = oy + ly, ek = oz + lz;
+            const MpmMaterial &m = mats[mat];
+            const int mtype = MAT ? MAT : m.type;
+            PState s;
+            if (SH != MPMGPU_SHAPE_LCPDI) load_state<DIM>(P, p, mtype, s);
             double L[3][3];
             particle_gradient<DIM, SH>(g, gp, P, p, ei, ej, ek, lx, ly, lz, s_v, L);
             scale_gradient<DIM>(L, g.strainLast);
-            const MpmMaterial &m = mats[P.mat[p]];
-            const int mtype = MAT ? MAT : m.type;
-            PState s;
-            load_state<DIM>(P, p, mtype, s);
+            if (SH == MPMGPU_SHAPE_LCPDI) load_state<DIM>(P, p, mtype, s);
             constitutive<DIM, MAT>(L, m, s);
             store_state<DIM>(P, p, mtype, s);
 
