@@ -145,11 +145,14 @@ void mpmi::enqueue_step(MpmCtx *c) {
         launch_xpic(c->dim, c->kg, c->kp, c->kb, c->kn, c->kbc, xo, fmpm, forcePass, par, s);
     };
     if (fmpm && xo > 1) xpic(false);
-    launch_usf(c->dim, c->kg, c->kp, c->kb, c->kn, c->dmats, s);
-    done(MPMGPU_KG_USF);
-    if (c->kld.nl) launch_particle_loads(c->kg, c->kld, par, s);    // InitializationTask's pFext
-    launch_p2g_force(c->dim, c->kg, c->kp, c->kb, c->kn, c->kld, par, s);
-    done(MPMGPU_KG_P2G_FORCE);
+    // one pass for both where there is one (profiling times the two groups apart)
+    if (c->profiling || !launch_usf_force(c->dim, c->kg, c->kp, c->kb, c->kn, c->kld, c->dmats, s)) {
+        launch_usf(c->dim, c->kg, c->kp, c->kb, c->kn, c->dmats, s);
+        done(MPMGPU_KG_USF);
+        if (c->kld.nl) launch_particle_loads(c->kg, c->kld, par, s);    // InitializationTask's pFext
+        launch_p2g_force(c->dim, c->kg, c->kp, c->kb, c->kn, c->kld, par, s);
+        done(MPMGPU_KG_P2G_FORCE);
+    }
     launch_node_force(c->dim, c->kg, c->kb, c->kn, s);
     // the UPDATE_MOMENTUM pass is left out in XPIC and FMPM steps of order > 1 (NodalVelBC.cpp:365-370)
     vel_bcs(mm || xo > 1 ? BC_PASS_GRID_FORCES : BC_PASS_FORCES_MOMENTA);

@@ -1930,6 +1930,102 @@ __global__ __launch_bounds__(64 * UGIMP_NW, FX ? 2 : WAVES4) void k_p2g_force(KG
     for_each_tile(B, tile);
 }
 
+// The first strain half step and the internal forces of uGIMP and classic particles without loads, in one
+// pass: nothing on the grid changes between the two, so a particle's words, cell and shape factors are
+// taken once and the stress goes to the scatter from registers. The same operations in the same order as
+// k_usf and k_p2g_force, to the bit (task by task, with profiling, loads or lCPDI those two run). Its LDS
+// holds two blocks a CU where the two kernels have three, yet steps gain, apart and in one pass: 4k 2D
+// elastic 66 and 63 us, 1.7M 2D 529 and 516, 74k J2 129 and 122.5, 885k neo-Hookean 568 and 542, 7.08M J2
+// 3,341 and 3,254; only tiles that three blocks a CU take in one go and two do not lose (262k J2 with
+// XPIC(3) 253 and 259). Three waves per SIMD hold the 2D laws without volume terms (1.7M: 516, two 530).
+template <int DIM, int MAT>
+__global__ __launch_bounds__(64 * UGIMP_NW, DIM == 2 && (MAT == MPMGPU_MAT_ISOTROPIC || MAT == MPMGPU_MAT_ISOPLASTICITY) ? 3 : 2)
+void k_usf_force(KGrid g0, KPart P, KBins B, KNodes N, const MpmMaterial *mats, int only) {
+    using G = TileGeom<DIM>;
+    constexpr int NW = UGIMP_NW;
+    __shared__ int s_cs[G::NC + 1];
+    __shared__ double s_v[3][G::FOOT];
+    __shared__ double2 s_F[NW][4 * DIM][WROW]; // as in k_p2g_force
+    __shared__ double s_a[NW][6][WROW];
+    __shared__ double s_acc[NW][NQ_FORCE][WaveFoot<DIM, NW>::SIZE];
+    static_assert(64 * NW == NT, "load_foot's threads");
+    const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
+    auto tile = [&](const int tall) {      // (field, context tile) pair
+        if (only >= 0 && g0.tileType[tall % g0.tilesTotal] != only) return;   // another launch's type
+        const int fld = tall / g0.tilesTotal;
+        const int tc = tall - fld * g0.tilesTotal;
+        const GridPtr gp = tile_grid_ptr(g0, tc);
+        const KGrid g = grid_copy(gp);
+        const KNodes Nf = field_view(g, N, fld);
+        load_tile_starts<DIM, 64 * NW>(B, tall, s_cs);
+        if (s_cs[0] == s_cs[G::NC]) return;
+        int ox, oy, oz;
+        tile_origin<DIM>(g, tc - g.tileBase, ox, oy, oz);
+        WaveCells<DIM, NW> W;
+        W.begin(s_cs);
+        WaveForce<DIM, NW, false, WROW> sc;
+        sc.begin(&s_F[w][0][0], &s_a[w][0][0], nullptr, s_acc);
+        int p = W.particle(B, W.b + l);
+        {
+            const double *src[3] = {Nf.vk, Nf.vk, Nf.vk};
+            const long long st[3] = {0, g.nstride, 2 * g.nstride};
+            load_foot<DIM, 3>(g, ox, oy, oz, src, st, s_v);
+        }
+        zero_wave_acc<DIM, NW, NQ_FORCE>(s_acc);
+        __syncthreads();
+        for (int r = W.b; r < W.e; r += 64) {
+            AxisFactors f[DIM];
+            double invd[DIM], a[6];
+            if (p >= 0) {
+                const int mat = P.mat[p];
+                int lx, ly, lz;
+                tile_cell<DIM>(B.key[p], tall, lx, ly, lz);
+                double pos[3];
+#pragma unroll
+                for (int c = 0; c < 3; c++) pos[c] = c < DIM ? P.f(MPF_POS_X + c)[p] : 0.;
+                const double nm = -P.f(MPF_MASS)[p];
+                const MpmMaterial &m = mats[mat];
+                const int mtype = MAT ? MAT : m.type;
+                // (stays 0 for small-strain elastic particles, whose law does not touch it)
+                double pr = mtype == MPMGPU_MAT_ISOTROPIC ? P.f(MPF_PRESSURE)[p] : 0.;
+                PState s;
+                load_state<DIM>(P, p, mtype, s);
+                double L[3][3];
+                {
+                    double Sw[3][3], Dw[3][3];
+                    int wd[3];
+                    particle_axes<DIM>(gp, P, p, ox + lx, oy + ly, oz + lz, pos, f, invd);
+                    particle_window<DIM>(f, invd, wd, Sw, Dw);
+                    velocity_gradient<DIM>(wd, Sw, Dw, lx, ly, lz, s_v, L);
+                }
+                scale_gradient<DIM>(L, g.strainFirst);
+                constitutive<DIM, MAT>(L, m, s);
+                store_state<DIM>(P, p, mtype, s);
+                if (mtype != MPMGPU_MAT_ISOTROPIC) pr = s.P;
+                a[0] = nm * (s.sp[0] - pr);
+                a[1] = nm * (s.sp[1] - pr);
+                a[2] = nm * s.sp[5];
+                if (DIM == 3) {
+                    a[3] = nm * (s.sp[2] - pr);
+                    a[4] = nm * s.sp[4];
+                    a[5] = nm * s.sp[3];
+                }
+            }
+            for (int r0 = r; r0 < min(r + 64, W.e); r0 += WREC) {
+                if (l / WREC == (r0 - r) / WREC && p >= 0) stage_force<DIM>(s_F[w], s_a[w], l % WREC, f, invd, a);
+                if (r0 + WREC >= min(r + 64, W.e)) p = W.particle(B, r + 64 + l);
+                wave_sync();
+                sc.scatter(W, r0, min(r0 + WREC, W.e), NoExtra());
+                wave_sync();
+            }
+        }
+        sc.finish(W);
+        __syncthreads();
+        write_partials<DIM, NW, NQ_FORCE>(N, tall, s_acc);
+    };
+    for_each_tile(B, tile);
+}
+
 // lCPDI: a corner's payload is the force -mp (sigma - P) . its gradient weight (+ pFext)
 template <int DIM> struct CornerForceWords { int p, key; double x[DIM], m, pr, s[6], r[9]; };
 
@@ -3509,10 +3605,18 @@ void launch_bin_finish(int dim, const KGrid &g, const KPart &p, const KBins &b, 
 
 void set_tile_cus(int cus) { g_cus = cus > 0 ? cus : 256; }
 
-// workgroups of one tile-kernel launch: eight per CU (at least as many as the device holds at once
-// for any of the tile kernels), at most one per (field, tile) pair
-static dim3 tile_grid_dim(const KBins &b) {
-    const long long want = 8LL * g_cus;
+// Workgroups of one tile-kernel launch, at most one per (field, tile) pair. Kernels that fill a CU with one
+// or two blocks take no more than the device holds at once: further blocks would wait for the end of those
+// to find no tile left (262k particles in 512 tiles: 204 us per step with twice as many, 195 without).
+// Others take twice as many, whose start hides the claims between short tiles (1.7M particles of 2D
+// instances: 523 without, 516; eight blocks per CU for every kernel: 518, and 885k particles 449 for 445).
+static int kernel_blocks(const void *kernel, int threads) {
+    int n = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, threads, 0) != hipSuccess || n < 1) return 8;
+    return n <= 2 ? n : 2 * n;
+}
+static dim3 tile_grid_dim(const KBins &b, int perCu) {
+    const long long want = (long long)perCu * g_cus;
     return dim3((unsigned)(b.ntall < want ? b.ntall : want));
 }
 static KBins tile_bins(const KBins &b, int slot) {
@@ -3520,7 +3624,11 @@ static KBins tile_bins(const KBins &b, int slot) {
     r.slot = slot;
     return r;
 }
-#define TILE_LAUNCH_NT(NT, KERNEL, B, S, ...) hipLaunchKernelGGL(KERNEL, tile_grid_dim(B), dim3(NT), 0, S, __VA_ARGS__)
+#define TILE_LAUNCH_NT(NT, KERNEL, B, S, ...)                                                                    \
+    do {                                                                                                         \
+        static const int perCu = kernel_blocks(reinterpret_cast<const void *>(&KERNEL), NT);                     \
+        hipLaunchKernelGGL(KERNEL, tile_grid_dim(B, perCu), dim3(NT), 0, S, __VA_ARGS__);                        \
+    } while (0)
 #define TILE_LAUNCH(KERNEL, B, S, ...) TILE_LAUNCH_NT(NT, KERNEL, B, S, __VA_ARGS__)
 
 void launch_p2g_mass(int dim, const KGrid &g, const KPart &p, const KBins &b, const KNodes &nd,
@@ -3571,6 +3679,31 @@ static void by_type(const KGrid &g, int firstTypedSlot, int plainSlot, L launch)
     }
     for (int j = 0; j < g.ntypes; j++) launch(g.types[j], g.types[j], firstTypedSlot + j);
     if (g.anyMixed) launch(0, 0, plainSlot);
+}
+
+template <int DIM>
+static void usf_force_mat(int mat, const KGrid &g, const KPart &p, const KBins &b, const KNodes &nd, const MpmMaterial *mats,
+                          int only, int slot, hipStream_t s) {
+    const KBins tb = tile_bins(b, slot);
+#define FUSED_LAUNCH(MAT) TILE_LAUNCH_NT(64 * UGIMP_NW, (k_usf_force<DIM, MAT>), tb, s, g, p, tb, nd, mats, only)
+    switch (mat) {
+        case MPMGPU_MAT_ISOTROPIC: FUSED_LAUNCH(MPMGPU_MAT_ISOTROPIC); break;
+        case MPMGPU_MAT_ISOPLASTICITY: FUSED_LAUNCH(MPMGPU_MAT_ISOPLASTICITY); break;
+        case MPMGPU_MAT_NEOHOOKEAN: FUSED_LAUNCH(MPMGPU_MAT_NEOHOOKEAN); break;
+        case MPMGPU_MAT_MOONEY: FUSED_LAUNCH(MPMGPU_MAT_MOONEY); break;
+        default: FUSED_LAUNCH(0); break;
+    }
+#undef FUSED_LAUNCH
+}
+
+bool launch_usf_force(int dim, const KGrid &g, const KPart &p, const KBins &b, const KNodes &nd, const KLoads &L,
+                      const MpmMaterial *mats, hipStream_t s) {
+    if (g.shape == MPMGPU_SHAPE_LCPDI || L.nl > 0) return false;
+    by_type(g, TILE_SLOT_TYPED, TILE_SLOT_USF, [&](int mat, int only, int slot) {
+        if (dim == 3) usf_force_mat<3>(mat, g, p, b, nd, mats, only, slot, s);
+        else usf_force_mat<2>(mat, g, p, b, nd, mats, only, slot, s);
+    });
+    return true;
 }
 
 void launch_usf(int dim, const KGrid &g, const KPart &p, const KBins &b, const KNodes &nd,

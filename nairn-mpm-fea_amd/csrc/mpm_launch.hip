@@ -24,6 +24,10 @@ void launch_p2g_mass(int dim, const KGrid &g, const KPart &p, const KBins &b, co
 void launch_node_mass(int dim, const KGrid &g, const KBins &b, const KNodes &nd, hipStream_t s) {
     BY_SHAPE(g, launch_node_mass(dim, g, b, nd, s));
 }
+bool launch_usf_force(int dim, const KGrid &g, const KPart &p, const KBins &b, const KNodes &nd, const KLoads &L,
+                      const MpmMaterial *mats, hipStream_t s) {
+    return BY_SHAPE(g, launch_usf_force(dim, g, p, b, nd, L, mats, s));
+}
 void launch_usf(int dim, const KGrid &g, const KPart &p, const KBins &b, const KNodes &nd,
                 const MpmMaterial *mats, hipStream_t s) {
     BY_SHAPE(g, launch_usf(dim, g, p, b, nd, mats, s));
