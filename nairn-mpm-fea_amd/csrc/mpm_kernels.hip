@@ -933,25 +933,36 @@ __global__ void k_bin_sort_cells(KBins B, int nc, int nb) {
 // A tile kernel's blocks walk the list of non-empty tiles, so no workgroup is spent on an empty
 // tile. Block b takes entry b first, then further entries claimed from one of eight cursors (the
 // block's cursor is b mod 8, so the blocks sharing a cursor sit on one XCD and a claim never waits
-// behind the whole device), entry gridDim.x + c + 8 k for the k-th claim on cursor c. The claim for
-// the next tile is made while the current one runs. Results do not depend on which block takes a tile.
-template <typename F>
+// behind the whole device), entry gridDim.x + c + 8 k for the k-th claim on cursor c. Results do not
+// depend on which block takes a tile. A wave's memory operations return in order, so a claim (an atomic
+// on a contended word) holds up the loads after it: a 3D tile's is made after its particles, a 2D tile's,
+// which are short, before (885k particles in 3D: 548 us per step with it before, 537 after; 1.7M in 2D: 506
+// and 511), none where every entry has its block, and claims two tiles ahead cost more than the wait they
+// spare (559). The first entry is read beside the list's length: a grid has no more blocks than the list
+// has room.
+template <int DIM, typename F>
 __device__ __forceinline__ void for_each_tile(const KBins &B, F &tile) {
+    __shared__ int s_li[2];
     const int n = B.ntiles[0];
-    __shared__ int s_li;
+    int t = B.tiles[blockIdx.x];
+    if ((int)blockIdx.x >= n) return;
     const int cur = blockIdx.x & 7;
     int *cursor = &B.work[(B.slot * 8 + cur) * TILE_SLOT_STRIDE];
-    int li = blockIdx.x;
-    while (li < n) {
-        int next = 0;
-        if (threadIdx.x == 0) next = (int)gridDim.x + cur + 8 * atomicAdd(cursor, 1);
+    for (int k = 0;; k ^= 1) {
+        int next = n > (int)gridDim.x ? -1 : n;            // no claims where every entry has its block
+        auto claim = [&] {
+            if (threadIdx.x == 0 && next < 0) next = (int)gridDim.x + cur + 8 * atomicAdd(cursor, 1);
+        };
         // one tile per block: a scalar for the compiler, so an instance's grid and the node views
         // built from it stay in scalar registers
-        tile(__builtin_amdgcn_readfirstlane(B.tiles[li]));
-        if (threadIdx.x == 0) s_li = next;
-        __syncthreads();
-        li = __builtin_amdgcn_readfirstlane(s_li);
-        __syncthreads();
+        if (DIM == 2) claim();
+        tile(__builtin_amdgcn_readfirstlane(t), claim);
+        claim();                           // unless it has been made
+        if (threadIdx.x == 0) s_li[k] = next;
+        __syncthreads();                   // (the two slots alternate, so one barrier a tile is enough)
+        const int li = __builtin_amdgcn_readfirstlane(s_li[k]);
+        if (li >= n) return;
+        t = B.tiles[li];
     }
 }
 
@@ -1013,9 +1024,10 @@ template <int DIM, int NW> struct WaveCells {
     int bounds, it, at;
     bool open;
     int b, e;                   // the wave's particles: sorted slots b..e-1
-    __device__ __forceinline__ void begin(const int *s_cs) {
+    // starts: the tile's cells' first sorted slots, and the next tile's first
+    __device__ __forceinline__ void begin(const int *starts) {
         const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
-        bounds = s_cs[w * ITS + l % ITS + (l / ITS > 0 ? 1 : 0)];
+        bounds = starts[w * ITS + l % ITS + (l / ITS > 0 ? 1 : 0)];
         it = 0;
         open = false;
         b = start(0);
@@ -1263,13 +1275,6 @@ __device__ __forceinline__ void write_partials(const KNodes &N, int t, double (*
     }
 }
 
-template <int DIM, int NTB = NT>
-__device__ __forceinline__ void load_tile_starts(const KBins &B, int t, int *s_cs) {
-    using G = TileGeom<DIM>;
-    for (int i = threadIdx.x; i <= G::NC; i += NTB) s_cs[i] = B.cellStart[t * G::NC + i];
-    __syncthreads();
-}
-
 // ---------------------------------------------------------------------------------------
 // P2G #1: mass and momentum (MassAndMomentumTask -> NodalPoint::AddMassMomentum,
 // NodalPointMPM.cpp:419-453). The point count of a node is not summed: every particle has
@@ -1310,20 +1315,17 @@ template <int DIM>
 __global__ __launch_bounds__(64 * UGIMP_NW, WAVES4) void k_p2g_mass(KGrid g0, KPart P, KBins B, KNodes N) {
     using G = TileGeom<DIM>;
     constexpr int NW = UGIMP_NW;
-    __shared__ int s_cs[G::NC + 1];
     __shared__ double s_S[NW][4 * DIM + 4][WROW];       // per wave: [axis*4 + offset][record], then mass and momentum
     __shared__ double s_acc[NW][NQ_MASS][WaveFoot<DIM, NW>::SIZE];
     const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
-    auto tile = [&](const int tall) {      // (field, context tile) pair
+    auto tile = [&](const int tall, auto &&claim) {      // (field, context tile) pair
         const int tc = tall % g0.tilesTotal;
         const GridPtr gp = tile_grid_ptr(g0, tc);
         const KGrid g = grid_copy(gp);
-        load_tile_starts<DIM, 64 * NW>(B, tall, s_cs);
-        if (s_cs[0] == s_cs[G::NC]) return;
         int ox, oy, oz;
         tile_origin<DIM>(g, tc - g.tileBase, ox, oy, oz);
         WaveCells<DIM, NW> W;
-        W.begin(s_cs);
+        W.begin(B.cellStart + (size_t)tall * G::NC);
         WaveScatter<DIM, NW, NQ_MASS, 1, WROW> sc;
         sc.begin(&s_S[w][0][0], s_acc);
         MassWords<DIM> cur;
@@ -1354,11 +1356,12 @@ __global__ __launch_bounds__(64 * UGIMP_NW, WAVES4) void k_p2g_mass(KGrid g0, KP
                 wave_sync();
             }
         }
+        claim();
         sc.finish(W);
         __syncthreads();
         write_partials<DIM, NW, NQ_MASS>(N, tall, s_acc);
     };
-    for_each_tile(B, tile);
+    for_each_tile<DIM>(B, tile);
 }
 
 // strains and rotations in the order of get_F3 (2D: those out of the plane are zero)
@@ -1392,20 +1395,17 @@ template <int DIM>
 __global__ __launch_bounds__(64 * CORNER_NW(DIM), WAVES8) void k_p2g_mass_corners(KGrid g0, KPart P, KBins B, KNodes N, KStats st) {
     using G = TileGeom<DIM>;
     constexpr int NW = CORNER_NW(DIM);
-    __shared__ int s_cs[G::NC + 1];
     __shared__ double s_S[NW][4 * DIM + 4][WROW];       // per wave: [axis*4 + offset][corner], then mass and momentum over 64
     __shared__ double s_acc[NW][NQ_MASS][WaveFoot<DIM, NW>::SIZE];
     const int w = threadIdx.x >> 6, l = threadIdx.x & 63, i = l / Corners<DIM>::N, c = l % Corners<DIM>::N;
-    auto tile = [&](const int tall) {      // (field, context tile) pair
+    auto tile = [&](const int tall, auto &&claim) {      // (field, context tile) pair
         const int tc = tall % g0.tilesTotal;
         const GridPtr gp = tile_grid_ptr(g0, tc);
         const KGrid g = grid_copy(gp);
-        load_tile_starts<DIM, 64 * NW>(B, tall, s_cs);
-        if (s_cs[0] == s_cs[G::NC]) return;
         int ox, oy, oz;
         tile_origin<DIM>(g, tc - g.tileBase, ox, oy, oz);
         WaveCells<DIM, NW> W;
-        W.begin(s_cs);
+        W.begin(B.cellStart + (size_t)tall * G::NC);
         WaveScatter<DIM, NW, NQ_MASS, Corners<DIM>::N, WROW> sc;
         sc.begin(&s_S[w][0][0], s_acc);
         CornerMassWords<DIM> cur;
@@ -1447,11 +1447,12 @@ __global__ __launch_bounds__(64 * CORNER_NW(DIM), WAVES8) void k_p2g_mass_corner
                 wave_sync();
             }
         }
+        claim();
         sc.finish(W);
         __syncthreads();
         write_partials<DIM, NW, NQ_MASS>(N, tall, s_acc);
     };
-    for_each_tile(B, tile);
+    for_each_tile<DIM>(B, tile);
 }
 
 // sum the partials of the tiles that cover node (i,j,k), in fixed tile order
@@ -1759,18 +1760,15 @@ template <int DIM, int MAT, int SH>
 __global__ __launch_bounds__(NT, MAT == MPMGPU_MAT_ISOTROPIC || MAT == MPMGPU_MAT_ISOPLASTICITY ? 3 : 2) void k_usf(KGrid g0, KPart P, KBins B, KNodes N, const MpmMaterial *mats,
                                                int only) {
     using G = TileGeom<DIM>;
-    __shared__ int s_cs[G::NC + 1];
     __shared__ double s_v[3][G::FOOT];
-    auto tile = [&](const int tall) {      // (field, context tile) pair
+    auto tile = [&](const int tall, auto &&claim) {      // (field, context tile) pair
         if (only >= 0 && g0.tileType[tall % g0.tilesTotal] != only) return;   // another launch's type
         const int fld = tall / g0.tilesTotal;
         const GridPtr gp = tile_grid_ptr(g0, tall - fld * g0.tilesTotal);
         const KGrid g = grid_copy(gp);
         const int t = tall - fld * g0.tilesTotal - g.tileBase;
         const KNodes Nf = field_view(g, N, fld);
-        load_tile_starts<DIM>(B, tall, s_cs);
-        const int tb = s_cs[0], te = s_cs[G::NC];
-        if (tb == te) return;
+        const int tb = const_int(B.cellStart + (size_t)tall * G::NC), te = const_int(B.cellStart + (size_t)(tall + 1) * G::NC);
         int ox, oy, oz;
         tile_origin<DIM>(g, t, ox, oy, oz);
         int p = tb + (int)threadIdx.x < te ? B.order[tb + threadIdx.x] : -1;
@@ -1796,7 +1794,7 @@ __global__ __launch_bounds__(NT, MAT == MPMGPU_MAT_ISOTROPIC || MAT == MPMGPU_MA
             store_state<DIM>(P, p, mtype, s);
         }
     };
-    for_each_tile(B, tile);
+    for_each_tile<DIM>(B, tile);
 }
 
 // internal-force scatter (GridForcesTask::Execute, GridForcesTask.cpp:40-153 ->
@@ -1860,25 +1858,22 @@ __global__ __launch_bounds__(64 * UGIMP_NW, FX ? 2 : WAVES4) void k_p2g_force(KG
                                                                        const int *loaded) {
     using G = TileGeom<DIM>;
     constexpr int NW = UGIMP_NW;
-    __shared__ int s_cs[G::NC + 1];
     __shared__ double2 s_F[NW][4 * DIM][WROW]; // per wave: [axis*4 + offset][record] (factor, derivative)
     __shared__ double s_a[NW][6][WROW];
     __shared__ double s_e[FX ? NW : 1][3][WROW];   // pFext of the staged particles
     __shared__ int s_tt[FX ? NW : 1][WREC];        // their traction tables (-1: none)
     __shared__ double s_acc[NW][NQ_FORCE][WaveFoot<DIM, NW>::SIZE];
     const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
-    auto tile = [&](const int tall) {      // (field, context tile) pair
+    auto tile = [&](const int tall, auto &&claim) {      // (field, context tile) pair
         // with loads: the launch with the load term takes the marked tiles, the other the rest
         if (loaded && (loaded[tall] != 0) != FX) return;
         const int tc = tall % g0.tilesTotal;
         const GridPtr gp = tile_grid_ptr(g0, tc);
         const KGrid g = grid_copy(gp);
-        load_tile_starts<DIM, 64 * NW>(B, tall, s_cs);
-        if (s_cs[0] == s_cs[G::NC]) return;
         int ox, oy, oz;
         tile_origin<DIM>(g, tc - g.tileBase, ox, oy, oz);
         WaveCells<DIM, NW> W;
-        W.begin(s_cs);
+        W.begin(B.cellStart + (size_t)tall * G::NC);
         WaveForce<DIM, NW, FX, WROW> sc;
         sc.begin(&s_F[w][0][0], &s_a[w][0][0], &s_e[FX ? w : 0][0][0], s_acc);
         // tractions: lane (q, iz, ix), in 2D (q, iy, ix), adds the tables of the cell's particles to its nodes
@@ -1923,11 +1918,12 @@ __global__ __launch_bounds__(64 * UGIMP_NW, FX ? 2 : WAVES4) void k_p2g_force(KG
                 wave_sync();
             }
         }
+        claim();
         sc.finish(W);
         __syncthreads();
         write_partials<DIM, NW, NQ_FORCE>(N, tall, s_acc);
     };
-    for_each_tile(B, tile);
+    for_each_tile<DIM>(B, tile);
 }
 
 // The first strain half step and the internal forces of uGIMP and classic particles without loads, in one
@@ -1943,26 +1939,23 @@ __global__ __launch_bounds__(64 * UGIMP_NW, DIM == 2 && (MAT == MPMGPU_MAT_ISOTR
 void k_usf_force(KGrid g0, KPart P, KBins B, KNodes N, const MpmMaterial *mats, int only) {
     using G = TileGeom<DIM>;
     constexpr int NW = UGIMP_NW;
-    __shared__ int s_cs[G::NC + 1];
     __shared__ double s_v[3][G::FOOT];
     __shared__ double2 s_F[NW][4 * DIM][WROW]; // as in k_p2g_force
     __shared__ double s_a[NW][6][WROW];
     __shared__ double s_acc[NW][NQ_FORCE][WaveFoot<DIM, NW>::SIZE];
     static_assert(64 * NW == NT, "load_foot's threads");
     const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
-    auto tile = [&](const int tall) {      // (field, context tile) pair
+    auto tile = [&](const int tall, auto &&claim) {      // (field, context tile) pair
         if (only >= 0 && g0.tileType[tall % g0.tilesTotal] != only) return;   // another launch's type
         const int fld = tall / g0.tilesTotal;
         const int tc = tall - fld * g0.tilesTotal;
         const GridPtr gp = tile_grid_ptr(g0, tc);
         const KGrid g = grid_copy(gp);
         const KNodes Nf = field_view(g, N, fld);
-        load_tile_starts<DIM, 64 * NW>(B, tall, s_cs);
-        if (s_cs[0] == s_cs[G::NC]) return;
         int ox, oy, oz;
         tile_origin<DIM>(g, tc - g.tileBase, ox, oy, oz);
         WaveCells<DIM, NW> W;
-        W.begin(s_cs);
+        W.begin(B.cellStart + (size_t)tall * G::NC);
         WaveForce<DIM, NW, false, WROW> sc;
         sc.begin(&s_F[w][0][0], &s_a[w][0][0], nullptr, s_acc);
         int p = W.particle(B, W.b + l);
@@ -2019,11 +2012,12 @@ void k_usf_force(KGrid g0, KPart P, KBins B, KNodes N, const MpmMaterial *mats, 
                 wave_sync();
             }
         }
+        claim();
         sc.finish(W);
         __syncthreads();
         write_partials<DIM, NW, NQ_FORCE>(N, tall, s_acc);
     };
-    for_each_tile(B, tile);
+    for_each_tile<DIM>(B, tile);
 }
 
 // lCPDI: a corner's payload is the force -mp (sigma - P) . its gradient weight (+ pFext)
@@ -2050,22 +2044,19 @@ __global__ __launch_bounds__(64 * CORNER_NW(DIM), FX ? 2 : WAVES8) void k_p2g_fo
                                                                         const int *loaded) {
     using G = TileGeom<DIM>;
     constexpr int NW = CORNER_NW(DIM);
-    __shared__ int s_cs[G::NC + 1];
     __shared__ double s_S[NW][4 * DIM + 4][WROW];
     __shared__ int s_tt[FX ? NW : 1][WREC / Corners<DIM>::N];    // traction tables of the staged particles (-1: none)
     __shared__ double s_acc[NW][NQ_FORCE][WaveFoot<DIM, NW>::SIZE];
     const int w = threadIdx.x >> 6, l = threadIdx.x & 63, i = l / Corners<DIM>::N, c = l % Corners<DIM>::N;
-    auto tile = [&](const int tall) {      // (field, context tile) pair
+    auto tile = [&](const int tall, auto &&claim) {      // (field, context tile) pair
         if (loaded && (loaded[tall] != 0) != FX) return;
         const int tc = tall % g0.tilesTotal;
         const GridPtr gp = tile_grid_ptr(g0, tc);
         const KGrid g = grid_copy(gp);
-        load_tile_starts<DIM, 64 * NW>(B, tall, s_cs);
-        if (s_cs[0] == s_cs[G::NC]) return;
         int ox, oy, oz;
         tile_origin<DIM>(g, tc - g.tileBase, ox, oy, oz);
         WaveCells<DIM, NW> W;
-        W.begin(s_cs);
+        W.begin(B.cellStart + (size_t)tall * G::NC);
         WaveScatter<DIM, NW, NQ_FORCE, Corners<DIM>::N, WROW> sc;
         sc.begin(&s_S[w][0][0], s_acc);
         auto trac = [&](int kb, int ke, int q, int hi, int ix, auto &f) {
@@ -2117,11 +2108,12 @@ __global__ __launch_bounds__(64 * CORNER_NW(DIM), FX ? 2 : WAVES8) void k_p2g_fo
                 wave_sync();
             }
         }
+        claim();
         sc.finish(W);
         __syncthreads();
         write_partials<DIM, NW, NQ_FORCE>(N, tall, s_acc);
     };
-    for_each_tile(B, tile);
+    for_each_tile<DIM>(B, tile);
 }
 
 // node pass after the forces: ftot, restore p (identity without BCs), p += f dt, v = p/m
@@ -2335,23 +2327,20 @@ __global__ __launch_bounds__(64 * G2P_NW(DIM), WAVES8) void k_g2p_p2g(KGrid g0, 
                                                             int mode) {
     using G = TileGeom<DIM>;
     constexpr int NW = G2P_NW(DIM);
-    __shared__ int s_cs[G::NC + 1];
     __shared__ double2 s_n[3][G::FOOT];        // (velocity, f/m) of each component
     __shared__ double s_S[NW][4 * DIM + 4][WROW];       // [axis*4 + offset][record], then the momentum (the last row is not used)
     __shared__ double s_acc[NW][NQ_MOM][WaveFoot<DIM, NW>::SIZE];
     const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
-    auto tile = [&](const int tall) {      // (field, context tile) pair
+    auto tile = [&](const int tall, auto &&claim) {      // (field, context tile) pair
         const int fld = tall / g0.tilesTotal;
         const int tc = tall - fld * g0.tilesTotal;
         const GridPtr gp = tile_grid_ptr(g0, tc);
         const KGrid g = grid_copy(gp);
         const KNodes Nf = field_view(g, N, fld);
-        load_tile_starts<DIM, 64 * NW>(B, tall, s_cs);
-        if (s_cs[0] == s_cs[G::NC]) return;
         int ox, oy, oz;
         tile_origin<DIM>(g, tc - g.tileBase, ox, oy, oz);
         WaveCells<DIM, NW> W;
-        W.begin(s_cs);
+        W.begin(B.cellStart + (size_t)tall * G::NC);
         WaveScatter<DIM, NW, NQ_MOM, 1, WROW> sc;
         sc.begin(&s_S[w][0][0], s_acc);
         MassWords<DIM> cur;
@@ -2391,11 +2380,12 @@ __global__ __launch_bounds__(64 * G2P_NW(DIM), WAVES8) void k_g2p_p2g(KGrid g0, 
                 wave_sync();
             }
         }
+        claim();
         sc.finish(W);
         __syncthreads();
         write_partials<DIM, NW, NQ_MOM>(N, tall, s_acc);
     };
-    for_each_tile(B, tile);
+    for_each_tile<DIM>(B, tile);
 }
 
 // lCPDI: the gather is taken corner by corner, a lane each, and added over the particle's lanes
@@ -2422,23 +2412,20 @@ __global__ __launch_bounds__(64 * CORNER_NW(DIM), WAVES8) void k_g2p_p2g_corners
                                                              const MpmMaterial *mats, int mode) {
     using G = TileGeom<DIM>;
     constexpr int NW = CORNER_NW(DIM);
-    __shared__ int s_cs[G::NC + 1];
     __shared__ double s_n[6][G::FOOT];         // v(3), f/m(3)
     __shared__ double s_S[NW][4 * DIM + 4][WROW];
     __shared__ double s_acc[NW][NQ_MOM][WaveFoot<DIM, NW>::SIZE];
     const int w = threadIdx.x >> 6, l = threadIdx.x & 63, i = l / Corners<DIM>::N, c = l % Corners<DIM>::N;
-    auto tile = [&](const int tall) {      // (field, context tile) pair
+    auto tile = [&](const int tall, auto &&claim) {      // (field, context tile) pair
         const int fld = tall / g0.tilesTotal;
         const int tc = tall - fld * g0.tilesTotal;
         const GridPtr gp = tile_grid_ptr(g0, tc);
         const KGrid g = grid_copy(gp);
         const KNodes Nf = field_view(g, N, fld);
-        load_tile_starts<DIM, 64 * NW>(B, tall, s_cs);
-        if (s_cs[0] == s_cs[G::NC]) return;
         int ox, oy, oz;
         tile_origin<DIM>(g, tc - g.tileBase, ox, oy, oz);
         WaveCells<DIM, NW> W;
-        W.begin(s_cs);
+        W.begin(B.cellStart + (size_t)tall * G::NC);
         WaveScatter<DIM, NW, NQ_MOM, Corners<DIM>::N, WROW> sc;
         sc.begin(&s_S[w][0][0], s_acc);
         CornerMoveWords<DIM> cur;
@@ -2477,11 +2464,12 @@ __global__ __launch_bounds__(64 * CORNER_NW(DIM), WAVES8) void k_g2p_p2g_corners
                 wave_sync();
             }
         }
+        claim();
         sc.finish(W);
         __syncthreads();
         write_partials<DIM, NW, NQ_MOM>(N, tall, s_acc);
     };
-    for_each_tile(B, tile);
+    for_each_tile<DIM>(B, tile);
 }
 
 // node pass of the USL re-extrapolation: p (rezeroed, RezeroNodeTask6) and v = p/m
@@ -2560,23 +2548,20 @@ template <int DIM>
 __global__ __launch_bounds__(64 * UGIMP_NW, WAVES4) void k_xpic_p2g(KGrid g0, KPart P, KBins B, KNodes N) {
     using G = TileGeom<DIM>;
     constexpr int NW = UGIMP_NW;
-    __shared__ int s_cs[G::NC + 1];
     __shared__ double s_n[3][G::FOOT];         // vprev
     __shared__ double s_S[NW][4 * DIM + 4][WROW];       // [axis*4 + offset][record], then the momentum (the last row is not used)
     __shared__ double s_acc[NW][NQ_MOM][WaveFoot<DIM, NW>::SIZE];
     const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
-    auto tile = [&](const int tall) {      // (field, context tile) pair
+    auto tile = [&](const int tall, auto &&claim) {      // (field, context tile) pair
         const int fld = tall / g0.tilesTotal;
         const int tc = tall - fld * g0.tilesTotal;
         const GridPtr gp = tile_grid_ptr(g0, tc);
         const KGrid g = grid_copy(gp);
         const KNodes Nf = field_view(g, N, fld);
-        load_tile_starts<DIM, 64 * NW>(B, tall, s_cs);
-        if (s_cs[0] == s_cs[G::NC]) return;
         int ox, oy, oz;
         tile_origin<DIM>(g, tc - g.tileBase, ox, oy, oz);
         WaveCells<DIM, NW> W;
-        W.begin(s_cs);
+        W.begin(B.cellStart + (size_t)tall * G::NC);
         WaveScatter<DIM, NW, NQ_MOM, 1, WROW> sc;
         sc.begin(&s_S[w][0][0], s_acc);
         MassWords<DIM> cur;
@@ -2611,34 +2596,32 @@ __global__ __launch_bounds__(64 * UGIMP_NW, WAVES4) void k_xpic_p2g(KGrid g0, KP
                 wave_sync();
             }
         }
+        claim();
         sc.finish(W);
         __syncthreads();
         write_partials<DIM, NW, NQ_MOM>(N, tall, s_acc);
     };
-    for_each_tile(B, tile);
+    for_each_tile<DIM>(B, tile);
 }
 
 template <int DIM>
 __global__ __launch_bounds__(64 * CORNER_NW(DIM), WAVES8) void k_xpic_p2g_corners(KGrid g0, KPart P, KBins B, KNodes N) {
     using G = TileGeom<DIM>;
     constexpr int NW = CORNER_NW(DIM);
-    __shared__ int s_cs[G::NC + 1];
     __shared__ double s_n[3][G::FOOT];         // vprev
     __shared__ double s_S[NW][4 * DIM + 4][WROW];
     __shared__ double s_acc[NW][NQ_MOM][WaveFoot<DIM, NW>::SIZE];
     const int w = threadIdx.x >> 6, l = threadIdx.x & 63, i = l / Corners<DIM>::N, c = l % Corners<DIM>::N;
-    auto tile = [&](const int tall) {      // (field, context tile) pair
+    auto tile = [&](const int tall, auto &&claim) {      // (field, context tile) pair
         const int fld = tall / g0.tilesTotal;
         const int tc = tall - fld * g0.tilesTotal;
         const GridPtr gp = tile_grid_ptr(g0, tc);
         const KGrid g = grid_copy(gp);
         const KNodes Nf = field_view(g, N, fld);
-        load_tile_starts<DIM, 64 * NW>(B, tall, s_cs);
-        if (s_cs[0] == s_cs[G::NC]) return;
         int ox, oy, oz;
         tile_origin<DIM>(g, tc - g.tileBase, ox, oy, oz);
         WaveCells<DIM, NW> W;
-        W.begin(s_cs);
+        W.begin(B.cellStart + (size_t)tall * G::NC);
         WaveScatter<DIM, NW, NQ_MOM, Corners<DIM>::N, WROW> sc;
         sc.begin(&s_S[w][0][0], s_acc);
         CornerMoveWords<DIM> cur;
@@ -2670,11 +2653,12 @@ __global__ __launch_bounds__(64 * CORNER_NW(DIM), WAVES8) void k_xpic_p2g_corner
                 wave_sync();
             }
         }
+        claim();
         sc.finish(W);
         __syncthreads();
         write_partials<DIM, NW, NQ_MOM>(N, tall, s_acc);
     };
-    for_each_tile(B, tile);
+    for_each_tile<DIM>(B, tile);
 }
 
 // Node pass of one increment (GetDeltaV and UpdateXStar, XPICExtrapolationTask.cpp:222-240;
@@ -2729,18 +2713,15 @@ template <int DIM, int MAT, int SH>
 __global__ __launch_bounds__(NT, 2) void k_usl_reset(KGrid g0, KPart P, KBins B, KNodes N, const MpmMaterial *mats,
                                                   KStats st, int only) {
     using G = TileGeom<DIM>;
-    __shared__ int s_cs[G::NC + 1];
     __shared__ double s_v[3][G::FOOT];
-    auto tile = [&](const int tall) {      // (field, context tile) pair
+    auto tile = [&](const int tall, auto &&claim) {      // (field, context tile) pair
         if (only >= 0 && g0.tileType[tall % g0.tilesTotal] != only) return;   // another launch's type
         const int fld = tall / g0.tilesTotal;
         const GridPtr gp = tile_grid_ptr(g0, tall - fld * g0.tilesTotal);
         const KGrid g = grid_copy(gp);
         const int t = tall - fld * g0.tilesTotal - g.tileBase;
         const KNodes Nf = field_view(g, N, fld);
-        load_tile_starts<DIM>(B, tall, s_cs);
-        const int tb = s_cs[0], te = s_cs[G::NC];
-        if (tb == te) return;
+        const int tb = const_int(B.cellStart + (size_t)tall * G::NC), te = const_int(B.cellStart + (size_t)(tall + 1) * G::NC);
         int ox, oy, oz;
         tile_origin<DIM>(g, t, ox, oy, oz);
         int p = tb + (int)threadIdx.x < te ? B.order[tb + threadIdx.x] : -1;
@@ -2854,7 +2835,7 @@ __global__ __launch_bounds__(NT, 2) void k_usl_reset(KGrid g0, KPart P, KBins B,
             wave_count(B.count, key);
         }
     };
-    for_each_tile(B, tile);
+    for_each_tile<DIM>(B, tile);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -2894,20 +2875,17 @@ __global__ __launch_bounds__(64 * UGIMP_NW, MPM_TILE_SHAPE == 0 ? 2 : 1) void k_
     constexpr int NW = UGIMP_NW;
     constexpr bool CP = SH == MPMGPU_SHAPE_LCPDI;
     constexpr int PPR = CP ? Corners<DIM>::N : 4, PB = 64 / PPR;     // records per particle, particles per 64 lanes
-    __shared__ int s_cs[G::NC + 1];
     __shared__ double s_S[NW][4 * DIM + 8][WROW];
     __shared__ double s_acc[NW][NQ_CONTACT][WaveFoot<DIM, NW>::SIZE];
     const int w = threadIdx.x >> 6, l = threadIdx.x & 63, i = l / PPR, c = l % PPR;
-    auto tile = [&](const int tall) {      // (field, context tile) pair
+    auto tile = [&](const int tall, auto &&claim) {      // (field, context tile) pair
         const int tc = tall % g0.tilesTotal;
         const GridPtr gp = tile_grid_ptr(g0, tc);
         const KGrid g = grid_copy(gp);
-        load_tile_starts<DIM, 64 * NW>(B, tall, s_cs);
-        if (s_cs[0] == s_cs[G::NC]) return;
         int ox, oy, oz;
         tile_origin<DIM>(g, tc - g.tileBase, ox, oy, oz);
         WaveCells<DIM, NW> W;
-        W.begin(s_cs);
+        W.begin(B.cellStart + (size_t)tall * G::NC);
         WaveScatter<DIM, NW, NQ_CONTACT, PPR, WROW> sc;
         sc.begin(&s_S[w][0][0], s_acc);
         ContactWords<DIM> cur;
@@ -2973,11 +2951,12 @@ __global__ __launch_bounds__(64 * UGIMP_NW, MPM_TILE_SHAPE == 0 ? 2 : 1) void k_
                 wave_sync();
             }
         }
+        claim();
         sc.finish(W);
         __syncthreads();
         write_partials<DIM, NW, NQ_CONTACT>(N, tall, s_acc);
     };
-    for_each_tile(B, tile);
+    for_each_tile<DIM>(B, tile);
 }
 
 template <int DIM>
