@@ -50,7 +50,7 @@ struct MpmCtx {
     double *pbuf = nullptr;           // particle double fields + second position buffer
     int *ibuf = nullptr;              // particle int fields
     double *cbuf = nullptr;           // lCPDI semi-side vectors of the step
-    double *scr = nullptr;            // one particle row of scratch (row permutations)
+    double *scr = nullptr;            // one particle row of scratch (the places of a download)
     RowDownload rows;                 // staging of mpmgpu_download_particles
     int sortInterval = 50;           // steps between sorts of the rows into tile order (0: never)
     int sinceSort = 0;

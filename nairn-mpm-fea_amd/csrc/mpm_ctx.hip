@@ -981,18 +981,19 @@ int mpmi::sort_rows(MpmCtx *c) {
     c->sinceSort = 0;
     if (n == 0) return 0;
     hipStream_t s = c->stream;
-    for (int r = 0; r < PROWS; r++) {
-        double *row = c->pbuf + (size_t)r * n;
-        launch_gather_row(row, c->scr, c->kb.order, n, s);
-        HIPCHECK(c, hipMemcpyAsync(row, c->scr, n * sizeof(double), hipMemcpyDeviceToDevice, s));
-    }
-    int *iscr = reinterpret_cast<int *>(c->scr);
-    for (int r = 0; r < IROWS; r++) {
-        if (r == IROW_ORDER || r == IROW_SHOME) continue;      // per slot, not per particle
-        int *row = c->ibuf + (size_t)r * n;
-        launch_gather_irow(row, iscr, c->kb.order, n, s);
-        HIPCHECK(c, hipMemcpyAsync(row, iscr, n * sizeof(int), hipMemcpyDeviceToDevice, s));
-    }
+    // three rows at a time through the position rows that no step needs meanwhile (one row at a time, with
+    // a copy each, 90 launches and copies cost 4 us of every 61 us step on 4k particles); a run that has
+    // stopped keeps its rows, as its last positions may be in those
+    const unsigned long long *stop = c->kb.stop;
+    double *now = c->parity == 0 ? c->posA[0] : c->posB[0], *other = c->parity == 0 ? c->posB[0] : c->posA[0];
+    int *itmp = reinterpret_cast<int *>(other);
+    launch_reorder_rows(false, now, other, c->kb.order, 3, n, stop, s);
+    for (int r = 3; r < MPF_NUM_FIELDS; r += 3)
+        launch_reorder_rows(false, c->kp.d + (size_t)r * n, other, c->kb.order, std::min(3, MPF_NUM_FIELDS - r), n, stop, s);
+    static_assert(MPI_ELEM == 0 && IROW_KEY == MPI_NUM_FIELDS && IROW_KEY < 6, "int rows to the key, in three double rows");
+    launch_reorder_rows(false, c->ibuf, itmp, c->kb.order, IROW_KEY + 1, n, stop, s);
+    launch_reorder_rows(false, c->ibuf + (size_t)IROW_HOME * n, itmp, c->kb.order, 1, n, stop, s);
+    if (c->dim == 2) launch_copy_row(now + 2 * n, other + 2 * n, n, stop, s);      // a step does not write this row
     launch_iota(c->kb.order, n, 0, s);
     HIPCHECK(c, hipGetLastError());
     return 0;

@@ -279,3 +279,11 @@ namespace mpmk_s1 {
 #include "mpm_launch.inc"
 }
 #include "mpm_launch.inc"
+
+// m rows of n words, one after another, into the order at[] (row[k] = row[at[k]]) or back out of it
+// (row[at[k]] = row[k]) through the m rows of tmp; a set *stop (may be null) leaves them as they are
+void launch_reorder_rows(bool back, double *rows, double *tmp, const int *at, int m, long long n,
+                         const unsigned long long *stop, hipStream_t s);
+void launch_reorder_rows(bool back, int *rows, int *tmp, const int *at, int m, long long n,
+                         const unsigned long long *stop, hipStream_t s);
+void launch_copy_row(const double *src, double *dst, long long n, const unsigned long long *stop, hipStream_t s);

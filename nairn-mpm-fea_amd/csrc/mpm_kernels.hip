@@ -644,12 +644,16 @@ __global__ void k_bin_keys(KGrid g0, KPart P, KBins B) {
     long long p = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= P.n) return;
     if (B.stop[0]) { B.key[p] = 0; return; }   // input refused on the device: nothing is binned
-    const KGrid g = g0.inst ? g0.inst[g0.matInst[P.mat[p]]] : g0;
+    // (only the words used are read: a copy of the grid, whose table is indexed by the material, would go
+    // through 520 bytes of private memory per particle)
+    const int mat = P.mat[p];
+    const GridPtr gp = g0.inst ? (GridPtr)(g0.inst + g0.matInst[mat]) : (GridPtr)__builtin_amdgcn_kernarg_segment_ptr();
+    const KGrid g = grid_copy(gp);
     int i, j, k;
     elem_ijk(g, P.elem[p], i, j, k);
     // fieldOf covers the materials of one multimaterial context; batch instances are single-field
     // and their material numbers run past its end
-    const int fld = g.nfields > 1 ? g.fieldOf[P.mat[p]] : 0;
+    const int fld = g.nfields > 1 ? gp->fieldOf[mat] : 0;
     int key = cell_key<DIM>(g, fld, i, j, DIM == 3 ? k : 0);
     B.key[p] = key;
     wave_count(B.count, key);
@@ -4199,23 +4203,11 @@ void launch_move(const KMove &m, hipStream_t s) {
     hipLaunchKernelGGL(k_move, dim3(blocks_for(m.cnt, NT), MPF_NUM_FIELDS + MPI_NUM_FIELDS + 1), dim3(NT), 0, s, m);
 }
 
-template <typename T>
-__global__ void k_gather_row(const T *src, T *dst, const int *order, long long n) {
-    const long long k = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k < n) dst[k] = src[order[k]];
-}
-
 __global__ void k_iota(int *a, long long n, int base) {
     const long long k = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (k < n) a[k] = base + (int)k;
 }
 
-void launch_gather_row(const double *src, double *dst, const int *order, long long n, hipStream_t s) {
-    if (n > 0) hipLaunchKernelGGL(k_gather_row<double>, dim3(blocks_for(n, NT)), dim3(NT), 0, s, src, dst, order, n);
-}
-void launch_gather_irow(const int *src, int *dst, const int *order, long long n, hipStream_t s) {
-    if (n > 0) hipLaunchKernelGGL(k_gather_row<int>, dim3(blocks_for(n, NT)), dim3(NT), 0, s, src, dst, order, n);
-}
 void launch_iota(int *a, long long n, int base, hipStream_t s) {
     if (n > 0) hipLaunchKernelGGL(k_iota, dim3(blocks_for(n, NT)), dim3(NT), 0, s, a, n, base);
 }

@@ -3,6 +3,8 @@
 // not depend on the shape and run shape 0's copy.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "mpm_kernels.h"
 
 #define BY_SHAPE(G, CALL) ((G).tileShape ? mpmk_s1::CALL : mpmk_s0::CALL)
@@ -75,10 +77,47 @@ void launch_particle_loads(const KGrid &g, const KLoads &L, int par, hipStream_t
     BY_SHAPE(g, launch_particle_loads(g, L, par, s));
 }
 void launch_move(const KMove &m, hipStream_t s) { mpmk_s0::launch_move(m, s); }
-void launch_gather_row(const double *src, double *dst, const int *order, long long n, hipStream_t s) {
-    mpmk_s0::launch_gather_row(src, dst, order, n, s);
-}
-void launch_gather_irow(const int *src, int *dst, const int *order, long long n, hipStream_t s) {
-    mpmk_s0::launch_gather_irow(src, dst, order, n, s);
-}
 void launch_iota(int *a, long long n, int base, hipStream_t s) { mpmk_s0::launch_iota(a, n, base, s); }
+
+namespace {
+
+// Rows of n words taken in another order, and back: dst[a][k] = src[a][at[k]], or dst[a][at[k]] = src[a][k].
+// A run that has stopped (*stop set, if stop is given) keeps its rows where they are: its last positions
+// may be in the buffer that serves as scratch.
+template <typename T, bool BACK>
+__global__ void k_reorder_rows(const T *src, T *dst, const int *at, int rows, long long n, const unsigned long long *stop) {
+    const long long k = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= n || (stop && *stop)) return;
+    const long long from = BACK ? k : at[k], to = BACK ? at[k] : k;
+    for (int a = 0; a < rows; a++) dst[a * n + to] = src[a * n + from];
+}
+
+template <typename T>
+__global__ void k_copy_unless(const T *src, T *dst, long long n, const unsigned long long *stop) {
+    if (stop && *stop) return;
+    for (long long k = (long long)blockIdx.x * blockDim.x + threadIdx.x; k < n; k += (long long)gridDim.x * blockDim.x)
+        dst[k] = src[k];
+}
+
+template <typename T>
+void reorder(bool back, T *rows, T *tmp, const int *at, int m, long long n, const unsigned long long *stop, hipStream_t s) {
+    const dim3 grid((unsigned)((n + 255) / 256)), block(256);
+    if (back) hipLaunchKernelGGL((k_reorder_rows<T, true>), grid, block, 0, s, rows, tmp, at, m, n, stop);
+    else hipLaunchKernelGGL((k_reorder_rows<T, false>), grid, block, 0, s, rows, tmp, at, m, n, stop);
+    hipLaunchKernelGGL(k_copy_unless<T>, dim3((unsigned)std::min<long long>((m * n + 255) / 256, 2048)), block, 0, s, tmp, rows,
+                       m * n, stop);
+}
+
+}  // namespace
+
+void launch_reorder_rows(bool back, double *rows, double *tmp, const int *at, int m, long long n,
+                         const unsigned long long *stop, hipStream_t s) {
+    reorder(back, rows, tmp, at, m, n, stop, s);
+}
+void launch_reorder_rows(bool back, int *rows, int *tmp, const int *at, int m, long long n,
+                         const unsigned long long *stop, hipStream_t s) {
+    reorder(back, rows, tmp, at, m, n, stop, s);
+}
+void launch_copy_row(const double *src, double *dst, long long n, const unsigned long long *stop, hipStream_t s) {
+    hipLaunchKernelGGL(k_copy_unless<double>, dim3((unsigned)std::min<long long>((n + 255) / 256, 2048)), dim3(256), 0, s, src, dst, n, stop);
+}

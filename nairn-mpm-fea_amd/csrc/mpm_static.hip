@@ -95,39 +95,15 @@ __global__ void k_copy_rows(const double *src, double *dst, long long n) {
         dst[k] = src[k];
 }
 
-// Rows of n words taken in another order, and back: dst[a][k] = src[a][at[k]], or dst[a][at[k]] = src[a][k].
-// A run that has stopped (*stop set, if stop is given) keeps its rows where they are: its last positions
-// may be in the buffer that serves as scratch.
-template <typename T, bool BACK>
-__global__ void k_reorder_rows(const T *src, T *dst, const int *at, int rows, long long n, const unsigned long long *stop) {
-    const long long k = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= n || (stop && *stop)) return;
-    const long long from = BACK ? k : at[k], to = BACK ? at[k] : k;
-    for (int a = 0; a < rows; a++) dst[a * n + to] = src[a * n + from];
-}
-
-template <typename T>
-__global__ void k_copy_unless(const T *src, T *dst, long long n, const unsigned long long *stop) {
-    if (stop && *stop) return;
-    for (long long k = (long long)blockIdx.x * blockDim.x + threadIdx.x; k < n; k += (long long)gridDim.x * blockDim.x)
-        dst[k] = src[k];
-}
-
-template <bool BACK, typename T>
-void reorder(T *rows, T *tmp, const int *at, int m, long long n, const unsigned long long *stop, hipStream_t s) {
-    hipLaunchKernelGGL((k_reorder_rows<T, BACK>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, rows, tmp, at, m, n, stop);
-    hipLaunchKernelGGL(k_copy_unless<T>, dim3(1024), dim3(256), 0, s, tmp, rows, m * n, stop);
-}
-
 // The caller's rows in the order at[], or out of it, three at a time through the three rows of tmp; pos
 // holds the positions
 template <bool BACK>
 void reorder_particles(const KPart &P, double *pos, double *tmp, const int *at, const unsigned long long *stop, hipStream_t s) {
     for (int f = 0; f < MPF_NUM_FIELDS; f += 3)
-        reorder<BACK>(f == 0 ? pos : P.d + f * P.n, tmp, at, MPF_NUM_FIELDS - f < 3 ? MPF_NUM_FIELDS - f : 3, P.n, stop, s);
+        launch_reorder_rows(BACK, f == 0 ? pos : P.d + f * P.n, tmp, at, MPF_NUM_FIELDS - f < 3 ? MPF_NUM_FIELDS - f : 3, P.n, stop, s);
     // the int rows lie one after another in ifields, from the first of them
     static_assert(MPI_ELEM == 0 && MPI_NUM_FIELDS == 4, "four int rows, two doubles a particle");
-    reorder<BACK>(P.elem, reinterpret_cast<int *>(tmp), at, MPI_NUM_FIELDS, P.n, stop, s);
+    launch_reorder_rows(BACK, P.elem, reinterpret_cast<int *>(tmp), at, MPI_NUM_FIELDS, P.n, stop, s);
 }
 
 // A solve of this many particles and steps works on its rows in tile order, renewed at the interval, and
@@ -271,12 +247,12 @@ int mpmgpu_solve_static(const MpmGridDesc *grid, const MpmMaterial *mats, int32_
         double *now = c.parity == 0 ? c.posA[0] : c.posB[0], *other = c.parity == 0 ? c.posB[0] : c.posA[0];
         int *tmp = reinterpret_cast<int *>(other);
         reorder_particles<false>(P, now, other, c.kb.order, c.kb.stop, s);
-        reorder<false>(key, tmp, c.kb.order, 1, (long long)n, c.kb.stop, s);
-        reorder<false>(home, tmp, c.kb.order, 1, (long long)n, c.kb.stop, s);
+        launch_reorder_rows(false, key, tmp, c.kb.order, 1, (long long)n, c.kb.stop, s);
+        launch_reorder_rows(false, home, tmp, c.kb.order, 1, (long long)n, c.kb.stop, s);
         launch_iota(c.kb.order, (long long)n, 0, s);        // (a stopped run's order is not used again)
         // in 2D a step does not write the z row
         if (c.dim == 2)
-            hipLaunchKernelGGL(k_copy_unless<double>, dim3(1024), dim3(256), 0, s, now + 2 * nn, other + 2 * nn, (long long)n, c.kb.stop);
+            launch_copy_row(now + 2 * nn, other + 2 * nn, (long long)n, c.kb.stop, s);
     };
     for (int32_t k = 0; k < nsteps; k++) {
         if (sorted && k % STATIC_SORT_INTERVAL == 0) sort_rows();
