@@ -104,7 +104,7 @@ struct KBins {
     int *cellStart;            // nkeys + 1
     int *count;                // nkeys histogram
     int *cursor;               // nkeys scatter cursor
-    int *blockSums;            // scan scratch
+    int *blockSums;            // the scan's states, one per block, and its ticket
     const int *home;           // particle -> its index at upload: the order inside a cell
     int *shome;                // sorted slot -> upload index of its particle
     int *tiles;                // the non-empty (field, tile) pairs of the binning, in no fixed order
@@ -114,7 +114,7 @@ struct KBins {
     // (need), at this or the previous one (needAny: the pairs whose nodes the node passes visit)
     int *need;
     int *needAny;
-    int *tileOn;               // per (field, tile): non-empty at this binning (k_tile_list)
+    int *tileOn;               // per (field, tile): non-empty at this binning (k_bin_scan)
     // run stop (ResetElementsTask's exceptions): stop[0] the reason and its rank (stop_run; 0 while running),
     // stop[1] the steps completed before the step that stopped, stop[2] the steps completed since
     // the upload (counted by the tile list). Once stop[0] is set, binning builds an empty tile

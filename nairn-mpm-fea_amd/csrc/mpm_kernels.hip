@@ -1500,7 +1500,7 @@ __device__ __forceinline__ void gather_partials(const KGrid &g, const KBins &B, 
 }
 
 // Node passes visit the nodes of the (field, tile) pairs that a non-empty pair's footprint reached at
-// this binning or the one before (k_tile_need): a node of any other pair was cleared when its pair
+// this binning or the one before (tile_need): a node of any other pair was cleared when its pair
 // last was visited, or was never written, so it is skipped and stays zero. A node's own pair is the
 // tile holding it (the grid's last node row belongs to the last tile); the pairs whose footprints
 // can reach it are that tile and its neighbours.
@@ -1937,7 +1937,7 @@ __global__ __launch_bounds__(64 * UGIMP_NW, FX ? 2 : WAVES4) void k_p2g_force(KG
 // holds two blocks a CU where the two kernels have three, yet steps gain, apart and in one pass: 4k 2D
 // elastic 66 and 63 us, 1.7M 2D 529 and 516, 74k J2 129 and 122.5, 885k neo-Hookean 568 and 542, 7.08M J2
 // 3,341 and 3,254; only tiles that three blocks a CU take in one go and two do not lose (262k J2 with
-// XPIC(3) 253 and 259). Three waves per SIMD hold the 2D laws without volume terms (1.7M: 516, two 530).
+// XPIC(2) 253 and 259). Three waves per SIMD hold the 2D laws without volume terms (1.7M: 516, two 530).
 template <int DIM, int MAT>
 __global__ __launch_bounds__(64 * UGIMP_NW, DIM == 2 && (MAT == MPMGPU_MAT_ISOTROPIC || MAT == MPMGPU_MAT_ISOPLASTICITY) ? 3 : 2)
 void k_usf_force(KGrid g0, KPart P, KBins B, KNodes N, const MpmMaterial *mats, int only) {
