@@ -1641,6 +1641,7 @@ int mpmgpu_download_particles(MpmCtx *c, double *dfields, int32_t *ifields) {
     if (read_stop(c, &why)) return 1;      // a stopped run's particles are still downloaded
     size_t nn = (size_t)c->kp.n;
     if (nn == 0) return 0;
+    if (!dfields) return c->fail("null particle rows");
     set_positions(c);
     // rows back to upload order
     HIPCHECK(c, c->rows.run(c->kp.pos, c->kp.d, c->ibuf, c->kb.home, reinterpret_cast<int *>(c->scr), (long long)nn, 0, 0,

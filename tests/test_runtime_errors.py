@@ -1,0 +1,63 @@
+"""What the library does when a call of the HIP runtime fails, on the CPU: a stand-in for the runtime
+(native/hip_stand_in.cpp) takes its calls and fails the one that a test names. Each case runs in a process
+of its own, which loads the stand-in before the library."""
+import os
+import shutil
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(HERE)
+
+pytestmark = pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++")
+
+PRELUDE = """
+import ctypes, sys
+sys.path.insert(0, {package!r})
+fake = ctypes.CDLL({stand_in!r}, mode=ctypes.RTLD_GLOBAL)
+fake.stand_in_count.restype = ctypes.c_long
+fake.stand_in_fail.argtypes = [ctypes.c_char_p, ctypes.c_long, ctypes.c_int]
+fail = lambda what, nth=0, error=1: fake.stand_in_fail(what.encode(), nth, error)     # 1: hipErrorInvalidValue
+count = lambda part: fake.stand_in_count(part.encode())
+import numpy as np
+import nairnmpm as nm
+from nairnmpm import configs
+lib = nm.library()
+prob = nm.Problem.from_xml(configs.elastic_block_2d(cells=16, block=8))
+g, mats, run, n, _ = prob.describe()
+d, i = prob.particles()
+def message(call):
+    try:
+        call()
+    except nm.MPMError as e:
+        return str(e)
+    return None
+"""
+
+
+@pytest.fixture(scope="module")
+def stand_in(tmp_path_factory):
+    out = tmp_path_factory.mktemp("hip") / "libhip_stand_in.so"
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__", "-I" + rocm + "/include",
+                    os.path.join(HERE, "native", "hip_stand_in.cpp"), "-o", str(out)], check=True)
+    return str(out)
+
+
+def _run(stand_in, body):
+    text = PRELUDE.format(package=os.path.join(ROOT, "nairn-mpm-fea_amd"), stand_in=stand_in) + body + "\nprint('done')\n"
+    r = subprocess.run([sys.executable, "-c", text], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0 and r.stdout.endswith("done\n"), (r.returncode, r.stdout, r.stderr)
+
+
+def test_download_without_rows_is_an_error(stand_in):
+    _run(stand_in, """
+sim = nm.Simulation(g, mats, run)
+sim.upload(d, i)
+assert lib.mpmgpu_download_particles(sim._h, None, None) != 0
+assert lib.mpmgpu_last_error(sim._h)
+a, b = sim.particles()
+assert a.shape == d.shape and b.shape == i.shape
+""")
