@@ -22,9 +22,10 @@ public:
     void free();
     // The rows of n particles: double rows from d (positions from pos), MPI_* rows from iv, home[] the
     // particles' places in the result (less homeBase), inv n ints of device scratch; matShift is taken
-    // off the material numbers. iOut may be null. Work already on the stream s comes first; returns
-    // when the arrays hold the rows. Errors of the runtime come back as they are; hipErrorInvalidValue
-    // if a place lies outside the result.
+    // off the material numbers. The arrays lie in host memory or, which is slower, in a device's; iOut may
+    // be null. Work already on the stream s comes first; returns when the arrays hold the rows. Errors of
+    // the runtime come back as they are; hipErrorInvalidValue for a null dOut and if a place lies outside
+    // the result.
     hipError_t run(const double *pos, const double *d, const int *iv, const int *home, int *inv, long long n,
                    long long homeBase, int matShift, double *dOut, int32_t *iOut, hipStream_t s);
 

@@ -50,6 +50,22 @@ __global__ __launch_bounds__(256) void k_result_words(const double *pos, const d
     }
 }
 
+// whether the runtime has to copy to p, because the host cannot write there
+bool on_device(const void *p) {
+    hipPointerAttribute_t a{};
+    if (!p || hipPointerGetAttributes(&a, p) != hipSuccess) {
+        (void)hipGetLastError();               // memory that the runtime does not know
+        return false;
+    }
+    return a.type == hipMemoryTypeDevice;
+}
+
+hipError_t put(void *to, const void *from, size_t bytes, bool device) {
+    if (device) return hipMemcpy(to, from, bytes, hipMemcpyHostToDevice);
+    std::memcpy(to, from, bytes);
+    return hipSuccess;
+}
+
 }  // namespace
 
 void RowDownload::free() {
@@ -61,6 +77,7 @@ void RowDownload::free() {
 hipError_t RowDownload::run(const double *pos, const double *d, const int *iv, const int *home, int *inv, long long n,
                             long long homeBase, int matShift, double *dOut, int32_t *iOut, hipStream_t s) {
     if (n <= 0) return hipStreamSynchronize(s);
+    if (!dOut) return hipErrorInvalidValue;
     const long long nd = (long long)MPF_NUM_FIELDS * n, total = nd + (iOut ? MPI_NUM_FIELDS / 2 * n : 0);
     const long long words = CHUNK / 8, chunks = (total + words - 1) / words;
     const int want = (int)std::min<long long>(THREADS, chunks);
@@ -80,6 +97,7 @@ hipError_t RowDownload::run(const double *pos, const double *d, const int *iv, c
                        reinterpret_cast<int *>(slots));
     if ((rc = hipGetLastError()) != hipSuccess) return rc;
 
+    const bool dDev = on_device(dOut), iDev = on_device(iOut);
     std::atomic<long long> next{0};
     std::atomic<int> failed{(int)hipSuccess};
     // takes chunks in turn: its launch, the wait for it, the copy; other threads' chunks fill the stream
@@ -100,8 +118,8 @@ hipError_t RowDownload::run(const double *pos, const double *d, const int *iv, c
                 break;
             if (*bad) { e = hipErrorInvalidValue; break; }
             const long long db = std::max<long long>(0, std::min(cnt, nd - w0));
-            if (db) std::memcpy(dOut + w0, at, (size_t)db * 8);
-            if (db < cnt) std::memcpy(iOut + 2 * (w0 + db - nd), at + db * 8, (size_t)(cnt - db) * 8);
+            if (db) e = put(dOut + w0, at, (size_t)db * 8, dDev);
+            if (e == hipSuccess && db < cnt) e = put(iOut + 2 * (w0 + db - nd), at + db * 8, (size_t)(cnt - db) * 8, iDev);
         }
         if (done) (void)hipEventDestroy(done);
         if (e != hipSuccess) failed.store((int)e);
