@@ -25,9 +25,10 @@ public:
     // off the material numbers. The arrays lie in host memory or, which is slower, in a device's; iOut may
     // be null. Work already on the stream s comes first; returns when the arrays hold the rows. Errors of
     // the runtime come back as they are; hipErrorInvalidValue for a null dOut and if a place lies outside
-    // the result.
+    // the result, which outside then tells.
     hipError_t run(const double *pos, const double *d, const int *iv, const int *home, int *inv, long long n,
                    long long homeBase, int matShift, double *dOut, int32_t *iOut, hipStream_t s);
+    bool outside = false;      // the last run found a place outside its result
 
 private:
     static constexpr int THREADS = 8;

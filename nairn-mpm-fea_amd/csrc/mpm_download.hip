@@ -76,6 +76,7 @@ void RowDownload::free() {
 
 hipError_t RowDownload::run(const double *pos, const double *d, const int *iv, const int *home, int *inv, long long n,
                             long long homeBase, int matShift, double *dOut, int32_t *iOut, hipStream_t s) {
+    outside = false;
     if (n <= 0) return hipStreamSynchronize(s);
     if (!dOut) return hipErrorInvalidValue;
     const long long nd = (long long)MPF_NUM_FIELDS * n, total = nd + (iOut ? MPI_NUM_FIELDS / 2 * n : 0);
@@ -134,5 +135,6 @@ hipError_t RowDownload::run(const double *pos, const double *d, const int *iv, c
     for (std::thread &t : team) t.join();
     rc = (hipError_t)failed.load();
     const hipError_t end = hipStreamSynchronize(s);     // nothing writes a slot after the return
+    outside = *bad != 0;
     return rc != hipSuccess ? rc : end;
 }

@@ -586,14 +586,17 @@ int mpmgpu_server_collect(MpmServer *s, int64_t id, double *dfields, int32_t *if
     // complete (the loop waits for their copies), and their order row is free for the places
     const size_t n = (size_t)r->n;
     hipError_t rc;
+    bool outside = false;
     {
         std::lock_guard<std::mutex> lk(s->downMutex);
         int dev = s->device;
         (void)hipGetDevice(&dev);
         rc = hipSetDevice(s->device);
-        if (rc == hipSuccess)
+        if (rc == hipSuccess) {
             rc = s->rows.run(r->dd, r->dd, r->di, r->di + IROW_HOME * n, r->di + IROW_ORDER * n, r->n, r->homeBase,
                              r->resultFirstMat, dfields, ifields, s->downStream);
+            outside = rc != hipSuccess && s->rows.outside;
+        }
         if (dev != s->device) (void)hipSetDevice(dev);
     }
     free_rows(r);
@@ -601,7 +604,7 @@ int mpmgpu_server_collect(MpmServer *s, int64_t id, double *dfields, int32_t *if
     s->deviceRowBytes -= r->devBytes;
     r->devBytes = 0;
     if (rc != hipSuccess) {
-        s->err = rc == hipErrorInvalidValue ? "particle rows of a solve left its range" : "result download failed";
+        s->err = outside ? "particle rows of a solve left its range" : "result download failed";
         return 1;
     }
     return 0;

@@ -61,3 +61,22 @@ assert lib.mpmgpu_last_error(sim._h)
 a, b = sim.particles()
 assert a.shape == d.shape and b.shape == i.shape
 """)
+
+
+@pytest.mark.parametrize("what,expect", [("hipEventRecord", "result download failed"), ("k_result_words", "result download failed"),
+                                         ("places", "left its range"), (None, None)])
+def test_message_of_a_failed_collect(stand_in, what, expect):
+    _run(stand_in, f"""
+what, expect = {what!r}, {expect!r}
+srv = nm.Server(nm.PLANE_STRAIN, nm.SHAPE_UGIMP)
+rid = srv.submit(g, mats, run, d, i, 4)
+for _ in range(10):
+    srv.advance(4)
+assert srv.info(rid)["state"] == 2
+if what == "places":
+    fake.stand_in_places_outside(1)
+elif what:
+    fail(what)                       # with hipErrorInvalidValue
+m = message(lambda: srv.collect(rid))
+assert (m is None) == (expect is None) and (m is None or expect in m), m
+""")
