@@ -427,8 +427,11 @@ void mpmgpu_destroy(MpmCtx *ctx);
    read as the initial state and overwritten with the final one. The grid, tile partials, bins,
    counters and second position buffer come from one static device array of
    MPMGPU_STATIC_SCRATCH_BYTES per device, held until the process ends; a solve needing more is
-   refused with a message giving its size. No velocity conditions or particle loads; no row
-   sorting (results do not depend on it). stream: a hipStream_t, or null for the null stream.
+   refused with a message giving its size. No velocity conditions or particle loads. A solve of
+   65,536 particles and 16 steps or more orders the caller's rows by grid tile while it steps and
+   puts them back in the caller's order before it returns (no result depends on their order). After
+   an error of the HIP runtime the rows' values are those of no particular step, and a launch of the
+   ordering that itself failed leaves them in no particular order. stream: a hipStream_t, or null for the null stream.
    Every call on a device shares its array: calls that overlap on one device race. Errors come
    from mpmgpu_global_error(); a run stopped on the device (ResetElementsTask's exceptions)
    returns its message with the stopping step's state in the rows. */

@@ -258,19 +258,32 @@ int mpmgpu_solve_static(const MpmGridDesc *grid, const MpmMaterial *mats, int32_
         if (sorted && k % STATIC_SORT_INTERVAL == 0) sort_rows();
         mpmi::enqueue_step(&c);
     }
-    if ((e = hipGetLastError()) != hipSuccess) return hipfail("step launch", e);
+    auto put_back = [&] {
+        if (sorted) reorder_particles<true>(P, c.posA[0], c.posB[0], home, nullptr, s);
+        return hipGetLastError();
+    };
+    // an error of the runtime leaves the rows in the caller's order too, if the stream still works
+    auto stepfail = [&](const char *what, hipError_t err) {
+        (void)put_back();
+        (void)hipStreamSynchronize(s);
+        return hipfail(what, err);
+    };
+    if ((e = hipGetLastError()) != hipSuccess) return stepfail("step launch", e);
 
     // a run stopped on the device keeps the stopping step's state, as mpmgpu_step does
     unsigned long long st[STATS_WORDS] = {};
-    if ((e = hipMemcpyAsync(st, sbuf, sizeof(st), hipMemcpyDeviceToHost, s)) != hipSuccess) return hipfail("counter copy", e);
-    if ((e = hipStreamSynchronize(s)) != hipSuccess) return hipfail("step", e);
+    if ((e = hipMemcpyAsync(st, sbuf, sizeof(st), hipMemcpyDeviceToHost, s)) != hipSuccess) return stepfail("counter copy", e);
+    if ((e = hipStreamSynchronize(s)) != hipSuccess) return stepfail("step", e);
     const unsigned long long why = stop_reason(st[3]);
     const int parity = why ? (int)((st[4] + 1) & 1ull) : (int)(nsteps & 1);
     if (parity == 1) {
         for (int k = 0; k < 3; k++)
             hipLaunchKernelGGL(k_copy_rows, dim3(1024), dim3(256), 0, s, c.posB[k], c.posA[k], (long long)n);
     }
-    if (sorted) reorder_particles<true>(P, c.posA[0], c.posB[0], home, nullptr, s);
+    if ((e = put_back()) != hipSuccess) {
+        (void)hipStreamSynchronize(s);
+        return hipfail("row order", e);
+    }
     if ((e = hipStreamSynchronize(s)) != hipSuccess) return hipfail("position copy", e);
     if (st[6])
         return fail_global("a contact node is seen by more than 1024 particles, more than the regression normals' "

@@ -80,3 +80,23 @@ elif what:
 m = message(lambda: srv.collect(rid))
 assert (m is None) == (expect is None) and (m is None or expect in m), m
 """)
+
+
+@pytest.mark.parametrize("what,nth", [("k_p2g_mass", 3), ("k_reorder_rows", 20), ("hipStreamSynchronize", 1), ("hipMemcpyAsync", 6),
+                                      ("k_reorder_rowsIdLb1", 2), ("k_copy_unless", -2)])
+def test_static_solve_puts_the_rows_back(stand_in, what, nth):
+    """a solve that orders the caller's rows: one that fails orders them back, and says so if that fails"""
+    _run(stand_in, f"""
+what, nth = {what!r}, {nth}
+prob = nm.Problem.from_xml(configs.j2_block_2d(cells=144, block=128))
+g, mats, run, n, _ = prob.describe()
+d, i = prob.particles()
+d, i = np.ascontiguousarray(d), np.ascontiguousarray(i)
+solve = lambda: nm.solve_static(g, mats, run, n, d.ctypes.data, i.ctypes.data, 16)
+assert n >= 65536 and message(solve) is None
+back = count("k_reorder_rowsIdLb1") + count("k_reorder_rowsIiLb1")
+assert back == -(-nm.NUM_FIELDS // 3) + 1
+fail(what, nth if nth >= 0 else count(what) + nth)
+assert message(solve)
+assert count("k_reorder_rowsIdLb1") + count("k_reorder_rowsIiLb1") == 2 * back
+""")
