@@ -545,10 +545,10 @@ template <int DIM> struct Corners {
     static constexpr double W = 1. / N, WW = W * W;             // a corner's share; times its function's factor
 };
 
-// n/d from r = 1/d, correctly rounded as a division
+// n/d from r = 1/d, correctly rounded as a division (an infinite one has no remainder to correct it by)
 __device__ __forceinline__ double quotient(double n, double d, double r) {
-    const double q = n * r;
-    return fma(fma(-q, d, n), r, q);
+    const double q = n * r, c = fma(fma(-q, d, n), r, q);
+    return c == c ? c : q;
 }
 
 // corner c of a particle at pos in cell (cx, cy, cz): cpdi_corner without its divisions
