@@ -1646,6 +1646,7 @@ int mpmgpu_download_particles(MpmCtx *c, double *dfields, int32_t *ifields) {
     // rows back to upload order
     HIPCHECK(c, c->rows.run(c->kp.pos, c->kp.d, c->ibuf, c->kb.home, reinterpret_cast<int *>(c->scr), (long long)nn, 0, 0,
                             dfields, ifields, c->stream));
+    HIPCHECK(c, hipGetLastError());
     return 0;
 }
 

@@ -6,6 +6,7 @@
 #include <cstring>
 #include <system_error>
 #include <thread>
+#include <tuple>
 #include <vector>
 
 namespace {
@@ -50,11 +51,23 @@ __global__ __launch_bounds__(256) void k_result_words(const double *pos, const d
     }
 }
 
+// a launch's own error, not one that an earlier call left for its caller to read
+template <typename... P, typename... A>
+hipError_t launch(void (*kernel)(P...), unsigned blocks, hipStream_t s, A... a) {
+    std::tuple<P...> values(static_cast<P>(a)...);
+    return std::apply([&](auto &...v) {
+        void *args[] = {&v...};
+        return hipLaunchKernel(reinterpret_cast<const void *>(kernel), dim3(blocks), dim3(256), args, 0, s);
+    }, values);
+}
+
 // whether the runtime has to copy to p, because the host cannot write there
 bool on_device(const void *p) {
     hipPointerAttribute_t a{};
-    if (!p || hipPointerGetAttributes(&a, p) != hipSuccess) {
-        (void)hipGetLastError();               // memory that the runtime does not know
+    if (!p) return false;
+    const bool clean = hipPeekAtLastError() == hipSuccess;
+    if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+        if (clean) (void)hipGetLastError();      // memory that the runtime does not know
         return false;
     }
     return a.type == hipMemoryTypeDevice;
@@ -94,9 +107,8 @@ hipError_t RowDownload::run(const double *pos, const double *d, const int *iv, c
     }
     volatile int *bad = reinterpret_cast<int *>(slots);
     *bad = 0;
-    hipLaunchKernelGGL(k_places, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, home, inv, n, homeBase,
-                       reinterpret_cast<int *>(slots));
-    if ((rc = hipGetLastError()) != hipSuccess) return rc;
+    if ((rc = launch(k_places, (unsigned)((n + 255) / 256), s, home, inv, n, homeBase, reinterpret_cast<int *>(slots))) != hipSuccess)
+        return rc;
 
     const bool dDev = on_device(dOut), iDev = on_device(iOut);
     std::atomic<long long> next{0};
@@ -112,10 +124,9 @@ hipError_t RowDownload::run(const double *pos, const double *d, const int *iv, c
             if (c >= chunks) break;
             const long long w0 = c * words, cnt = std::min(words, total - w0);
             const unsigned blocks = (unsigned)std::min<long long>((cnt + 255) / 256, 512);
-            hipLaunchKernelGGL(k_result_words, dim3(blocks), dim3(256), 0, s, pos, d, iv, inv, n, matShift, w0, cnt,
-                               reinterpret_cast<unsigned long long *>(at));
-            if ((e = hipGetLastError()) != hipSuccess || (e = hipEventRecord(done, s)) != hipSuccess ||
-                (e = hipEventSynchronize(done)) != hipSuccess)
+            if ((e = launch(k_result_words, blocks, s, pos, d, iv, inv, n, matShift, w0, cnt,
+                            reinterpret_cast<unsigned long long *>(at))) != hipSuccess ||
+                (e = hipEventRecord(done, s)) != hipSuccess || (e = hipEventSynchronize(done)) != hipSuccess)
                 break;
             if (*bad) { e = hipErrorInvalidValue; break; }
             const long long db = std::max<long long>(0, std::min(cnt, nd - w0));

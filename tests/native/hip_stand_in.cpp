@@ -88,6 +88,7 @@ hipError_t hipGetDevice(int *d) { *d = 0; return hipSuccess; }
 hipError_t hipSetDevice(int) { return hipSuccess; }
 hipError_t hipDeviceGetAttribute(int *v, hipDeviceAttribute_t, int) { *v = 4; return hipSuccess; }
 hipError_t hipGetLastError(void) { hipError_t e = last; last = hipSuccess; return e; }
+hipError_t hipPeekAtLastError(void) { return last; }
 const char *hipGetErrorString(hipError_t e) { return e == hipErrorInvalidValue ? "invalid argument" : "stand-in error"; }
 hipError_t hipGetSymbolAddress(void **p, const void *) { *p = symbol; return hipSuccess; }
 hipError_t hipPointerGetAttributes(hipPointerAttribute_t *a, const void *) {

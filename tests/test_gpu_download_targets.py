@@ -38,3 +38,20 @@ def test_rows_into_device_memory(n, doubles, ints):
     assert np.array_equal(a, d)
     assert np.array_equal(b, i) if ints else not b.any()
     sim.close()
+
+
+def test_collect_after_an_unread_error():
+    print("case: server collect after an unread error of the runtime", flush=True)
+    prob = nm.Problem.from_xml(configs.elastic_block_2d(cells=24, block=12))
+    g, mats, run, _, _ = prob.describe()
+    d, i = prob.particles()
+    srv = nm.Server(nm.PLANE_STRAIN, nm.SHAPE_UGIMP)
+    rid = srv.submit(g, mats, run, d, i, 4)
+    while srv.info(rid)["state"] < 2:
+        srv.advance(4)
+    hip = _Hip()
+    assert hip.lib.hipMemcpy(None, d.ctypes.data, 8, hip.D2H) != 0          # refused, and kept as the last error
+    a, b = srv.collect(rid)
+    assert np.array_equal(a[nm.F["orig_x"]], d[nm.F["orig_x"]]) and np.array_equal(b[nm.I["id"]], i[nm.I["id"]])
+    hip.lib.hipGetLastError()
+    srv.close()

@@ -100,3 +100,28 @@ fail(what, nth if nth >= 0 else count(what) + nth)
 assert message(solve)
 assert count("k_reorder_rowsIdLb1") + count("k_reorder_rowsIiLb1") == 2 * back
 """)
+
+
+def test_unread_error_before_a_collect(stand_in):
+    """an error of the caller's own that nobody has read fails no collect and stays for its caller; a context's
+    download reports it, with the rows"""
+    _run(stand_in, """
+def unread():
+    assert fake.hipMemcpy(None, None, 8, 0) != 0
+srv = nm.Server(nm.PLANE_STRAIN, nm.SHAPE_UGIMP)
+rid = srv.submit(g, mats, run, d, i, 4)
+for _ in range(10):
+    srv.advance(4)
+assert srv.info(rid)["state"] == 2
+unread()
+a, b = srv.collect(rid)
+assert a.shape == d.shape
+assert fake.hipGetLastError() == 1
+sim = nm.Simulation(g, mats, run)
+sim.upload(d, i)
+unread()
+before = count("k_result_words")
+assert "invalid argument" in message(sim.particles)
+assert count("k_result_words") > before
+assert message(sim.particles) is None
+""")
