@@ -100,11 +100,17 @@ hipError_t RowDownload::run(const double *pos, const double *d, const int *iv, c
     if ((rc = hipGetDevice(&device)) != hipSuccess) return rc;
     if (nslots < want) {
         free();
-        void *p = nullptr;
-        if ((rc = hipHostMalloc(&p, FLAG_BYTES + (size_t)want * CHUNK, hipHostMallocCoherent)) != hipSuccess) return rc;
-        slots = static_cast<char *>(p);
-        nslots = want;
+        const bool clean = hipPeekAtLastError() == hipSuccess;
+        for (int k = want; !slots && k > 0; k /= 2) {      // as many as the host will pin
+            void *p = nullptr;
+            if ((rc = hipHostMalloc(&p, FLAG_BYTES + (size_t)k * CHUNK, hipHostMallocCoherent)) != hipSuccess) continue;
+            slots = static_cast<char *>(p);
+            nslots = k;
+        }
+        if (clean) (void)hipGetLastError();
+        if (!slots) return rc;
     }
+    const int threads = std::min(want, nslots);
     volatile int *bad = reinterpret_cast<int *>(slots);
     *bad = 0;
     if ((rc = launch(k_places, (unsigned)((n + 255) / 256), s, home, inv, n, homeBase, reinterpret_cast<int *>(slots))) != hipSuccess)
@@ -138,8 +144,8 @@ hipError_t RowDownload::run(const double *pos, const double *d, const int *iv, c
     };
     std::vector<std::thread> team;
     try {
-        team.reserve(want - 1);
-        for (int k = 1; k < want; k++) team.emplace_back(work, k);
+        team.reserve(threads - 1);
+        for (int k = 1; k < threads; k++) team.emplace_back(work, k);
     } catch (const std::exception &) {                  // fewer threads than wanted: the others take its chunks
     }
     work(0);

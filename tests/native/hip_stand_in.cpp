@@ -19,6 +19,7 @@ long failAt = -1;
 hipError_t failWith = hipSuccess;
 hipError_t last = hipSuccess;                 // (one for all threads, where the runtime has one each)
 bool placesBad = false;
+int refusePinned = 0;
 unsigned long long handle = 1;
 void *symbol = nullptr;
 
@@ -43,6 +44,7 @@ void stand_in_fail(const char *what, long nth, int error) {
     failWith = (hipError_t)error;
     last = hipSuccess;
 }
+void stand_in_refuse_pinned(int calls) { refusePinned = calls; }
 void stand_in_places_outside(int on) { placesBad = on != 0; }
 long stand_in_count(const char *part) {
     std::lock_guard<std::mutex> lk(m);
@@ -70,7 +72,14 @@ hipError_t hipMalloc(void **p, size_t n) {
     return called("hipMalloc");
 }
 hipError_t hipFree(void *p) { free(p); return hipSuccess; }
-hipError_t hipHostMalloc(void **p, size_t n, unsigned) { *p = calloc(n, 1); return called("hipHostMalloc"); }
+hipError_t hipHostMalloc(void **p, size_t n, unsigned) {
+    if (refusePinned > 0) {
+        refusePinned--;
+        return last = hipErrorOutOfMemory;
+    }
+    *p = calloc(n, 1);
+    return called("hipHostMalloc");
+}
 hipError_t hipHostFree(void *p) { free(p); return hipSuccess; }
 hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind) {
     if (!d || !s) return last = hipErrorInvalidValue;

@@ -125,3 +125,20 @@ assert "invalid argument" in message(sim.particles)
 assert count("k_result_words") > before
 assert message(sim.particles) is None
 """)
+
+
+def test_download_with_less_pinned_memory(stand_in):
+    """slots that cannot be pinned are done without, down to one"""
+    _run(stand_in, """
+prob = nm.Problem.from_xml(configs.j2_block_2d(cells=144, block=128))
+g, mats, run, n, _ = prob.describe()
+d, i = prob.particles()
+for refused in (1, 2, 3, 4):
+    sim = nm.Simulation(g, mats, run)
+    sim.upload(d, i)
+    fake.stand_in_refuse_pinned(refused)
+    m = message(sim.particles)
+    assert (m is None) == (refused < 4), (refused, m)
+    fake.stand_in_refuse_pinned(0)
+    assert message(sim.particles) is None
+""")
