@@ -2193,8 +2193,8 @@ __global__ void k_node_force(KGrid g0, KBins B, KNodes N) {
     gather_partials<DIM, NQ_FORCE>(g, B, N, fld, i, j, k, f);
     long long nn = g.nstride;
     if (DIM == 2) f[2] = 0.;
-    if (DIM == 3 && g.shape == MPMGPU_SHAPE_LCPDI && Nf.mass[n] == 0.) f[0] = f[1] = f[2] = 0.;   // (stage_corner)
     int cnt = Nf.cnt[n];
+    if (DIM == 3 && cnt <= 0 && g.shape == MPMGPU_SHAPE_LCPDI && Nf.mass[n] == 0.) f[0] = f[1] = f[2] = 0.;   // (stage_corner)
     if (g.hasGravity && cnt > 0) {         // PostForcesTask.cpp:62-91 -> AddGravityAndBodyForceTask3
         const double m = Nf.mass[n];       // (MatVelocityField.cpp:254-258): ftot += mass g
         for (int c = 0; c < 3; c++) f[c] += m * g.gravity[c];
