@@ -1293,6 +1293,86 @@ template <int DIM, int NW, bool FX, int STR> struct WaveForce {
     }
 };
 
+// The contact sums of uGIMP and classic particles: volume and displacement as the mass scatter's components,
+// and the volume gradient as the force scatter's with Vp alone (component q takes the derivative along q),
+// four products (2D: three) for four particles. F: rows of pairs as in WaveForce; U: 4 rows, the volume and
+// the displacement's components. A lane per node took 82 us per launch on 202k particles in 3D and 32 on
+// 192k in 2D; four records a particle (its factors, and each axis's derivative in turn beside the others'
+// factors), two products each and eight particles a round, 96 and 39; this takes 48 and 18. Bit for bit the
+// sums of the four records: a component's terms come in the same order, without the zeros between.
+template <int DIM, int NW, int STR> struct WaveContact {
+    using F = WaveFoot<DIM, NW>;
+    const double2 *flo, *fhi;
+    const double *ulo;
+    double *acc;
+    int k4, lo;
+    typename MatSums<DIM>::T c[2];
+    struct Quad { double2 x, y, z; double u, v; };
+    __device__ __forceinline__ void begin(const double2 *S, const double *U, double (*s_acc)[NQ_CONTACT][F::SIZE]) {
+        const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
+        const int hi = (l >> 2) & 3;
+        lo = l & 3;
+        k4 = l >> 4;
+        flo = S + lo * STR + k4;
+        fhi = S + hi * STR + k4;
+        ulo = U + lo * STR + k4;
+        // nodes as in WaveScatter
+        acc = &s_acc[w][lo][hi * (DIM == 3 ? F::PLANE : F::WX) + k4];
+    }
+    __device__ __forceinline__ Quad load(int k, int e) const {
+        const bool in = k + k4 < e;
+        const int at = in ? k : e - 1 - k4;
+        Quad t;
+        t.x = flo[at]; t.y = fhi[4 * STR + at];
+        t.z = DIM == 3 ? fhi[8 * STR + at] : make_double2(1., 0.);
+        t.u = ulo[at]; t.v = ulo[at - lo * STR];
+        if (!in) t.x = make_double2(0., 0.);
+        return t;
+    }
+    __device__ __forceinline__ void fold(const Quad &t) {
+        const double v0 = lo == 0 ? t.v : 0., v1 = lo == 1 ? t.v : 0., v2 = lo == 2 ? t.v : 0.;
+        if constexpr (DIM == 3) {
+            c[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(t.x.x * t.y.x, t.z.x * t.u, c[0], 0, 0, 0);
+            c[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(t.x.y * t.y.x, t.z.x * v0, c[1], 0, 0, 0);
+            c[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(t.x.x * t.y.y, t.z.x * v1, c[1], 0, 0, 0);
+            c[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(t.x.x * t.y.x, t.z.y * v2, c[1], 0, 0, 0);
+        } else {
+            c[0] = __builtin_amdgcn_mfma_f64_4x4x4f64(t.x.x * t.y.x, t.u, c[0], 0, 0, 0);
+            c[1] = __builtin_amdgcn_mfma_f64_4x4x4f64(t.x.y * t.y.x, v0, c[1], 0, 0, 0);
+            c[1] = __builtin_amdgcn_mfma_f64_4x4x4f64(t.x.x * t.y.y, v1, c[1], 0, 0, 0);
+        }
+    }
+    __device__ __forceinline__ void flush(int at) const {
+#pragma unroll
+        for (int b = 0; b < 2; b++) {
+            if (b == 1 && lo >= DIM) continue;
+            double *p = acc + b * 4 * F::SIZE + at;
+            if constexpr (DIM == 3) {
+#pragma unroll
+                for (int r = 0; r < 4; r++) lds_add(p + r * F::WX, c[b][r]);
+            } else lds_add(p, c[b]);
+        }
+    }
+    __device__ __forceinline__ void scatter(WaveCells<DIM, NW> &W, int r0, int r1) {
+        auto add = [&](int k, int e) {
+#pragma unroll 1
+            for (; k < e; k += 4) fold(load(k, e));
+        };
+        wave_walk(W, r0, r1,
+            [&](int kb, int ke, bool open) {
+                const Quad t = load(kb, ke);
+                if (open) flush(W.at);
+                c[0] = c[1] = typename MatSums<DIM>::T{};
+                fold(t);
+                add(kb + 4, ke);
+            },
+            [&](int kb, int ke) { add(kb, ke); });
+    }
+    __device__ __forceinline__ void finish(const WaveCells<DIM, NW> &W) const {
+        if (W.open) flush(W.at);
+    }
+};
+
 // a wave's own copy (the wave's later LDS instructions follow in order)
 template <int DIM, int NW, int NQ>
 __device__ __forceinline__ void zero_wave_acc(double (*s_acc)[NQ][(WaveFoot<DIM, NW>::SIZE)]) {
@@ -1859,11 +1939,9 @@ __global__ __launch_bounds__(NT, MAT == MPMGPU_MAT_ISOTROPIC || MAT == MPMGPU_MA
 // MatPoint3D::GetFintPlusFext, MatPoint3D.cpp:248-270; MatPoint2D.cpp:242-263) with the stress
 // just updated by k_usf; FX adds N * pFext of the loaded particles (pFext is zero otherwise)
 
-// uGIMP and classic: stages -mp times the stress terms (xx, yy, xy, zz, xz, yz of sigma - P; 2D: three)
-// and the factor pairs of one particle at record i of its wave's rows
+// uGIMP and classic: the (factor, derivative) pairs of one particle at record i of its wave's rows
 template <int DIM>
-__device__ __forceinline__ void stage_force(double2 (*F)[WROW], double (*A)[WROW], int i, const AxisFactors f[DIM],
-                                            const double invd[DIM], const double s[6]) {
+__device__ __forceinline__ void stage_pairs(double2 (*F)[WROW], int i, const AxisFactors f[DIM], const double invd[DIM]) {
 #pragma unroll
     for (int a = 0; a < DIM; a++) {
         AxisFactors t = f[a];
@@ -1871,6 +1949,13 @@ __device__ __forceinline__ void stage_force(double2 (*F)[WROW], double (*A)[WROW
 #pragma unroll
         for (int o = 0; o < 4; o++) F[a * 4 + o][i] = make_double2(t.s4(o), t.d4(o) * invd[a]);
     }
+}
+
+// and -mp times the stress terms (xx, yy, xy, zz, xz, yz of sigma - P; 2D: three)
+template <int DIM>
+__device__ __forceinline__ void stage_force(double2 (*F)[WROW], double (*A)[WROW], int i, const AxisFactors f[DIM],
+                                            const double invd[DIM], const double s[6]) {
+    stage_pairs<DIM>(F, i, f, invd);
 #pragma unroll
     for (int c = 0; c < (DIM == 3 ? 6 : 3); c++) A[c][i] = s[c];
 }
@@ -2904,10 +2989,6 @@ __global__ __launch_bounds__(NT, 2) void k_usl_reset(KGrid g0, KPart P, KBins B,
 // volume sum N Vp, displacement sum (x - x0) N mp and volume gradient sum grad N Vp, with
 // Vp = det(F) mp / rho (MatPoint3D::GetVolume, MatPoint2D::GetVolume) and the start-of-step
 // shape functions. The displacement uses the new positions in the USL pass.
-// Seven components are two products with the same rows. A particle's records are its lCPDI corners
-// (weights and the gradient weight times Vp), or, for uGIMP and classic, four: its factors with the
-// volume and the displacement's momentum-like terms, and with each axis's derivative in turn, which
-// carry the three components of the volume gradient (2D: the last is zero).
 template <int DIM> struct ContactWords { int p, key; double x[DIM], m, ep[6], wr[3], u[DIM], rho; };
 
 template <int DIM>
@@ -2927,13 +3008,86 @@ __device__ __forceinline__ void load_contact_words(const KPart &rows, const KBin
     t.rho = mats[P.mat[t.p]].rho;
 }
 
-template <int DIM, int SH>
+// Vp of the words' particle
+template <int DIM>
+__device__ __forceinline__ double contact_volume(const ContactWords<DIM> &t) {
+    double Fm[3][3], J;
+    get_F3(t.ep, t.wr, Fm);
+    if (DIM == 3)
+        J = Fm[0][0] * (Fm[1][1] * Fm[2][2] - Fm[2][1] * Fm[1][2])
+            - Fm[0][1] * (Fm[1][0] * Fm[2][2] - Fm[2][0] * Fm[1][2])
+            + Fm[0][2] * (Fm[1][0] * Fm[2][1] - Fm[2][0] * Fm[1][1]);
+    else J = Fm[0][0] * Fm[1][1] - Fm[1][0] * Fm[0][1];
+    return J * t.m / t.rho;
+}
+
+// uGIMP and classic
+template <int DIM>
 __global__ __launch_bounds__(64 * UGIMP_NW, MPM_TILE_SHAPE == 0 ? 2 : 1) void k_p2g_contact(KGrid g0, KPart P, KBins B, KNodes N, const MpmMaterial *mats,
                                                         int newPositions) {
     using G = TileGeom<DIM>;
     constexpr int NW = UGIMP_NW;
-    constexpr bool CP = SH == MPMGPU_SHAPE_LCPDI;
-    constexpr int PPR = CP ? Corners<DIM>::N : 4, PB = 64 / PPR;     // records per particle, particles per 64 lanes
+    __shared__ double2 s_F[NW][4 * DIM][WROW]; // per wave: [axis*4 + offset][record] (factor, derivative)
+    __shared__ double s_u[NW][4][WROW];        // volume and displacement
+    __shared__ double s_acc[NW][NQ_CONTACT][WaveFoot<DIM, NW>::SIZE];
+    const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
+    auto tile = [&](const int tall, auto &&claim) {      // (field, context tile) pair
+        const int tc = tall % g0.tilesTotal;
+        const GridPtr gp = tile_grid_ptr(g0, tc);
+        const KGrid g = grid_copy(gp);
+        int ox, oy, oz;
+        tile_origin<DIM>(g, tc - g.tileBase, ox, oy, oz);
+        WaveCells<DIM, NW> W;
+        W.begin(B.cellStart + (size_t)tall * G::NC);
+        WaveContact<DIM, NW, WROW> sc;
+        sc.begin(&s_F[w][0][0], &s_u[w][0][0], s_acc);
+        ContactWords<DIM> cur;
+        int ahead = W.particle(B, W.b + 64 + l);       // the order is read a round before the words
+        load_contact_words<DIM>(P, B, mats, newPositions, W.particle(B, W.b + l), cur);
+        zero_wave_acc<DIM, NW, NQ_CONTACT>(s_acc);
+        for (int r = W.b; r < W.e; r += 64) {
+            AxisFactors f[DIM];
+            double invd[DIM], u[4];
+            if (cur.p >= 0) {
+                int lx, ly, lz;
+                tile_cell<DIM>(cur.key, tall, lx, ly, lz);
+                u[0] = contact_volume<DIM>(cur);
+#pragma unroll
+                for (int a = 0; a < 3; a++) u[1 + a] = a < DIM ? cur.m * cur.u[a < DIM ? a : 0] : 0.;
+                particle_axes<DIM>(gp, P, cur.p, ox + lx, oy + ly, oz + lz, cur.x, f, invd);
+            }
+            for (int r0 = r; r0 < min(r + 64, W.e); r0 += WREC) {
+                if (l / WREC == (r0 - r) / WREC && cur.p >= 0) {
+                    stage_pairs<DIM>(s_F[w], l % WREC, f, invd);
+#pragma unroll
+                    for (int q = 0; q < 4; q++) s_u[w][q][l % WREC] = u[q];
+                }
+                // the next particles' loads pass over the last scatter
+                if (r0 + WREC >= min(r + 64, W.e)) {
+                    load_contact_words<DIM>(P, B, mats, newPositions, ahead, cur);
+                    ahead = W.particle(B, r + 2 * 64 + l);
+                }
+                wave_sync();
+                sc.scatter(W, r0, min(r0 + WREC, W.e));
+                wave_sync();
+            }
+        }
+        claim();
+        sc.finish(W);
+        __syncthreads();
+        write_partials<DIM, NW, NQ_CONTACT>(N, tall, s_acc);
+    };
+    for_each_tile<DIM>(B, tile);
+}
+
+// lCPDI: seven components are two products with the same rows, a particle's corners its records (weights and
+// the gradient weight times Vp)
+template <int DIM>
+__global__ __launch_bounds__(64 * UGIMP_NW, MPM_TILE_SHAPE == 0 ? 2 : 1) void k_p2g_contact_corners(KGrid g0, KPart P, KBins B, KNodes N,
+                                                        const MpmMaterial *mats, int newPositions) {
+    using G = TileGeom<DIM>;
+    constexpr int NW = UGIMP_NW;
+    constexpr int PPR = Corners<DIM>::N, PB = Corners<DIM>::PB;
     __shared__ double s_S[NW][4 * DIM + 8][WROW];
     __shared__ double s_acc[NW][NQ_CONTACT][WaveFoot<DIM, NW>::SIZE];
     const int w = threadIdx.x >> 6, l = threadIdx.x & 63, i = l / PPR, c = l % PPR;
@@ -2945,62 +3099,33 @@ __global__ __launch_bounds__(64 * UGIMP_NW, MPM_TILE_SHAPE == 0 ? 2 : 1) void k_
         tile_origin<DIM>(g, tc - g.tileBase, ox, oy, oz);
         WaveCells<DIM, NW> W;
         W.begin(B.cellStart + (size_t)tall * G::NC);
-        WaveScatter<DIM, NW, NQ_CONTACT, PPR, WROW, CP && DIM == 2> sc;
+        WaveScatter<DIM, NW, NQ_CONTACT, PPR, WROW, DIM == 2> sc;
         sc.begin(&s_S[w][0][0], s_acc);
         ContactWords<DIM> cur;
         int ahead = W.particle(B, W.b + PB + i);       // the order is read a round before the words
         load_contact_words<DIM>(P, B, mats, newPositions, W.particle(B, W.b + i), cur);
         zero_wave_acc<DIM, NW, NQ_CONTACT>(s_acc);
         for (int r = W.b; r < W.e; r += PB) {
-            double xi[3], u[NQ_CONTACT], invd[DIM];
+            double xi[3], u[NQ_CONTACT];
             int off[3];
-            AxisFactors f[DIM];
             if (cur.p >= 0) {
                 int lx, ly, lz;
                 tile_cell<DIM>(cur.key, tall, lx, ly, lz);
-                double Fm[3][3], J;
-                get_F3(cur.ep, cur.wr, Fm);
-                if (DIM == 3)
-                    J = Fm[0][0] * (Fm[1][1] * Fm[2][2] - Fm[2][1] * Fm[1][2])
-                        - Fm[0][1] * (Fm[1][0] * Fm[2][2] - Fm[2][0] * Fm[1][2])
-                        + Fm[0][2] * (Fm[1][0] * Fm[2][1] - Fm[2][0] * Fm[1][1]);
-                else J = Fm[0][0] * Fm[1][1] - Fm[1][0] * Fm[0][1];
-                const double Vp = J * cur.m / cur.rho;
-                if constexpr (CP) {
-                    double s[9], wg[3];
+                const double Vp = contact_volume<DIM>(cur);
+                double s[9], wg[3];
 #pragma unroll
-                    for (int a = 0; a < 9; a++) s[a] = DIM == 3 || (a < 6 && a % 3 < 2) ? P.cpr(a)[cur.p] : 0.;
-                    corner_lane<DIM>(gp, cur.x, s, ox + lx, oy + ly, oz + lz, c, xi, off);
-                    cpdi_wg_staged<DIM>(s, c, wg);
-                    u[0] = Corners<DIM>::WW * Vp;
+                for (int a = 0; a < 9; a++) s[a] = DIM == 3 || (a < 6 && a % 3 < 2) ? P.cpr(a)[cur.p] : 0.;
+                corner_lane<DIM>(gp, cur.x, s, ox + lx, oy + ly, oz + lz, c, xi, off);
+                cpdi_wg_staged<DIM>(s, c, wg);
+                u[0] = Corners<DIM>::WW * Vp;
 #pragma unroll
-                    for (int a = 0; a < 3; a++) {
-                        u[1 + a] = a < DIM ? Corners<DIM>::WW * cur.m * cur.u[a < DIM ? a : 0] : 0.;
-                        u[4 + a] = wg[a] * Vp;
-                    }
-                } else {
-                    particle_axes<DIM>(gp, P, cur.p, ox + lx, oy + ly, oz + lz, cur.x, f, invd);
-                    u[0] = c == 0 ? Vp : 0.;
-#pragma unroll
-                    for (int a = 0; a < 3; a++) {
-                        u[1 + a] = a < DIM && c == 0 ? cur.m * cur.u[a < DIM ? a : 0] : 0.;
-                        u[4 + a] = a < DIM && c == 1 + a ? Vp : 0.;
-                    }
+                for (int a = 0; a < 3; a++) {
+                    u[1 + a] = a < DIM ? Corners<DIM>::WW * cur.m * cur.u[a < DIM ? a : 0] : 0.;
+                    u[4 + a] = wg[a] * Vp;
                 }
             }
             for (int r0 = r; r0 < min(r + PB, W.e); r0 += WREC / PPR) {
-                if (l / WREC == (r0 - r) / (WREC / PPR) && cur.p >= 0) {
-                    if constexpr (CP) stage_corner<DIM, NQ_CONTACT>(s_S[w], l % WREC, xi, off, u);
-                    else {
-#pragma unroll
-                        for (int a = 0; a < DIM; a++)
-#pragma unroll
-                            for (int o = 0; o < 4; o++)
-                                s_S[w][a * 4 + o][l % WREC] = c == 1 + a ? f[a].d4(o) * invd[a] : f[a].s4(o);
-#pragma unroll
-                        for (int q = 0; q < NQ_CONTACT; q++) s_S[w][4 * DIM + q][l % WREC] = u[q];
-                    }
-                }
+                if (l / WREC == (r0 - r) / (WREC / PPR) && cur.p >= 0) stage_corner<DIM, NQ_CONTACT>(s_S[w], l % WREC, xi, off, u);
                 if (r0 + WREC / PPR >= min(r + PB, W.e)) {
                     load_contact_words<DIM>(P, B, mats, newPositions, ahead, cur);
                     ahead = W.particle(B, r + 2 * PB + i);
@@ -4032,11 +4157,11 @@ void launch_p2g_contact(int dim, const KGrid &g, const KPart &p, const KBins &b,
     int np = newPositions ? 1 : 0;
     const bool cp = g.shape == MPMGPU_SHAPE_LCPDI;
     if (dim == 3) {
-        if (cp) TILE_LAUNCH_NT(64 * UGIMP_NW, (k_p2g_contact<3, MPMGPU_SHAPE_LCPDI>), tb, s, g, p, tb, nd, mats, np);
-        else TILE_LAUNCH_NT(64 * UGIMP_NW, (k_p2g_contact<3, MPMGPU_SHAPE_UGIMP>), tb, s, g, p, tb, nd, mats, np);
+        if (cp) TILE_LAUNCH_NT(64 * UGIMP_NW, k_p2g_contact_corners<3>, tb, s, g, p, tb, nd, mats, np);
+        else TILE_LAUNCH_NT(64 * UGIMP_NW, k_p2g_contact<3>, tb, s, g, p, tb, nd, mats, np);
     } else {
-        if (cp) TILE_LAUNCH_NT(64 * UGIMP_NW, (k_p2g_contact<2, MPMGPU_SHAPE_LCPDI>), tb, s, g, p, tb, nd, mats, np);
-        else TILE_LAUNCH_NT(64 * UGIMP_NW, (k_p2g_contact<2, MPMGPU_SHAPE_UGIMP>), tb, s, g, p, tb, nd, mats, np);
+        if (cp) TILE_LAUNCH_NT(64 * UGIMP_NW, k_p2g_contact_corners<2>, tb, s, g, p, tb, nd, mats, np);
+        else TILE_LAUNCH_NT(64 * UGIMP_NW, k_p2g_contact<2>, tb, s, g, p, tb, nd, mats, np);
     }
 }
 
