@@ -408,7 +408,10 @@ int mpmgpu_download_grid(MpmCtx *ctx, double *mass, double *pk, double *ftot);
 int mpmgpu_download_contact(MpmCtx *ctx, double *volume, double *disp, double *grad);
 /* Per-kernel-group HIP event timing on the context's stream (MPMTask::TrackTimes,
    MPMTask.cpp:51-72). Turning it on or off clears the totals; mpmgpu_step then launches
-   eagerly (no graph replay) with an event between kernel groups. */
+   eagerly (no graph replay) with an event between kernel groups. Where a step takes the first
+   strain half step and the internal forces in one kernel (uGIMP and classic without loads), a
+   profiled step takes the two kernels that time MPMGPU_KG_USF and MPMGPU_KG_P2G_FORCE apart: the
+   results are the same bit for bit, the step is a few percent slower. */
 int mpmgpu_set_profiling(MpmCtx *ctx, int32_t on);
 /* totals (ms) and launch counts per MPMGPU_KG_* group since profiling was turned on */
 int mpmgpu_kernel_times(MpmCtx *ctx, double *totalMs, int64_t *launches);

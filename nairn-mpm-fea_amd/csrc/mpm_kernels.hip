@@ -52,7 +52,8 @@ template <int DIM> using TileGeom = TileShape<DIM, MPM_TILE_SHAPE>;
 // rows and footprint copy, so they need 1.5 times the LDS, and with 32 particles a wave (2D) half of its
 // lanes idle. us per launch with 4 and 8 waves: 7.08M uGIMP particles, update 670 and 600, mass 356 and
 // 375, force 540 and 870 (its registers and LDS then leave one block); 87k lCPDI particles, mass 74 and 59,
-// force 73 and 59, update 90 and 70 (16 waves: 60, 56, 69); 1.7M 2D particles, mass 73 and 110.
+// force 73 and 59, update 90 and 70 (16 waves: 60, 56, 69); 1.7M 2D particles, mass 73 and 110. The 3D lCPDI
+// scatters hold four waves per SIMD with 128 registers and 20 (XPIC) to 88 (mass) bytes of scratch a lane.
 // One choice per kernel: the order of a sum must not depend on the number of particles.
 #define WAVES4 (MPM_TILE_SHAPE == 0 ? 3 : 2)
 #define WAVES8 (MPM_TILE_SHAPE == 0 ? 4 : 2)
@@ -1024,9 +1025,9 @@ template <int DIM, int NW> struct WaveFoot {
 // A wave works on its own: it takes its particles 64 at a time (a lane each for the loads and the
 // shape factors), stages their factors in its own LDS rows and scatters its own cells, so no barrier
 // stands between loads, factors and sums and the waves of a CU overlap them. The rows hold WREC
-// records, so that three blocks fit in a CU's LDS. On the 128^3 J2 block the mass scatter went from
-// 0.65 to 0.35 ms per launch, the force scatter from 0.83 to 0.53 and the particle update from 0.92
-// to 0.60; on 87k lCPDI particles from 0.13, 0.18 and 0.18 to 0.059, 0.059 and 0.070.
+// records, so that three blocks fit in a CU's LDS. On the 128^3 J2 block (kernel traces of 205 steps) the
+// mass scatter went from 0.60 to 0.30 ms per launch, the force scatter from 0.76 to 0.45 and the particle
+// update from 0.86 to 0.48; on 202k lCPDI particles from 0.147, 0.196 and 0.245 to 0.116, 0.091 and 0.115.
 typedef double mat4d __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ void lds_add(double *a, double v) {
@@ -2076,7 +2077,9 @@ __global__ __launch_bounds__(64 * UGIMP_NW, FX ? 2 : WAVES4) void k_p2g_force(KG
 // holds two blocks a CU where the two kernels have three, yet steps gain, apart and in one pass: 4k 2D
 // elastic 66 and 63 us, 1.7M 2D 529 and 516, 74k J2 129 and 122.5, 885k neo-Hookean 568 and 542, 7.08M J2
 // 3,341 and 3,254; only tiles that three blocks a CU take in one go and two do not lose (262k J2 with
-// XPIC(2) 253 and 259). Three waves per SIMD hold the 2D laws without volume terms (1.7M: 516, two 530).
+// XPIC(2) 253 and 259; it is taken there too, as the launch does not know how many tiles hold particles).
+// On the 128^3 J2 block it moves 2.7 GB in 0.974 ms, 2.75 TB/s: 249 to 254 registers and 61.6 KB of LDS leave
+// two waves per SIMD. Three waves per SIMD hold the 2D laws without volume terms (1.7M: 516, two 530).
 template <int DIM, int MAT>
 __global__ __launch_bounds__(64 * UGIMP_NW, DIM == 2 && (MAT == MPMGPU_MAT_ISOTROPIC || MAT == MPMGPU_MAT_ISOPLASTICITY) ? 3 : 2)
 void k_usf_force(KGrid g0, KPart P, KBins B, KNodes N, const MpmMaterial *mats, int only) {

@@ -252,7 +252,7 @@ int relayout(MpmServer *s, const std::vector<Request *> &members) {
 }
 
 // Final rows of a finished solve, copied on the device to its result buffer (in layout order;
-// mpmgpu_server_collect puts them in the solve's own order on the host).
+// mpmgpu_server_collect brings them to the host in the solve's own order).
 int keep_result(MpmServer *s, Request *r) {
     MpmCtx *c = s->ctx;
     mpmi::set_positions(c);

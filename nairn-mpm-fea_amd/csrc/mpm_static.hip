@@ -107,10 +107,12 @@ void reorder_particles(const KPart &P, double *pos, double *tmp, const int *at, 
 }
 
 // A solve of this many particles and steps works on its rows in tile order, renewed at the interval, and
-// puts them back in the caller's order at its end; no result depends on the order. ms per solve without
-// and with it: 74k particles, 8 steps 1.37 and 1.45, 16 steps 2.55 and 2.45, 40 steps 6.2 and 5.6; 262k, 8
-// steps 2.24 and 2.14, 16 steps 4.3 and 3.7; 885k, 8 steps 5.6 and 5.1, 40 steps 28.6 and 23.5. Fewer
-// particles leave each launch too short for the order to matter, and two reorderings are 60 launches.
+// puts them back in the caller's order at its end; no result depends on the order. The two orderings are 60
+// launches, 0.25 to 0.3 ms. ms per solve without and with them, rows in random order: 8k particles, 16 steps
+// 2.24 and 2.01, 40 steps 5.4 and 4.4; 64k, 16 steps 3.06 and 2.25, 40 steps 7.5 and 4.8; 885k, 8 steps 5.6
+// and 5.1, 40 steps 28.6 and 23.5. Rows in the grid's order, as a generator leaves them, gain only once the
+// particles have moved: 64k, 16 steps 1.95 and 2.19, 40 steps 4.58 and 4.83; 176k, 16 steps 2.5 and 2.8, 40
+// steps 6.3 and 6.0. The line keeps small solves in either order from paying for it.
 constexpr long long STATIC_SORT_PARTICLES = 1 << 16;
 constexpr int STATIC_SORT_STEPS = 16, STATIC_SORT_INTERVAL = 50;
 
