@@ -108,11 +108,11 @@ void reorder_particles(const KPart &P, double *pos, double *tmp, const int *at, 
 
 // A solve of this many particles and steps works on its rows in tile order, renewed at the interval, and
 // puts them back in the caller's order at its end; no result depends on the order. The two orderings are 60
-// launches, 0.25 to 0.3 ms. ms per solve without and with them, rows in random order: 8k particles, 16 steps
-// 2.24 and 2.01, 40 steps 5.4 and 4.4; 64k, 16 steps 3.06 and 2.25, 40 steps 7.5 and 4.8; 885k, 8 steps 5.6
-// and 5.1, 40 steps 28.6 and 23.5. Rows in the grid's order, as a generator leaves them, gain only once the
-// particles have moved: 64k, 16 steps 1.95 and 2.19, 40 steps 4.58 and 4.83; 176k, 16 steps 2.5 and 2.8, 40
-// steps 6.3 and 6.0. The line keeps small solves in either order from paying for it.
+// launches, 0.2 to 0.3 ms. ms per solve without and with them, rows in random order: 8k particles, 16 steps
+// 2.24 and 2.01, 40 steps 5.4 and 4.4; 64k, 16 steps 3.06 and 2.25, 40 steps 7.5 and 4.8; 176k, 16 steps 6.1
+// and 2.8, 40 steps 15.6 and 6.1. Rows still in the grid's order, as a generator leaves them, only pay for it:
+// 64k, 16 steps 1.95 and 2.19, 40 steps 4.6 and 4.8; 176k, 16 steps 2.46 and 2.67, 40 steps 5.87 and 5.94. The
+// line keeps small and short solves, of which that is a tenth or more, from it.
 constexpr long long STATIC_SORT_PARTICLES = 1 << 16;
 constexpr int STATIC_SORT_STEPS = 16, STATIC_SORT_INTERVAL = 50;
 
